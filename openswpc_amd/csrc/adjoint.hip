@@ -833,14 +833,12 @@ extern "C" int swpc_adj_accumulate(swpc_ctx *c, int nt, const float *obs, int ck
     };
     // one forward step n (time step it = n + 1), the order of main.f90:119-139
     auto stress_phase = [&](int it) -> hipError_t {
-        hipError_t e = launch_stress_side(c, nullptr);
-        if (e == hipSuccess) e = launch_stress_cols(c, 3);
+        hipError_t e = launch_stress(c, true, 3);
         if (e == hipSuccess) e = launch_stressglut(c, it, nullptr);
         return e;
     };
     auto vel_phase = [&](int it) -> hipError_t {
-        hipError_t e = launch_vel_side(c, nullptr);
-        if (e == hipSuccess) e = launch_vel_cols(c, 3);
+        hipError_t e = launch_vel(c, true, 3);
         if (e == hipSuccess) e = launch_bodyforce(c, it, nullptr);
         return e;
     };

@@ -127,13 +127,13 @@ static int build_pml_tiles(swpc_ctx *c)
     const bool slab_tiles = na > 0 && na <= 64 && slab_rows > 0;
     for (int k0 = 1; k0 <= nz; k0 += kc) {
         const int k1 = std::min(nz, k0 + kc - 1);
-        // y-slab rows as full-row tiles over the full depth; the bottom band
-        // of interior columns is marched by the interior kernels
-        for (int j0 = 1; j0 <= ny; j0 += by) {
-            const int jl = std::min(j0 + by - 1, ny);
-            if (j0 <= na || jl > ny - na)
-                for (int i0 = 1; i0 <= nx; i0 += 64) add(i0, 64, 0, j0, k0, k1);
-        }
+        // y-slab rows as full-row tiles over the full depth, each within its
+        // slab; the bottom band of interior columns is marched by the interior
+        // kernels
+        for (int j0 = 1; j0 <= na; j0 += by)
+            for (int i0 = 1; i0 <= nx; i0 += 64) add(i0, 64, 0, j0, k0, k1);
+        for (int j0 = ny - na + 1; j0 <= ny; j0 += by)
+            for (int i0 = 1; i0 <= nx; i0 += 64) add(i0, 64, 0, j0, k0, k1);
         if (slab_tiles)
             for (int j0 = na + 1; j0 <= ny - na; j0 += slab_rows) {
                 add(1, na, 1, j0, k0, k1);
@@ -397,7 +397,6 @@ extern "C" int swpc_create(const swpc_desc *d, swpc_ctx **out)
     if (hipStreamSynchronize(c->stream) != hipSuccess) { rc = SWPC_EHIP; goto bad; }
     if ((rc = build_pml_tiles(c)) != SWPC_OK) goto bad;
     if ((rc = build_zchunks(c)) != SWPC_OK) goto bad;
-    if ((rc = build_schedule(c)) != SWPC_OK) goto bad;
     *out = c;
     return SWPC_OK;
 bad:
@@ -435,7 +434,6 @@ extern "C" int swpc_destroy(swpc_ctx *c)
     dfree(c->rho); dfree(c->lam); dfree(c->mu); dfree(c->taup); dfree(c->taus);
     dfree(c->kfs_top); dfree(c->kfs_bot); dfree(c->kob_top); dfree(c->kob_bot); dfree(c->kob);
     dfree(c->R); dfree(c->ade); dfree(c->d_pml_tiles); dfree(c->d_zchunks);
-    dfree(c->d_sched[0]); dfree(c->d_sched[1]);
     dfree(c->gxc); dfree(c->gxe); dfree(c->gyc); dfree(c->gye); dfree(c->gzc); dfree(c->gze);
     dfree(c->cgx_c); dfree(c->cgx_b); dfree(c->cgy_c); dfree(c->cgy_b); dfree(c->cgz_c); dfree(c->cgz_b);
     dfree(c->d_targets); dfree(c->d_contrib); dfree(c->d_comp); dfree(c->d_mo); dfree(c->d_stf);
@@ -936,7 +934,7 @@ extern "C" int swpc_kernel_update_stress(swpc_ctx *c)
     if (!c) return SWPC_EINVAL;
     int rc = ready(c);
     if (rc) return rc;
-    HIPCHK(c, launch_kernel_stress(c));
+    HIPCHK(c, launch_stress(c, false, 1));
     return SWPC_OK;
 }
 
@@ -945,7 +943,7 @@ extern "C" int swpc_absorb_update_stress(swpc_ctx *c)
     if (!c) return SWPC_EINVAL;
     int rc = ready(c);
     if (rc) return rc;
-    if (c->desc.abc == SWPC_ABC_PML) HIPCHK(c, launch_pml_stress(c));
+    if (c->desc.abc == SWPC_ABC_PML) HIPCHK(c, launch_stress(c, true, 2));
     else HIPCHK(c, launch_cerjan_stress(c));
     return SWPC_OK;
 }
@@ -955,7 +953,7 @@ extern "C" int swpc_kernel_update_vel(swpc_ctx *c)
     if (!c) return SWPC_EINVAL;
     int rc = ready(c);
     if (rc) return rc;
-    HIPCHK(c, launch_kernel_vel(c));
+    HIPCHK(c, launch_vel(c, false, 1));
     return SWPC_OK;
 }
 
@@ -964,7 +962,7 @@ extern "C" int swpc_absorb_update_vel(swpc_ctx *c)
     if (!c) return SWPC_EINVAL;
     int rc = ready(c);
     if (rc) return rc;
-    if (c->desc.abc == SWPC_ABC_PML) HIPCHK(c, launch_pml_vel(c));
+    if (c->desc.abc == SWPC_ABC_PML) HIPCHK(c, launch_vel(c, true, 2));
     else HIPCHK(c, launch_cerjan_vel(c));
     return SWPC_OK;
 }
@@ -975,9 +973,9 @@ extern "C" int swpc_update_stress(swpc_ctx *c)
     int rc = ready(c);
     if (rc) return rc;
     if (c->desc.abc == SWPC_ABC_PML) {
-        HIPCHK(c, launch_stress(c, 3, nullptr));
+        HIPCHK(c, launch_stress(c, true, 3));
     } else {
-        HIPCHK(c, launch_stress(c, 1, nullptr));
+        HIPCHK(c, launch_stress(c, false, 1));
         HIPCHK(c, launch_cerjan_stress(c));
     }
     return SWPC_OK;
@@ -989,9 +987,9 @@ extern "C" int swpc_update_vel(swpc_ctx *c)
     int rc = ready(c);
     if (rc) return rc;
     if (c->desc.abc == SWPC_ABC_PML) {
-        HIPCHK(c, launch_vel(c, 3, nullptr));
+        HIPCHK(c, launch_vel(c, true, 3));
     } else {
-        HIPCHK(c, launch_vel(c, 1, nullptr));
+        HIPCHK(c, launch_vel(c, false, 1));
         HIPCHK(c, launch_cerjan_vel(c));
     }
     return SWPC_OK;
@@ -1049,28 +1047,20 @@ static hipError_t enqueue_step(swpc_ctx *c, int it, const int *d_it, hipEvent_t 
     if ((e = launch_green_store(c, it, d_it)) != hipSuccess) return e;
     if ((e = launch_wav_store(c, it, d_it)) != hipSuccess || (e = mark()) != hipSuccess) return e;
     if ((e = launch_snap(c, it, d_it)) != hipSuccess || (e = mark()) != hipSuccess) return e;
-    const bool merged = pml && merged_launch_ready(c);
+    const bool merged = (c->variant & 32) && !fork;
     if ((e = fork_to_side()) != hipSuccess) return e;
-    if (pml && !merged && (e = launch_stress_side(c, side)) != hipSuccess) return e;
+    if (pml && !merged && (e = launch_stress(c, true, 0, side)) != hipSuccess) return e;
     if ((e = mark()) != hipSuccess) return e;
-    if (merged) {
-        if ((e = launch_stress_all(c)) != hipSuccess) return e;
-    } else if ((e = launch_stress_cols(c, pml ? 3 : 1)) != hipSuccess) {
-        return e;
-    }
+    if ((e = launch_stress(c, pml && merged, pml ? 3 : 1)) != hipSuccess) return e;
     if ((e = join_side()) != hipSuccess) return e;
     if ((e = mark()) != hipSuccess) return e;
     if (!pml && (e = launch_cerjan_stress(c)) != hipSuccess) return e;
     if ((e = mark()) != hipSuccess) return e;
     if ((e = launch_stressglut(c, it, d_it)) != hipSuccess || (e = mark()) != hipSuccess) return e;
     if ((e = fork_to_side()) != hipSuccess) return e;
-    if (pml && !merged && (e = launch_vel_side(c, side)) != hipSuccess) return e;
+    if (pml && !merged && (e = launch_vel(c, true, 0, side)) != hipSuccess) return e;
     if ((e = mark()) != hipSuccess) return e;
-    if (merged) {
-        if ((e = launch_vel_all(c)) != hipSuccess) return e;
-    } else if ((e = launch_vel_cols(c, pml ? 3 : 1)) != hipSuccess) {
-        return e;
-    }
+    if ((e = launch_vel(c, pml && merged, pml ? 3 : 1)) != hipSuccess) return e;
     if ((e = join_side()) != hipSuccess) return e;
     if ((e = mark()) != hipSuccess) return e;
     if (!pml && (e = launch_cerjan_vel(c)) != hipSuccess) return e;
@@ -1115,7 +1105,7 @@ static hipError_t enqueue_fused_steps(swpc_ctx *c, int it, int n, const int *d_i
     // step it up to its stress glut, as in enqueue_step
     if ((e = launch_green_store(c, step_no(0), d_it)) != hipSuccess ||
         (e = launch_wav_store(c, step_no(0), d_it)) != hipSuccess || (e = launch_snap(c, step_no(0), d_it)) != hipSuccess ||
-        (e = launch_stress_side(c, nullptr)) != hipSuccess || (e = launch_stress_cols(c, 3)) != hipSuccess ||
+        (e = launch_stress(c, true, 0)) != hipSuccess || (e = launch_stress(c, false, 3)) != hipSuccess ||
         (e = launch_stressglut(c, step_no(0), d_it)) != hipSuccess)
         return e;
     const int nf = (n - 1) & ~1;
@@ -1124,12 +1114,12 @@ static hipError_t enqueue_fused_steps(swpc_ctx *c, int it, int n, const int *d_i
         float *const *nxt = (s & 1) ? A : B;
         // step it+s: velocities of the side columns and the bottom band (2: band only)
         view(nxt, cur, cur);
-        if ((e = launch_vel_side(c, nullptr)) != hipSuccess || (e = launch_vel_cols(c, 2)) != hipSuccess) break;
+        if ((e = launch_vel(c, true, 0)) != hipSuccess || (e = launch_vel(c, false, 2)) != hipSuccess) break;
         // interior: velocities of step it+s and stresses of step it+s+1
         view(nxt, nxt, cur);
         if ((e = launch_fused(c)) != hipSuccess) break;
         // step it+s+1: stresses of the side columns and the bottom band
-        if ((e = launch_stress_side(c, nullptr)) != hipSuccess || (e = launch_stress_cols(c, 2)) != hipSuccess) break;
+        if ((e = launch_stress(c, true, 0)) != hipSuccess || (e = launch_stress(c, false, 2)) != hipSuccess) break;
         if (d_it && (e = launch_step_advance(c)) != hipSuccess) break;
         view(nxt, cur, nullptr);
         if ((e = launch_wav_store(c, step_no(s + 1), d_it)) != hipSuccess ||
@@ -1141,7 +1131,7 @@ static hipError_t enqueue_fused_steps(swpc_ctx *c, int it, int n, const int *d_i
     view(A, A, nullptr);
     if (e != hipSuccess) return e;
     // step it+nf from its velocity update on, in place
-    if ((e = launch_vel_side(c, nullptr)) != hipSuccess || (e = launch_vel_cols(c, 3)) != hipSuccess ||
+    if ((e = launch_vel(c, true, 0)) != hipSuccess || (e = launch_vel(c, false, 3)) != hipSuccess ||
         (e = launch_bodyforce(c, step_no(nf), d_it)) != hipSuccess ||
         (e = launch_green_source(c, step_no(nf), d_it)) != hipSuccess || (d_it && (e = launch_step_advance(c)) != hipSuccess))
         return e;
@@ -1333,6 +1323,5 @@ extern "C" int swpc_set_tuning(swpc_ctx *c, int kchunk, int by, int variant)
     HIPCHK(c, hipStreamSynchronize(c->stream));
     int rc = build_pml_tiles(c);
     if (rc == SWPC_OK) rc = build_zchunks(c);
-    if (rc == SWPC_OK && (rc = build_schedule(c)) != SWPC_OK) rc = fail(c, rc, "swpc_set_tuning: launch schedule");
     return rc;
 }

@@ -6,21 +6,27 @@
 // first cell sits on a 128-byte line, and marches a chunk of planes along z,
 // keeping the z-neighbours of its column in a rotating register queue while
 // the x/y neighbours come from the plane the tile is streaming (L1/L2
-// resident).  Loop bodies are branch free so every load of an iteration is
-// issued at once.  Every arithmetic expression keeps the reference's FP32
+// resident).  Loop bodies are branch free and load everything before they
+// store, so every load of an iteration is in flight at once: with each stress
+// component loaded between the stores of its neighbours a wave made six
+// memory round trips per cell (elastic 256 x 256 x 192, 20-cell PML: stress
+// launch 262 us, 195 us with the loads first).  Every arithmetic expression keeps the reference's FP32
 // evaluation order; the library is compiled with -ffp-contract=off so no FMA
 // changes the rounding.
 //
 // Cerjan tapers (m_absorb_c) are separate per-cell sweeps, as in the
 // reference.
-#include <vector>
-
 #include "swpc_internal.h"
 
 #define BX 64
 #define MASK_INT 1
 #define MASK_PML 2
 
+
+// Four waves per SIMD: 128 registers, which every NM <= 4 form fits without a
+// spill; asking for no more lets the scheduler keep a cell's loads together.
+#define WAVES4 __attribute__((amdgpu_waves_per_eu(4, 4)))
+#define WAVES_NM __attribute__((amdgpu_waves_per_eu(NM <= 4 ? 4 : 3, NM <= 4 ? 4 : 3)))
 
 // isign of m_kernel.f90:103-104: true inside the 2nd-order band
 __device__ static inline bool in_band(int k, int kft, int kfb, int kot, int kob)
@@ -41,18 +47,77 @@ __device__ static inline float hmean4(float a, float b, float c, float d, float 
 typedef float f4v __attribute__((ext_vector_type(4)));
 typedef float f2v __attribute__((ext_vector_type(2)));
 
+// Loads and stores through explicit global pointers: a batch launch reads its
+// arrays' addresses from memory, where the compiler only knows generic ones
+// and would make every access a flat one, which waits for all others.  NT:
+// streams read or written once per step (memory variables, stress, the
+// per-cell medium) bypass cache retention so the L2 keeps the V and mu rows
+// that neighbouring tiles re-read.
+template <typename T>
+using GlobalPtr = __attribute__((address_space(1))) T *;
+
 template <bool NT, typename T>
 __device__ static inline T ldv(const T *p)
 {
-    if constexpr (NT) return __builtin_nontemporal_load(p);
-    else return *p;
+    const GlobalPtr<const T> q = (GlobalPtr<const T>)p;
+    if constexpr (NT) return __builtin_nontemporal_load(q);
+    else return *q;
 }
 template <bool NT, typename T>
 __device__ static inline void stv(T *p, T v)
 {
-    if constexpr (NT) __builtin_nontemporal_store(v, p);
-    else *p = v;
+    const GlobalPtr<T> q = (GlobalPtr<T>)p;
+    if constexpr (NT) __builtin_nontemporal_store(v, q);
+    else *q = v;
 }
+// one cell's PML profile
+__device__ static inline float4 ldp(const float4 *p)
+{
+    const f4v v = ldv<false>((const f4v *)p);
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+
+// Where a lane reads: u is the element offset all lanes of the block share
+// (plane and tile origin, kept in scalar registers), o the lane's byte offset
+// from there and y the bytes of a row.  F + u is a scalar pointer and o a
+// 32-bit register, so an access is one instruction with the x neighbour as
+// its immediate offset; y neighbours add rows to o and z neighbours planes to
+// u.  No array costs 64-bit vector arithmetic or a register pair of its own:
+// the NM = 3 stress update fell from 201 registers to 106 and four waves per
+// SIMD instead of two (1024 x 1024 x 512 class grids: 9.22 -> 8.83 ms per
+// 264 M cells; 128^3: 58 -> 50 us).
+struct Loc {
+    long long u;
+    unsigned o, y;
+};
+// F d elements (the same for every lane), dx cells and dy rows from the lane's
+// place; u starts two rows before the tile so that o stays positive
+template <bool NT = false>
+__device__ __forceinline__ float ld(const float *F, const Loc &l, long long d = 0, int dx = 0, int dy = 0)
+{
+    return ldv<NT>((const float *)((const char *)(F + (l.u + d)) + (l.o + (unsigned)dy * l.y)) + dx);
+}
+template <bool NT>
+__device__ __forceinline__ void st(float *F, const Loc &l, float v, long long d = 0)
+{
+    stv<NT>((float *)((char *)(F + (l.u + d)) + l.o), v);
+}
+// The compiler selects the scalar-pointer form only where it sees the 32-bit
+// offset being widened; hoisted out of the loop, the widened offset costs a
+// 64-bit vector add per access.  An offset that looks new in every iteration
+// is widened at its uses.
+__device__ __forceinline__ void fresh(Loc &l) { asm("" : "+v"(l.o)); }
+
+// the place of cell (i0 + col, j0 + row) on plane k, (i0, j0, k) the same for
+// every lane of the block
+__device__ __forceinline__ Loc field_loc(const Grid &g, int i0, int j0, int k, int col, int row)
+{
+    return Loc{gidx(g, i0, j0 - 2, k), 4u * (unsigned)((row + 2) * g.pitch + col), 4u * (unsigned)g.pitch};
+}
+
+// a value that every lane of the block holds, in a scalar register
+__device__ static inline int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ static inline int4 uni(int4 v) { return make_int4(uni(v.x), uni(v.y), uni(v.z), uni(v.w)); }
 
 // The 6*NM memory variables of one cell, value v = c*NM + m for component
 // c = xx yy zz yz xz xy and mechanism m, packed as 16-byte vectors: value v
@@ -66,50 +131,34 @@ struct RCell {
     float v[NV > 0 ? NV : 1];
 
     template <bool NT>
-    __device__ __forceinline__ void load(const float *R, long long rn, long long r)
+    __device__ __forceinline__ void load(const float *R, long long rn, const Loc &r)
     {
 #pragma unroll
         for (int s = 0; s < N4; ++s) {
-            const f4v t = ldv<NT>((const f4v *)R + s * rn + r);
+            const f4v t = ldv<NT>((const f4v *)((const char *)((const f4v *)R + (s * rn + r.u)) + 4 * r.o));
             v[4 * s] = t.x; v[4 * s + 1] = t.y; v[4 * s + 2] = t.z; v[4 * s + 3] = t.w;
         }
         if constexpr (N2 == 1) {
-            const f2v t = ldv<NT>((const f2v *)(R + 4 * N4 * rn) + r);
+            const f2v t = ldv<NT>((const f2v *)((const char *)((const f2v *)(R + 4 * N4 * rn) + r.u) + 2 * r.o));
             v[4 * N4] = t.x; v[4 * N4 + 1] = t.y;
         }
     }
     template <bool NT>
-    __device__ __forceinline__ void store(float *R, long long rn, long long r) const
+    __device__ __forceinline__ void store(float *R, long long rn, const Loc &r) const
     {
 #pragma unroll
         for (int s = 0; s < N4; ++s) {
             f4v t;
             t.x = v[4 * s]; t.y = v[4 * s + 1]; t.z = v[4 * s + 2]; t.w = v[4 * s + 3];
-            stv<NT>((f4v *)R + s * rn + r, t);
+            stv<NT>((f4v *)((char *)((f4v *)R + (s * rn + r.u)) + 4 * r.o), t);
         }
         if constexpr (N2 == 1) {
             f2v t;
             t.x = v[4 * N4]; t.y = v[4 * N4 + 1];
-            stv<NT>((f2v *)(R + 4 * N4 * rn) + r, t);
+            stv<NT>((f2v *)((char *)((f2v *)(R + 4 * N4 * rn) + r.u) + 2 * r.o), t);
         }
     }
 };
-
-// Streams read or written once per step (memory variables, stress, the
-// per-cell medium) can bypass cache retention so the L2 keeps the V and mu
-// rows that neighbouring tiles re-read.
-template <bool NT>
-__device__ static inline float ld1(const float *p)
-{
-    if constexpr (NT) return __builtin_nontemporal_load(p);
-    else return *p;
-}
-template <bool NT>
-__device__ static inline void st1(float *p, float v)
-{
-    if constexpr (NT) __builtin_nontemporal_store(v, p);
-    else *p = v;
-}
 
 struct StepArgs {
     Grid g;
@@ -131,11 +180,32 @@ struct StepArgs {
     float r20x, r20y, r20z;
     const int4 *tiles;   // side-column PML tiles: (i0 | width << 20, j0, k0, k1)
     int ntiles;
+    int sideb;           // blocks of a launch that walk the side tiles (a multiple of 8, >= ntiles; 0: none)
     int has_pml, mask;
     // interior launch shape
     const int *zc;       // first plane of each k chunk (nbz + 1 entries, last = nz + 1)
     int bx0, nbx, nby, nbz, by;
     int bxw, byi;        // interior tiles: bxw (64 or 32) cells wide, byi rows (bxw * byi = 64 * by threads)
+};
+
+// The 4th-order coefficients of a cell (near and far per axis) by its band
+// state.  Both states are held in vector registers across the march: left in
+// the arguments, the selects become loads at a per-lane address or, short of
+// scalar registers, lane reads of spilled ones.
+struct Coefs {
+    float v[2][6];
+
+    __device__ explicit Coefs(const StepArgs &a)
+    {
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            v[b][0] = a.c.re40x[b]; v[b][1] = a.c.re41x[b]; v[b][2] = a.c.re40y[b];
+            v[b][3] = a.c.re41y[b]; v[b][4] = a.c.re40z[b]; v[b][5] = a.c.re41z[b];
+#pragma unroll
+            for (int q = 0; q < 6; ++q) asm("" : "+v"(v[b][q]));
+        }
+    }
+    __device__ float at(bool in, int q) const { return in ? v[1][q] : v[0][q]; }
 };
 
 // ---------------------------------------------------------------------------
@@ -151,7 +221,7 @@ __device__ static inline PmlBox pick_box(const StepArgs &a, int q)
 // passes its z-queue values: V at k (and k+1 for Vx, Vy; k-1 for Vz) and mu
 // on planes k, k+1.
 template <bool NT, bool OOP>
-__device__ __forceinline__ void pml_stress_cell(const StepArgs &a, long long p, long long q, int k, float vx_0,
+__device__ __forceinline__ void pml_stress_cell(const StepArgs &a, const Loc &p, const Loc &q, int k, float vx_0,
                                                 float vx_p1, float vy_0, float vy_p1, float vz_m1, float vz_0,
                                                 float mu00, float mu00n, float mu10, float mu10n, float mu01,
                                                 float mu01n, float mu11, float4 gxc, float4 gxe, float4 gyc,
@@ -163,19 +233,19 @@ __device__ __forceinline__ void pml_stress_cell(const StepArgs &a, long long p, 
     const float *__restrict__ Vy = a.f.Vy;
     const float *__restrict__ Vz = a.f.Vz;
     const long long n = a.npml;
-    float *__restrict__ A = a.ade + q;
-    const float *__restrict__ AI = OOP ? a.ade_in + q : A;
+    float *__restrict__ A = a.ade;
+    const float *__restrict__ AI = OOP ? a.ade_in : A;
     const float dt = a.dt;
     (void)P;
-    const float vx_im1 = Vx[p - 1], vy_jm1 = Vy[p - Y];
-    const float vy_ip1 = Vy[p + 1], vz_ip1 = Vz[p + 1];
-    const float vx_jp1 = Vx[p + Y], vz_jp1 = Vz[p + Y];
-    const float4 gzc = a.gzc[k - 1], gze = a.gze[k - 1];
-    const float lam0 = ld1<NT>(a.m.lam + p);
-    const float axVx = ld1<NT>(AI + A_axVx * n), ayVy = ld1<NT>(AI + A_ayVy * n), azVz = ld1<NT>(AI + A_azVz * n);
-    const float ayVx = ld1<NT>(AI + A_ayVx * n), azVx = ld1<NT>(AI + A_azVx * n);
-    const float axVy = ld1<NT>(AI + A_axVy * n), azVy = ld1<NT>(AI + A_azVy * n);
-    const float axVz = ld1<NT>(AI + A_axVz * n), ayVz = ld1<NT>(AI + A_ayVz * n);
+    const float vx_im1 = ld(Vx, p, 0, -1), vy_jm1 = ld(Vy, p, 0, 0, -1);
+    const float vy_ip1 = ld(Vy, p, 0, 1), vz_ip1 = ld(Vz, p, 0, 1);
+    const float vx_jp1 = ld(Vx, p, 0, 0, 1), vz_jp1 = ld(Vz, p, 0, 0, 1);
+    const float4 gzc = ldp(a.gzc + (k - 1)), gze = ldp(a.gze + (k - 1));
+    const float lam0 = ld<NT>(a.m.lam, p);
+    const float axVx = ld<NT>(AI, q, A_axVx * n), ayVy = ld<NT>(AI, q, A_ayVy * n), azVz = ld<NT>(AI, q, A_azVz * n);
+    const float ayVx = ld<NT>(AI, q, A_ayVx * n), azVx = ld<NT>(AI, q, A_azVx * n);
+    const float axVy = ld<NT>(AI, q, A_axVy * n), azVy = ld<NT>(AI, q, A_azVy * n);
+    const float axVz = ld<NT>(AI, q, A_axVz * n), ayVz = ld<NT>(AI, q, A_ayVz * n);
     float *__restrict__ Sxx = a.f.Sxx;
     float *__restrict__ Syy = a.f.Syy;
     float *__restrict__ Szz = a.f.Szz;
@@ -188,6 +258,9 @@ __device__ __forceinline__ void pml_stress_cell(const StepArgs &a, long long p, 
     const float *__restrict__ SyzI = OOP ? a.fin.Syz : Syz;
     const float *__restrict__ SxzI = OOP ? a.fin.Sxz : Sxz;
     const float *__restrict__ SxyI = OOP ? a.fin.Sxy : Sxy;
+    // every load before the first store (see stress_cell)
+    const float sxx = ld<NT>(SxxI, p), syy = ld<NT>(SyyI, p), szz = ld<NT>(SzzI, p);
+    const float syz = ld<NT>(SyzI, p), sxz = ld<NT>(SxzI, p), sxy = ld<NT>(SxyI, p);
 
     // normal components
     const float dxVx = (vx_0 - vx_im1) * a.r20x;
@@ -198,12 +271,12 @@ __device__ __forceinline__ void pml_stress_cell(const StepArgs &a, long long p, 
     const float dxVx_ade = gxc.x * dxVx + gxc.y * axVx;
     const float dyVy_ade = gyc.x * dyVy + gyc.y * ayVy;
     const float dzVz_ade = gzc.x * dzVz + gzc.y * azVz;
-    st1<NT>(Sxx + p, ld1<NT>(SxxI + p) + (lam2mu_R * dxVx_ade + lam_R * (dyVy_ade + dzVz_ade)) * dt);
-    st1<NT>(Syy + p, ld1<NT>(SyyI + p) + (lam2mu_R * dyVy_ade + lam_R * (dxVx_ade + dzVz_ade)) * dt);
-    st1<NT>(Szz + p, ld1<NT>(SzzI + p) + (lam2mu_R * dzVz_ade + lam_R * (dxVx_ade + dyVy_ade)) * dt);
-    st1<NT>(A + A_axVx * n, gxc.z * axVx + gxc.w * dxVx * dt);
-    st1<NT>(A + A_ayVy * n, gyc.z * ayVy + gyc.w * dyVy * dt);
-    st1<NT>(A + A_azVz * n, gzc.z * azVz + gzc.w * dzVz * dt);
+    st<NT>(Sxx, p, sxx + (lam2mu_R * dxVx_ade + lam_R * (dyVy_ade + dzVz_ade)) * dt);
+    st<NT>(Syy, p, syy + (lam2mu_R * dyVy_ade + lam_R * (dxVx_ade + dzVz_ade)) * dt);
+    st<NT>(Szz, p, szz + (lam2mu_R * dzVz_ade + lam_R * (dxVx_ade + dyVy_ade)) * dt);
+    st<NT>(A, q, gxc.z * axVx + gxc.w * dxVx * dt, A_axVx * n);
+    st<NT>(A, q, gyc.z * ayVy + gyc.w * dyVy * dt, A_ayVy * n);
+    st<NT>(A, q, gzc.z * azVz + gzc.w * dzVz * dt, A_azVz * n);
 
     // shear components
     const float dxVy = (vy_ip1 - vy_0) * a.r20x;
@@ -215,21 +288,21 @@ __device__ __forceinline__ void pml_stress_cell(const StepArgs &a, long long p, 
     const float muxz = hmean4(mu00, mu00n, mu10, mu10n, EPSL);
     const float muxy = hmean4(mu00, mu10, mu01, mu11, EPSL);
     const float muyz = hmean4(mu00, mu00n, mu01, mu01n, EPSL);
-    st1<NT>(Syz + p, ld1<NT>(SyzI + p) + muyz * (gye.x * dyVz + gze.x * dzVy + gye.y * ayVz + gze.y * azVy) * dt);
-    st1<NT>(Sxz + p, ld1<NT>(SxzI + p) + muxz * (gxe.x * dxVz + gze.x * dzVx + gxe.y * axVz + gze.y * azVx) * dt);
-    st1<NT>(Sxy + p, ld1<NT>(SxyI + p) + muxy * (gxe.x * dxVy + gye.x * dyVx + gxe.y * axVy + gye.y * ayVx) * dt);
-    st1<NT>(A + A_ayVx * n, gye.z * ayVx + gye.w * dyVx * dt);
-    st1<NT>(A + A_azVx * n, gze.z * azVx + gze.w * dzVx * dt);
-    st1<NT>(A + A_axVy * n, gxe.z * axVy + gxe.w * dxVy * dt);
-    st1<NT>(A + A_azVy * n, gze.z * azVy + gze.w * dzVy * dt);
-    st1<NT>(A + A_axVz * n, gxe.z * axVz + gxe.w * dxVz * dt);
-    st1<NT>(A + A_ayVz * n, gye.z * ayVz + gye.w * dyVz * dt);
+    st<NT>(Syz, p, syz + muyz * (gye.x * dyVz + gze.x * dzVy + gye.y * ayVz + gze.y * azVy) * dt);
+    st<NT>(Sxz, p, sxz + muxz * (gxe.x * dxVz + gze.x * dzVx + gxe.y * axVz + gze.y * azVx) * dt);
+    st<NT>(Sxy, p, sxy + muxy * (gxe.x * dxVy + gye.x * dyVx + gxe.y * axVy + gye.y * ayVx) * dt);
+    st<NT>(A, q, gye.z * ayVx + gye.w * dyVx * dt, A_ayVx * n);
+    st<NT>(A, q, gze.z * azVx + gze.w * dzVx * dt, A_azVx * n);
+    st<NT>(A, q, gxe.z * axVy + gxe.w * dxVy * dt, A_axVy * n);
+    st<NT>(A, q, gze.z * azVy + gze.w * dzVy * dt, A_azVy * n);
+    st<NT>(A, q, gxe.z * axVz + gxe.w * dxVz * dt, A_axVz * n);
+    st<NT>(A, q, gye.z * ayVz + gye.w * dyVz * dt, A_ayVz * n);
 }
 
 // absorb_p__update_vel for one cell, m_absorb_p.f90:267-304.  Queue values:
 // Szz on k, k+1; Syz, Sxz on k-1, k; rho on k, k+1.
 template <bool OOP>
-__device__ __forceinline__ void pml_vel_cell(const StepArgs &a, long long p, long long q, int k, float szz_0,
+__device__ __forceinline__ void pml_vel_cell(const StepArgs &a, const Loc &p, const Loc &q, int k, float szz_0,
                                              float szz_p1, float syz_m1, float syz_0, float sxz_m1, float sxz_0,
                                              float rho0, float rho_kp, float4 gxc, float4 gxe, float4 gyc,
                                              float4 gye)
@@ -242,18 +315,23 @@ __device__ __forceinline__ void pml_vel_cell(const StepArgs &a, long long p, lon
     const float *__restrict__ Sxy = a.f.Sxy;
     const float *__restrict__ rho = a.m.rho;
     const long long n = a.npml;
-    float *__restrict__ A = a.ade + q;
-    const float *__restrict__ AI = OOP ? a.ade_in + q : A;
+    float *__restrict__ A = a.ade;
+    const float *__restrict__ AI = OOP ? a.ade_in : A;
     const float dt = a.dt;
-    const float sxx_0 = Sxx[p], sxx_ip1 = Sxx[p + 1];
-    const float syy_0 = Syy[p], syy_jp1 = Syy[p + Y];
-    const float syz_jm1 = Syz[p - Y], sxz_im1 = Sxz[p - 1];
-    const float sxy_0 = Sxy[p], sxy_im1 = Sxy[p - 1], sxy_jm1 = Sxy[p - Y];
-    const float rho_ip = rho[p + 1], rho_jp = rho[p + Y];
-    const float4 gzc = a.gzc[k - 1], gze = a.gze[k - 1];
-    const float axSxx = ld1<true>(AI + A_axSxx * n), aySxy = ld1<true>(AI + A_aySxy * n), azSxz = ld1<true>(AI + A_azSxz * n);
-    const float axSxy = ld1<true>(AI + A_axSxy * n), aySyy = ld1<true>(AI + A_aySyy * n), azSyz = ld1<true>(AI + A_azSyz * n);
-    const float axSxz = ld1<true>(AI + A_axSxz * n), aySyz = ld1<true>(AI + A_aySyz * n), azSzz = ld1<true>(AI + A_azSzz * n);
+    const float sxx_0 = ld(Sxx, p), sxx_ip1 = ld(Sxx, p, 0, 1);
+    const float syy_0 = ld(Syy, p), syy_jp1 = ld(Syy, p, 0, 0, 1);
+    const float syz_jm1 = ld(Syz, p, 0, 0, -1), sxz_im1 = ld(Sxz, p, 0, -1);
+    const float sxy_0 = ld(Sxy, p), sxy_im1 = ld(Sxy, p, 0, -1), sxy_jm1 = ld(Sxy, p, 0, 0, -1);
+    const float rho_ip = ld(rho, p, 0, 1), rho_jp = ld(rho, p, 0, 0, 1);
+    const float4 gzc = ldp(a.gzc + (k - 1)), gze = ldp(a.gze + (k - 1));
+    const float axSxx = ld<true>(AI, q, A_axSxx * n), aySxy = ld<true>(AI, q, A_aySxy * n), azSxz = ld<true>(AI, q, A_azSxz * n);
+    const float axSxy = ld<true>(AI, q, A_axSxy * n), aySyy = ld<true>(AI, q, A_aySyy * n), azSyz = ld<true>(AI, q, A_azSyz * n);
+    const float axSxz = ld<true>(AI, q, A_axSxz * n), aySyz = ld<true>(AI, q, A_aySyz * n), azSzz = ld<true>(AI, q, A_azSzz * n);
+    float *__restrict__ Vx = a.f.Vx;
+    float *__restrict__ Vy = a.f.Vy;
+    float *__restrict__ Vz = a.f.Vz;
+    const float vx = ld<true>(OOP ? a.fin.Vx : Vx, p), vy = ld<true>(OOP ? a.fin.Vy : Vy, p);
+    const float vz = ld<true>(OOP ? a.fin.Vz : Vz, p);
 
     const float dxSxx = (sxx_ip1 - sxx_0) * a.r20x;
     const float dySyy = (syy_jp1 - syy_0) * a.r20y;
@@ -268,24 +346,21 @@ __device__ __forceinline__ void pml_vel_cell(const StepArgs &a, long long p, lon
     const float by = 2.0f / (rho0 + rho_jp);
     const float bz = 2.0f / (rho0 + rho_kp);
 
-    float *__restrict__ Vx = a.f.Vx;
-    float *__restrict__ Vy = a.f.Vy;
-    float *__restrict__ Vz = a.f.Vz;
-    st1<true>(Vx + p, ld1<true>((OOP ? a.fin.Vx : Vx) + p) + bx * (gxe.x * dxSxx + gyc.x * dySxy + gzc.x * dzSxz
+    st<true>(Vx, p, vx + bx * (gxe.x * dxSxx + gyc.x * dySxy + gzc.x * dzSxz
                                                 + gxe.y * axSxx + gyc.y * aySxy + gzc.y * azSxz) * dt);
-    st1<true>(Vy + p, ld1<true>((OOP ? a.fin.Vy : Vy) + p) + by * (gxc.x * dxSxy + gye.x * dySyy + gzc.x * dzSyz
+    st<true>(Vy, p, vy + by * (gxc.x * dxSxy + gye.x * dySyy + gzc.x * dzSyz
                                                 + gxc.y * axSxy + gye.y * aySyy + gzc.y * azSyz) * dt);
-    st1<true>(Vz + p, ld1<true>((OOP ? a.fin.Vz : Vz) + p) + bz * (gxc.x * dxSxz + gyc.x * dySyz + gze.x * dzSzz
+    st<true>(Vz, p, vz + bz * (gxc.x * dxSxz + gyc.x * dySyz + gze.x * dzSzz
                                                 + gxc.y * axSxz + gyc.y * aySyz + gze.y * azSzz) * dt);
-    st1<true>(A + A_axSxx * n, gxe.z * axSxx + gxe.w * dxSxx * dt);
-    st1<true>(A + A_aySxy * n, gyc.z * aySxy + gyc.w * dySxy * dt);
-    st1<true>(A + A_azSxz * n, gzc.z * azSxz + gzc.w * dzSxz * dt);
-    st1<true>(A + A_axSxy * n, gxc.z * axSxy + gxc.w * dxSxy * dt);
-    st1<true>(A + A_aySyy * n, gye.z * aySyy + gye.w * dySyy * dt);
-    st1<true>(A + A_azSyz * n, gzc.z * azSyz + gzc.w * dzSyz * dt);
-    st1<true>(A + A_axSxz * n, gxc.z * axSxz + gxc.w * dxSxz * dt);
-    st1<true>(A + A_aySyz * n, gyc.z * aySyz + gyc.w * dySyz * dt);
-    st1<true>(A + A_azSzz * n, gze.z * azSzz + gze.w * dzSzz * dt);
+    st<true>(A, q, gxe.z * axSxx + gxe.w * dxSxx * dt, A_axSxx * n);
+    st<true>(A, q, gyc.z * aySxy + gyc.w * dySxy * dt, A_aySxy * n);
+    st<true>(A, q, gzc.z * azSxz + gzc.w * dzSxz * dt, A_azSxz * n);
+    st<true>(A, q, gxc.z * axSxy + gxc.w * dxSxy * dt, A_axSxy * n);
+    st<true>(A, q, gye.z * aySyy + gye.w * dySyy * dt, A_aySyy * n);
+    st<true>(A, q, gzc.z * azSyz + gzc.w * dzSyz * dt, A_azSyz * n);
+    st<true>(A, q, gxc.z * axSxz + gxc.w * dxSxz * dt, A_axSxz * n);
+    st<true>(A, q, gyc.z * aySyz + gyc.w * dySyz * dt, A_aySyz * n);
+    st<true>(A, q, gze.z * azSzz + gze.w * dzSzz * dt, A_azSzz * n);
 }
 
 // ---------------------------------------------------------------------------
@@ -312,7 +387,8 @@ struct VStencil {
 // at (i,j), (i+1,j), (i,j+1) on planes k and k+1 (n) and at (i+1,j+1) on
 // plane k.  OOP: the old stresses are read from a.fin.
 template <int NM, bool NT, bool OOP>
-__device__ __forceinline__ void stress_cell(const StepArgs &a, long long p, long long r, bool in, const VStencil &v,
+__device__ __forceinline__ void stress_cell(const StepArgs &a, const Loc &p, const Loc &r, bool in, const Coefs &cf,
+                                            const VStencil &v,
                                             float mu00, float mu00n, float mu10, float mu10n, float mu01, float mu01n,
                                             float mu11)
 {
@@ -331,12 +407,22 @@ __device__ __forceinline__ void stress_cell(const StepArgs &a, long long p, long
     const float dt = a.dt;
     const float d2 = a.v.d2;
     const long long rn = a.g.rn;
-    const float re40x = in ? a.c.re40x[1] : a.c.re40x[0];
-    const float re41x = in ? a.c.re41x[1] : a.c.re41x[0];
-    const float re40y = in ? a.c.re40y[1] : a.c.re40y[0];
-    const float re41y = in ? a.c.re41y[1] : a.c.re41y[0];
-    const float re40z = in ? a.c.re40z[1] : a.c.re40z[0];
-    const float re41z = in ? a.c.re41z[1] : a.c.re41z[0];
+    // every load comes before the first store: the fields may alias for the
+    // compiler, and a load left between two stores waits for both
+    const float lam1 = ld<NT>(a.m.lam, p);
+    const float taup1 = ld<NT>(a.m.taup, p);
+    const float taus1 = ld<NT>(a.m.taus, p);
+    const float sxx = ld<NT>(SxxI, p), syy = ld<NT>(SyyI, p), szz = ld<NT>(SzzI, p);
+    const float syz = ld<NT>(SyzI, p), sxz = ld<NT>(SxzI, p), sxy = ld<NT>(SxyI, p);
+    RCell<NM> R;
+    R.template load<NT>(a.R, rn, r);
+
+    const float re40x = cf.at(in, 0);
+    const float re41x = cf.at(in, 1);
+    const float re40y = cf.at(in, 2);
+    const float re41y = cf.at(in, 3);
+    const float re40z = cf.at(in, 4);
+    const float re41z = cf.at(in, 5);
 
     // normal components, m_kernel.f90:198-238
     const float dxVx = (v.vx_0 - v.vx_im1) * re40x - (v.vx_ip1 - v.vx_im2) * re41x;
@@ -344,16 +430,12 @@ __device__ __forceinline__ void stress_cell(const StepArgs &a, long long p, long
     const float dzVz = (v.vz_0 - v.vz_m1) * re40z - (v.vz_p1 - v.vz_m2) * re41z;
 
     const float mu2 = 2.0f * mu00;
-    const float lam2mu = ld1<NT>(a.m.lam + p) + mu2;
-    const float taup1 = ld1<NT>(a.m.taup + p);
-    const float taus1 = ld1<NT>(a.m.taus + p);
+    const float lam2mu = lam1 + mu2;
     const float d3v3 = dxVx + dyVy + dzVz;
     const float dyVy_dzVz = dyVy + dzVz;
     const float dxVx_dzVz = dxVx + dzVz;
     const float dxVx_dyVy = dxVx + dyVy;
 
-    RCell<NM> R;
-    R.template load<NT>(a.R, rn, r);
     float Rxx_n = 0.0f, Ryy_n = 0.0f, Rzz_n = 0.0f;
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
@@ -370,9 +452,9 @@ __device__ __forceinline__ void stress_cell(const StepArgs &a, long long p, long
     }
     const float taup_plus1 = 1.0f + taup1 * (1.0f + d2);
     const float taus_plus1 = 1.0f + taus1 * (1.0f + d2);
-    st1<NT>(Sxx + p, ld1<NT>(SxxI + p) + (lam2mu * taup_plus1 * d3v3 - mu2 * taus_plus1 * dyVy_dzVz + Rxx_n) * dt);
-    st1<NT>(Syy + p, ld1<NT>(SyyI + p) + (lam2mu * taup_plus1 * d3v3 - mu2 * taus_plus1 * dxVx_dzVz + Ryy_n) * dt);
-    st1<NT>(Szz + p, ld1<NT>(SzzI + p) + (lam2mu * taup_plus1 * d3v3 - mu2 * taus_plus1 * dxVx_dyVy + Rzz_n) * dt);
+    st<NT>(Sxx, p, sxx + (lam2mu * taup_plus1 * d3v3 - mu2 * taus_plus1 * dyVy_dzVz + Rxx_n) * dt);
+    st<NT>(Syy, p, syy + (lam2mu * taup_plus1 * d3v3 - mu2 * taus_plus1 * dxVx_dzVz + Ryy_n) * dt);
+    st<NT>(Szz, p, szz + (lam2mu * taup_plus1 * d3v3 - mu2 * taus_plus1 * dxVx_dyVy + Rzz_n) * dt);
 
     // shear components, m_kernel.f90:285-333
     const float dxVy_dyVx = (v.vy_ip1 - v.vy_0) * re40x - (v.vy_ip2 - v.vy_im1) * re41x
@@ -401,16 +483,16 @@ __device__ __forceinline__ void stress_cell(const StepArgs &a, long long p, long
         Rxy_n = Rxy_n + d1 * nxy;
     }
     R.template store<NT>(a.R, rn, r);
-    st1<NT>(Syz + p, ld1<NT>(SyzI + p) + (muyz * taus_plus1 * dyVz_dzVy + Ryz_n) * dt);
-    st1<NT>(Sxz + p, ld1<NT>(SxzI + p) + (muxz * taus_plus1 * dxVz_dzVx + Rxz_n) * dt);
-    st1<NT>(Sxy + p, ld1<NT>(SxyI + p) + (muxy * taus_plus1 * dxVy_dyVx + Rxy_n) * dt);
+    st<NT>(Syz, p, syz + (muyz * taus_plus1 * dyVz_dzVy + Ryz_n) * dt);
+    st<NT>(Sxz, p, sxz + (muxz * taus_plus1 * dxVz_dzVx + Rxz_n) * dt);
+    st<NT>(Sxy, p, sxy + (muxy * taus_plus1 * dxVy_dyVx + Rxy_n) * dt);
 }
 
-// logical tile (bx, by, bz) of a plain launch: blocks of one XCD take a
-// contiguous run of tiles, x fastest
+// logical tile (bx, by, bz) of the interior blocks of a launch (those after
+// its side blocks): blocks of one XCD take a contiguous run of tiles, x fastest
 __device__ static inline void plain_tile(const StepArgs &a, int &bx, int &byy, int &bz)
 {
-    const int bid = xcd_remap(blockIdx.x, gridDim.x);
+    const int bid = xcd_remap(blockIdx.x - a.sideb, gridDim.x - a.sideb);
     bx = bid % a.nbx;
     const int t = bid / a.nbx;
     byy = t % a.nby;
@@ -421,11 +503,11 @@ template <int NM, bool NT, bool OOP>
 __device__ __forceinline__ void stress_int_body(const StepArgs &a, int bx, int byy, int bz)
 {
     const Grid &g = a.g;
-    const int i = 1 + (a.bx0 + bx) * a.bxw + threadIdx.x;
-    const int j = g.jb + byy * a.byi + threadIdx.y;
+    const int it = 1 + (a.bx0 + bx) * a.bxw, jt = g.jb + byy * a.byi;   // the tile's first cell
+    const int i = it + threadIdx.x, j = jt + threadIdx.y;
     if (i < g.ib || i > g.ie || j > g.je) return;
-    const int k0 = a.zc[bz];
-    const int k1 = a.zc[bz + 1] - 1;
+    const int k0 = uni(ldv<false>(a.zc + bz));
+    const int k1 = uni(ldv<false>(a.zc + bz + 1)) - 1;
     const int ka1 = (a.mask & MASK_INT) ? min(k1, g.ke) : k0 - 1;      // interior planes k0..ka1
     const int kb0 = max(k0, g.ke + 1);
     const int kb1 = (a.has_pml && (a.mask & MASK_PML)) ? k1 : kb0 - 1;  // bottom PML planes kb0..kb1
@@ -439,80 +521,79 @@ __device__ __forceinline__ void stress_int_body(const StepArgs &a, int bx, int b
     const float *__restrict__ Vz = a.f.Vz;
     const float *__restrict__ mu = a.m.mu;
 
-    long long p = gidx(g, i, j, ks);
-    float vx_m1 = Vx[p - P], vx_0 = Vx[p], vx_p1 = Vx[p + P];
-    float vy_m1 = Vy[p - P], vy_0 = Vy[p], vy_p1 = Vy[p + P];
-    float vz_m2 = Vz[p - 2 * P], vz_m1 = Vz[p - P], vz_0 = Vz[p];
-    float mu00 = mu[p], mu10 = mu[p + 1], mu01 = mu[p + Y], mu11 = mu[p + 1 + Y];
+    Loc p = field_loc(g, it, jt, ks, threadIdx.x, threadIdx.y);
+    float vx_m1 = ld(Vx, p, -P), vx_0 = ld(Vx, p), vx_p1 = ld(Vx, p, P);
+    float vy_m1 = ld(Vy, p, -P), vy_0 = ld(Vy, p), vy_p1 = ld(Vy, p, P);
+    float vz_m2 = ld(Vz, p, -2 * P), vz_m1 = ld(Vz, p, -P), vz_0 = ld(Vz, p);
+    float mu00 = ld(mu, p), mu10 = ld(mu, p, 0, 1), mu01 = ld(mu, p, 0, 0, 1), mu11 = ld(mu, p, 0, 1, 1);
 
     if (ka1 >= k0) {
         const long long c2 = g2idx(g, i, j);
-        const int kft = a.m.kfs_top[c2], kfb = a.m.kfs_bot[c2];
-        const int kot = a.m.kob_top[c2], kobb = a.m.kob_bot[c2];
-        long long r = ((long long)(k0 - g.kb) * g.nyk + (j - g.jb)) * g.rpitch + (i - 1);
-        for (int k = k0; k <= ka1; ++k, p += P, r += g.rplane) {
-            const float vx_p2 = Vx[p + 2 * P], vy_p2 = Vy[p + 2 * P], vz_p1 = Vz[p + P];
-            const float mu00n = mu[p + P], mu10n = mu[p + P + 1], mu01n = mu[p + P + Y];
+        const int kft = ldv<false>(a.m.kfs_top + c2), kfb = ldv<false>(a.m.kfs_bot + c2);
+        const int kot = ldv<false>(a.m.kob_top + c2), kobb = ldv<false>(a.m.kob_bot + c2);
+        const Coefs cf(a);
+        Loc r = {((long long)(k0 - g.kb) * g.nyk + (jt - g.jb)) * g.rpitch + (it - 1),
+                 4u * (threadIdx.y * g.rpitch + threadIdx.x), 0u};
+        for (int k = k0; k <= ka1; ++k, p.u += P, r.u += g.rplane) {
+            fresh(p);
+            fresh(r);
+            const float vx_p2 = ld(Vx, p, 2 * P), vy_p2 = ld(Vy, p, 2 * P), vz_p1 = ld(Vz, p, P);
+            const float mu00n = ld(mu, p, P), mu10n = ld(mu, p, P, 1), mu01n = ld(mu, p, P, 0, 1);
+            const float mu11n = ld(mu, p, P, 1, 1);
 
             VStencil v;
             v.vx_m1 = vx_m1; v.vx_0 = vx_0; v.vx_p1 = vx_p1; v.vx_p2 = vx_p2;
             v.vy_m1 = vy_m1; v.vy_0 = vy_0; v.vy_p1 = vy_p1; v.vy_p2 = vy_p2;
             v.vz_m2 = vz_m2; v.vz_m1 = vz_m1; v.vz_0 = vz_0; v.vz_p1 = vz_p1;
-            v.vx_im2 = Vx[p - 2]; v.vx_im1 = Vx[p - 1]; v.vx_ip1 = Vx[p + 1];
-            v.vx_jm1 = Vx[p - Y]; v.vx_jp1 = Vx[p + Y]; v.vx_jp2 = Vx[p + 2 * Y];
-            v.vy_jm2 = Vy[p - 2 * Y]; v.vy_jm1 = Vy[p - Y]; v.vy_jp1 = Vy[p + Y];
-            v.vy_im1 = Vy[p - 1]; v.vy_ip1 = Vy[p + 1]; v.vy_ip2 = Vy[p + 2];
-            v.vz_im1 = Vz[p - 1]; v.vz_ip1 = Vz[p + 1]; v.vz_ip2 = Vz[p + 2];
-            v.vz_jm1 = Vz[p - Y]; v.vz_jp1 = Vz[p + Y]; v.vz_jp2 = Vz[p + 2 * Y];
-            stress_cell<NM, NT, OOP>(a, p, r, in_band(k, kft, kfb, kot, kobb), v, mu00, mu00n, mu10, mu10n, mu01, mu01n,
+            v.vx_im2 = ld(Vx, p, 0, -2); v.vx_im1 = ld(Vx, p, 0, -1); v.vx_ip1 = ld(Vx, p, 0, 1);
+            v.vx_jm1 = ld(Vx, p, 0, 0, -1); v.vx_jp1 = ld(Vx, p, 0, 0, 1); v.vx_jp2 = ld(Vx, p, 0, 0, 2);
+            v.vy_jm2 = ld(Vy, p, 0, 0, -2); v.vy_jm1 = ld(Vy, p, 0, 0, -1); v.vy_jp1 = ld(Vy, p, 0, 0, 1);
+            v.vy_im1 = ld(Vy, p, 0, -1); v.vy_ip1 = ld(Vy, p, 0, 1); v.vy_ip2 = ld(Vy, p, 0, 2);
+            v.vz_im1 = ld(Vz, p, 0, -1); v.vz_ip1 = ld(Vz, p, 0, 1); v.vz_ip2 = ld(Vz, p, 0, 2);
+            v.vz_jm1 = ld(Vz, p, 0, 0, -1); v.vz_jp1 = ld(Vz, p, 0, 0, 1); v.vz_jp2 = ld(Vz, p, 0, 0, 2);
+            stress_cell<NM, NT, OOP>(a, p, r, in_band(k, kft, kfb, kot, kobb), cf, v, mu00, mu00n, mu10, mu10n, mu01, mu01n,
                                      mu11);
 
             // rotate the z queues
             vx_m1 = vx_0; vx_0 = vx_p1; vx_p1 = vx_p2;
             vy_m1 = vy_0; vy_0 = vy_p1; vy_p1 = vy_p2;
             vz_m2 = vz_m1; vz_m1 = vz_0; vz_0 = vz_p1;
-            mu00 = mu00n; mu10 = mu10n; mu01 = mu01n;
-            mu11 = mu[p + P + 1 + Y];
+            mu00 = mu00n; mu10 = mu10n; mu01 = mu01n; mu11 = mu11n;
         }
     }
     if (kb1 >= kb0) {
         // bottom PML band of the interior columns (box 4)
         const PmlBox b = a.box[4];
         const long long astride = (long long)b.nxb * b.nyb;
-        long long q = b.off + (long long)(j - b.j0) * b.nxb + (i - b.i0) + (long long)(kb0 - b.k0) * astride;
-        const float4 gxc = a.gxc[i - 1], gxe = a.gxe[i - 1];
-        const float4 gyc = a.gyc[j - 1], gye = a.gye[j - 1];
-        for (int k = kb0; k <= kb1; ++k, p += P, q += astride) {
-            const float vx_p2 = Vx[p + 2 * P], vy_p2 = Vy[p + 2 * P], vz_p1 = Vz[p + P];
-            const float mu00n = mu[p + P], mu10n = mu[p + P + 1], mu01n = mu[p + P + Y];
+        Loc q = {b.off + (long long)(jt - b.j0) * b.nxb + (it - b.i0) + (long long)(kb0 - b.k0) * astride,
+                 4u * (threadIdx.y * b.nxb + threadIdx.x), 0u};
+        const float4 gxc = ldp(a.gxc + (i - 1)), gxe = ldp(a.gxe + (i - 1));
+        const float4 gyc = ldp(a.gyc + (j - 1)), gye = ldp(a.gye + (j - 1));
+        for (int k = kb0; k <= kb1; ++k, p.u += P, q.u += astride) {
+            fresh(p);
+            fresh(q);
+            const float vx_p2 = ld(Vx, p, 2 * P), vy_p2 = ld(Vy, p, 2 * P), vz_p1 = ld(Vz, p, P);
+            const float mu00n = ld(mu, p, P), mu10n = ld(mu, p, P, 1), mu01n = ld(mu, p, P, 0, 1);
+            const float mu11n = ld(mu, p, P, 1, 1);
             pml_stress_cell<NT, OOP>(a, p, q, k, vx_0, vx_p1, vy_0, vy_p1, vz_m1, vz_0, mu00, mu00n, mu10, mu10n, mu01,
                                 mu01n, mu11, gxc, gxe, gyc, gye);
             vx_m1 = vx_0; vx_0 = vx_p1; vx_p1 = vx_p2;
             vy_m1 = vy_0; vy_0 = vy_p1; vy_p1 = vy_p2;
             vz_m2 = vz_m1; vz_m1 = vz_0; vz_0 = vz_p1;
-            mu00 = mu00n; mu10 = mu10n; mu01 = mu01n;
-            mu11 = mu[p + P + 1 + Y];
+            mu00 = mu00n; mu10 = mu10n; mu01 = mu01n; mu11 = mu11n;
         }
     }
 }
 
-template <int NM, bool NT, bool OOP>
-__global__ void __launch_bounds__(256) k_stress_int(StepArgs a)
-{
-    int bx, byy, bz;
-    plain_tile(a, bx, byy, bz);
-    stress_int_body<NM, NT, OOP>(a, bx, byy, bz);
-}
-
 // batched launch: tile = (member, bx, by, bz), member arguments in HBM
 template <int NM, bool NT>
-__global__ void __launch_bounds__(256) k_stress_int_b(const StepArgs *__restrict__ mem, const int4 *__restrict__ tiles)
+__global__ void __launch_bounds__(256) WAVES_NM k_stress_int_b(const StepArgs *__restrict__ mem, const int4 *__restrict__ tiles)
 {
-    const int4 t = tiles[xcd_remap(blockIdx.x, gridDim.x)];
+    const int4 t = uni(tiles[xcd_remap(blockIdx.x, gridDim.x)]);
     stress_int_body<NM, NT, false>(mem[t.x], t.y, t.z, t.w);
 }
 
-// Every load of one plane of the interior velocity update: the z-queue
+// Every load of one plane (d elements on from p) of the interior velocity update: the z-queue
 // entries the plane adds, the x/y neighbours, the buoyancy densities and the
 // old velocities.  Loading the next plane's set before computing this one's
 // keeps two planes of loads in flight per wave.
@@ -528,8 +609,9 @@ struct VelLoads {
 };
 
 template <bool OOP>
-__device__ __forceinline__ void vel_loads(const StepArgs &a, long long p, VelLoads &L)
+__device__ __forceinline__ void vel_loads(const StepArgs &a, Loc p, VelLoads &L, long long d)
 {
+    fresh(p);
     const long long P = a.g.plane;
     const int Y = a.g.pitch;
     const float *__restrict__ Sxx = a.f.Sxx;
@@ -539,18 +621,18 @@ __device__ __forceinline__ void vel_loads(const StepArgs &a, long long p, VelLoa
     const float *__restrict__ Sxz = a.f.Sxz;
     const float *__restrict__ Sxy = a.f.Sxy;
     const float *__restrict__ rho = a.m.rho;
-    L.sxz_p1 = Sxz[p + P]; L.syz_p1 = Syz[p + P]; L.szz_p2 = Szz[p + 2 * P]; L.rho_kp = rho[p + P];
-    L.sxx_im1 = Sxx[p - 1]; L.sxx_0 = Sxx[p]; L.sxx_ip1 = Sxx[p + 1]; L.sxx_ip2 = Sxx[p + 2];
-    L.sxy_0 = Sxy[p];
-    L.sxy_jm2 = Sxy[p - 2 * Y]; L.sxy_jm1 = Sxy[p - Y]; L.sxy_jp1 = Sxy[p + Y];
-    L.sxy_im2 = Sxy[p - 2]; L.sxy_im1 = Sxy[p - 1]; L.sxy_ip1 = Sxy[p + 1];
-    L.syy_jm1 = Syy[p - Y]; L.syy_0 = Syy[p]; L.syy_jp1 = Syy[p + Y]; L.syy_jp2 = Syy[p + 2 * Y];
-    L.syz_jm2 = Syz[p - 2 * Y]; L.syz_jm1 = Syz[p - Y]; L.syz_jp1 = Syz[p + Y];
-    L.sxz_im2 = Sxz[p - 2]; L.sxz_im1 = Sxz[p - 1]; L.sxz_ip1 = Sxz[p + 1];
-    L.rho_ip = rho[p + 1]; L.rho_jp = rho[p + Y];
-    L.vx = ld1<true>((OOP ? a.fin.Vx : a.f.Vx) + p);
-    L.vy = ld1<true>((OOP ? a.fin.Vy : a.f.Vy) + p);
-    L.vz = ld1<true>((OOP ? a.fin.Vz : a.f.Vz) + p);
+    L.sxz_p1 = ld(Sxz, p, d + P); L.syz_p1 = ld(Syz, p, d + P); L.szz_p2 = ld(Szz, p, d + 2 * P); L.rho_kp = ld(rho, p, d + P);
+    L.sxx_im1 = ld(Sxx, p, d, -1); L.sxx_0 = ld(Sxx, p, d); L.sxx_ip1 = ld(Sxx, p, d, 1); L.sxx_ip2 = ld(Sxx, p, d, 2);
+    L.sxy_0 = ld(Sxy, p, d);
+    L.sxy_jm2 = ld(Sxy, p, d, 0, -2); L.sxy_jm1 = ld(Sxy, p, d, 0, -1); L.sxy_jp1 = ld(Sxy, p, d, 0, 1);
+    L.sxy_im2 = ld(Sxy, p, d, -2); L.sxy_im1 = ld(Sxy, p, d, -1); L.sxy_ip1 = ld(Sxy, p, d, 1);
+    L.syy_jm1 = ld(Syy, p, d, 0, -1); L.syy_0 = ld(Syy, p, d); L.syy_jp1 = ld(Syy, p, d, 0, 1); L.syy_jp2 = ld(Syy, p, d, 0, 2);
+    L.syz_jm2 = ld(Syz, p, d, 0, -2); L.syz_jm1 = ld(Syz, p, d, 0, -1); L.syz_jp1 = ld(Syz, p, d, 0, 1);
+    L.sxz_im2 = ld(Sxz, p, d, -2); L.sxz_im1 = ld(Sxz, p, d, -1); L.sxz_ip1 = ld(Sxz, p, d, 1);
+    L.rho_ip = ld(rho, p, d, 1); L.rho_jp = ld(rho, p, d, 0, 1);
+    L.vx = ld<true>(OOP ? a.fin.Vx : a.f.Vx, p, d);
+    L.vy = ld<true>(OOP ? a.fin.Vy : a.f.Vy, p, d);
+    L.vz = ld<true>(OOP ? a.fin.Vz : a.f.Vz, p, d);
 }
 
 // kernel__update_vel, m_kernel.f90:75-140, then the bottom PML band.
@@ -559,11 +641,11 @@ template <bool OOP, bool PF>
 __device__ __forceinline__ void vel_int_body(const StepArgs &a, int bx, int byy, int bz)
 {
     const Grid &g = a.g;
-    const int i = 1 + (a.bx0 + bx) * a.bxw + threadIdx.x;
-    const int j = g.jb + byy * a.byi + threadIdx.y;
+    const int it = 1 + (a.bx0 + bx) * a.bxw, jt = g.jb + byy * a.byi;   // the tile's first cell
+    const int i = it + threadIdx.x, j = jt + threadIdx.y;
     if (i < g.ib || i > g.ie || j > g.je) return;
-    const int k0 = a.zc[bz];
-    const int k1 = a.zc[bz + 1] - 1;
+    const int k0 = uni(ldv<false>(a.zc + bz));
+    const int k1 = uni(ldv<false>(a.zc + bz + 1)) - 1;
     const int ka1 = (a.mask & MASK_INT) ? min(k1, g.ke) : k0 - 1;
     const int kb0 = max(k0, g.ke + 1);
     const int kb1 = (a.has_pml && (a.mask & MASK_PML)) ? k1 : kb0 - 1;
@@ -584,30 +666,32 @@ __device__ __forceinline__ void vel_int_body(const StepArgs &a, int bx, int byy,
     float *__restrict__ Vz = a.f.Vz;
     const float dt = a.dt;
 
-    long long p = gidx(g, i, j, ks);
-    float sxz_m2 = Sxz[p - 2 * P], sxz_m1 = Sxz[p - P], sxz_0 = Sxz[p];
-    float syz_m2 = Syz[p - 2 * P], syz_m1 = Syz[p - P], syz_0 = Syz[p];
-    float szz_m1 = Szz[p - P], szz_0 = Szz[p], szz_p1 = Szz[p + P];
-    float rho0 = rho[p];
+    Loc p = field_loc(g, it, jt, ks, threadIdx.x, threadIdx.y);
+    float sxz_m2 = ld(Sxz, p, -2 * P), sxz_m1 = ld(Sxz, p, -P), sxz_0 = ld(Sxz, p);
+    float syz_m2 = ld(Syz, p, -2 * P), syz_m1 = ld(Syz, p, -P), syz_0 = ld(Syz, p);
+    float szz_m1 = ld(Szz, p, -P), szz_0 = ld(Szz, p), szz_p1 = ld(Szz, p, P);
+    float rho0 = ld(rho, p);
 
     if (PF && ka1 >= k0) {
         const long long c2 = g2idx(g, i, j);
-        const int kft = a.m.kfs_top[c2], kfb = a.m.kfs_bot[c2];
-        const int kot = a.m.kob_top[c2], kobb = a.m.kob_bot[c2];
+        const int kft = ldv<false>(a.m.kfs_top + c2), kfb = ldv<false>(a.m.kfs_bot + c2);
+        const int kot = ldv<false>(a.m.kob_top + c2), kobb = ldv<false>(a.m.kob_bot + c2);
+        const Coefs cf(a);
         VelLoads L;
-        vel_loads<OOP>(a, p, L);
-        for (int k = k0; k <= ka1; ++k, p += P) {
+        vel_loads<OOP>(a, p, L, 0);
+        for (int k = k0; k <= ka1; ++k, p.u += P) {
+            fresh(p);
             // plane k+1 <= nz + 1: its loads stay within the -2..nz+3 halo
             VelLoads N;
-            if (k < ka1) vel_loads<OOP>(a, p + P, N);
+            if (k < ka1) vel_loads<OOP>(a, p, N, P);
 
             const bool in = in_band(k, kft, kfb, kot, kobb);
-            const float re40x = in ? a.c.re40x[1] : a.c.re40x[0];
-            const float re41x = in ? a.c.re41x[1] : a.c.re41x[0];
-            const float re40y = in ? a.c.re40y[1] : a.c.re40y[0];
-            const float re41y = in ? a.c.re41y[1] : a.c.re41y[0];
-            const float re40z = in ? a.c.re40z[1] : a.c.re40z[0];
-            const float re41z = in ? a.c.re41z[1] : a.c.re41z[0];
+            const float re40x = cf.at(in, 0);
+            const float re41x = cf.at(in, 1);
+            const float re40y = cf.at(in, 2);
+            const float re41y = cf.at(in, 3);
+            const float re40z = cf.at(in, 4);
+            const float re41z = cf.at(in, 5);
 
             const float d3Sx3 = (L.sxx_ip1 - L.sxx_0) * re40x - (L.sxx_ip2 - L.sxx_im1) * re41x
                               + (L.sxy_0 - L.sxy_jm1) * re40y - (L.sxy_jp1 - L.sxy_jm2) * re41y
@@ -619,9 +703,9 @@ __device__ __forceinline__ void vel_int_body(const StepArgs &a, int bx, int byy,
                               + (syz_0 - L.syz_jm1) * re40y - (L.syz_jp1 - L.syz_jm2) * re41y
                               + (szz_p1 - szz_0) * re40z - (L.szz_p2 - szz_m1) * re41z;
 
-            st1<true>(Vx + p, L.vx + 2.0f / (rho0 + L.rho_ip) * d3Sx3 * dt);
-            st1<true>(Vy + p, L.vy + 2.0f / (rho0 + L.rho_jp) * d3Sy3 * dt);
-            st1<true>(Vz + p, L.vz + 2.0f / (rho0 + L.rho_kp) * d3Sz3 * dt);
+            st<true>(Vx, p, L.vx + 2.0f / (rho0 + L.rho_ip) * d3Sx3 * dt);
+            st<true>(Vy, p, L.vy + 2.0f / (rho0 + L.rho_jp) * d3Sy3 * dt);
+            st<true>(Vz, p, L.vz + 2.0f / (rho0 + L.rho_kp) * d3Sz3 * dt);
 
             sxz_m2 = sxz_m1; sxz_m1 = sxz_0; sxz_0 = L.sxz_p1;
             syz_m2 = syz_m1; syz_m1 = syz_0; syz_0 = L.syz_p1;
@@ -631,27 +715,32 @@ __device__ __forceinline__ void vel_int_body(const StepArgs &a, int bx, int byy,
         }
     } else if (ka1 >= k0) {
         const long long c2 = g2idx(g, i, j);
-        const int kft = a.m.kfs_top[c2], kfb = a.m.kfs_bot[c2];
-        const int kot = a.m.kob_top[c2], kobb = a.m.kob_bot[c2];
-        for (int k = k0; k <= ka1; ++k, p += P) {
-            const float sxz_p1 = Sxz[p + P], syz_p1 = Syz[p + P], szz_p2 = Szz[p + 2 * P];
-            const float rho_kp = rho[p + P];
+        const int kft = ldv<false>(a.m.kfs_top + c2), kfb = ldv<false>(a.m.kfs_bot + c2);
+        const int kot = ldv<false>(a.m.kob_top + c2), kobb = ldv<false>(a.m.kob_bot + c2);
+        const Coefs cf(a);
+        for (int k = k0; k <= ka1; ++k, p.u += P) {
+            fresh(p);
+            const float sxz_p1 = ld(Sxz, p, P), syz_p1 = ld(Syz, p, P), szz_p2 = ld(Szz, p, 2 * P);
+            const float rho_kp = ld(rho, p, P);
 
             const bool in = in_band(k, kft, kfb, kot, kobb);
-            const float re40x = in ? a.c.re40x[1] : a.c.re40x[0];
-            const float re41x = in ? a.c.re41x[1] : a.c.re41x[0];
-            const float re40y = in ? a.c.re40y[1] : a.c.re40y[0];
-            const float re41y = in ? a.c.re41y[1] : a.c.re41y[0];
-            const float re40z = in ? a.c.re40z[1] : a.c.re40z[0];
-            const float re41z = in ? a.c.re41z[1] : a.c.re41z[0];
+            const float re40x = cf.at(in, 0);
+            const float re41x = cf.at(in, 1);
+            const float re40y = cf.at(in, 2);
+            const float re41y = cf.at(in, 3);
+            const float re40z = cf.at(in, 4);
+            const float re41z = cf.at(in, 5);
 
-            const float sxx_im1 = Sxx[p - 1], sxx_0 = Sxx[p], sxx_ip1 = Sxx[p + 1], sxx_ip2 = Sxx[p + 2];
-            const float sxy_0 = Sxy[p];
-            const float sxy_jm2 = Sxy[p - 2 * Y], sxy_jm1 = Sxy[p - Y], sxy_jp1 = Sxy[p + Y];
-            const float sxy_im2 = Sxy[p - 2], sxy_im1 = Sxy[p - 1], sxy_ip1 = Sxy[p + 1];
-            const float syy_jm1 = Syy[p - Y], syy_0 = Syy[p], syy_jp1 = Syy[p + Y], syy_jp2 = Syy[p + 2 * Y];
-            const float syz_jm2 = Syz[p - 2 * Y], syz_jm1 = Syz[p - Y], syz_jp1 = Syz[p + Y];
-            const float sxz_im2 = Sxz[p - 2], sxz_im1 = Sxz[p - 1], sxz_ip1 = Sxz[p + 1];
+            const float rho_ip = ld(rho, p, 0, 1), rho_jp = ld(rho, p, 0, 0, 1);
+            const float vx = ld<true>(OOP ? a.fin.Vx : Vx, p), vy = ld<true>(OOP ? a.fin.Vy : Vy, p);
+            const float vz = ld<true>(OOP ? a.fin.Vz : Vz, p);
+            const float sxx_im1 = ld(Sxx, p, 0, -1), sxx_0 = ld(Sxx, p), sxx_ip1 = ld(Sxx, p, 0, 1), sxx_ip2 = ld(Sxx, p, 0, 2);
+            const float sxy_0 = ld(Sxy, p);
+            const float sxy_jm2 = ld(Sxy, p, 0, 0, -2), sxy_jm1 = ld(Sxy, p, 0, 0, -1), sxy_jp1 = ld(Sxy, p, 0, 0, 1);
+            const float sxy_im2 = ld(Sxy, p, 0, -2), sxy_im1 = ld(Sxy, p, 0, -1), sxy_ip1 = ld(Sxy, p, 0, 1);
+            const float syy_jm1 = ld(Syy, p, 0, 0, -1), syy_0 = ld(Syy, p), syy_jp1 = ld(Syy, p, 0, 0, 1), syy_jp2 = ld(Syy, p, 0, 0, 2);
+            const float syz_jm2 = ld(Syz, p, 0, 0, -2), syz_jm1 = ld(Syz, p, 0, 0, -1), syz_jp1 = ld(Syz, p, 0, 0, 1);
+            const float sxz_im2 = ld(Sxz, p, 0, -2), sxz_im1 = ld(Sxz, p, 0, -1), sxz_ip1 = ld(Sxz, p, 0, 1);
 
             const float d3Sx3 = (sxx_ip1 - sxx_0) * re40x - (sxx_ip2 - sxx_im1) * re41x
                               + (sxy_0 - sxy_jm1) * re40y - (sxy_jp1 - sxy_jm2) * re41y
@@ -663,9 +752,9 @@ __device__ __forceinline__ void vel_int_body(const StepArgs &a, int bx, int byy,
                               + (syz_0 - syz_jm1) * re40y - (syz_jp1 - syz_jm2) * re41y
                               + (szz_p1 - szz_0) * re40z - (szz_p2 - szz_m1) * re41z;
 
-            st1<true>(Vx + p, ld1<true>((OOP ? a.fin.Vx : Vx) + p) + 2.0f / (rho0 + rho[p + 1]) * d3Sx3 * dt);
-            st1<true>(Vy + p, ld1<true>((OOP ? a.fin.Vy : Vy) + p) + 2.0f / (rho0 + rho[p + Y]) * d3Sy3 * dt);
-            st1<true>(Vz + p, ld1<true>((OOP ? a.fin.Vz : Vz) + p) + 2.0f / (rho0 + rho_kp) * d3Sz3 * dt);
+            st<true>(Vx, p, vx + 2.0f / (rho0 + rho_ip) * d3Sx3 * dt);
+            st<true>(Vy, p, vy + 2.0f / (rho0 + rho_jp) * d3Sy3 * dt);
+            st<true>(Vz, p, vz + 2.0f / (rho0 + rho_kp) * d3Sz3 * dt);
 
             sxz_m2 = sxz_m1; sxz_m1 = sxz_0; sxz_0 = sxz_p1;
             syz_m2 = syz_m1; syz_m1 = syz_0; syz_0 = syz_p1;
@@ -676,12 +765,15 @@ __device__ __forceinline__ void vel_int_body(const StepArgs &a, int bx, int byy,
     if (kb1 >= kb0) {
         const PmlBox b = a.box[4];
         const long long astride = (long long)b.nxb * b.nyb;
-        long long q = b.off + (long long)(j - b.j0) * b.nxb + (i - b.i0) + (long long)(kb0 - b.k0) * astride;
-        const float4 gxc = a.gxc[i - 1], gxe = a.gxe[i - 1];
-        const float4 gyc = a.gyc[j - 1], gye = a.gye[j - 1];
-        for (int k = kb0; k <= kb1; ++k, p += P, q += astride) {
-            const float sxz_p1 = Sxz[p + P], syz_p1 = Syz[p + P], szz_p2 = Szz[p + 2 * P];
-            const float rho_kp = rho[p + P];
+        Loc q = {b.off + (long long)(jt - b.j0) * b.nxb + (it - b.i0) + (long long)(kb0 - b.k0) * astride,
+                 4u * (threadIdx.y * b.nxb + threadIdx.x), 0u};
+        const float4 gxc = ldp(a.gxc + (i - 1)), gxe = ldp(a.gxe + (i - 1));
+        const float4 gyc = ldp(a.gyc + (j - 1)), gye = ldp(a.gye + (j - 1));
+        for (int k = kb0; k <= kb1; ++k, p.u += P, q.u += astride) {
+            fresh(p);
+            fresh(q);
+            const float sxz_p1 = ld(Sxz, p, P), syz_p1 = ld(Syz, p, P), szz_p2 = ld(Szz, p, 2 * P);
+            const float rho_kp = ld(rho, p, P);
             pml_vel_cell<OOP>(a, p, q, k, szz_0, szz_p1, syz_m1, syz_0, sxz_m1, sxz_0, rho0, rho_kp, gxc, gxe, gyc, gye);
             sxz_m2 = sxz_m1; sxz_m1 = sxz_0; sxz_0 = sxz_p1;
             syz_m2 = syz_m1; syz_m1 = syz_0; syz_0 = syz_p1;
@@ -691,20 +783,10 @@ __device__ __forceinline__ void vel_int_body(const StepArgs &a, int bx, int byy,
     }
 }
 
-// 4 waves per SIMD: the velocity update fits 128 VGPRs without spilling and
-// runs about 6 % faster than at the compiler's default of 3 waves
-template <bool OOP, bool PF>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PF ? 3 : 4))) k_vel_int(StepArgs a)
-{
-    int bx, byy, bz;
-    plain_tile(a, bx, byy, bz);
-    vel_int_body<OOP, PF>(a, bx, byy, bz);
-}
-
 template <bool PF>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PF ? 3 : 4))) k_vel_int_b(const StepArgs *__restrict__ mem, const int4 *__restrict__ tiles)
+__global__ void __launch_bounds__(256) WAVES4 k_vel_int_b(const StepArgs *__restrict__ mem, const int4 *__restrict__ tiles)
 {
-    const int4 t = tiles[xcd_remap(blockIdx.x, gridDim.x)];
+    const int4 t = uni(tiles[xcd_remap(blockIdx.x, gridDim.x)]);
     vel_int_body<false, PF>(mem[t.x], t.y, t.z, t.w);
 }
 
@@ -748,6 +830,7 @@ __global__ void __launch_bounds__(256) k_fused(StepArgs a)
     const float *__restrict__ rho = a.m.rho;
     const float *__restrict__ mu = a.m.mu;
 
+    const Coefs cf(a);
     // velocity points of this thread: column iv, rows j0 - 2 + ty + 4 r.
     // vf: 0 not needed by the tile, 1 read from a.f, 2 computed, 3 computed
     // and stored (the tile's own cells)
@@ -811,12 +894,12 @@ __global__ void __launch_bounds__(256) k_fused(StepArgs a)
                 const float sxz_p1 = Sxz[p + P], syz_p1 = Syz[p + P], szz_p2 = Szz[p + 2 * P];
                 const float rho_kp = rho[p + P];
                 const bool in = in_band(kv, vb[r][0], vb[r][1], vb[r][2], vb[r][3]);
-                const float re40x = in ? a.c.re40x[1] : a.c.re40x[0];
-                const float re41x = in ? a.c.re41x[1] : a.c.re41x[0];
-                const float re40y = in ? a.c.re40y[1] : a.c.re40y[0];
-                const float re41y = in ? a.c.re41y[1] : a.c.re41y[0];
-                const float re40z = in ? a.c.re40z[1] : a.c.re40z[0];
-                const float re41z = in ? a.c.re41z[1] : a.c.re41z[0];
+                const float re40x = cf.at(in, 0);
+                const float re41x = cf.at(in, 1);
+                const float re40y = cf.at(in, 2);
+                const float re41y = cf.at(in, 3);
+                const float re40z = cf.at(in, 4);
+                const float re41z = cf.at(in, 5);
 
                 const float sxx_im1 = Sxx[p - 1], sxx_0 = Sxx[p], sxx_ip1 = Sxx[p + 1], sxx_ip2 = Sxx[p + 2];
                 const float sxy_0 = Sxy[p];
@@ -836,13 +919,13 @@ __global__ void __launch_bounds__(256) k_fused(StepArgs a)
                                   + (syz_0[r] - syz_jm1) * re40y - (syz_jp1 - syz_jm2) * re41y
                                   + (szz_p1[r] - szz_0[r]) * re40z - (szz_p2 - szz_m1[r]) * re41z;
 
-                vx = ld1<true>(a.fin.Vx + p) + 2.0f / (rho0[r] + rho[p + 1]) * d3Sx3 * dt;
-                vy = ld1<true>(a.fin.Vy + p) + 2.0f / (rho0[r] + rho[p + Y]) * d3Sy3 * dt;
-                vz = ld1<true>(a.fin.Vz + p) + 2.0f / (rho0[r] + rho_kp) * d3Sz3 * dt;
+                vx = ldv<true>(a.fin.Vx + p) + 2.0f / (rho0[r] + rho[p + 1]) * d3Sx3 * dt;
+                vy = ldv<true>(a.fin.Vy + p) + 2.0f / (rho0[r] + rho[p + Y]) * d3Sy3 * dt;
+                vz = ldv<true>(a.fin.Vz + p) + 2.0f / (rho0[r] + rho_kp) * d3Sz3 * dt;
                 if (vf[r] == 3 && kv >= k0 && kv <= k1) {
-                    st1<true>(a.f.Vx + p, vx);
-                    st1<true>(a.f.Vy + p, vy);
-                    st1<true>(a.f.Vz + p, vz);
+                    stv<true>(a.f.Vx + p, vx);
+                    stv<true>(a.f.Vy + p, vy);
+                    stv<true>(a.f.Vz + p, vz);
                 }
                 sxz_m2[r] = sxz_m1[r]; sxz_m1[r] = sxz_0[r]; sxz_0[r] = sxz_p1;
                 syz_m2[r] = syz_m1[r]; syz_m1[r] = syz_0[r]; syz_0[r] = syz_p1;
@@ -891,7 +974,7 @@ __global__ void __launch_bounds__(256) k_fused(StepArgs a)
             v.vz_jm1 = vs[s0][2][row - 1][col]; v.vz_jp1 = vs[s0][2][row + 1][col];
             v.vz_jp2 = vs[s0][2][row + 2][col];
             const long long rr = ((long long)(k - g.kb) * g.nyk + (js - g.jb)) * g.rpitch + (is - 1);
-            stress_cell<NM, true, true>(a, p, rr, in_band(k, sb[s][0], sb[s][1], sb[s][2], sb[s][3]), v, mu00[s],
+            stress_cell<NM, true, true>(a, Loc{p, 0u, 0u}, Loc{rr, 0u, 0u}, in_band(k, sb[s][0], sb[s][1], sb[s][2], sb[s][3]), cf, v, mu00[s],
                                         mu00n, mu10[s], mu10n, mu01[s], mu01n, mu11[s]);
             mu00[s] = mu00n; mu10[s] = mu10n; mu01[s] = mu01n;
             mu11[s] = mu[p + P + 1 + Y];
@@ -907,34 +990,33 @@ __global__ void __launch_bounds__(256) k_fused(StepArgs a)
 // ---------------------------------------------------------------------------
 struct PmlLane {
     int i, j, kb, ke;
-    long long abase, astride;
+    Loc p, q;            // field and auxiliary places on plane kb
+    long long astride;
 };
 
 __device__ static inline bool pml_lane(const StepArgs &a, const int4 tl, PmlLane &L)
 {
     const Grid &g = a.g;
-    const int w = (tl.x >> 20) & 0xFF;
+    const int i0 = tl.x & 0xFFFFF, w = (tl.x >> 20) & 0xFF, j0 = tl.y;
     const bool xslab = (tl.x >> 28) & 1;
     const int lane = threadIdx.y * blockDim.x + threadIdx.x;
     const int rows = (blockDim.x * blockDim.y) / w;
     if (lane >= rows * w) return false;
-    L.i = (tl.x & 0xFFFFF) + lane % w;
-    L.j = tl.y + lane / w;
-    if (L.i > g.nx || L.j > g.ny) return false;
+    const int col = lane % w, row = lane / w;
+    L.i = i0 + col;
+    L.j = j0 + row;
+    // a tile lies in one box: x slabs hold the interior rows, y slabs their own
     const int na = g.na;
-    int q;
-    if (L.j <= na) q = 0;
-    else if (L.j > g.ny - na) q = 1;
-    else if (L.i <= na) q = 2;
-    else if (L.i > g.nx - na) q = 3;
-    else return false;  // interior column: its bottom band belongs to the interior kernels
-    // x-slab cells of interior rows belong to the slab tiles, y-slab cells to full-row tiles
-    if (xslab != (q >= 2)) return false;
+    const int q = xslab ? (i0 <= na ? 2 : 3) : (j0 <= na ? 0 : 1);
+    const int jl = q == 0 ? na : q == 1 ? g.ny : g.ny - na;
+    if (L.i > g.nx || L.j > jl) return false;
     const PmlBox b = pick_box(a, q);
     L.kb = tl.z;
     L.ke = min(tl.w, g.nz);
     L.astride = (long long)b.nxb * b.nyb;
-    L.abase = b.off + (long long)(L.j - b.j0) * b.nxb + (L.i - b.i0) - (long long)b.k0 * L.astride;
+    L.p = field_loc(g, i0, j0, L.kb, col, row);
+    L.q = {b.off + (long long)(j0 - b.j0) * b.nxb + (i0 - b.i0) + (long long)(L.kb - b.k0) * L.astride,
+           4u * (unsigned)(row * b.nxb + col), 0u};
     return L.kb <= L.ke;
 }
 
@@ -952,21 +1034,22 @@ __device__ __forceinline__ void stress_pml_body(const StepArgs &a, const int4 tl
     const float *__restrict__ Vy = a.f.Vy;
     const float *__restrict__ Vz = a.f.Vz;
     const float *__restrict__ mu = a.m.mu;
-    const float4 gxc = a.gxc[i - 1], gxe = a.gxe[i - 1];
-    const float4 gyc = a.gyc[j - 1], gye = a.gye[j - 1];
+    const float4 gxc = ldp(a.gxc + (i - 1)), gxe = ldp(a.gxe + (i - 1));
+    const float4 gyc = ldp(a.gyc + (j - 1)), gye = ldp(a.gye + (j - 1));
 
-    long long p = gidx(g, i, j, L.kb);
-    long long q = L.abase + (long long)L.kb * L.astride;
-    float vx_0 = Vx[p], vy_0 = Vy[p], vz_m1 = Vz[p - P];
-    float mu00 = mu[p], mu10 = mu[p + 1], mu01 = mu[p + Y], mu11 = mu[p + 1 + Y];
-    for (int k = L.kb; k <= L.ke; ++k, p += P, q += L.astride) {
-        const float vx_p1 = Vx[p + P], vy_p1 = Vy[p + P], vz_0 = Vz[p];
-        const float mu00n = mu[p + P], mu10n = mu[p + P + 1], mu01n = mu[p + P + Y];
+    Loc p = L.p, q = L.q;
+    float vx_0 = ld(Vx, p), vy_0 = ld(Vy, p), vz_m1 = ld(Vz, p, -P);
+    float mu00 = ld(mu, p), mu10 = ld(mu, p, 0, 1), mu01 = ld(mu, p, 0, 0, 1), mu11 = ld(mu, p, 0, 1, 1);
+    for (int k = L.kb; k <= L.ke; ++k, p.u += P, q.u += L.astride) {
+        fresh(p);
+        fresh(q);
+        const float vx_p1 = ld(Vx, p, P), vy_p1 = ld(Vy, p, P), vz_0 = ld(Vz, p);
+        const float mu00n = ld(mu, p, P), mu10n = ld(mu, p, P, 1), mu01n = ld(mu, p, P, 0, 1);
+        const float mu11n = ld(mu, p, P, 1, 1);
         pml_stress_cell<true, OOP>(a, p, q, k, vx_0, vx_p1, vy_0, vy_p1, vz_m1, vz_0, mu00, mu00n, mu10, mu10n, mu01,
                               mu01n, mu11, gxc, gxe, gyc, gye);
         vx_0 = vx_p1; vy_0 = vy_p1; vz_m1 = vz_0;
-        mu00 = mu00n; mu10 = mu10n; mu01 = mu01n;
-        mu11 = mu[p + P + 1 + Y];
+        mu00 = mu00n; mu10 = mu10n; mu01 = mu01n; mu11 = mu11n;
     }
 }
 
@@ -983,29 +1066,49 @@ __device__ __forceinline__ void vel_pml_body(const StepArgs &a, const int4 tl)
     const float *__restrict__ Syz = a.f.Syz;
     const float *__restrict__ Sxz = a.f.Sxz;
     const float *__restrict__ rho = a.m.rho;
-    const float4 gxc = a.gxc[i - 1], gxe = a.gxe[i - 1];
-    const float4 gyc = a.gyc[j - 1], gye = a.gye[j - 1];
+    const float4 gxc = ldp(a.gxc + (i - 1)), gxe = ldp(a.gxe + (i - 1));
+    const float4 gyc = ldp(a.gyc + (j - 1)), gye = ldp(a.gye + (j - 1));
 
-    long long p = gidx(g, i, j, L.kb);
-    long long q = L.abase + (long long)L.kb * L.astride;
-    float szz_0 = Szz[p], syz_m1 = Syz[p - P], sxz_m1 = Sxz[p - P], rho0 = rho[p];
-    for (int k = L.kb; k <= L.ke; ++k, p += P, q += L.astride) {
-        const float szz_p1 = Szz[p + P], syz_0 = Syz[p], sxz_0 = Sxz[p], rho_kp = rho[p + P];
+    Loc p = L.p, q = L.q;
+    float szz_0 = ld(Szz, p), syz_m1 = ld(Syz, p, -P), sxz_m1 = ld(Sxz, p, -P), rho0 = ld(rho, p);
+    for (int k = L.kb; k <= L.ke; ++k, p.u += P, q.u += L.astride) {
+        fresh(p);
+        fresh(q);
+        const float szz_p1 = ld(Szz, p, P), syz_0 = ld(Syz, p), sxz_0 = ld(Sxz, p), rho_kp = ld(rho, p, P);
         pml_vel_cell<OOP>(a, p, q, k, szz_0, szz_p1, syz_m1, syz_0, sxz_m1, sxz_0, rho0, rho_kp, gxc, gxe, gyc, gye);
         szz_0 = szz_p1; syz_m1 = syz_0; sxz_m1 = sxz_0; rho0 = rho_kp;
     }
 }
 
-template <bool OOP>
-__global__ void __launch_bounds__(256) k_stress_pml(StepArgs a)
+// One launch of a phase: its first sideb blocks walk the side tiles, the rest
+// the interior columns.  The two kinds update disjoint cells from the other
+// phase's fields, so their order does not change any result.  Each kind is
+// dealt to the XCDs by itself (sideb is a multiple of 8), so every XCD gets an
+// eighth of both.
+template <int NM, bool NT, bool OOP>
+__global__ void __launch_bounds__(256) WAVES_NM k_stress(StepArgs a)
 {
-    stress_pml_body<OOP>(a, a.tiles[xcd_remap(blockIdx.x, gridDim.x)]);
+    if ((int)blockIdx.x < a.sideb) {
+        const int t = xcd_remap(blockIdx.x, a.sideb);
+        if (t < a.ntiles) stress_pml_body<OOP>(a, uni(a.tiles[t]));
+        return;
+    }
+    int bx, byy, bz;
+    plain_tile(a, bx, byy, bz);
+    stress_int_body<NM, NT, OOP>(a, bx, byy, bz);
 }
 
-template <bool OOP>
-__global__ void __launch_bounds__(256) k_vel_pml(StepArgs a)
+template <bool OOP, bool PF>
+__global__ void __launch_bounds__(256) WAVES4 k_vel(StepArgs a)
 {
-    vel_pml_body<OOP>(a, a.tiles[xcd_remap(blockIdx.x, gridDim.x)]);
+    if ((int)blockIdx.x < a.sideb) {
+        const int t = xcd_remap(blockIdx.x, a.sideb);
+        if (t < a.ntiles) vel_pml_body<OOP>(a, uni(a.tiles[t]));
+        return;
+    }
+    int bx, byy, bz;
+    plain_tile(a, bx, byy, bz);
+    vel_int_body<OOP, PF>(a, bx, byy, bz);
 }
 
 // batched side-column tiles: (i0 | width << 20 | xslab << 28, j0, k0 | k1 << 16, member)
@@ -1013,54 +1116,31 @@ __device__ static inline int4 unpack_bside(const int4 t) { return make_int4(t.x,
 
 __global__ void __launch_bounds__(256) k_stress_pml_b(const StepArgs *__restrict__ mem, const int4 *__restrict__ tiles)
 {
-    const int4 t = tiles[xcd_remap(blockIdx.x, gridDim.x)];
+    const int4 t = uni(tiles[xcd_remap(blockIdx.x, gridDim.x)]);
     stress_pml_body<false>(mem[t.w], unpack_bside(t));
 }
 
 __global__ void __launch_bounds__(256) k_vel_pml_b(const StepArgs *__restrict__ mem, const int4 *__restrict__ tiles)
 {
-    const int4 t = tiles[xcd_remap(blockIdx.x, gridDim.x)];
+    const int4 t = uni(tiles[xcd_remap(blockIdx.x, gridDim.x)]);
     vel_pml_body<false>(mem[t.w], unpack_bside(t));
 }
 
-// One launch per phase for the interior columns and the side columns
-// together (variant bit 5): a schedule lists interior tiles (bx, by, bz, -1)
-// and side tiles (i0 | width << 20 | xslab << 28, j0, k0 | k1 << 16, 0), the
-// x-slab tiles of a k chunk next to the interior tile rows they border, so
-// the 128-byte lines the two kinds share are fetched once through the L2 of
-// one XCD.  The two kinds update disjoint cells from the other phase's
-// fields, so their order does not change any result.
-template <int NM, bool NT>
-__global__ void __launch_bounds__(256) k_stress_all(StepArgs a, const int4 *__restrict__ sched)
-{
-    const int4 t = sched[xcd_remap(blockIdx.x, gridDim.x)];
-    if (t.w < 0) stress_int_body<NM, NT, false>(a, t.x, t.y, t.z);
-    else stress_pml_body<false>(a, make_int4(t.x, t.y, t.z & 0xFFFF, t.z >> 16));
-}
-
-template <bool PF>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PF ? 3 : 4))) k_vel_all(StepArgs a, const int4 *__restrict__ sched)
-{
-    const int4 t = sched[xcd_remap(blockIdx.x, gridDim.x)];
-    if (t.w < 0) vel_int_body<false, PF>(a, t.x, t.y, t.z);
-    else vel_pml_body<false>(a, make_int4(t.x, t.y, t.z & 0xFFFF, t.z >> 16));
-}
-
-// batched form of the merged launch: entries (m, bx, by, bz) are interior
+// one launch per phase for the tiles of both kinds: entries (m, bx, by, bz) are interior
 // tiles of member m, entries (-(m+1), i0 | width << 20 | xslab << 28, j0,
 // k0 | k1 << 16) its side tiles
 template <int NM, bool NT>
-__global__ void __launch_bounds__(256) k_stress_all_b(const StepArgs *__restrict__ mem, const int4 *__restrict__ tiles)
+__global__ void __launch_bounds__(256) WAVES_NM k_stress_all_b(const StepArgs *__restrict__ mem, const int4 *__restrict__ tiles)
 {
-    const int4 t = tiles[xcd_remap(blockIdx.x, gridDim.x)];
+    const int4 t = uni(tiles[xcd_remap(blockIdx.x, gridDim.x)]);
     if (t.x >= 0) stress_int_body<NM, NT, false>(mem[t.x], t.y, t.z, t.w);
     else stress_pml_body<false>(mem[-t.x - 1], make_int4(t.y, t.z, t.w & 0xFFFF, t.w >> 16));
 }
 
 template <bool PF>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PF ? 3 : 4))) k_vel_all_b(const StepArgs *__restrict__ mem, const int4 *__restrict__ tiles)
+__global__ void __launch_bounds__(256) WAVES4 k_vel_all_b(const StepArgs *__restrict__ mem, const int4 *__restrict__ tiles)
 {
-    const int4 t = tiles[xcd_remap(blockIdx.x, gridDim.x)];
+    const int4 t = uni(tiles[xcd_remap(blockIdx.x, gridDim.x)]);
     if (t.x >= 0) vel_int_body<false, PF>(mem[t.x], t.y, t.z, t.w);
     else vel_pml_body<false>(mem[-t.x - 1], make_int4(t.y, t.z, t.w & 0xFFFF, t.w >> 16));
 }
@@ -1097,6 +1177,7 @@ void fill_step_args(swpc_ctx *c, StepArgs &a, int mask)
     a.r20z = 1.0f / (float)c->desc.dz;
     a.tiles = (const int4 *)c->d_pml_tiles;
     a.ntiles = c->npml_tiles;
+    a.sideb = 0;
     a.has_pml = (c->desc.abc == SWPC_ABC_PML && c->npml > 0) ? 1 : 0;
     a.mask = mask;
     a.by = c->by;
@@ -1112,45 +1193,38 @@ void fill_step_args(swpc_ctx *c, StepArgs &a, int mask)
     a.nbz = c->nbz;
 }
 
-// side-column PML tiles of one phase (y slabs, x slabs)
-hipError_t launch_stress_side(swpc_ctx *c, hipStream_t s)
+// One launch of a phase over the side tiles (side), over the interior columns'
+// interior planes (mask & MASK_INT) and their bottom PML band (mask &
+// MASK_PML), or over all of them.  The batch's and the fused launch's tiles
+// use the same bodies.
+static bool phase_grid(swpc_ctx *c, StepArgs &a, int phase, bool side, int mask, dim3 &grid, dim3 &block)
 {
-    if (c->desc.abc != SWPC_ABC_PML || c->npml == 0 || c->npml_tiles <= 0) return hipSuccess;
-    StepArgs a;
-    step_args(c, a, MASK_PML);
-    if (c->fields_in[0]) hipLaunchKernelGGL(k_stress_pml<true>, dim3(c->npml_tiles), dim3(BX, a.by), 0, s ? s : c->stream, a);
-    else hipLaunchKernelGGL(k_stress_pml<false>, dim3(c->npml_tiles), dim3(BX, a.by), 0, s ? s : c->stream, a);
-    return hipGetLastError();
-}
-
-hipError_t launch_vel_side(swpc_ctx *c, hipStream_t s)
-{
-    if (c->desc.abc != SWPC_ABC_PML || c->npml == 0 || c->npml_tiles <= 0) return hipSuccess;
-    StepArgs a;
-    step_args(c, a, MASK_PML);
-    if (c->fields_in[0]) hipLaunchKernelGGL(k_vel_pml<true>, dim3(c->npml_tiles), dim3(BX, a.by), 0, s ? s : c->stream, a);
-    else hipLaunchKernelGGL(k_vel_pml<false>, dim3(c->npml_tiles), dim3(BX, a.by), 0, s ? s : c->stream, a);
-    return hipGetLastError();
-}
-
-// interior columns: interior planes (mask & 1) and their bottom PML band (mask & 2)
-hipError_t launch_stress_cols(swpc_ctx *c, int mask)
-{
-    StepArgs a;
     step_args(c, a, mask);
+    if (phase == 1) a.zc = c->d_zchunks + c->nbz + 1;
     if (mask == MASK_PML) {   // the bottom band alone: only the chunks that reach below the interior box
-        a.zc += c->zband[0];
-        a.nbz -= c->zband[0];
+        a.zc += c->zband[phase];
+        a.nbz -= c->zband[phase];
     }
-    if (c->g.nxk <= 0 || c->g.nyk <= 0 || !((mask & MASK_INT) || a.has_pml)) return hipSuccess;
-    dim3 block(a.bxw, a.byi), grid(a.nbx * a.nby * a.nbz);
+    const bool cols = c->g.nxk > 0 && c->g.nyk > 0 && ((mask & MASK_INT) || ((mask & MASK_PML) && a.has_pml));
+    a.sideb = side && a.has_pml ? (c->npml_tiles + 7) & ~7 : 0;
+    block = dim3(a.bxw, a.byi);
+    grid = dim3(a.sideb + (cols ? a.nbx * a.nby * a.nbz : 0));
+    return grid.x > 0;
+}
+
+hipError_t launch_stress(swpc_ctx *c, bool side, int mask, hipStream_t s)
+{
+    StepArgs a;
+    dim3 grid, block;
+    if (!phase_grid(c, a, 0, side, mask, grid, block)) return hipSuccess;
+    if (!s) s = c->stream;
     const bool nt = (c->variant & 1) != 0;
     const bool oop = c->fields_in[0] != nullptr;   // out of place: non-temporal streams as well
-#define SWPC_STRESS_CASE(NMV)                                                                       \
-    case NMV:                                                                                       \
-        if (oop) hipLaunchKernelGGL((k_stress_int<NMV, true, true>), grid, block, 0, c->stream, a); \
-        else if (nt) hipLaunchKernelGGL((k_stress_int<NMV, true, false>), grid, block, 0, c->stream, a); \
-        else hipLaunchKernelGGL((k_stress_int<NMV, false, false>), grid, block, 0, c->stream, a); \
+#define SWPC_STRESS_CASE(NMV)                                                                   \
+    case NMV:                                                                                   \
+        if (oop) hipLaunchKernelGGL((k_stress<NMV, true, true>), grid, block, 0, s, a);         \
+        else if (nt) hipLaunchKernelGGL((k_stress<NMV, true, false>), grid, block, 0, s, a);    \
+        else hipLaunchKernelGGL((k_stress<NMV, false, false>), grid, block, 0, s, a);           \
         break;
     switch (c->g.nm) {
         SWPC_STRESS_CASE(0) SWPC_STRESS_CASE(1) SWPC_STRESS_CASE(2) SWPC_STRESS_CASE(3) SWPC_STRESS_CASE(4)
@@ -1161,24 +1235,19 @@ hipError_t launch_stress_cols(swpc_ctx *c, int mask)
     return hipGetLastError();
 }
 
-hipError_t launch_vel_cols(swpc_ctx *c, int mask)
+hipError_t launch_vel(swpc_ctx *c, bool side, int mask, hipStream_t s)
 {
     StepArgs a;
-    step_args(c, a, mask);
-    a.zc = c->d_zchunks + c->nbz + 1;
-    if (mask == MASK_PML) {
-        a.zc += c->zband[1];
-        a.nbz -= c->zband[1];
-    }
-    if (c->g.nxk <= 0 || c->g.nyk <= 0 || !((mask & MASK_INT) || a.has_pml)) return hipSuccess;
-    const dim3 grid(a.nbx * a.nby * a.nbz), block(a.bxw, a.byi);
+    dim3 grid, block;
+    if (!phase_grid(c, a, 1, side, mask, grid, block)) return hipSuccess;
+    if (!s) s = c->stream;
     const bool pf = (c->variant & 8) != 0;
     if (c->fields_in[0]) {
-        if (pf) hipLaunchKernelGGL((k_vel_int<true, true>), grid, block, 0, c->stream, a);
-        else hipLaunchKernelGGL((k_vel_int<true, false>), grid, block, 0, c->stream, a);
+        if (pf) hipLaunchKernelGGL((k_vel<true, true>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((k_vel<true, false>), grid, block, 0, s, a);
     } else {
-        if (pf) hipLaunchKernelGGL((k_vel_int<false, true>), grid, block, 0, c->stream, a);
-        else hipLaunchKernelGGL((k_vel_int<false, false>), grid, block, 0, c->stream, a);
+        if (pf) hipLaunchKernelGGL((k_vel<false, true>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((k_vel<false, false>), grid, block, 0, s, a);
     }
     return hipGetLastError();
 }
@@ -1210,125 +1279,6 @@ hipError_t launch_fused(swpc_ctx *c)
 #undef SWPC_FUSED_CASE
     return hipGetLastError();
 }
-
-// schedules of the merged launches, one per phase (see k_stress_all)
-int build_schedule(swpc_ctx *c)
-{
-    for (int ph = 0; ph < 2; ++ph) {
-        if (c->d_sched[ph]) (void)hipFree(c->d_sched[ph]);
-        c->d_sched[ph] = nullptr;
-        c->nsched[ph] = 0;
-    }
-    const Grid &g = c->g;
-    if (c->desc.abc != SWPC_ABC_PML || c->npml == 0 || c->npml_tiles <= 0 || g.nxk <= 0 || g.nyk <= 0 ||
-        g.nz > 0x7FFF)
-        return SWPC_OK;
-    StepArgs a;
-    step_args(c, a, MASK_INT | MASK_PML);
-    std::vector<int4> side(c->npml_tiles);
-    std::vector<int> zc(2 * (c->nbz + 1));
-    if (hipMemcpy(side.data(), c->d_pml_tiles, side.size() * sizeof(int4), hipMemcpyDeviceToHost) != hipSuccess ||
-        hipMemcpy(zc.data(), c->d_zchunks, zc.size() * sizeof(int), hipMemcpyDeviceToHost) != hipSuccess)
-        return SWPC_EHIP;
-    for (int ph = 0; ph < 2; ++ph) {
-        const int *z = zc.data() + ph * (c->nbz + 1);
-        std::vector<int4> out;
-        std::vector<char> used(side.size(), 0);
-        for (int bz = 0; bz < a.nbz; ++bz) {
-            const int kb = z[bz], ke = z[bz + 1] - 1;
-            std::vector<int> low, high, xs;
-            for (size_t n = 0; n < side.size(); ++n) {
-                const int4 t = side[n];
-                if (used[n] || t.z < kb || t.z > ke) continue;
-                used[n] = 1;
-                const bool xslab = (t.x >> 28) & 1;
-                if (xslab) xs.push_back((int)n);
-                else if (t.y <= g.na) low.push_back((int)n);
-                else high.push_back((int)n);
-            }
-            auto emit_side = [&](int n) {
-                const int4 t = side[n];
-                out.push_back(make_int4(t.x, t.y, t.z | (t.w << 16), 0));
-            };
-            for (int n : low) emit_side(n);
-            size_t q = 0;
-            for (int by = 0; by < a.nby; ++by) {
-                const int j1 = g.jb + (by + 1) * a.byi - 1;
-                while (q < xs.size() && side[xs[q]].y <= j1) emit_side(xs[q++]);
-                for (int bx = 0; bx < a.nbx; ++bx) out.push_back(make_int4(bx, by, bz, -1));
-            }
-            for (; q < xs.size(); ++q) emit_side(xs[q]);
-            for (int n : high) emit_side(n);
-        }
-        for (size_t n = 0; n < side.size(); ++n)
-            if (!used[n]) {
-                const int4 t = side[n];
-                out.push_back(make_int4(t.x, t.y, t.z | (t.w << 16), 0));
-            }
-        if (hipMalloc((void **)&c->d_sched[ph], out.size() * sizeof(int4)) != hipSuccess) return SWPC_ENOMEM;
-        if (hipMemcpy(c->d_sched[ph], out.data(), out.size() * sizeof(int4), hipMemcpyHostToDevice) != hipSuccess)
-            return SWPC_EHIP;
-        c->nsched[ph] = (int)out.size();
-    }
-    return SWPC_OK;
-}
-
-// both kinds of columns of a phase in one launch, when the schedule exists
-// and the step is in place
-bool merged_launch_ready(const swpc_ctx *c)
-{
-    return (c->variant & 32) && c->d_sched[0] && c->d_sched[1] && !c->fields_in[0];
-}
-
-hipError_t launch_stress_all(swpc_ctx *c)
-{
-    StepArgs a;
-    step_args(c, a, MASK_INT | MASK_PML);
-    const dim3 grid(c->nsched[0]), block(a.bxw, a.byi);
-    const bool nt = (c->variant & 1) != 0;
-#define SWPC_ALL_CASE(NMV)                                                                                 \
-    case NMV:                                                                                              \
-        if (nt) hipLaunchKernelGGL((k_stress_all<NMV, true>), grid, block, 0, c->stream, a, c->d_sched[0]); \
-        else hipLaunchKernelGGL((k_stress_all<NMV, false>), grid, block, 0, c->stream, a, c->d_sched[0]);   \
-        break;
-    switch (c->g.nm) {
-        SWPC_ALL_CASE(0) SWPC_ALL_CASE(1) SWPC_ALL_CASE(2) SWPC_ALL_CASE(3) SWPC_ALL_CASE(4)
-        SWPC_ALL_CASE(5) SWPC_ALL_CASE(6) SWPC_ALL_CASE(7) SWPC_ALL_CASE(8)
-    default: return hipErrorInvalidValue;
-    }
-#undef SWPC_ALL_CASE
-    return hipGetLastError();
-}
-
-hipError_t launch_vel_all(swpc_ctx *c)
-{
-    StepArgs a;
-    step_args(c, a, MASK_INT | MASK_PML);
-    a.zc = c->d_zchunks + c->nbz + 1;
-    const dim3 grid(c->nsched[1]), block(a.bxw, a.byi);
-    if (c->variant & 8) hipLaunchKernelGGL((k_vel_all<true>), grid, block, 0, c->stream, a, c->d_sched[1]);
-    else hipLaunchKernelGGL((k_vel_all<false>), grid, block, 0, c->stream, a, c->d_sched[1]);
-    return hipGetLastError();
-}
-
-hipError_t launch_stress(swpc_ctx *c, int mask, hipStream_t pml_stream)
-{
-    hipError_t e;
-    if ((mask & MASK_PML) && (e = launch_stress_side(c, pml_stream)) != hipSuccess) return e;
-    return launch_stress_cols(c, mask);
-}
-
-hipError_t launch_vel(swpc_ctx *c, int mask, hipStream_t pml_stream)
-{
-    hipError_t e;
-    if ((mask & MASK_PML) && (e = launch_vel_side(c, pml_stream)) != hipSuccess) return e;
-    return launch_vel_cols(c, mask);
-}
-
-hipError_t launch_kernel_stress(swpc_ctx *c) { return launch_stress(c, MASK_INT, nullptr); }
-hipError_t launch_pml_stress(swpc_ctx *c) { return launch_stress(c, MASK_PML, nullptr); }
-hipError_t launch_kernel_vel(swpc_ctx *c) { return launch_vel(c, MASK_INT, nullptr); }
-hipError_t launch_pml_vel(swpc_ctx *c) { return launch_vel(c, MASK_PML, nullptr); }
 
 // ---------------------------------------------------------------------------
 // Cerjan sponge (m_absorb_c.f90:113-198).  Profiles carry the 3-cell halo:

@@ -196,8 +196,6 @@ struct swpc_ctx {
     int *d_fzc;        // chunks of the fused launch over the interior planes (nfz + 1 entries)
     int nfz;
     float *fields2[SWPC_NFIELD];  // second field set of the fused steps (variant bit 7)
-    int4 *d_sched[2];  // merged interior + side-column schedules of the two phases (variant bit 5)
-    int nsched[2];
     int variant;       // bit 0: non-temporal single-use streams in the interior stress kernel,
                        // bit 1: side-column PML kernels on a second stream,
                        // bit 2: 32-wide interior tiles, bit 3: velocity loads one plane ahead,
@@ -230,23 +228,12 @@ int64_t arena_granule_bytes(int device, const void *who);
 bool arena_free(void *p);
 
 // ---- launchers (stencil.hip / aux.hip) ----
-// mask: 1 interior, 2 PML, 3 both; the PML kernel goes to pml_stream when
-// given (it updates cells disjoint from the interior kernel's)
-hipError_t launch_stress(swpc_ctx *c, int mask, hipStream_t pml_stream);
-hipError_t launch_vel(swpc_ctx *c, int mask, hipStream_t pml_stream);
-hipError_t launch_stress_side(swpc_ctx *c, hipStream_t s);
-hipError_t launch_vel_side(swpc_ctx *c, hipStream_t s);
-hipError_t launch_stress_cols(swpc_ctx *c, int mask);
-int build_schedule(swpc_ctx *c);
-bool merged_launch_ready(const swpc_ctx *c);
-hipError_t launch_stress_all(swpc_ctx *c);
-hipError_t launch_vel_all(swpc_ctx *c);
-hipError_t launch_vel_cols(swpc_ctx *c, int mask);
+// one launch of the stress or velocity update: the side columns when `side`,
+// and of the interior columns mask 1 the interior planes, 2 the bottom PML
+// band, 3 both, 0 none; on the context's stream unless s is given
+hipError_t launch_stress(swpc_ctx *c, bool side, int mask, hipStream_t s = nullptr);
+hipError_t launch_vel(swpc_ctx *c, bool side, int mask, hipStream_t s = nullptr);
 hipError_t launch_fused(swpc_ctx *c);
-hipError_t launch_kernel_stress(swpc_ctx *c);
-hipError_t launch_kernel_vel(swpc_ctx *c);
-hipError_t launch_pml_stress(swpc_ctx *c);
-hipError_t launch_pml_vel(swpc_ctx *c);
 hipError_t launch_cerjan_stress(swpc_ctx *c, hipStream_t s = nullptr);
 hipError_t launch_cerjan_vel(swpc_ctx *c, hipStream_t s = nullptr);
 hipError_t launch_stressglut(swpc_ctx *c, int it, const int *d_it, hipStream_t s = nullptr);
