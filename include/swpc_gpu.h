@@ -402,24 +402,20 @@ int swpc_stripe_release(int device);
 int64_t swpc_stripe_free_bytes(int device, int region);
 
 /* Launch-shape tuning knobs.  kchunk: k-planes marched per thread block
-   (0 = keep, -1 = the default: 16, 32 when nm = 0, halved on small grids
-   until the interior launch has two blocks per CU); by: rows per 64-wide tile, 1, 2
-   or 4 (0 = keep; default 4); variant: kernel variant flags (-1 = keep;
-   default 9): bit 0 = non-temporal loads and
-   stores for the single-use streams of the stress update, bit 1 = side-column
-   PML kernels on a second stream alongside the interior ones, bit 2 =
-   interior tiles 32 cells wide with 2 by rows (narrow grids idle fewer
-   lanes), bit 3 = the interior velocity update loads plane k+1 while it
-   computes plane k, bit 4 = the adjoint copies its step records instead of
-   stepping out of place into them, bit 5 = the interior and side columns of
-   a phase in one launch, x-slab tiles next to the interior rows they
-   border, bit 7 = the velocity update of a step and the stress update of
-   the next in one interior launch (PML runs without body forces or the
-   reciprocity mode; the context then holds a second set of the 9 fields,
-   taken from the striped arena when it has room; kchunk sets the launch's
-   chunk depth), bit 8 = that launch with 8-row tiles instead of 4.  All
-   variants give bit-identical results.  Fails with SWPC_ENOMEM when the
-   second field set does not fit. */
+   (0 = keep, -1 = the default: 16, halved on small grids until a phase's
+   launch has 14 blocks per CU); by: rows per 64-wide tile, 1, 2 or 4 (0 =
+   keep; default 4); variant: kernel variant flags (-1 = keep; default 1):
+   bit 0 = non-temporal loads and stores for the single-use streams of the
+   stress update, bit 2 = interior tiles 32 cells wide with 2 by rows (narrow
+   grids idle fewer lanes), bit 4 = the adjoint copies its step records
+   instead of stepping out of place into them, bit 7 = the velocity update of
+   a step and the stress update of the next in one interior launch (PML runs
+   without body forces or the reciprocity mode; the context then holds a
+   second set of the 9 fields, taken from the striped arena when it has room;
+   kchunk sets the launch's chunk depth), bit 8 = that launch with 8-row
+   tiles instead of 4; other bits have no effect.  All variants give
+   bit-identical results.  Fails with SWPC_ENOMEM when the second field set
+   does not fit. */
 int swpc_set_tuning(swpc_ctx *ctx, int kchunk, int by, int variant);
 
 /* The HIP stream the context launches on (hipStream_t as void*), so a

@@ -226,25 +226,32 @@ extern "C" void *swpc_staging_buffer(swpc_ctx *ctx, int64_t *nfloats)
     return ctx ? (void *)ctx->staging : nullptr;
 }
 
-// The default k chunk of a context.  16 planes was fastest on 1024x1024x512
-// with NM = 3 among 8..128 (the stress and side-column launches favour short
-// chunks); an elastic update streams far fewer arrays, so each chunk's
-// priming loads weigh more and 32 planes is faster there (256x256x192,
-// NM = 0).  Small grids halve it until the interior launch has two blocks per
-// CU: 128^3 with a 20-cell PML took 0.233 ms/step in 352 blocks of 16 planes
-// and 0.161 in 704 blocks of 8.
+// The default k chunk of a context: 16 planes, halved until a phase's launch
+// has 14 blocks per CU (four are resident at a time), down to one plane.  A
+// march spares reading its z neighbours again, but its planes follow one
+// another, so a grid that gives the chip few blocks waits for them: us/step
+// at 16, 8, 4, 2, 1 planes per chunk
+//   48 x 44 x 40   (NM = 3):  -, 88, 41, 19, 17
+//   128^3          (NM = 3):  162 (8), 129 (4), 127 (2)
+//   168 x 152 x 120 (NM = 2): 183 (8), 173 (4), 175 (2)
+//   256 x 256 x 192 (NM = 0): 510 (16), 505 (8), 510 (4)
+//   384 x 384 x 256 (NM = 3): 2020 (16), 2010 (8), 2320 (4)
+// and 13.21, 13.29, 13.32 ms at 16, 12 and 24 on 768 x 768 x 448.
 static int default_kchunk(const swpc_ctx *c)
 {
     const Grid &g = c->g;
-    int kc = g.nm > 0 ? 16 : 32;
     int ncu = 0;
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess || ncu <= 0) {
         (void)hipGetLastError();
         ncu = 256;
     }
-    const long long tiles =
+    // tiles of one chunk: interior columns, and the side columns' y and x slabs
+    long long tiles =
         g.nxk > 0 && g.nyk > 0 ? (long long)((g.ie - 1) / 64 - (g.ib - 1) / 64 + 1) * ((g.nyk + 3) / 4) : 0;
-    while (tiles > 0 && kc > 4 && tiles * ((g.nz + kc - 1) / kc) < 2LL * ncu) kc /= 2;
+    if (c->desc.abc == SWPC_ABC_PML && g.na > 0 && g.na <= 64)
+        tiles += 2LL * ((g.na + 3) / 4) * ((g.nx + 63) / 64) + 2LL * ((g.nyk + 256 / g.na - 1) / (256 / g.na));
+    int kc = 16;
+    while (tiles > 0 && kc > 1 && tiles * ((g.nz + kc - 1) / kc) < 14LL * ncu) kc /= 2;
     return kc;
 }
 
@@ -263,11 +270,8 @@ extern "C" int swpc_create(const swpc_desc *d, swpc_ctx **out)
     c->desc = *d;
     c->device = d->device;
     c->by = 4;
-    c->variant = 1 | 8;
-    if (hipSetDevice(d->device) != hipSuccess || hipStreamCreate(&c->stream) != hipSuccess ||
-        hipStreamCreate(&c->stream2) != hipSuccess ||
-        hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming) != hipSuccess) {
+    c->variant = 1;
+    if (hipSetDevice(d->device) != hipSuccess || hipStreamCreate(&c->stream) != hipSuccess) {
         swpc_destroy(c);
         return SWPC_EHIP;
     }
@@ -442,10 +446,6 @@ extern "C" int swpc_destroy(swpc_ctx *c)
     dfree(c->d_green_ijk); dfree(c->d_green_acc); dfree(c->d_gf); dfree(c->d_green_stf);
     dfree(c->staging); dfree(c->d_vmax); dfree(c->d_it);
     free_snapshots(c);
-    if (c->stream2) (void)hipStreamSynchronize(c->stream2);
-    if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
-    if (c->ev_join) (void)hipEventDestroy(c->ev_join);
-    if (c->stream2) (void)hipStreamDestroy(c->stream2);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     // the arena this context reserved for itself goes with it (it stays, to
     // be released at process exit or by swpc_stripe_release, while another
@@ -1019,49 +1019,31 @@ extern "C" int swpc_wav_store(swpc_ctx *c, int it)
 // one step in the order of src/swpc_3d/main.f90:122-138.  d_it != nullptr:
 // kernels read the step number from device memory and the step ends by
 // advancing it (graph-capturable).  marks != nullptr: an event is recorded
-// before the step and after each of the SWPC_NTIMER launch slots (timing;
-// no second stream then).
+// before the step and after each of the SWPC_NTIMER launch slots.
 static hipError_t enqueue_step(swpc_ctx *c, int it, const int *d_it, hipEvent_t *marks = nullptr)
 {
     // kernel__update_stress and absorb__update_stress touch disjoint cells
-    // and only read V: with the PML the interior columns (interior planes and
-    // bottom band) are one launch and the side columns another; the Cerjan
-    // taper is a separate sweep over the updated stress, as in the reference.
+    // and only read V: with the PML they are one launch (two when timed, the
+    // side columns first); the Cerjan taper is a separate sweep over the
+    // updated stress, as in the reference.
     hipError_t e;
     const bool pml = c->desc.abc == SWPC_ABC_PML;
-    const bool fork = !marks && pml && (c->variant & 2) && c->npml_tiles > 0;
-    hipStream_t side = fork ? c->stream2 : c->stream;
     int slot = 0;
     auto mark = [&]() -> hipError_t { return marks ? hipEventRecord(marks[slot++], c->stream) : hipSuccess; };
-    auto fork_to_side = [&]() -> hipError_t {
-        if (!fork) return hipSuccess;
-        hipError_t r = hipEventRecord(c->ev_fork, c->stream);
-        return r != hipSuccess ? r : hipStreamWaitEvent(c->stream2, c->ev_fork, 0);
-    };
-    auto join_side = [&]() -> hipError_t {
-        if (!fork) return hipSuccess;
-        hipError_t r = hipEventRecord(c->ev_join, c->stream2);
-        return r != hipSuccess ? r : hipStreamWaitEvent(c->stream, c->ev_join, 0);
-    };
     if ((e = mark()) != hipSuccess) return e;
     if ((e = launch_green_store(c, it, d_it)) != hipSuccess) return e;
     if ((e = launch_wav_store(c, it, d_it)) != hipSuccess || (e = mark()) != hipSuccess) return e;
     if ((e = launch_snap(c, it, d_it)) != hipSuccess || (e = mark()) != hipSuccess) return e;
-    const bool merged = (c->variant & 32) && !fork;
-    if ((e = fork_to_side()) != hipSuccess) return e;
-    if (pml && !merged && (e = launch_stress(c, true, 0, side)) != hipSuccess) return e;
+    if (marks && (e = launch_stress(c, pml, 0)) != hipSuccess) return e;
     if ((e = mark()) != hipSuccess) return e;
-    if ((e = launch_stress(c, pml && merged, pml ? 3 : 1)) != hipSuccess) return e;
-    if ((e = join_side()) != hipSuccess) return e;
+    if ((e = launch_stress(c, pml && !marks, pml ? 3 : 1)) != hipSuccess) return e;
     if ((e = mark()) != hipSuccess) return e;
     if (!pml && (e = launch_cerjan_stress(c)) != hipSuccess) return e;
     if ((e = mark()) != hipSuccess) return e;
     if ((e = launch_stressglut(c, it, d_it)) != hipSuccess || (e = mark()) != hipSuccess) return e;
-    if ((e = fork_to_side()) != hipSuccess) return e;
-    if (pml && !merged && (e = launch_vel(c, true, 0, side)) != hipSuccess) return e;
+    if (marks && (e = launch_vel(c, pml, 0)) != hipSuccess) return e;
     if ((e = mark()) != hipSuccess) return e;
-    if ((e = launch_vel(c, pml && merged, pml ? 3 : 1)) != hipSuccess) return e;
-    if ((e = join_side()) != hipSuccess) return e;
+    if ((e = launch_vel(c, pml && !marks, pml ? 3 : 1)) != hipSuccess) return e;
     if ((e = mark()) != hipSuccess) return e;
     if (!pml && (e = launch_cerjan_vel(c)) != hipSuccess) return e;
     if ((e = mark()) != hipSuccess) return e;
@@ -1105,7 +1087,7 @@ static hipError_t enqueue_fused_steps(swpc_ctx *c, int it, int n, const int *d_i
     // step it up to its stress glut, as in enqueue_step
     if ((e = launch_green_store(c, step_no(0), d_it)) != hipSuccess ||
         (e = launch_wav_store(c, step_no(0), d_it)) != hipSuccess || (e = launch_snap(c, step_no(0), d_it)) != hipSuccess ||
-        (e = launch_stress(c, true, 0)) != hipSuccess || (e = launch_stress(c, false, 3)) != hipSuccess ||
+        (e = launch_stress(c, true, 3)) != hipSuccess ||
         (e = launch_stressglut(c, step_no(0), d_it)) != hipSuccess)
         return e;
     const int nf = (n - 1) & ~1;
@@ -1114,12 +1096,12 @@ static hipError_t enqueue_fused_steps(swpc_ctx *c, int it, int n, const int *d_i
         float *const *nxt = (s & 1) ? A : B;
         // step it+s: velocities of the side columns and the bottom band (2: band only)
         view(nxt, cur, cur);
-        if ((e = launch_vel(c, true, 0)) != hipSuccess || (e = launch_vel(c, false, 2)) != hipSuccess) break;
+        if ((e = launch_vel(c, true, 2)) != hipSuccess) break;
         // interior: velocities of step it+s and stresses of step it+s+1
         view(nxt, nxt, cur);
         if ((e = launch_fused(c)) != hipSuccess) break;
         // step it+s+1: stresses of the side columns and the bottom band
-        if ((e = launch_stress(c, true, 0)) != hipSuccess || (e = launch_stress(c, false, 2)) != hipSuccess) break;
+        if ((e = launch_stress(c, true, 2)) != hipSuccess) break;
         if (d_it && (e = launch_step_advance(c)) != hipSuccess) break;
         view(nxt, cur, nullptr);
         if ((e = launch_wav_store(c, step_no(s + 1), d_it)) != hipSuccess ||
@@ -1131,7 +1113,7 @@ static hipError_t enqueue_fused_steps(swpc_ctx *c, int it, int n, const int *d_i
     view(A, A, nullptr);
     if (e != hipSuccess) return e;
     // step it+nf from its velocity update on, in place
-    if ((e = launch_vel(c, true, 0)) != hipSuccess || (e = launch_vel(c, false, 3)) != hipSuccess ||
+    if ((e = launch_vel(c, true, 3)) != hipSuccess ||
         (e = launch_bodyforce(c, step_no(nf), d_it)) != hipSuccess ||
         (e = launch_green_source(c, step_no(nf), d_it)) != hipSuccess || (d_it && (e = launch_step_advance(c)) != hipSuccess))
         return e;

@@ -593,51 +593,10 @@ __global__ void __launch_bounds__(256) WAVES_NM k_stress_int_b(const StepArgs *_
     stress_int_body<NM, NT, false>(mem[t.x], t.y, t.z, t.w);
 }
 
-// Every load of one plane (d elements on from p) of the interior velocity update: the z-queue
-// entries the plane adds, the x/y neighbours, the buoyancy densities and the
-// old velocities.  Loading the next plane's set before computing this one's
-// keeps two planes of loads in flight per wave.
-struct VelLoads {
-    float sxz_p1, syz_p1, szz_p2, rho_kp;
-    float sxx_im1, sxx_0, sxx_ip1, sxx_ip2;
-    float sxy_0, sxy_jm2, sxy_jm1, sxy_jp1, sxy_im2, sxy_im1, sxy_ip1;
-    float syy_jm1, syy_0, syy_jp1, syy_jp2;
-    float syz_jm2, syz_jm1, syz_jp1;
-    float sxz_im2, sxz_im1, sxz_ip1;
-    float rho_ip, rho_jp;
-    float vx, vy, vz;
-};
-
-template <bool OOP>
-__device__ __forceinline__ void vel_loads(const StepArgs &a, Loc p, VelLoads &L, long long d)
-{
-    fresh(p);
-    const long long P = a.g.plane;
-    const int Y = a.g.pitch;
-    const float *__restrict__ Sxx = a.f.Sxx;
-    const float *__restrict__ Syy = a.f.Syy;
-    const float *__restrict__ Szz = a.f.Szz;
-    const float *__restrict__ Syz = a.f.Syz;
-    const float *__restrict__ Sxz = a.f.Sxz;
-    const float *__restrict__ Sxy = a.f.Sxy;
-    const float *__restrict__ rho = a.m.rho;
-    L.sxz_p1 = ld(Sxz, p, d + P); L.syz_p1 = ld(Syz, p, d + P); L.szz_p2 = ld(Szz, p, d + 2 * P); L.rho_kp = ld(rho, p, d + P);
-    L.sxx_im1 = ld(Sxx, p, d, -1); L.sxx_0 = ld(Sxx, p, d); L.sxx_ip1 = ld(Sxx, p, d, 1); L.sxx_ip2 = ld(Sxx, p, d, 2);
-    L.sxy_0 = ld(Sxy, p, d);
-    L.sxy_jm2 = ld(Sxy, p, d, 0, -2); L.sxy_jm1 = ld(Sxy, p, d, 0, -1); L.sxy_jp1 = ld(Sxy, p, d, 0, 1);
-    L.sxy_im2 = ld(Sxy, p, d, -2); L.sxy_im1 = ld(Sxy, p, d, -1); L.sxy_ip1 = ld(Sxy, p, d, 1);
-    L.syy_jm1 = ld(Syy, p, d, 0, -1); L.syy_0 = ld(Syy, p, d); L.syy_jp1 = ld(Syy, p, d, 0, 1); L.syy_jp2 = ld(Syy, p, d, 0, 2);
-    L.syz_jm2 = ld(Syz, p, d, 0, -2); L.syz_jm1 = ld(Syz, p, d, 0, -1); L.syz_jp1 = ld(Syz, p, d, 0, 1);
-    L.sxz_im2 = ld(Sxz, p, d, -2); L.sxz_im1 = ld(Sxz, p, d, -1); L.sxz_ip1 = ld(Sxz, p, d, 1);
-    L.rho_ip = ld(rho, p, d, 1); L.rho_jp = ld(rho, p, d, 0, 1);
-    L.vx = ld<true>(OOP ? a.fin.Vx : a.f.Vx, p, d);
-    L.vy = ld<true>(OOP ? a.fin.Vy : a.f.Vy, p, d);
-    L.vz = ld<true>(OOP ? a.fin.Vz : a.f.Vz, p, d);
-}
-
 // kernel__update_vel, m_kernel.f90:75-140, then the bottom PML band.
-// PF: the interior loop loads plane k+1 while it computes plane k.
-template <bool OOP, bool PF>
+// (Loading plane k+1 while computing plane k gained 1 % at three waves per
+// SIMD and nothing at four.)
+template <bool OOP>
 __device__ __forceinline__ void vel_int_body(const StepArgs &a, int bx, int byy, int bz)
 {
     const Grid &g = a.g;
@@ -672,48 +631,7 @@ __device__ __forceinline__ void vel_int_body(const StepArgs &a, int bx, int byy,
     float szz_m1 = ld(Szz, p, -P), szz_0 = ld(Szz, p), szz_p1 = ld(Szz, p, P);
     float rho0 = ld(rho, p);
 
-    if (PF && ka1 >= k0) {
-        const long long c2 = g2idx(g, i, j);
-        const int kft = ldv<false>(a.m.kfs_top + c2), kfb = ldv<false>(a.m.kfs_bot + c2);
-        const int kot = ldv<false>(a.m.kob_top + c2), kobb = ldv<false>(a.m.kob_bot + c2);
-        const Coefs cf(a);
-        VelLoads L;
-        vel_loads<OOP>(a, p, L, 0);
-        for (int k = k0; k <= ka1; ++k, p.u += P) {
-            fresh(p);
-            // plane k+1 <= nz + 1: its loads stay within the -2..nz+3 halo
-            VelLoads N;
-            if (k < ka1) vel_loads<OOP>(a, p, N, P);
-
-            const bool in = in_band(k, kft, kfb, kot, kobb);
-            const float re40x = cf.at(in, 0);
-            const float re41x = cf.at(in, 1);
-            const float re40y = cf.at(in, 2);
-            const float re41y = cf.at(in, 3);
-            const float re40z = cf.at(in, 4);
-            const float re41z = cf.at(in, 5);
-
-            const float d3Sx3 = (L.sxx_ip1 - L.sxx_0) * re40x - (L.sxx_ip2 - L.sxx_im1) * re41x
-                              + (L.sxy_0 - L.sxy_jm1) * re40y - (L.sxy_jp1 - L.sxy_jm2) * re41y
-                              + (sxz_0 - sxz_m1) * re40z - (L.sxz_p1 - sxz_m2) * re41z;
-            const float d3Sy3 = (L.sxy_0 - L.sxy_im1) * re40x - (L.sxy_ip1 - L.sxy_im2) * re41x
-                              + (L.syy_jp1 - L.syy_0) * re40y - (L.syy_jp2 - L.syy_jm1) * re41y
-                              + (syz_0 - syz_m1) * re40z - (L.syz_p1 - syz_m2) * re41z;
-            const float d3Sz3 = (sxz_0 - L.sxz_im1) * re40x - (L.sxz_ip1 - L.sxz_im2) * re41x
-                              + (syz_0 - L.syz_jm1) * re40y - (L.syz_jp1 - L.syz_jm2) * re41y
-                              + (szz_p1 - szz_0) * re40z - (L.szz_p2 - szz_m1) * re41z;
-
-            st<true>(Vx, p, L.vx + 2.0f / (rho0 + L.rho_ip) * d3Sx3 * dt);
-            st<true>(Vy, p, L.vy + 2.0f / (rho0 + L.rho_jp) * d3Sy3 * dt);
-            st<true>(Vz, p, L.vz + 2.0f / (rho0 + L.rho_kp) * d3Sz3 * dt);
-
-            sxz_m2 = sxz_m1; sxz_m1 = sxz_0; sxz_0 = L.sxz_p1;
-            syz_m2 = syz_m1; syz_m1 = syz_0; syz_0 = L.syz_p1;
-            szz_m1 = szz_0; szz_0 = szz_p1; szz_p1 = L.szz_p2;
-            rho0 = L.rho_kp;
-            L = N;
-        }
-    } else if (ka1 >= k0) {
+    if (ka1 >= k0) {
         const long long c2 = g2idx(g, i, j);
         const int kft = ldv<false>(a.m.kfs_top + c2), kfb = ldv<false>(a.m.kfs_bot + c2);
         const int kot = ldv<false>(a.m.kob_top + c2), kobb = ldv<false>(a.m.kob_bot + c2);
@@ -783,11 +701,10 @@ __device__ __forceinline__ void vel_int_body(const StepArgs &a, int bx, int byy,
     }
 }
 
-template <bool PF>
 __global__ void __launch_bounds__(256) WAVES4 k_vel_int_b(const StepArgs *__restrict__ mem, const int4 *__restrict__ tiles)
 {
     const int4 t = uni(tiles[xcd_remap(blockIdx.x, gridDim.x)]);
-    vel_int_body<false, PF>(mem[t.x], t.y, t.z, t.w);
+    vel_int_body<false>(mem[t.x], t.y, t.z, t.w);
 }
 
 // ---------------------------------------------------------------------------
@@ -1084,7 +1001,9 @@ __device__ __forceinline__ void vel_pml_body(const StepArgs &a, const int4 tl)
 // the interior columns.  The two kinds update disjoint cells from the other
 // phase's fields, so their order does not change any result.  Each kind is
 // dealt to the XCDs by itself (sideb is a multiple of 8), so every XCD gets an
-// eighth of both.
+// eighth of both.  Launched one after the other, each kind's last blocks leave
+// CUs idle: 128^3 took 140 us/step in two launches per phase and 127 in one,
+// elastic 256 x 256 x 192 525 and 505, 768 x 768 x 448 13.26 and 13.21 ms.
 template <int NM, bool NT, bool OOP>
 __global__ void __launch_bounds__(256) WAVES_NM k_stress(StepArgs a)
 {
@@ -1098,7 +1017,7 @@ __global__ void __launch_bounds__(256) WAVES_NM k_stress(StepArgs a)
     stress_int_body<NM, NT, OOP>(a, bx, byy, bz);
 }
 
-template <bool OOP, bool PF>
+template <bool OOP>
 __global__ void __launch_bounds__(256) WAVES4 k_vel(StepArgs a)
 {
     if ((int)blockIdx.x < a.sideb) {
@@ -1108,7 +1027,7 @@ __global__ void __launch_bounds__(256) WAVES4 k_vel(StepArgs a)
     }
     int bx, byy, bz;
     plain_tile(a, bx, byy, bz);
-    vel_int_body<OOP, PF>(a, bx, byy, bz);
+    vel_int_body<OOP>(a, bx, byy, bz);
 }
 
 // batched side-column tiles: (i0 | width << 20 | xslab << 28, j0, k0 | k1 << 16, member)
@@ -1137,11 +1056,10 @@ __global__ void __launch_bounds__(256) WAVES_NM k_stress_all_b(const StepArgs *_
     else stress_pml_body<false>(mem[-t.x - 1], make_int4(t.y, t.z, t.w & 0xFFFF, t.w >> 16));
 }
 
-template <bool PF>
 __global__ void __launch_bounds__(256) WAVES4 k_vel_all_b(const StepArgs *__restrict__ mem, const int4 *__restrict__ tiles)
 {
     const int4 t = uni(tiles[xcd_remap(blockIdx.x, gridDim.x)]);
-    if (t.x >= 0) vel_int_body<false, PF>(mem[t.x], t.y, t.z, t.w);
+    if (t.x >= 0) vel_int_body<false>(mem[t.x], t.y, t.z, t.w);
     else vel_pml_body<false>(mem[-t.x - 1], make_int4(t.y, t.z, t.w & 0xFFFF, t.w >> 16));
 }
 
@@ -1212,19 +1130,18 @@ static bool phase_grid(swpc_ctx *c, StepArgs &a, int phase, bool side, int mask,
     return grid.x > 0;
 }
 
-hipError_t launch_stress(swpc_ctx *c, bool side, int mask, hipStream_t s)
+hipError_t launch_stress(swpc_ctx *c, bool side, int mask)
 {
     StepArgs a;
     dim3 grid, block;
     if (!phase_grid(c, a, 0, side, mask, grid, block)) return hipSuccess;
-    if (!s) s = c->stream;
     const bool nt = (c->variant & 1) != 0;
     const bool oop = c->fields_in[0] != nullptr;   // out of place: non-temporal streams as well
 #define SWPC_STRESS_CASE(NMV)                                                                   \
     case NMV:                                                                                   \
-        if (oop) hipLaunchKernelGGL((k_stress<NMV, true, true>), grid, block, 0, s, a);         \
-        else if (nt) hipLaunchKernelGGL((k_stress<NMV, true, false>), grid, block, 0, s, a);    \
-        else hipLaunchKernelGGL((k_stress<NMV, false, false>), grid, block, 0, s, a);           \
+        if (oop) hipLaunchKernelGGL((k_stress<NMV, true, true>), grid, block, 0, c->stream, a);       \
+        else if (nt) hipLaunchKernelGGL((k_stress<NMV, true, false>), grid, block, 0, c->stream, a);  \
+        else hipLaunchKernelGGL((k_stress<NMV, false, false>), grid, block, 0, c->stream, a);         \
         break;
     switch (c->g.nm) {
         SWPC_STRESS_CASE(0) SWPC_STRESS_CASE(1) SWPC_STRESS_CASE(2) SWPC_STRESS_CASE(3) SWPC_STRESS_CASE(4)
@@ -1235,20 +1152,13 @@ hipError_t launch_stress(swpc_ctx *c, bool side, int mask, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t launch_vel(swpc_ctx *c, bool side, int mask, hipStream_t s)
+hipError_t launch_vel(swpc_ctx *c, bool side, int mask)
 {
     StepArgs a;
     dim3 grid, block;
     if (!phase_grid(c, a, 1, side, mask, grid, block)) return hipSuccess;
-    if (!s) s = c->stream;
-    const bool pf = (c->variant & 8) != 0;
-    if (c->fields_in[0]) {
-        if (pf) hipLaunchKernelGGL((k_vel<true, true>), grid, block, 0, s, a);
-        else hipLaunchKernelGGL((k_vel<true, false>), grid, block, 0, s, a);
-    } else {
-        if (pf) hipLaunchKernelGGL((k_vel<false, true>), grid, block, 0, s, a);
-        else hipLaunchKernelGGL((k_vel<false, false>), grid, block, 0, s, a);
-    }
+    if (c->fields_in[0]) hipLaunchKernelGGL(k_vel<true>, grid, block, 0, c->stream, a);
+    else hipLaunchKernelGGL(k_vel<false>, grid, block, 0, c->stream, a);
     return hipGetLastError();
 }
 
@@ -1433,8 +1343,7 @@ hipError_t launch_batch_phase_all(int phase, int nm, int variant, int by, int bx
     const dim3 block(bxw, by * (BX / bxw));
     const bool nt = (variant & 1) != 0;
     if (phase == 1) {
-        if (variant & 8) hipLaunchKernelGGL(k_vel_all_b<true>, dim3(nall), block, 0, s, mem, d_all);
-        else hipLaunchKernelGGL(k_vel_all_b<false>, dim3(nall), block, 0, s, mem, d_all);
+        hipLaunchKernelGGL(k_vel_all_b, dim3(nall), block, 0, s, mem, d_all);
         return hipGetLastError();
     }
 #define SWPC_BALL_CASE(NMV)                                                                           \
@@ -1465,8 +1374,7 @@ hipError_t launch_batch_phase(int phase, int nm, int variant, int by, int bxw, c
     }
     if (ncols <= 0) return hipSuccess;
     if (phase == 1) {
-        if (variant & 8) hipLaunchKernelGGL(k_vel_int_b<true>, dim3(ncols), block, 0, s, mem, d_cols);
-        else hipLaunchKernelGGL(k_vel_int_b<false>, dim3(ncols), block, 0, s, mem, d_cols);
+        hipLaunchKernelGGL(k_vel_int_b, dim3(ncols), block, 0, s, mem, d_cols);
         return hipGetLastError();
     }
 #define SWPC_BSTRESS_CASE(NMV)                                                                      \

@@ -112,8 +112,6 @@ struct swpc_ctx {
     Grid g;
     int device;
     hipStream_t stream;
-    hipStream_t stream2;            // PML kernels alongside the interior ones
-    hipEvent_t ev_fork, ev_join;
     char err[512];
 
     float *fields[SWPC_NFIELD];
@@ -197,11 +195,9 @@ struct swpc_ctx {
     int nfz;
     float *fields2[SWPC_NFIELD];  // second field set of the fused steps (variant bit 7)
     int variant;       // bit 0: non-temporal single-use streams in the interior stress kernel,
-                       // bit 1: side-column PML kernels on a second stream,
-                       // bit 2: 32-wide interior tiles, bit 3: velocity loads one plane ahead,
-                       // bit 4: adjoint records copied, bit 5: interior and side columns in one launch,
+                       // bit 2: 32-wide interior tiles, bit 4: adjoint records copied,
                        // bit 7: the velocity update fused to the next stress update (k_fused, two field
-                       // sets), bit 8: fused tiles of 8 rows instead of 4
+                       // sets), bit 8: fused tiles of 8 rows instead of 4; other bits have no effect
     long long bytes;
     int own_arena;     // the context reserved the device's striped arena itself (swpc_create)
     struct AdjWorkspace *adj_ws;  // adjoint state, gradient sums and checkpoints (adjoint.hip)
@@ -230,9 +226,9 @@ bool arena_free(void *p);
 // ---- launchers (stencil.hip / aux.hip) ----
 // one launch of the stress or velocity update: the side columns when `side`,
 // and of the interior columns mask 1 the interior planes, 2 the bottom PML
-// band, 3 both, 0 none; on the context's stream unless s is given
-hipError_t launch_stress(swpc_ctx *c, bool side, int mask, hipStream_t s = nullptr);
-hipError_t launch_vel(swpc_ctx *c, bool side, int mask, hipStream_t s = nullptr);
+// band, 3 both, 0 none
+hipError_t launch_stress(swpc_ctx *c, bool side, int mask);
+hipError_t launch_vel(swpc_ctx *c, bool side, int mask);
 hipError_t launch_fused(swpc_ctx *c);
 hipError_t launch_cerjan_stress(swpc_ctx *c, hipStream_t s = nullptr);
 hipError_t launch_cerjan_vel(swpc_ctx *c, hipStream_t s = nullptr);
