@@ -975,8 +975,7 @@ extern "C" int swpc_update_stress(swpc_ctx *c)
     if (c->desc.abc == SWPC_ABC_PML) {
         HIPCHK(c, launch_stress(c, true, 3));
     } else {
-        HIPCHK(c, launch_stress(c, false, 1));
-        HIPCHK(c, launch_cerjan_stress(c));
+        HIPCHK(c, launch_stress(c, false, 5));
     }
     return SWPC_OK;
 }
@@ -989,8 +988,7 @@ extern "C" int swpc_update_vel(swpc_ctx *c)
     if (c->desc.abc == SWPC_ABC_PML) {
         HIPCHK(c, launch_vel(c, true, 3));
     } else {
-        HIPCHK(c, launch_vel(c, false, 1));
-        HIPCHK(c, launch_cerjan_vel(c));
+        HIPCHK(c, launch_vel(c, false, 5));
     }
     return SWPC_OK;
 }
@@ -1024,8 +1022,8 @@ static hipError_t enqueue_step(swpc_ctx *c, int it, const int *d_it, hipEvent_t 
 {
     // kernel__update_stress and absorb__update_stress touch disjoint cells
     // and only read V: with the PML they are one launch (two when timed, the
-    // side columns first); the Cerjan taper is a separate sweep over the
-    // updated stress, as in the reference.
+    // side columns first).  The Cerjan taper is part of the update's launch (a
+    // sweep of its own when timed).
     hipError_t e;
     const bool pml = c->desc.abc == SWPC_ABC_PML;
     int slot = 0;
@@ -1036,16 +1034,16 @@ static hipError_t enqueue_step(swpc_ctx *c, int it, const int *d_it, hipEvent_t 
     if ((e = launch_snap(c, it, d_it)) != hipSuccess || (e = mark()) != hipSuccess) return e;
     if (marks && (e = launch_stress(c, pml, 0)) != hipSuccess) return e;
     if ((e = mark()) != hipSuccess) return e;
-    if ((e = launch_stress(c, pml && !marks, pml ? 3 : 1)) != hipSuccess) return e;
+    if ((e = launch_stress(c, pml && !marks, pml ? 3 : marks ? 1 : 5)) != hipSuccess) return e;
     if ((e = mark()) != hipSuccess) return e;
-    if (!pml && (e = launch_cerjan_stress(c)) != hipSuccess) return e;
+    if (!pml && marks && (e = launch_cerjan_stress(c)) != hipSuccess) return e;
     if ((e = mark()) != hipSuccess) return e;
     if ((e = launch_stressglut(c, it, d_it)) != hipSuccess || (e = mark()) != hipSuccess) return e;
     if (marks && (e = launch_vel(c, pml, 0)) != hipSuccess) return e;
     if ((e = mark()) != hipSuccess) return e;
-    if ((e = launch_vel(c, pml && !marks, pml ? 3 : 1)) != hipSuccess) return e;
+    if ((e = launch_vel(c, pml && !marks, pml ? 3 : marks ? 1 : 5)) != hipSuccess) return e;
     if ((e = mark()) != hipSuccess) return e;
-    if (!pml && (e = launch_cerjan_vel(c)) != hipSuccess) return e;
+    if (!pml && marks && (e = launch_cerjan_vel(c)) != hipSuccess) return e;
     if ((e = mark()) != hipSuccess) return e;
     if ((e = launch_bodyforce(c, it, d_it)) != hipSuccess) return e;
     if ((e = launch_green_source(c, it, d_it)) != hipSuccess || (e = mark()) != hipSuccess) return e;

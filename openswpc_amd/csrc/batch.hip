@@ -5,9 +5,8 @@
 // members: the launch walks a tile table whose entries carry the member
 // index, and each member's launch arguments sit in HBM.  Uneven grids pack
 // into one grid of blocks with no per-member launch tail.  Receivers,
-// sources, sections, Green's-function stores and Cerjan sponges are
-// member-tagged launches too: one per kind and step for every member that
-// has them.
+// sources, sections and Green's-function stores are member-tagged launches
+// too: one per kind and step for every member that has them.
 // Steps replay from a HIP graph of `block` steps driven by one device step
 // counter shared by all members.
 //
@@ -35,6 +34,7 @@ struct swpc_batch {
     int device;
     hipStream_t stream;
     int nm, by;
+    bool tp;                       // Cerjan members: the update applies their taper
     int packing;                   // tile order of the tables (see above)
     void *d_args[2];               // StepArgs of every member: stress, velocity
     int4 *d_cols, *d_side;
@@ -45,9 +45,6 @@ struct swpc_batch {
     int naux[BATCH_AUX_N], maxaux[BATCH_AUX_N];
     void *d_snap;                  // section arguments of the members with sections
     int nsnap, maxsnap;
-    void *d_cerj[2];               // sponge arguments (stress, velocity phase) of the Cerjan members
-    int *d_cerj_blk0[2];           // their first blocks in the flat sponge launch (ncerj + 1 entries)
-    int ncerj, ncerj_blocks[2];
     int *d_it;
     hipGraphExec_t graph;
     int graph_block;
@@ -103,14 +100,6 @@ static void free_tables(swpc_batch *b)
     }
     bfree(b->d_snap);
     b->nsnap = b->maxsnap = 0;
-    for (int ph = 0; ph < 2; ++ph) {
-        bfree(b->d_cerj[ph]);
-        p = b->d_cerj_blk0[ph];
-        bfree(p);
-        b->d_cerj_blk0[ph] = nullptr;
-        b->ncerj_blocks[ph] = 0;
-    }
-    b->ncerj = 0;
 }
 
 // interior tile width of the members (variant bit 2: 32 cells, else 64)
@@ -258,31 +247,6 @@ static int build_tables(swpc_batch *b)
         b->nsnap = cnt;
         b->maxsnap = mx;
     }
-    // Cerjan sponges: one flat launch per phase over the sponge members' blocks
-    for (int ph = 0; ph < 2; ++ph) {
-        const size_t sz = batch_cerjan_size();
-        std::vector<char> buf(sz * n);
-        std::vector<int> blk0(1, 0);
-        long long total = 0;
-        int cnt = 0;
-        for (int m = 0; m < n; ++m) {
-            const int t = batch_cerjan_fill(b->mem[m], ph, buf.data() + sz * cnt);
-            if (t > 0) {
-                ++cnt;
-                total += t;
-                if (total > 0x7FFFFFFFLL) return bfail(b, SWPC_EINVAL, "sponge members too large for one launch");
-                blk0.push_back((int)total);
-            }
-        }
-        if (cnt > 0) {
-            BCHK(b, hipMalloc(&b->d_cerj[ph], sz * cnt));
-            BCHK(b, hipMemcpy(b->d_cerj[ph], buf.data(), sz * cnt, hipMemcpyHostToDevice));
-            BCHK(b, hipMalloc((void **)&b->d_cerj_blk0[ph], blk0.size() * sizeof(int)));
-            BCHK(b, hipMemcpy(b->d_cerj_blk0[ph], blk0.data(), blk0.size() * sizeof(int), hipMemcpyHostToDevice));
-        }
-        b->ncerj = cnt;
-        b->ncerj_blocks[ph] = (int)total;
-    }
     for (int m = 0; m < n; ++m) b->gen[m] = b->mem[m]->gen;
     return SWPC_OK;
 }
@@ -307,25 +271,20 @@ static hipError_t enqueue_batch_step(swpc_batch *b, int it, const int *d_it)
     if ((e = launch_batch_aux(BATCH_AUX_WAV, b->d_aux[BATCH_AUX_WAV], b->naux[BATCH_AUX_WAV],
                               b->maxaux[BATCH_AUX_WAV], it, d_it, s)) != hipSuccess)
         return e;
-    if (b->packing == 2) e = launch_batch_phase_all(0, b->nm, b->mem[0]->variant, b->by, batch_bxw(b), b->d_args[0],
+    if (b->packing == 2) e = launch_batch_phase_all(0, b->nm, b->mem[0]->variant, b->tp, b->by, batch_bxw(b), b->d_args[0],
                                                     b->d_all, b->nall, s);
-    else e = launch_batch_phase(0, b->nm, b->mem[0]->variant, b->by, batch_bxw(b), b->d_args[0], b->d_cols, b->ncols,
+    else e = launch_batch_phase(0, b->nm, b->mem[0]->variant, b->tp, b->by, batch_bxw(b), b->d_args[0], b->d_cols, b->ncols,
                                 b->d_side, b->nside, s);
     if (e != hipSuccess) return e;
-    if ((e = launch_batch_cerjan(0, b->d_cerj[0], b->d_cerj_blk0[0], b->ncerj, b->ncerj_blocks[0], s)) != hipSuccess)
-        return e;
-    // each member's sponge before its stress glut, as in its own step
     if ((e = launch_batch_aux(BATCH_AUX_GLUT, b->d_aux[BATCH_AUX_GLUT], b->naux[BATCH_AUX_GLUT],
                               b->maxaux[BATCH_AUX_GLUT], it, d_it, s)) != hipSuccess)
         return e;
-    if (b->packing == 2) e = launch_batch_phase_all(1, b->nm, b->mem[0]->variant, b->by, batch_bxw(b), b->d_args[1],
+    if (b->packing == 2) e = launch_batch_phase_all(1, b->nm, b->mem[0]->variant, b->tp, b->by, batch_bxw(b), b->d_args[1],
                                                     b->d_all, b->nall, s);
-    else e = launch_batch_phase(1, b->nm, b->mem[0]->variant, b->by, batch_bxw(b), b->d_args[1], b->d_cols, b->ncols,
+    else e = launch_batch_phase(1, b->nm, b->mem[0]->variant, b->tp, b->by, batch_bxw(b), b->d_args[1], b->d_cols, b->ncols,
                                 b->d_side, b->nside, s);
     if (e != hipSuccess) return e;
-    if ((e = launch_batch_cerjan(1, b->d_cerj[1], b->d_cerj_blk0[1], b->ncerj, b->ncerj_blocks[1], s)) != hipSuccess)
-        return e;
-    // sponge, body force, then the Green's-function source, per member as in its own step
+    // body force, then the Green's-function source, per member as in its own step
     if ((e = launch_batch_aux(BATCH_AUX_BODYFORCE, b->d_aux[BATCH_AUX_BODYFORCE], b->naux[BATCH_AUX_BODYFORCE],
                               b->maxaux[BATCH_AUX_BODYFORCE], it, d_it, s)) != hipSuccess)
         return e;
@@ -374,6 +333,7 @@ extern "C" int swpc_batch_create(swpc_ctx *const *members, int n, swpc_batch **o
     b->device = members[0]->desc.device;
     b->nm = members[0]->desc.nm;
     b->by = members[0]->by;
+    for (const swpc_ctx *c : b->mem) b->tp |= c->desc.abc == SWPC_ABC_CERJAN;
     int rc = SWPC_OK;
     if (hipSetDevice(b->device) != hipSuccess || hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess ||
         hipMalloc((void **)&b->d_it, sizeof(int)) != hipSuccess) {

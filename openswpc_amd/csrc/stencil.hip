@@ -14,13 +14,15 @@
 // evaluation order; the library is compiled with -ffp-contract=off so no FMA
 // changes the rounding.
 //
-// Cerjan tapers (m_absorb_c) are separate per-cell sweeps, as in the
-// reference.
+// A whole step's Cerjan taper (m_absorb_c) is applied by the update itself
+// before it stores; called routine by routine it is a sweep of its own, as in
+// the reference.
 #include "swpc_internal.h"
 
 #define BX 64
 #define MASK_INT 1
 #define MASK_PML 2
+#define MASK_TAPER 4  // the update applies the Cerjan taper to the values it stores
 
 
 // Four waves per SIMD: 128 registers, which every NM <= 4 form fits without a
@@ -182,6 +184,8 @@ struct StepArgs {
     int ntiles;
     int sideb;           // blocks of a launch that walk the side tiles (a multiple of 8, >= ntiles; 0: none)
     int has_pml, mask;
+    // Cerjan profiles at cell centres (c) and boundaries (b), halo of 3: entry of cell n is n + 2
+    const float *cgx_c, *cgx_b, *cgy_c, *cgy_b, *cgz_c, *cgz_b;
     // interior launch shape
     const int *zc;       // first plane of each k chunk (nbz + 1 entries, last = nz + 1)
     int bx0, nbx, nby, nbz, by;
@@ -206,6 +210,23 @@ struct Coefs {
         }
     }
     __device__ float at(bool in, int q) const { return in ? v[1][q] : v[0][q]; }
+};
+
+// Cerjan profile values of a column (m_absorb_c.f90:113-198).  Folded into the
+// update the taper costs no traffic; as sweeps of their own the two tapers
+// read and wrote all nine fields again (181 x 149 x 117: 163 us/step, 122
+// folded).  TP: the launch may hold such members; other launches leave the
+// test out, which cost PML runs 4-8 % on small grids.
+template <bool TP>
+struct Taper {
+    float xc, xb, yc, yb;
+
+    __device__ Taper(const StepArgs &a, int i, int j) : xc(1.0f), xb(1.0f), yc(1.0f), yb(1.0f)
+    {
+        if (!TP || !(a.mask & MASK_TAPER)) return;
+        xc = ldv<false>(a.cgx_c + (i + 2)); xb = ldv<false>(a.cgx_b + (i + 2));
+        yc = ldv<false>(a.cgy_c + (j + 2)); yb = ldv<false>(a.cgy_b + (j + 2));
+    }
 };
 
 // ---------------------------------------------------------------------------
@@ -386,9 +407,9 @@ struct VStencil {
 // r: memory-variable index, in: the cell is in the 2nd-order band, mu..: mu
 // at (i,j), (i+1,j), (i,j+1) on planes k and k+1 (n) and at (i+1,j+1) on
 // plane k.  OOP: the old stresses are read from a.fin.
-template <int NM, bool NT, bool OOP>
-__device__ __forceinline__ void stress_cell(const StepArgs &a, const Loc &p, const Loc &r, bool in, const Coefs &cf,
-                                            const VStencil &v,
+template <int NM, bool NT, bool OOP, bool TP>
+__device__ __forceinline__ void stress_cell(const StepArgs &a, const Loc &p, const Loc &r, int k, bool in, const Coefs &cf,
+                                            const Taper<TP> &tp, const VStencil &v,
                                             float mu00, float mu00n, float mu10, float mu10n, float mu01, float mu01n,
                                             float mu11)
 {
@@ -412,8 +433,8 @@ __device__ __forceinline__ void stress_cell(const StepArgs &a, const Loc &p, con
     const float lam1 = ld<NT>(a.m.lam, p);
     const float taup1 = ld<NT>(a.m.taup, p);
     const float taus1 = ld<NT>(a.m.taus, p);
-    const float sxx = ld<NT>(SxxI, p), syy = ld<NT>(SyyI, p), szz = ld<NT>(SzzI, p);
-    const float syz = ld<NT>(SyzI, p), sxz = ld<NT>(SxzI, p), sxy = ld<NT>(SxyI, p);
+    float sxx = ld<NT>(SxxI, p), syy = ld<NT>(SyyI, p), szz = ld<NT>(SzzI, p);
+    float syz = ld<NT>(SyzI, p), sxz = ld<NT>(SxzI, p), sxy = ld<NT>(SxyI, p);
     RCell<NM> R;
     R.template load<NT>(a.R, rn, r);
 
@@ -452,9 +473,9 @@ __device__ __forceinline__ void stress_cell(const StepArgs &a, const Loc &p, con
     }
     const float taup_plus1 = 1.0f + taup1 * (1.0f + d2);
     const float taus_plus1 = 1.0f + taus1 * (1.0f + d2);
-    st<NT>(Sxx, p, sxx + (lam2mu * taup_plus1 * d3v3 - mu2 * taus_plus1 * dyVy_dzVz + Rxx_n) * dt);
-    st<NT>(Syy, p, syy + (lam2mu * taup_plus1 * d3v3 - mu2 * taus_plus1 * dxVx_dzVz + Ryy_n) * dt);
-    st<NT>(Szz, p, szz + (lam2mu * taup_plus1 * d3v3 - mu2 * taus_plus1 * dxVx_dyVy + Rzz_n) * dt);
+    sxx = sxx + (lam2mu * taup_plus1 * d3v3 - mu2 * taus_plus1 * dyVy_dzVz + Rxx_n) * dt;
+    syy = syy + (lam2mu * taup_plus1 * d3v3 - mu2 * taus_plus1 * dxVx_dzVz + Ryy_n) * dt;
+    szz = szz + (lam2mu * taup_plus1 * d3v3 - mu2 * taus_plus1 * dxVx_dyVy + Rzz_n) * dt;
 
     // shear components, m_kernel.f90:285-333
     const float dxVy_dyVx = (v.vy_ip1 - v.vy_0) * re40x - (v.vy_ip2 - v.vy_im1) * re41x
@@ -483,9 +504,25 @@ __device__ __forceinline__ void stress_cell(const StepArgs &a, const Loc &p, con
         Rxy_n = Rxy_n + d1 * nxy;
     }
     R.template store<NT>(a.R, rn, r);
-    st<NT>(Syz, p, syz + (muyz * taus_plus1 * dyVz_dzVy + Ryz_n) * dt);
-    st<NT>(Sxz, p, sxz + (muxz * taus_plus1 * dxVz_dzVx + Rxz_n) * dt);
-    st<NT>(Sxy, p, sxy + (muxy * taus_plus1 * dxVy_dyVx + Rxy_n) * dt);
+    syz = syz + (muyz * taus_plus1 * dyVz_dzVy + Ryz_n) * dt;
+    sxz = sxz + (muxz * taus_plus1 * dxVz_dzVx + Rxz_n) * dt;
+    sxy = sxy + (muxy * taus_plus1 * dxVy_dyVx + Rxy_n) * dt;
+    if (TP && (a.mask & MASK_TAPER)) {
+        const float zc = ldv<false>(a.cgz_c + (k + 2)), zb = ldv<false>(a.cgz_b + (k + 2));
+        const float ccc = tp.xc * tp.yc * zc;
+        sxx = sxx * ccc;
+        syy = syy * ccc;
+        szz = szz * ccc;
+        syz = syz * tp.xc * tp.yb * zb;
+        sxz = sxz * tp.xb * tp.yc * zb;
+        sxy = sxy * tp.xb * tp.yb * zc;
+    }
+    st<NT>(Sxx, p, sxx);
+    st<NT>(Syy, p, syy);
+    st<NT>(Szz, p, szz);
+    st<NT>(Syz, p, syz);
+    st<NT>(Sxz, p, sxz);
+    st<NT>(Sxy, p, sxy);
 }
 
 // logical tile (bx, by, bz) of the interior blocks of a launch (those after
@@ -499,7 +536,7 @@ __device__ static inline void plain_tile(const StepArgs &a, int &bx, int &byy, i
     bz = t / a.nby;
 }
 
-template <int NM, bool NT, bool OOP>
+template <int NM, bool NT, bool OOP, bool TP>
 __device__ __forceinline__ void stress_int_body(const StepArgs &a, int bx, int byy, int bz)
 {
     const Grid &g = a.g;
@@ -532,6 +569,7 @@ __device__ __forceinline__ void stress_int_body(const StepArgs &a, int bx, int b
         const int kft = ldv<false>(a.m.kfs_top + c2), kfb = ldv<false>(a.m.kfs_bot + c2);
         const int kot = ldv<false>(a.m.kob_top + c2), kobb = ldv<false>(a.m.kob_bot + c2);
         const Coefs cf(a);
+        const Taper<TP> tp(a, i, j);
         Loc r = {((long long)(k0 - g.kb) * g.nyk + (jt - g.jb)) * g.rpitch + (it - 1),
                  4u * (threadIdx.y * g.rpitch + threadIdx.x), 0u};
         for (int k = k0; k <= ka1; ++k, p.u += P, r.u += g.rplane) {
@@ -551,7 +589,7 @@ __device__ __forceinline__ void stress_int_body(const StepArgs &a, int bx, int b
             v.vy_im1 = ld(Vy, p, 0, -1); v.vy_ip1 = ld(Vy, p, 0, 1); v.vy_ip2 = ld(Vy, p, 0, 2);
             v.vz_im1 = ld(Vz, p, 0, -1); v.vz_ip1 = ld(Vz, p, 0, 1); v.vz_ip2 = ld(Vz, p, 0, 2);
             v.vz_jm1 = ld(Vz, p, 0, 0, -1); v.vz_jp1 = ld(Vz, p, 0, 0, 1); v.vz_jp2 = ld(Vz, p, 0, 0, 2);
-            stress_cell<NM, NT, OOP>(a, p, r, in_band(k, kft, kfb, kot, kobb), cf, v, mu00, mu00n, mu10, mu10n, mu01, mu01n,
+            stress_cell<NM, NT, OOP, TP>(a, p, r, k, in_band(k, kft, kfb, kot, kobb), cf, tp, v, mu00, mu00n, mu10, mu10n, mu01, mu01n,
                                      mu11);
 
             // rotate the z queues
@@ -586,17 +624,17 @@ __device__ __forceinline__ void stress_int_body(const StepArgs &a, int bx, int b
 }
 
 // batched launch: tile = (member, bx, by, bz), member arguments in HBM
-template <int NM, bool NT>
+template <int NM, bool NT, bool TP>
 __global__ void __launch_bounds__(256) WAVES_NM k_stress_int_b(const StepArgs *__restrict__ mem, const int4 *__restrict__ tiles)
 {
     const int4 t = uni(tiles[xcd_remap(blockIdx.x, gridDim.x)]);
-    stress_int_body<NM, NT, false>(mem[t.x], t.y, t.z, t.w);
+    stress_int_body<NM, NT, false, TP>(mem[t.x], t.y, t.z, t.w);
 }
 
 // kernel__update_vel, m_kernel.f90:75-140, then the bottom PML band.
 // (Loading plane k+1 while computing plane k gained 1 % at three waves per
 // SIMD and nothing at four.)
-template <bool OOP>
+template <bool OOP, bool TP>
 __device__ __forceinline__ void vel_int_body(const StepArgs &a, int bx, int byy, int bz)
 {
     const Grid &g = a.g;
@@ -636,6 +674,7 @@ __device__ __forceinline__ void vel_int_body(const StepArgs &a, int bx, int byy,
         const int kft = ldv<false>(a.m.kfs_top + c2), kfb = ldv<false>(a.m.kfs_bot + c2);
         const int kot = ldv<false>(a.m.kob_top + c2), kobb = ldv<false>(a.m.kob_bot + c2);
         const Coefs cf(a);
+        const Taper<TP> tp(a, i, j);
         for (int k = k0; k <= ka1; ++k, p.u += P) {
             fresh(p);
             const float sxz_p1 = ld(Sxz, p, P), syz_p1 = ld(Syz, p, P), szz_p2 = ld(Szz, p, 2 * P);
@@ -670,9 +709,18 @@ __device__ __forceinline__ void vel_int_body(const StepArgs &a, int bx, int byy,
                               + (syz_0 - syz_jm1) * re40y - (syz_jp1 - syz_jm2) * re41y
                               + (szz_p1 - szz_0) * re40z - (szz_p2 - szz_m1) * re41z;
 
-            st<true>(Vx, p, vx + 2.0f / (rho0 + rho_ip) * d3Sx3 * dt);
-            st<true>(Vy, p, vy + 2.0f / (rho0 + rho_jp) * d3Sy3 * dt);
-            st<true>(Vz, p, vz + 2.0f / (rho0 + rho_kp) * d3Sz3 * dt);
+            float nx = vx + 2.0f / (rho0 + rho_ip) * d3Sx3 * dt;
+            float ny = vy + 2.0f / (rho0 + rho_jp) * d3Sy3 * dt;
+            float nz = vz + 2.0f / (rho0 + rho_kp) * d3Sz3 * dt;
+            if (TP && (a.mask & MASK_TAPER)) {
+                const float zc = ldv<false>(a.cgz_c + (k + 2)), zb = ldv<false>(a.cgz_b + (k + 2));
+                nx = nx * tp.xb * tp.yc * zc;
+                ny = ny * tp.xc * tp.yb * zc;
+                nz = nz * tp.xc * tp.yc * zb;
+            }
+            st<true>(Vx, p, nx);
+            st<true>(Vy, p, ny);
+            st<true>(Vz, p, nz);
 
             sxz_m2 = sxz_m1; sxz_m1 = sxz_0; sxz_0 = sxz_p1;
             syz_m2 = syz_m1; syz_m1 = syz_0; syz_0 = syz_p1;
@@ -701,10 +749,11 @@ __device__ __forceinline__ void vel_int_body(const StepArgs &a, int bx, int byy,
     }
 }
 
+template <bool TP>
 __global__ void __launch_bounds__(256) WAVES4 k_vel_int_b(const StepArgs *__restrict__ mem, const int4 *__restrict__ tiles)
 {
     const int4 t = uni(tiles[xcd_remap(blockIdx.x, gridDim.x)]);
-    vel_int_body<false>(mem[t.x], t.y, t.z, t.w);
+    vel_int_body<false, TP>(mem[t.x], t.y, t.z, t.w);
 }
 
 // ---------------------------------------------------------------------------
@@ -748,6 +797,7 @@ __global__ void __launch_bounds__(256) k_fused(StepArgs a)
     const float *__restrict__ mu = a.m.mu;
 
     const Coefs cf(a);
+    const Taper<false> tp(a, 1, 1);
     // velocity points of this thread: column iv, rows j0 - 2 + ty + 4 r.
     // vf: 0 not needed by the tile, 1 read from a.f, 2 computed, 3 computed
     // and stored (the tile's own cells)
@@ -891,7 +941,7 @@ __global__ void __launch_bounds__(256) k_fused(StepArgs a)
             v.vz_jm1 = vs[s0][2][row - 1][col]; v.vz_jp1 = vs[s0][2][row + 1][col];
             v.vz_jp2 = vs[s0][2][row + 2][col];
             const long long rr = ((long long)(k - g.kb) * g.nyk + (js - g.jb)) * g.rpitch + (is - 1);
-            stress_cell<NM, true, true>(a, Loc{p, 0u, 0u}, Loc{rr, 0u, 0u}, in_band(k, sb[s][0], sb[s][1], sb[s][2], sb[s][3]), cf, v, mu00[s],
+            stress_cell<NM, true, true, false>(a, Loc{p, 0u, 0u}, Loc{rr, 0u, 0u}, k, in_band(k, sb[s][0], sb[s][1], sb[s][2], sb[s][3]), cf, tp, v, mu00[s],
                                         mu00n, mu10[s], mu10n, mu01[s], mu01n, mu11[s]);
             mu00[s] = mu00n; mu10[s] = mu10n; mu01[s] = mu01n;
             mu11[s] = mu[p + P + 1 + Y];
@@ -1004,7 +1054,7 @@ __device__ __forceinline__ void vel_pml_body(const StepArgs &a, const int4 tl)
 // eighth of both.  Launched one after the other, each kind's last blocks leave
 // CUs idle: 128^3 took 140 us/step in two launches per phase and 127 in one,
 // elastic 256 x 256 x 192 525 and 505, 768 x 768 x 448 13.26 and 13.21 ms.
-template <int NM, bool NT, bool OOP>
+template <int NM, bool NT, bool OOP, bool TP>
 __global__ void __launch_bounds__(256) WAVES_NM k_stress(StepArgs a)
 {
     if ((int)blockIdx.x < a.sideb) {
@@ -1014,10 +1064,10 @@ __global__ void __launch_bounds__(256) WAVES_NM k_stress(StepArgs a)
     }
     int bx, byy, bz;
     plain_tile(a, bx, byy, bz);
-    stress_int_body<NM, NT, OOP>(a, bx, byy, bz);
+    stress_int_body<NM, NT, OOP, TP>(a, bx, byy, bz);
 }
 
-template <bool OOP>
+template <bool OOP, bool TP>
 __global__ void __launch_bounds__(256) WAVES4 k_vel(StepArgs a)
 {
     if ((int)blockIdx.x < a.sideb) {
@@ -1027,7 +1077,7 @@ __global__ void __launch_bounds__(256) WAVES4 k_vel(StepArgs a)
     }
     int bx, byy, bz;
     plain_tile(a, bx, byy, bz);
-    vel_int_body<OOP>(a, bx, byy, bz);
+    vel_int_body<OOP, TP>(a, bx, byy, bz);
 }
 
 // batched side-column tiles: (i0 | width << 20 | xslab << 28, j0, k0 | k1 << 16, member)
@@ -1048,18 +1098,19 @@ __global__ void __launch_bounds__(256) k_vel_pml_b(const StepArgs *__restrict__ 
 // one launch per phase for the tiles of both kinds: entries (m, bx, by, bz) are interior
 // tiles of member m, entries (-(m+1), i0 | width << 20 | xslab << 28, j0,
 // k0 | k1 << 16) its side tiles
-template <int NM, bool NT>
+template <int NM, bool NT, bool TP>
 __global__ void __launch_bounds__(256) WAVES_NM k_stress_all_b(const StepArgs *__restrict__ mem, const int4 *__restrict__ tiles)
 {
     const int4 t = uni(tiles[xcd_remap(blockIdx.x, gridDim.x)]);
-    if (t.x >= 0) stress_int_body<NM, NT, false>(mem[t.x], t.y, t.z, t.w);
+    if (t.x >= 0) stress_int_body<NM, NT, false, TP>(mem[t.x], t.y, t.z, t.w);
     else stress_pml_body<false>(mem[-t.x - 1], make_int4(t.y, t.z, t.w & 0xFFFF, t.w >> 16));
 }
 
+template <bool TP>
 __global__ void __launch_bounds__(256) WAVES4 k_vel_all_b(const StepArgs *__restrict__ mem, const int4 *__restrict__ tiles)
 {
     const int4 t = uni(tiles[xcd_remap(blockIdx.x, gridDim.x)]);
-    if (t.x >= 0) vel_int_body<false>(mem[t.x], t.y, t.z, t.w);
+    if (t.x >= 0) vel_int_body<false, TP>(mem[t.x], t.y, t.z, t.w);
     else vel_pml_body<false>(mem[-t.x - 1], make_int4(t.y, t.z, t.w & 0xFFFF, t.w >> 16));
 }
 
@@ -1096,6 +1147,7 @@ void fill_step_args(swpc_ctx *c, StepArgs &a, int mask)
     a.tiles = (const int4 *)c->d_pml_tiles;
     a.ntiles = c->npml_tiles;
     a.sideb = 0;
+    a.cgx_c = c->cgx_c; a.cgx_b = c->cgx_b; a.cgy_c = c->cgy_c; a.cgy_b = c->cgy_b; a.cgz_c = c->cgz_c; a.cgz_b = c->cgz_b;
     a.has_pml = (c->desc.abc == SWPC_ABC_PML && c->npml > 0) ? 1 : 0;
     a.mask = mask;
     a.by = c->by;
@@ -1137,11 +1189,13 @@ hipError_t launch_stress(swpc_ctx *c, bool side, int mask)
     if (!phase_grid(c, a, 0, side, mask, grid, block)) return hipSuccess;
     const bool nt = (c->variant & 1) != 0;
     const bool oop = c->fields_in[0] != nullptr;   // out of place: non-temporal streams as well
-#define SWPC_STRESS_CASE(NMV)                                                                   \
-    case NMV:                                                                                   \
-        if (oop) hipLaunchKernelGGL((k_stress<NMV, true, true>), grid, block, 0, c->stream, a);       \
-        else if (nt) hipLaunchKernelGGL((k_stress<NMV, true, false>), grid, block, 0, c->stream, a);  \
-        else hipLaunchKernelGGL((k_stress<NMV, false, false>), grid, block, 0, c->stream, a);         \
+    const bool tp = (mask & MASK_TAPER) != 0;
+#define SWPC_STRESS_CASE(NMV)                                                                              \
+    case NMV:                                                                                              \
+        if (oop) hipLaunchKernelGGL((k_stress<NMV, true, true, false>), grid, block, 0, c->stream, a);       \
+        else if (tp) hipLaunchKernelGGL((k_stress<NMV, true, false, true>), grid, block, 0, c->stream, a);   \
+        else if (nt) hipLaunchKernelGGL((k_stress<NMV, true, false, false>), grid, block, 0, c->stream, a);  \
+        else hipLaunchKernelGGL((k_stress<NMV, false, false, false>), grid, block, 0, c->stream, a);         \
         break;
     switch (c->g.nm) {
         SWPC_STRESS_CASE(0) SWPC_STRESS_CASE(1) SWPC_STRESS_CASE(2) SWPC_STRESS_CASE(3) SWPC_STRESS_CASE(4)
@@ -1157,8 +1211,9 @@ hipError_t launch_vel(swpc_ctx *c, bool side, int mask)
     StepArgs a;
     dim3 grid, block;
     if (!phase_grid(c, a, 1, side, mask, grid, block)) return hipSuccess;
-    if (c->fields_in[0]) hipLaunchKernelGGL(k_vel<true>, grid, block, 0, c->stream, a);
-    else hipLaunchKernelGGL(k_vel<false>, grid, block, 0, c->stream, a);
+    if (c->fields_in[0]) hipLaunchKernelGGL((k_vel<true, false>), grid, block, 0, c->stream, a);
+    else if (mask & MASK_TAPER) hipLaunchKernelGGL((k_vel<false, true>), grid, block, 0, c->stream, a);
+    else hipLaunchKernelGGL((k_vel<false, false>), grid, block, 0, c->stream, a);
     return hipGetLastError();
 }
 
@@ -1239,28 +1294,6 @@ __global__ void __launch_bounds__(256) k_cerjan_vel(CerjanArgs a)
     cerjan_vel_cell(a, 1 + blockIdx.x * blockDim.x + threadIdx.x, 1 + blockIdx.y, 1 + blockIdx.z);
 }
 
-// batched sponges (swpc_batch): one flat launch over every member's blocks;
-// member m owns blocks blk0[m] .. blk0[m+1]-1, its (row chunk, j, k) blocks
-// in the order of its own launch
-__global__ void __launch_bounds__(256) k_cerjan_b(const CerjanArgs *__restrict__ args, const int *__restrict__ blk0,
-                                                  int nmem, int phase)
-{
-    const int b = blockIdx.x;
-    int lo = 0, hi = nmem - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (blk0[mid] <= b) lo = mid;
-        else hi = mid - 1;
-    }
-    const CerjanArgs &a = args[lo];
-    const int lb = b - blk0[lo];
-    const int gx = (a.g.nx + 255) / 256;
-    const int t = lb / gx;
-    const int i = 1 + (lb % gx) * 256 + threadIdx.x, j = 1 + t % a.g.ny, k = 1 + t / a.g.ny;
-    if (phase == 0) cerjan_stress_cell(a, i, j, k);
-    else cerjan_vel_cell(a, i, j, k);
-}
-
 static void cerjan_fill(swpc_ctx *c, CerjanArgs &a, int kend)
 {
     a.g = c->g;
@@ -1271,40 +1304,21 @@ static void cerjan_fill(swpc_ctx *c, CerjanArgs &a, int kend)
     a.kend = kend;
 }
 
-hipError_t launch_cerjan_stress(swpc_ctx *c, hipStream_t s)
+hipError_t launch_cerjan_stress(swpc_ctx *c)
 {
     CerjanArgs a;
     cerjan_fill(c, a, c->g.ke);
     dim3 grid((c->g.nx + 255) / 256, c->g.ny, c->g.ke);
-    hipLaunchKernelGGL(k_cerjan_stress, grid, dim3(256), 0, (s ? s : c->stream), a);
+    hipLaunchKernelGGL(k_cerjan_stress, grid, dim3(256), 0, c->stream, a);
     return hipGetLastError();
 }
 
-hipError_t launch_cerjan_vel(swpc_ctx *c, hipStream_t s)
+hipError_t launch_cerjan_vel(swpc_ctx *c)
 {
     CerjanArgs a;
     cerjan_fill(c, a, c->g.nz);
     dim3 grid((c->g.nx + 255) / 256, c->g.ny, c->g.nz);
-    hipLaunchKernelGGL(k_cerjan_vel, grid, dim3(256), 0, (s ? s : c->stream), a);
-    return hipGetLastError();
-}
-
-size_t batch_cerjan_size() { return sizeof(CerjanArgs); }
-
-int batch_cerjan_fill(swpc_ctx *c, int phase, void *out)
-{
-    if (c->desc.abc != SWPC_ABC_CERJAN) return 0;
-    CerjanArgs a;
-    const int kend = phase == 0 ? c->g.ke : c->g.nz;
-    cerjan_fill(c, a, kend);
-    *(CerjanArgs *)out = a;
-    return (c->g.nx + 255) / 256 * c->g.ny * kend;
-}
-
-hipError_t launch_batch_cerjan(int phase, const void *d_args, const int *d_blk0, int nmem, int nblocks, hipStream_t s)
-{
-    if (nmem <= 0 || nblocks <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_cerjan_b, dim3(nblocks), dim3(256), 0, s, (const CerjanArgs *)d_args, d_blk0, nmem, phase);
+    hipLaunchKernelGGL(k_cerjan_vel, grid, dim3(256), 0, c->stream, a);
     return hipGetLastError();
 }
 
@@ -1319,7 +1333,7 @@ size_t step_args_size() { return sizeof(StepArgs); }
 void fill_batch_args(swpc_ctx *c, void *out, int phase)
 {
     StepArgs a;
-    step_args(c, a, MASK_INT | MASK_PML);
+    step_args(c, a, MASK_INT | (c->desc.abc == SWPC_ABC_PML ? MASK_PML : MASK_TAPER));
     if (phase == 1) a.zc = c->d_zchunks + c->nbz + 1;
     *(StepArgs *)out = a;
 }
@@ -1335,7 +1349,7 @@ void member_tiles(swpc_ctx *c, int &nbx, int &nby, int &nbz)
 }
 
 // one launch per phase for both kinds of tiles (the batch's packing 2)
-hipError_t launch_batch_phase_all(int phase, int nm, int variant, int by, int bxw, const void *d_args,
+hipError_t launch_batch_phase_all(int phase, int nm, int variant, bool tp, int by, int bxw, const void *d_args,
                                   const int4 *d_all, int nall, hipStream_t s)
 {
     if (nall <= 0) return hipSuccess;
@@ -1343,13 +1357,15 @@ hipError_t launch_batch_phase_all(int phase, int nm, int variant, int by, int bx
     const dim3 block(bxw, by * (BX / bxw));
     const bool nt = (variant & 1) != 0;
     if (phase == 1) {
-        hipLaunchKernelGGL(k_vel_all_b, dim3(nall), block, 0, s, mem, d_all);
+        if (tp) hipLaunchKernelGGL(k_vel_all_b<true>, dim3(nall), block, 0, s, mem, d_all);
+        else hipLaunchKernelGGL(k_vel_all_b<false>, dim3(nall), block, 0, s, mem, d_all);
         return hipGetLastError();
     }
-#define SWPC_BALL_CASE(NMV)                                                                           \
-    case NMV:                                                                                         \
-        if (nt) hipLaunchKernelGGL((k_stress_all_b<NMV, true>), dim3(nall), block, 0, s, mem, d_all); \
-        else hipLaunchKernelGGL((k_stress_all_b<NMV, false>), dim3(nall), block, 0, s, mem, d_all);   \
+#define SWPC_BALL_CASE(NMV)                                                                                   \
+    case NMV:                                                                                                 \
+        if (tp) hipLaunchKernelGGL((k_stress_all_b<NMV, true, true>), dim3(nall), block, 0, s, mem, d_all);         \
+        else if (nt) hipLaunchKernelGGL((k_stress_all_b<NMV, true, false>), dim3(nall), block, 0, s, mem, d_all);   \
+        else hipLaunchKernelGGL((k_stress_all_b<NMV, false, false>), dim3(nall), block, 0, s, mem, d_all);          \
         break;
     switch (nm) {
         SWPC_BALL_CASE(0) SWPC_BALL_CASE(1) SWPC_BALL_CASE(2) SWPC_BALL_CASE(3) SWPC_BALL_CASE(4)
@@ -1360,8 +1376,8 @@ hipError_t launch_batch_phase_all(int phase, int nm, int variant, int by, int bx
     return hipGetLastError();
 }
 
-hipError_t launch_batch_phase(int phase, int nm, int variant, int by, int bxw, const void *d_args, const int4 *d_cols,
-                              int ncols, const int4 *d_side, int nside, hipStream_t s)
+hipError_t launch_batch_phase(int phase, int nm, int variant, bool tp, int by, int bxw, const void *d_args,
+                              const int4 *d_cols, int ncols, const int4 *d_side, int nside, hipStream_t s)
 {
     const bool nt = (variant & 1) != 0;
     const StepArgs *mem = (const StepArgs *)d_args;
@@ -1374,13 +1390,15 @@ hipError_t launch_batch_phase(int phase, int nm, int variant, int by, int bxw, c
     }
     if (ncols <= 0) return hipSuccess;
     if (phase == 1) {
-        hipLaunchKernelGGL(k_vel_int_b, dim3(ncols), block, 0, s, mem, d_cols);
+        if (tp) hipLaunchKernelGGL(k_vel_int_b<true>, dim3(ncols), block, 0, s, mem, d_cols);
+        else hipLaunchKernelGGL(k_vel_int_b<false>, dim3(ncols), block, 0, s, mem, d_cols);
         return hipGetLastError();
     }
-#define SWPC_BSTRESS_CASE(NMV)                                                                      \
-    case NMV:                                                                                       \
-        if (nt) hipLaunchKernelGGL((k_stress_int_b<NMV, true>), dim3(ncols), block, 0, s, mem, d_cols); \
-        else hipLaunchKernelGGL((k_stress_int_b<NMV, false>), dim3(ncols), block, 0, s, mem, d_cols);   \
+#define SWPC_BSTRESS_CASE(NMV)                                                                                \
+    case NMV:                                                                                                 \
+        if (tp) hipLaunchKernelGGL((k_stress_int_b<NMV, true, true>), dim3(ncols), block, 0, s, mem, d_cols);       \
+        else if (nt) hipLaunchKernelGGL((k_stress_int_b<NMV, true, false>), dim3(ncols), block, 0, s, mem, d_cols); \
+        else hipLaunchKernelGGL((k_stress_int_b<NMV, false, false>), dim3(ncols), block, 0, s, mem, d_cols);        \
         break;
     switch (nm) {
         SWPC_BSTRESS_CASE(0) SWPC_BSTRESS_CASE(1) SWPC_BSTRESS_CASE(2) SWPC_BSTRESS_CASE(3) SWPC_BSTRESS_CASE(4)

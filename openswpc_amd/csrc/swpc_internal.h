@@ -230,8 +230,8 @@ bool arena_free(void *p);
 hipError_t launch_stress(swpc_ctx *c, bool side, int mask);
 hipError_t launch_vel(swpc_ctx *c, bool side, int mask);
 hipError_t launch_fused(swpc_ctx *c);
-hipError_t launch_cerjan_stress(swpc_ctx *c, hipStream_t s = nullptr);
-hipError_t launch_cerjan_vel(swpc_ctx *c, hipStream_t s = nullptr);
+hipError_t launch_cerjan_stress(swpc_ctx *c);
+hipError_t launch_cerjan_vel(swpc_ctx *c);
 hipError_t launch_stressglut(swpc_ctx *c, int it, const int *d_it, hipStream_t s = nullptr);
 hipError_t launch_bodyforce(swpc_ctx *c, int it, const int *d_it, hipStream_t s = nullptr);
 hipError_t launch_wav_store(swpc_ctx *c, int it, const int *d_it, hipStream_t s = nullptr);
@@ -262,14 +262,11 @@ hipError_t launch_batch_green(int kind, const void *d_args, int nmem, int nmax, 
 size_t batch_snap_size();
 int batch_snap_fill(swpc_ctx *c, void *out);
 hipError_t launch_batch_snap(const void *d_args, int nmem, int maxblk, int it, const int *d_it, hipStream_t s);
-// batched Cerjan sponges (stencil.hip): phase 0 stress, 1 velocity; returns the member's block count
-size_t batch_cerjan_size();
-int batch_cerjan_fill(swpc_ctx *c, int phase, void *out);
-hipError_t launch_batch_cerjan(int phase, const void *d_args, const int *d_blk0, int nmem, int nblocks, hipStream_t s);
-hipError_t launch_batch_phase_all(int phase, int nm, int variant, int by, int bxw, const void *d_args,
+// a phase of every member; tp: Cerjan members are among them
+hipError_t launch_batch_phase_all(int phase, int nm, int variant, bool tp, int by, int bxw, const void *d_args,
                                   const int4 *d_all, int nall, hipStream_t s);
-hipError_t launch_batch_phase(int phase, int nm, int variant, int by, int bxw, const void *d_args, const int4 *d_cols,
-                              int ncols, const int4 *d_side, int nside, hipStream_t s);
+hipError_t launch_batch_phase(int phase, int nm, int variant, bool tp, int by, int bxw, const void *d_args,
+                              const int4 *d_cols, int ncols, const int4 *d_side, int nside, hipStream_t s);
 hipError_t launch_vmax(swpc_ctx *c);
 hipError_t launch_ref_to_dev(swpc_ctx *c, const float *src_ref, float *dst, hipStream_t s);
 hipError_t launch_dev_to_ref(swpc_ctx *c, const float *src, float *dst_ref, hipStream_t s);

@@ -1,0 +1,64 @@
+"""Edges of the phase launches: side and interior tiles in one launch on grids
+where a tile's rows, columns or planes run out (absorbers of one to twelve
+cells, slabs closer together than a tile is tall, a single interior column,
+k chunks of one plane up to the default), and the Cerjan taper applied by the
+update itself.  Bit for bit against the FP32 oracle."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from tests.gpu_helpers import compare_fields, gpu_from_model, small_config
+
+pytestmark = pytest.mark.gpu
+MT = dict(x=0.1, y=-0.1, z=1.6, t0=0.0, tr=0.4, mo=1e15, strike=30.0, dip=60.0, rake=90.0)
+BF = dict(x=0.1, y=-0.1, z=1.6, t0=0.0, tr=0.4, fx=0.3, fy=-1.0, fz=0.7)
+
+
+def _model(**kw):
+    cfg = small_config(nt=12, zbeg=-1.0, stations=[], wav_flags=0, **kw)
+    return O.build_model(cfg)
+
+
+def _same(g, run, label):
+    for n, (ulp, rel) in compare_fields(g, run).items():
+        assert ulp == 0, (label, n, ulp, rel)
+
+
+@pytest.mark.parametrize("kchunk", [0, 1, 5])
+@pytest.mark.parametrize("nx,ny,nz,na", [(13, 70, 14, 6), (70, 13, 14, 6), (9, 9, 12, 4), (67, 66, 12, 1),
+                                         (150, 31, 24, 12)])
+def test_tile_edges(orc, nx, ny, nz, na, kchunk):
+    m = _model(nx=nx, ny=ny, nz=nz, na=na, nm=2, sources=[MT])
+    run = O.OracleRun(m, 32)
+    run.run(12)
+    g = gpu_from_model(m, kchunk=kchunk)
+    g.step(1, 12, use_graph=True, block=5)
+    _same(g, run, f"{nx}x{ny}x{nz} na={na} kchunk={kchunk}")
+
+
+@pytest.mark.parametrize("force", [False, True])
+@pytest.mark.parametrize("nx,ny,nz,kchunk", [(33, 30, 27, 0), (65, 18, 9, 1), (64, 21, 16, 4), (129, 9, 11, 3)])
+def test_taper_applied_by_the_update(orc, nx, ny, nz, kchunk, force):
+    m = _model(nx=nx, ny=ny, nz=nz, na=4, nm=1, abc="cerjan", sources=[BF if force else MT], bf_mode=force)
+    run = O.OracleRun(m, 32)
+    run.run(12)
+    g = gpu_from_model(m, kchunk=kchunk)
+    g.step(1, 12)
+    _same(g, run, "steps")
+    # the fused routines against the reference's separate ones
+    h = gpu_from_model(m, kchunk=kchunk)
+    for it in range(1, 13):
+        if it % 2:
+            h.update_stress()
+        else:
+            h.kernel_update_stress()
+            h.absorb_update_stress()
+        h.source_stressglut(it)
+        if it % 2:
+            h.kernel_update_vel()
+            h.absorb_update_vel()
+        else:
+            h.update_vel()
+        h.source_bodyforce(it)
+    for n in O.FIELDS_V + O.FIELDS_S:
+        assert np.array_equal(h.get_field(n), g.get_field(n)), n
