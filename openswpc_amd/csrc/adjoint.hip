@@ -7,15 +7,21 @@
 //     R'_c[m] = c1[m] R_c[m] - c2[m] E_c dt,  S'_c = S_c + (F_c + sum d1[m] R'_c[m]) dt,
 // transpose to rho = aR' + d1 dt aS', aR = c1 rho, and -dt sum c2 rho on the
 // derivative combination E_c; they need no forward R for the gradients.
-// Per phase:
-//   1. density kernel (one thread per cell): the adjoint of every spatial
-//      derivative the cell's forward update used (9 per phase), the updated
-//      auxiliary adjoints, and the cell's gradient terms;
-//   2. gather kernel (one thread per field point): each point collects the
-//      densities of the cells whose stencils read it, with those cells'
-//      coefficients -- the band-switched 4th-order pair in the interior,
-//      1/h in the PML.
-// Gathers replace scatters, so no atomics and a fixed summation order.
+// Each phase works with densities, one per cell: the adjoint of every spatial
+// derivative the cell's forward update used (9 per phase).  Every field point
+// then gathers the densities of the cells whose stencils read it, with those
+// cells' own coefficients -- the band-switched 4th-order pair in the interior,
+// 1/h in the PML -- so there are no scatters, no atomics and a fixed summation
+// order.  A density depends on its own cell only, so one kernel gathers a
+// phase and leaves the next phase's densities:
+//   k_adj_s  gathers the velocity phase into the stress adjoints and writes
+//            the stress phase's densities from them;
+//   k_adj_v  gathers the stress phase into the velocity adjoints and writes
+//            the velocity densities of the step before (the trace adjoint is
+//            added to the velocity adjoints between the two).
+// The gradients of the shear moduli and buoyancies are summed over the steps
+// at their own staggered points, where a cell only touches its own entry, and
+// brought to the cells' mu and rho once per source (k_adj_finish).
 // The forward state the gradients need (V_n and its auxiliaries for the
 // stress update, S_{n+1} and the stress auxiliaries for the velocity
 // update) is recomputed segment by segment from checkpoints taken every
@@ -25,6 +31,7 @@
 #include <map>
 #include <vector>
 
+#include "device_access.h"
 #include "swpc_internal.h"
 
 namespace {
@@ -45,13 +52,14 @@ struct AdjArgs {
     const float4 *gxc, *gxe, *gyc, *gye, *gzc, *gze;
     float *aF[9];       // adjoint fields: Vx Vy Vz Sxx Syy Szz Syz Sxz Sxy
     float *aA;          // adjoint auxiliaries, 18 x npml
-    float *D[9];        // per-cell derivative adjoints
-    float *q[6];        // per-cell gradient terms gathered in phase 2 (velocity phase: 3, stress phase: 6)
-    const unsigned char *cls;  // class of every grid point (k_adj_class)
-    float tA[3][4], tB[3][4];  // per axis and class: near (p40 or 1/h) and far (p41) weights
+    float *W[9], *D[9]; // densities of the velocity and the stress phase
+    float *gb[3];       // gradients of 1 / buoyancy sums at the x, y, z velocity points
+    float *gh[3];       // gradients of the shear moduli at the yz, xz, xy points
+    const unsigned *nbr;  // what a gather needs to know of the cells around a point (k_adj_nbr)
+    float ratio;        // far over near 4th-order weight off the band
     const float *fF[9]; // forward fields of the step (same order as aF)
     const float *fA;    // forward auxiliaries of the phase, 9 x npml
-    float *g_lam, *g_mu, *g_rho;
+    float *g_lam, *g_mu;  // lam, and mu without its shear moduli
 };
 
 enum { FVX = 0, FVY, FVZ, FSXX, FSYY, FSZZ, FSYZ, FSXZ, FSXY };
@@ -84,14 +92,20 @@ __device__ static inline long long ade_index(const AdjArgs &a, int i, int j, int
     return b.off + ((long long)(k - b.k0) * b.nyb + (j - b.j0)) * b.nxb + (i - b.i0);
 }
 
-// 4th-order pair of a cell along an axis (the forward kernel's band switch)
-__device__ static inline void pair_at(const AdjArgs &a, int axis, int i, int j, int k, float &p40, float &p41)
+// 4th-order pairs of a cell (the forward kernel's band switch); returns
+// whether it is in the band
+__device__ static inline bool pairs_at(const AdjArgs &a, int i, int j, int k, float &ax, float &bx, float &ay,
+                                       float &by, float &az, float &bz)
 {
     const long long c2 = g2idx(a.g, i, j);
-    const int in = in_band(k, a.kfs_top[c2], a.kfs_bot[c2], a.kob_top[c2], a.kob_bot[c2]) ? 1 : 0;
-    if (axis == 0) { p40 = a.c.re40x[in]; p41 = a.c.re41x[in]; }
-    else if (axis == 1) { p40 = a.c.re40y[in]; p41 = a.c.re41y[in]; }
-    else { p40 = a.c.re40z[in]; p41 = a.c.re41z[in]; }
+    const bool in = in_band(k, a.kfs_top[c2], a.kfs_bot[c2], a.kob_top[c2], a.kob_bot[c2]);
+    ax = in ? a.c.re40x[1] : a.c.re40x[0];
+    bx = in ? a.c.re41x[1] : a.c.re41x[0];
+    ay = in ? a.c.re40y[1] : a.c.re40y[0];
+    by = in ? a.c.re41y[1] : a.c.re41y[0];
+    az = in ? a.c.re40z[1] : a.c.re40z[0];
+    bz = in ? a.c.re41z[1] : a.c.re41z[0];
+    return in;
 }
 
 // 0 = not updated, 1 = interior (4th order), 2 = PML (2nd order)
@@ -103,10 +117,25 @@ __device__ static inline int cell_kind(const AdjArgs &a, int i, int j, int k)
     return a.has_pml ? 2 : 0;
 }
 
-// Class of every grid point, for the gathers: 0 outside the updated cells
-// (halo), 1 interior off the free-surface band, 2 interior in the band, 3 PML.
-// A cell's weights in a gather depend only on its class and the axis.
-__global__ void k_adj_class(AdjArgs a, unsigned char *cls)
+// 0 outside the updated cells (halo), 1 interior off the 2nd-order band,
+// 2 interior in the band, 3 PML
+__device__ static inline int cell_class(const AdjArgs &a, int i, int j, int k)
+{
+    const int kind = cell_kind(a, i, j, k);
+    if (kind != 1) return kind == 2 ? 3 : 0;
+    const long long c2 = g2idx(a.g, i, j);
+    return in_band(k, a.kfs_top[c2], a.kfs_bot[c2], a.kob_top[c2], a.kob_bot[c2]) ? 2 : 1;
+}
+
+// One word per grid point about the twelve points at -2, -1, +1, +2 along each
+// axis (bit 4 * axis + 0..3 of a group) and the point itself: bits 0..11, off
+// the band (class 1: the only cells whose far weight is not zero); bits
+// 12..23 and 24 (itself), PML.  A gather reads this word where it read the
+// class bytes of thirteen points and looked two weights up for each.
+#define NBR_PML 12
+#define NBR_OWN 24
+#define NBR_ANY_PML 0x1FFF000u
+__global__ void k_adj_nbr(AdjArgs a, unsigned *nbr)
 {
     const Grid &g = a.g;
     for (long long p = blockIdx.x * (long long)blockDim.x + threadIdx.x; p < g.n; p += (long long)gridDim.x * blockDim.x) {
@@ -114,79 +143,67 @@ __global__ void k_adj_class(AdjArgs a, unsigned char *cls)
         const long long r = p % g.plane;
         const int j = (int)(r / g.pitch) - 2;
         const int i = (int)(r % g.pitch) - g.ox + 1;
-        const int kind = cell_kind(a, i, j, k);
-        unsigned char c = 0;
-        if (kind == 1) {
-            const long long c2 = g2idx(g, i, j);
-            c = in_band(k, a.kfs_top[c2], a.kfs_bot[c2], a.kob_top[c2], a.kob_bot[c2]) ? 2 : 1;
-        } else if (kind == 2) {
-            c = 3;
+        unsigned m = 0;
+        if (i >= 1 && i <= g.nx && j >= 1 && j <= g.ny && k >= 1 && k <= g.nz) {
+            for (int ax = 0; ax < 3; ++ax)
+                for (int o = 0; o < 4; ++o) {
+                    const int s = o < 2 ? o - 2 : o - 1;
+                    const int c = cell_class(a, i + (ax == 0 ? s : 0), j + (ax == 1 ? s : 0), k + (ax == 2 ? s : 0));
+                    if (c == 1) m |= 1u << (4 * ax + o);
+                    if (c == 3) m |= 1u << (NBR_PML + 4 * ax + o);
+                }
+            if (cell_class(a, i, j, k) == 3) m |= 1u << NBR_OWN;
         }
-        cls[p] = c;
+        nbr[p] = m;
     }
 }
 
-// weight of a class from a per-class table (t[0] = 0 for points outside)
-__device__ static inline float wt(const float t[4], int c) { return c == 1 ? t[1] : c == 2 ? t[2] : c == 3 ? t[3] : t[0]; }
+// Densities are stored times their cell's near weight in units of 1/h (9/8 off
+// the band, 1 in the band and in the PML), so a gather is differences of them:
+// its far terms take the ratio 1/27 of the cells off the band, or nothing.
+// Interior cells share one density for the derivatives that carry the same
+// value (the three of a velocity component; the two of a shear stress): it is
+// stored in Di only, and Dp holds the PML cells' own.  SEL: some lane of the
+// wave has a PML cell among its points and selects per point; the waves that
+// have none (most) read Di.
+template <int AX, bool SEL>
+struct Gather {
+    const AdjArgs &a;
+    const Loc &p;
+    unsigned m;
 
-// Gathers of one axis (stride s): the densities of the cells whose
-// derivative stencils read point p, times those cells' weights (A: the
-// near pair p40 or 1/h, B: the far pair p41 or 0).  Points outside the
-// updated cells hold density 0 and class 0.  The weights of the five
-// points p-2s .. p+2s are read once per axis and shared by its gathers.
-struct AxisW {
-    float A[5], B[5];
-    unsigned pml;   // bit o: point p + (o - 2) s is a PML cell
+    // the density at offset s (-2..2) along the axis
+    __device__ __forceinline__ float at(const float *Dp, const float *Di, int s) const
+    {
+        const float *F = Di;
+        if (SEL && Dp != Di) {
+            const int b = s == 0 ? NBR_OWN : NBR_PML + 4 * AX + (s < 0 ? s + 2 : s + 1);
+            F = (m >> b) & 1u ? Dp : Di;
+        }
+        return ld(F, p, AX == 2 ? s * a.g.plane : 0, AX == 0 ? s : 0, AX == 1 ? s : 0);
+    }
+    __device__ __forceinline__ float far(int s) const
+    {
+        const int b = 4 * AX + (s < 0 ? s + 2 : s + 1);
+        return __int_as_float(((int)(m << (31 - b)) >> 31) & __float_as_int(a.ratio));
+    }
+    __device__ __forceinline__ float h() const { return AX == 0 ? a.hx : AX == 1 ? a.hy : a.hz; }
+    // forward-type derivative (cell c reads c+1, c, c+2, c-1)
+    __device__ __forceinline__ float fwd(const float *Dp, const float *Di) const
+    {
+        return (at(Dp, Di, -1) - at(Dp, Di, 0) - far(-2) * at(Dp, Di, -2) + far(1) * at(Dp, Di, 1)) * h();
+    }
+    // backward-type derivative (cell c reads c, c-1, c+1, c-2)
+    __device__ __forceinline__ float bwd(const float *Dp, const float *Di) const
+    {
+        return (at(Dp, Di, 0) - at(Dp, Di, 1) - far(-1) * at(Dp, Di, -1) + far(2) * at(Dp, Di, 2)) * h();
+    }
+    __device__ __forceinline__ float fwd(const float *D) const { return fwd(D, D); }
+    __device__ __forceinline__ float bwd(const float *D) const { return bwd(D, D); }
 };
-__device__ static inline AxisW axis_w(const unsigned char *cls, long long p, long long s, const float tA[4],
-                                      const float tB[4])
-{
-    AxisW w;
-    w.pml = 0;
-#pragma unroll
-    for (int o = 0; o < 5; ++o) {
-        const int c = cls[p + (o - 2) * s];
-        w.A[o] = wt(tA, c);
-        w.B[o] = wt(tB, c);
-        w.pml |= (c == 3 ? 1u : 0u) << o;
-    }
-    return w;
-}
-// forward-type derivative (cell c reads c+1, c, c+2, c-1)
-__device__ static inline float gat_fwd(const float *D, long long p, long long s, const AxisW &w)
-{
-    return w.A[1] * D[p - s] - w.A[2] * D[p] - w.B[0] * D[p - 2 * s] + w.B[3] * D[p + s];
-}
-// backward-type derivative (cell c reads c, c-1, c+1, c-2)
-__device__ static inline float gat_bwd(const float *D, long long p, long long s, const AxisW &w)
-{
-    return w.A[2] * D[p] - w.A[3] * D[p + s] - w.B[1] * D[p - s] + w.B[4] * D[p + 2 * s];
-}
+#define NEAR_OFF_BAND 1.125f
 
-// The same gathers for a density that interior cells share with another
-// one (the velocity update's three derivatives of one component all carry
-// that component's weight; the stress update's two derivatives of one shear
-// component carry its weight): the density kernels store Dp for PML cells
-// only, and the gather reads point o from Dp where it is a PML cell and from
-// Di, which holds the same value, elsewhere.  Points outside the cells hold 0
-// in both.
-__device__ static inline float ld_sel(const float *Dp, const float *Di, long long p, long long s, int o,
-                                      const AxisW &w)
-{
-    return ((w.pml >> o) & 1u ? Dp : Di)[p + (o - 2) * s];
-}
-__device__ static inline float gat_fwd_s(const float *Dp, const float *Di, long long p, long long s, const AxisW &w)
-{
-    return w.A[1] * ld_sel(Dp, Di, p, s, 1, w) - w.A[2] * ld_sel(Dp, Di, p, s, 2, w)
-         - w.B[0] * ld_sel(Dp, Di, p, s, 0, w) + w.B[3] * ld_sel(Dp, Di, p, s, 3, w);
-}
-__device__ static inline float gat_bwd_s(const float *Dp, const float *Di, long long p, long long s, const AxisW &w)
-{
-    return w.A[2] * ld_sel(Dp, Di, p, s, 2, w) - w.A[3] * ld_sel(Dp, Di, p, s, 3, w)
-         - w.B[1] * ld_sel(Dp, Di, p, s, 1, w) + w.B[4] * ld_sel(Dp, Di, p, s, 4, w);
-}
-
-#define AT(F, di, dj, dk) (F)[gidx(g, i + (di), j + (dj), k + (dk))]
+#define AT(F, di, dj, dk) ld((F), p, (dk) * g.plane, (di), (dj))
 #define BWD4(F, di, dj, dk, p40, p41) ((AT(F, 0, 0, 0) - AT(F, -(di), -(dj), -(dk))) * (p40) \
                                        - (AT(F, di, dj, dk) - AT(F, -2 * (di), -2 * (dj), -2 * (dk))) * (p41))
 #define FWD4(F, di, dj, dk, p40, p41) ((AT(F, di, dj, dk) - AT(F, 0, 0, 0)) * (p40) \
@@ -216,107 +233,10 @@ __device__ static inline float4 prof(const float4 *p, int n) { return p[n - 1]; 
     const int k = 1 + (int)(blockIdx.x / tpp_);                    \
     const int t_ = (int)(blockIdx.x % tpp_);                       \
     if (t_ >= nbx_ * nby_) return;                                 \
-    const int i = 1 + (t_ % nbx_) * 64 + threadIdx.x;              \
-    const int j = 1 + (t_ / nbx_) * 4 + threadIdx.y;               \
-    if (i > g.nx || j > g.ny) return;
-
-// adjoint of the velocity update: densities, stress-auxiliary adjoints, rho terms
-// (the stores come after every load, which the compiler cannot reorder)
-__global__ void __launch_bounds__(256) k_adj_vel_dens(AdjArgs a)
-{
-    ADJ_CELL(a) {
-        const int kind = cell_kind(a, i, j, k);
-        const long long p = gidx(g, i, j, k);
-        const float r0 = a.rho[p];
-        const float sx = r0 + AT(a.rho, 1, 0, 0), sy = r0 + AT(a.rho, 0, 1, 0), sz = r0 + AT(a.rho, 0, 0, 1);
-        const float vx = a.aF[FVX][p], vy = a.aF[FVY][p], vz = a.aF[FVZ][p];
-        const float wx = 2.0f / sx * a.dt * vx, wy = 2.0f / sy * a.dt * vy, wz = 2.0f / sz * a.dt * vz;
-        const float *Sxx = a.fF[FSXX], *Syy = a.fF[FSYY], *Szz = a.fF[FSZZ];
-        const float *Syz = a.fF[FSYZ], *Sxz = a.fF[FSXZ], *Sxy = a.fF[FSXY];
-        float fx, fy, fz;
-        float d[9];
-        if (kind == 1) {
-            float ax, bx, ay, by, az, bz;
-            pair_at(a, 0, i, j, k, ax, bx);
-            pair_at(a, 1, i, j, k, ay, by);
-            pair_at(a, 2, i, j, k, az, bz);
-            fx = FWD4(Sxx, 1, 0, 0, ax, bx) + BWD4(Sxy, 0, 1, 0, ay, by) + BWD4(Sxz, 0, 0, 1, az, bz);
-            fy = BWD4(Sxy, 1, 0, 0, ax, bx) + FWD4(Syy, 0, 1, 0, ay, by) + BWD4(Syz, 0, 0, 1, az, bz);
-            fz = BWD4(Sxz, 1, 0, 0, ax, bx) + BWD4(Syz, 0, 1, 0, ay, by) + FWD4(Szz, 0, 0, 1, az, bz);
-            d[0] = wx; d[1] = wx; d[2] = wx;
-            d[3] = wy; d[4] = wy; d[5] = wy;
-            d[6] = wz; d[7] = wz; d[8] = wz;
-        } else {
-            const long long q = ade_index(a, i, j, k);
-            const long long n = a.npml;
-            const float4 gp[9] = {prof(a.gxe, i), prof(a.gyc, j), prof(a.gzc, k), prof(a.gxc, i), prof(a.gye, j),
-                                  prof(a.gzc, k), prof(a.gxc, i), prof(a.gyc, j), prof(a.gze, k)};
-            const float w[9] = {wx, wx, wx, wy, wy, wy, wz, wz, wz};
-            const float der[9] = {FWD2(Sxx, 1, 0, 0, a.hx), BWD2(Sxy, 0, 1, 0, a.hy), BWD2(Sxz, 0, 0, 1, a.hz),
-                                  BWD2(Sxy, 1, 0, 0, a.hx), FWD2(Syy, 0, 1, 0, a.hy), BWD2(Syz, 0, 0, 1, a.hz),
-                                  BWD2(Sxz, 1, 0, 0, a.hx), BWD2(Syz, 0, 1, 0, a.hy), FWD2(Szz, 0, 0, 1, a.hz)};
-            float ahat[9], fa[9];
-#pragma unroll
-            for (int c = 0; c < 9; ++c) {
-                ahat[c] = a.aA[(long long)(A_axSxx + c) * n + q];
-                fa[c] = a.fA[(long long)c * n + q];
-            }
-            float f[3] = {0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int c = 0; c < 9; ++c) {
-                d[c] = gp[c].x * w[c] + gp[c].w * a.dt * ahat[c];
-                f[c / 3] += gp[c].x * der[c] + gp[c].y * fa[c];
-            }
-#pragma unroll
-            for (int c = 0; c < 9; ++c) a.aA[(long long)(A_axSxx + c) * n + q] = gp[c].y * w[c] + gp[c].z * ahat[c];
-            fx = f[0]; fy = f[1]; fz = f[2];
-        }
-        // interior cells: d[0..2], d[3..5], d[6..8] are one value each, kept in D0, D3, D6
-        if (kind == 1) {
-            a.D[0][p] = d[0]; a.D[3][p] = d[3]; a.D[6][p] = d[6];
-        } else {
-#pragma unroll
-            for (int c = 0; c < 9; ++c) a.D[c][p] = d[c];
-        }
-        a.q[0][p] = -2.0f / (sx * sx) * a.dt * fx * vx;
-        a.q[1][p] = -2.0f / (sy * sy) * a.dt * fy * vy;
-        a.q[2][p] = -2.0f / (sz * sz) * a.dt * fz * vz;
-    }
-}
-
-// adjoint of the velocity update: stress adjoints and the rho gradient
-// (every load before the stores: the class bytes may alias anything)
-__global__ void __launch_bounds__(256) k_adj_vel_gather(AdjArgs a)
-{
-    ADJ_CELL(a) {
-        const long long p = gidx(g, i, j, k);
-        const long long sx = 1, sy = g.pitch, sz = g.plane;
-        const AxisW wx = axis_w(a.cls, p, sx, a.tA[0], a.tB[0]);
-        const AxisW wy = axis_w(a.cls, p, sy, a.tA[1], a.tB[1]);
-        const AxisW wz = axis_w(a.cls, p, sz, a.tA[2], a.tB[2]);
-        const float dxx = gat_fwd(a.D[0], p, sx, wx);
-        const float dyy = gat_fwd_s(a.D[4], a.D[3], p, sy, wy);
-        const float dzz = gat_fwd_s(a.D[8], a.D[6], p, sz, wz);
-        const float dxy = gat_bwd_s(a.D[1], a.D[0], p, sy, wy) + gat_bwd(a.D[3], p, sx, wx);
-        const float dxz = gat_bwd_s(a.D[2], a.D[0], p, sz, wz) + gat_bwd(a.D[6], p, sx, wx);
-        const float dyz = gat_bwd_s(a.D[5], a.D[3], p, sz, wz) + gat_bwd_s(a.D[7], a.D[6], p, sy, wy);
-        // each cell's density enters the buoyancy of its own point and of the
-        // point one cell back along each axis (q is 0 outside the cells)
-        float gr = a.q[0][p] + a.q[1][p] + a.q[2][p];
-        gr += a.q[0][p - sx];
-        gr += a.q[1][p - sy];
-        gr += a.q[2][p - sz];
-        const float oxx = a.aF[FSXX][p], oyy = a.aF[FSYY][p], ozz = a.aF[FSZZ][p];
-        const float oxy = a.aF[FSXY][p], oxz = a.aF[FSXZ][p], oyz = a.aF[FSYZ][p], org = a.g_rho[p];
-        a.aF[FSXX][p] = oxx + dxx;
-        a.aF[FSYY][p] = oyy + dyy;
-        a.aF[FSZZ][p] = ozz + dzz;
-        a.aF[FSXY][p] = oxy + dxy;
-        a.aF[FSXZ][p] = oxz + dxz;
-        a.aF[FSYZ][p] = oyz + dyz;
-        a.g_rho[p] = org + gr;
-    }
-}
+    const int i0_ = 1 + (t_ % nbx_) * 64, j0_ = 1 + (t_ / nbx_) * 4; \
+    const int i = i0_ + threadIdx.x, j = j0_ + threadIdx.y;        \
+    if (i > g.nx || j > g.ny) return;                              \
+    Loc p = field_loc(g, i0_, j0_, k, threadIdx.x, threadIdx.y);
 
 // harmonic mean of four moduli (the forward's shear modulus, m_kernel.f90:293-309)
 __device__ static inline float hmean4(float a, float b, float c, float d)
@@ -337,23 +257,135 @@ __device__ static inline void hmean4_w(float a, float b, float c, float d, float
     gr[3] = (4.0f * a * b * c * Dn - N * (a * b + a * c + b * c)) * r;
 }
 
-// adjoint of the stress update: densities, velocity-auxiliary adjoints,
-// lam and mu gradients of the cell, and the shear-mu terms of its
-// neighbours.  A shear point's modulus is the harmonic mean of four cells
-// (origin o and o + one or two unit steps); the cell adds the derivative
-// for its own corner to g_mu and leaves those for the other three corners
-// of each of its three quads, summed by target offset, in q[0..5]:
-//   q0 -> o+z, q1 -> o+y, q2 -> o+x, q3 -> o+y+z, q4 -> o+x+z, q5 -> o+x+y.
-// NM memory variables per component (a template argument, so their loops
-// unroll); the stores come after every load.
-template <int NM>
-__global__ void __launch_bounds__(256) k_adj_stress_dens(AdjArgs a)
+// k_adj_v: G gathers the stress phase into the velocity adjoints; D takes them
+// on to the velocity update of the step before: densities, stress-auxiliary
+// adjoints and the buoyancy gradients (D without G starts a segment of
+// records, G without D ends one).  The stores come after every load, which
+// the compiler cannot reorder.
+template <bool SEL>
+__device__ __forceinline__ void gather_vel(const AdjArgs &a, Loc p, unsigned m, float &vx, float &vy, float &vz)
+{
+    fresh(p);
+    const Gather<0, SEL> x{a, p, m};
+    const Gather<1, SEL> y{a, p, m};
+    const Gather<2, SEL> z{a, p, m};
+    vx = vx + (x.bwd(a.D[0]) + y.fwd(a.D[8], a.D[7]) + z.fwd(a.D[6], a.D[5]));
+    vy = vy + (y.bwd(a.D[1]) + x.fwd(a.D[7]) + z.fwd(a.D[4], a.D[3]));
+    vz = vz + (z.bwd(a.D[2]) + x.fwd(a.D[5]) + y.fwd(a.D[3]));
+}
+
+template <bool G, bool D>
+__global__ void __launch_bounds__(256) k_adj_v(AdjArgs a)
 {
     ADJ_CELL(a) {
+        float vx = ld(a.aF[FVX], p), vy = ld(a.aF[FVY], p), vz = ld(a.aF[FVZ], p);
+        if (G) {
+            const unsigned m = __float_as_uint(ld((const float *)a.nbr, p));
+            if (__any(m & NBR_ANY_PML)) gather_vel<true>(a, p, m, vx, vy, vz);
+            else gather_vel<false>(a, p, m, vx, vy, vz);
+        }
+        if (!D) {
+            fresh(p);
+            st<false>(a.aF[FVX], p, vx);
+            st<false>(a.aF[FVY], p, vy);
+            st<false>(a.aF[FVZ], p, vz);
+            return;
+        }
+        fresh(p);
         const int kind = cell_kind(a, i, j, k);
-        const long long p = gidx(g, i, j, k);
-        const float lam = a.lam[p], mu = a.mu[p];
-        const float sxx = a.aF[FSXX][p], syy = a.aF[FSYY][p], szz = a.aF[FSZZ][p];
+        const float r0 = ld(a.rho, p);
+        const float sx = r0 + AT(a.rho, 1, 0, 0), sy = r0 + AT(a.rho, 0, 1, 0), sz = r0 + AT(a.rho, 0, 0, 1);
+        const float bx = ld(a.gb[0], p), by = ld(a.gb[1], p), bz = ld(a.gb[2], p);
+        const float wx = 2.0f / sx * a.dt * vx, wy = 2.0f / sy * a.dt * vy, wz = 2.0f / sz * a.dt * vz;
+        const float *Sxx = a.fF[FSXX], *Syy = a.fF[FSYY], *Szz = a.fF[FSZZ];
+        const float *Syz = a.fF[FSYZ], *Sxz = a.fF[FSXZ], *Sxy = a.fF[FSXY];
+        float fx, fy, fz;
+        if (kind == 1) {
+            fresh(p);
+            float ax, bx4, ay, by4, az, bz4;
+            const bool in = pairs_at(a, i, j, k, ax, bx4, ay, by4, az, bz4);
+            fx = FWD4(Sxx, 1, 0, 0, ax, bx4) + BWD4(Sxy, 0, 1, 0, ay, by4) + BWD4(Sxz, 0, 0, 1, az, bz4);
+            fy = BWD4(Sxy, 1, 0, 0, ax, bx4) + FWD4(Syy, 0, 1, 0, ay, by4) + BWD4(Syz, 0, 0, 1, az, bz4);
+            fz = BWD4(Sxz, 1, 0, 0, ax, bx4) + BWD4(Syz, 0, 1, 0, ay, by4) + FWD4(Szz, 0, 0, 1, az, bz4);
+            // one density per component for its three derivatives, in W0, W3, W6
+            const float al = in ? 1.0f : NEAR_OFF_BAND;
+            st<false>(a.W[0], p, al * wx);
+            st<false>(a.W[3], p, al * wy);
+            st<false>(a.W[6], p, al * wz);
+        } else {
+            fresh(p);
+            const long long q = ade_index(a, i, j, k);
+            const long long n = a.npml;
+            const float4 gp[9] = {prof(a.gxe, i), prof(a.gyc, j), prof(a.gzc, k), prof(a.gxc, i), prof(a.gye, j),
+                                  prof(a.gzc, k), prof(a.gxc, i), prof(a.gyc, j), prof(a.gze, k)};
+            const float w[9] = {wx, wx, wx, wy, wy, wy, wz, wz, wz};
+            const float der[9] = {FWD2(Sxx, 1, 0, 0, a.hx), BWD2(Sxy, 0, 1, 0, a.hy), BWD2(Sxz, 0, 0, 1, a.hz),
+                                  BWD2(Sxy, 1, 0, 0, a.hx), FWD2(Syy, 0, 1, 0, a.hy), BWD2(Syz, 0, 0, 1, a.hz),
+                                  BWD2(Sxz, 1, 0, 0, a.hx), BWD2(Syz, 0, 1, 0, a.hy), FWD2(Szz, 0, 0, 1, a.hz)};
+            float ahat[9], fa[9];
+#pragma unroll
+            for (int c = 0; c < 9; ++c) {
+                ahat[c] = a.aA[(long long)(A_axSxx + c) * n + q];
+                fa[c] = a.fA[(long long)c * n + q];
+            }
+            float f[3] = {0.0f, 0.0f, 0.0f}, d[9];
+#pragma unroll
+            for (int c = 0; c < 9; ++c) {
+                d[c] = gp[c].x * w[c] + gp[c].w * a.dt * ahat[c];
+                f[c / 3] += gp[c].x * der[c] + gp[c].y * fa[c];
+            }
+#pragma unroll
+            for (int c = 0; c < 9; ++c) a.aA[(long long)(A_axSxx + c) * n + q] = gp[c].y * w[c] + gp[c].z * ahat[c];
+#pragma unroll
+            for (int c = 0; c < 9; ++c) st<false>(a.W[c], p, d[c]);
+            fx = f[0]; fy = f[1]; fz = f[2];
+        }
+        fresh(p);
+        if (G) {
+            st<false>(a.aF[FVX], p, vx);
+            st<false>(a.aF[FVY], p, vy);
+            st<false>(a.aF[FVZ], p, vz);
+        }
+        st<false>(a.gb[0], p, bx + -2.0f / (sx * sx) * a.dt * fx * vx);
+        st<false>(a.gb[1], p, by + -2.0f / (sy * sy) * a.dt * fy * vy);
+        st<false>(a.gb[2], p, bz + -2.0f / (sz * sz) * a.dt * fz * vz);
+    }
+}
+
+// k_adj_s: the velocity phase gathered into the stress adjoints, then the
+// stress update's densities, velocity- and memory-variable adjoints, and the
+// gradients of lam, of mu's own part and of the three shear moduli.
+// NM memory variables per component (a template argument, so their loops
+// unroll); the stores come after every load.
+template <bool SEL>
+__device__ __forceinline__ void gather_str(const AdjArgs &a, Loc p, unsigned m, float s[6])
+{
+    fresh(p);
+    const Gather<0, SEL> x{a, p, m};
+    const Gather<1, SEL> y{a, p, m};
+    const Gather<2, SEL> z{a, p, m};
+    s[0] = s[0] + x.fwd(a.W[0]);
+    s[1] = s[1] + y.fwd(a.W[4], a.W[3]);
+    s[2] = s[2] + z.fwd(a.W[8], a.W[6]);
+    s[3] = s[3] + (z.bwd(a.W[5], a.W[3]) + y.bwd(a.W[7], a.W[6]));
+    s[4] = s[4] + (z.bwd(a.W[2], a.W[0]) + x.bwd(a.W[6]));
+    s[5] = s[5] + (y.bwd(a.W[1], a.W[0]) + x.bwd(a.W[3]));
+}
+
+template <int NM>
+__global__ void __launch_bounds__(256) k_adj_s(AdjArgs a)
+{
+    ADJ_CELL(a) {
+        const unsigned m = __float_as_uint(ld((const float *)a.nbr, p));
+        float s[6];   // xx yy zz yz xz xy
+#pragma unroll
+        for (int c = 0; c < 6; ++c) s[c] = ld(a.aF[FSXX + c], p);
+        if (__any(m & NBR_ANY_PML)) gather_str<true>(a, p, m, s);
+        else gather_str<false>(a, p, m, s);
+        fresh(p);
+        const float sxx = s[0], syy = s[1], szz = s[2], syz = s[3], sxz = s[4], sxy = s[5];
+        const int kind = cell_kind(a, i, j, k);
+        const float lam = ld(a.lam, p), mu = ld(a.mu, p);
         const float X = a.dt * ((lam + 2.0f * mu) * sxx + lam * (syy + szz));
         const float Y = a.dt * ((lam + 2.0f * mu) * syy + lam * (sxx + szz));
         const float Z = a.dt * ((lam + 2.0f * mu) * szz + lam * (sxx + syy));
@@ -363,18 +395,18 @@ __global__ void __launch_bounds__(256) k_adj_stress_dens(AdjArgs a)
         const float hyz = hmean4(mu, m001, m010, m011);
         const float hxz = hmean4(mu, m001, m100, m101);
         const float hxy = hmean4(mu, m100, m010, m110);
-        const float syz = a.aF[FSYZ][p], sxz = a.aF[FSXZ][p], sxy = a.aF[FSXY][p];
         const float Wyz = a.dt * hyz * syz, Wxz = a.dt * hxz * sxz, Wxy = a.dt * hxy * sxy;
         const float *Vx = a.fF[FVX], *Vy = a.fF[FVY], *Vz = a.fF[FVZ];
-        const float glo = a.g_lam[p], gmo = a.g_mu[p];
+        const float glo = ld(a.g_lam, p), gmo = ld(a.g_mu, p);
+        const float hyo = ld(a.gh[0], p), hxo = ld(a.gh[1], p), hzo = ld(a.gh[2], p);
         float ex, ey, ez, tyz, txz, txy;
-        float qyz, qxz, qxy;   // shear-mu terms of the three quads
+        float qyz, qxz, qxy;   // gradients of the three shear moduli
         float d[9], dgl, dgm;
+        bool in = false;
         if (kind == 1) {
+            fresh(p);
             float ax, bx, ay, by, az, bz;
-            pair_at(a, 0, i, j, k, ax, bx);
-            pair_at(a, 1, i, j, k, ay, by);
-            pair_at(a, 2, i, j, k, az, bz);
+            in = pairs_at(a, i, j, k, ax, bx, ay, by, az, bz);
             ex = BWD4(Vx, 1, 0, 0, ax, bx);
             ey = BWD4(Vy, 0, 1, 0, ay, by);
             ez = BWD4(Vz, 0, 0, 1, az, bz);
@@ -383,7 +415,7 @@ __global__ void __launch_bounds__(256) k_adj_stress_dens(AdjArgs a)
             txy = FWD4(Vy, 1, 0, 0, ax, bx) + FWD4(Vx, 0, 1, 0, ay, by);
             if (NM > 0) {
                 // transposed memory variables and weighted stress sums
-                const float taup = a.taup[p], taus = a.taus[p];
+                const float taup = ld(a.taup, p), taus = ld(a.taus, p);
                 const float tp1 = 1.0f + taup * (1.0f + a.d2), ts1 = 1.0f + taus * (1.0f + a.d2);
                 const float as6[6] = {sxx, syy, szz, syz, sxz, sxy};
                 const long long r = ((long long)(k - g.kb) * g.nyk + (j - g.jb)) * g.rpitch + (i - 1);
@@ -463,53 +495,55 @@ __global__ void __launch_bounds__(256) k_adj_stress_dens(AdjArgs a)
             qxz = a.dt * txz * sxz;
             qxy = a.dt * txy * sxy;
         }
-        // quads: yz (o, o+z, o+y, o+y+z), xz (o, o+z, o+x, o+x+z), xy (o, o+x, o+y, o+x+y);
-        // their weights are taken here, late, to keep registers free above
-        float gyz[4], gxz[4], gxy[4];
-        hmean4_w(mu, m001, m010, m011, gyz);
-        hmean4_w(mu, m001, m100, m101, gxz);
-        hmean4_w(mu, m100, m010, m110, gxy);
+        fresh(p);
         // interior cells: d[3] = d[4], d[5] = d[6], d[7] = d[8], kept in D3, D5, D7
         if (kind == 1) {
-            a.D[0][p] = d[0]; a.D[1][p] = d[1]; a.D[2][p] = d[2];
-            a.D[3][p] = d[3]; a.D[5][p] = d[5]; a.D[7][p] = d[7];
+            const float al = in ? 1.0f : NEAR_OFF_BAND;
+            st<false>(a.D[0], p, al * d[0]); st<false>(a.D[1], p, al * d[1]); st<false>(a.D[2], p, al * d[2]);
+            st<false>(a.D[3], p, al * d[3]); st<false>(a.D[5], p, al * d[5]); st<false>(a.D[7], p, al * d[7]);
         } else {
 #pragma unroll
-            for (int c = 0; c < 9; ++c) a.D[c][p] = d[c];
+            for (int c = 0; c < 9; ++c) st<false>(a.D[c], p, d[c]);
         }
-        a.g_lam[p] = glo + dgl;
-        a.g_mu[p] = (gmo + dgm) + (qyz * gyz[0] + qxz * gxz[0] + qxy * gxy[0]);
-        a.q[0][p] = qyz * gyz[1] + qxz * gxz[1];
-        a.q[1][p] = qyz * gyz[2] + qxy * gxy[2];
-        a.q[2][p] = qxz * gxz[2] + qxy * gxy[1];
-        a.q[3][p] = qyz * gyz[3];
-        a.q[4][p] = qxz * gxz[3];
-        a.q[5][p] = qxy * gxy[3];
+        fresh(p);
+#pragma unroll
+        for (int c = 0; c < 6; ++c) st<false>(a.aF[FSXX + c], p, s[c]);
+        st<false>(a.g_lam, p, glo + dgl);
+        st<false>(a.g_mu, p, gmo + dgm);
+        st<false>(a.gh[0], p, hyo + qyz);
+        st<false>(a.gh[1], p, hxo + qxz);
+        st<false>(a.gh[2], p, hzo + qxy);
     }
 }
 
-// adjoint of the stress update: velocity adjoints and the shear terms of
-// the mu gradient left by the neighbouring cells (0 outside the cells)
-__global__ void __launch_bounds__(256) k_adj_stress_gather(AdjArgs a)
+
+// One source's gradients added to the sums: lam as it is; rho from the two
+// cells of each buoyancy; mu from its own part and, for each shear modulus
+// that a cell enters (the harmonic mean of four cells, an origin o and o + one
+// or two unit steps), that modulus's derivative with respect to the cell.
+// Entries outside the cells are zero.
+__global__ void __launch_bounds__(256) k_adj_finish(AdjArgs a, float *sl, float *sm, float *sr)
 {
     ADJ_CELL(a) {
-        const long long p = gidx(g, i, j, k);
-        const long long sx = 1, sy = g.pitch, sz = g.plane;
-        const AxisW wx = axis_w(a.cls, p, sx, a.tA[0], a.tB[0]);
-        const AxisW wy = axis_w(a.cls, p, sy, a.tA[1], a.tB[1]);
-        const AxisW wz = axis_w(a.cls, p, sz, a.tA[2], a.tB[2]);
-        const float vx = gat_bwd(a.D[0], p, sx, wx) + gat_fwd_s(a.D[8], a.D[7], p, sy, wy) +
-                         gat_fwd_s(a.D[6], a.D[5], p, sz, wz);
-        const float vy = gat_bwd(a.D[1], p, sy, wy) + gat_fwd(a.D[7], p, sx, wx) +
-                         gat_fwd_s(a.D[4], a.D[3], p, sz, wz);
-        const float vz = gat_bwd(a.D[2], p, sz, wz) + gat_fwd(a.D[5], p, sx, wx) + gat_fwd(a.D[3], p, sy, wy);
-        const float gm = a.q[0][p - sz] + a.q[1][p - sy] + a.q[2][p - sx] + a.q[3][p - sy - sz] + a.q[4][p - sx - sz] +
-                         a.q[5][p - sx - sy];
-        const float ox = a.aF[FVX][p], oy = a.aF[FVY][p], oz = a.aF[FVZ][p], om = a.g_mu[p];
-        a.aF[FVX][p] = ox + vx;
-        a.aF[FVY][p] = oy + vy;
-        a.aF[FVZ][p] = oz + vz;
-        a.g_mu[p] = om + gm;
+        const long long X = 1, Y = g.pitch, Z = g.plane, c = p.u + (p.o >> 2);
+        const float gr = a.gb[0][c] + a.gb[1][c] + a.gb[2][c] + a.gb[0][c - X] + a.gb[1][c - Y] + a.gb[2][c - Z];
+        float gm = a.g_mu[c];
+        // quads yz (o, o+z, o+y, o+y+z), xz (o, o+z, o+x, o+x+z), xy (o, o+x, o+y, o+x+y)
+        const long long e1[3] = {Z, Z, X}, e2[3] = {Y, X, Y};
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+#pragma unroll
+            for (int n = 0; n < 4; ++n) {
+                const long long o = c - ((n & 1) ? e1[q] : 0) - ((n & 2) ? e2[q] : 0);
+                const float gq = a.gh[q][o];
+                if (gq == 0.0f) continue;
+                float w[4];
+                hmean4_w(a.mu[o], a.mu[o + e1[q]], a.mu[o + e2[q]], a.mu[o + e1[q] + e2[q]], w);
+                gm += gq * w[n];
+            }
+        sl[c] = sl[c] + a.g_lam[c];
+        sm[c] = sm[c] + gm;
+        sr[c] = sr[c] + gr;
     }
 }
 
@@ -542,13 +576,6 @@ __global__ void k_fill(float *p, long long n)
         p[t] = 0.0f;
 }
 
-// sum += part, one rounding per element
-__global__ void k_add(float *sum, const float *part, long long n)
-{
-    for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < n; t += (long long)gridDim.x * blockDim.x)
-        sum[t] = sum[t] + part[t];
-}
-
 }  // namespace
 
 // ---------------------------------------------------------------------------
@@ -559,8 +586,9 @@ struct AdjSizes {
     long long nf, na18, nR;
     long long state() const { return 9 * nf + na18 + nR; }  // checkpoint: V, S, auxiliaries, R
     long long sstep() const { return 9 * nf + na18; }       // per-step record: V_n, S_{n+1}, aV_n, aS_n
-    long long cls() const { return (nf + 3) / 4; }           // point classes, one byte each
-    long long base() const { return 30 * nf + cls() + na18 + nR; }  // adjoint fields, densities, q, gradients, sums, classes, aR
+    // adjoint fields 9, velocity densities 9 (the stress phase's use the context's fields), staggered gradients 6,
+    // lam and mu 2, sums 3, neighbour words 1, and aA, aR
+    long long base() const { return 30 * nf + na18 + nR; }
 };
 
 namespace {
@@ -623,10 +651,11 @@ long long scheme_floats(const AdjSizes &z, int nt, int c1, int c2)
 // gradient sums, and checkpoint stores that grow to the largest scheme used.
 struct AdjWorkspace {
     AdjSizes z;
-    float *adjF = nullptr, *adjA = nullptr, *dens = nullptr, *qq = nullptr, *adjR = nullptr;
-    float *gsrc = nullptr;  // one source's gradients, summed over its steps
+    float *adjF = nullptr, *adjA = nullptr, *dens = nullptr, *adjR = nullptr;
+    float *gst = nullptr;   // one source's gradients at the staggered points: gb 3, gh 3
+    float *gsrc = nullptr;  // one source's gradients of lam and of mu's own part
     float *grad = nullptr;  // the sums over sources
-    float *cls = nullptr;   // point classes (bytes)
+    float *nbr = nullptr;   // neighbour words
     float *ck = nullptr, *seg = nullptr, *obs = nullptr;
     // record table for 6 nst targets: tgt (long long) | ptr (6 nst + 1 int) | src (6 nst int)
     float *rec = nullptr;
@@ -686,16 +715,12 @@ int ws_open(swpc_ctx *c)
     w.z = sizes_of(c);
     const long long nf = w.z.nf;
     if (!walloc(c, w.adjF, 9 * nf, nf) || !walloc(c, w.adjA, w.z.na18, c->npml) || !walloc(c, w.dens, 9 * nf, nf) ||
-        !walloc(c, w.qq, 6 * nf, nf) || !walloc(c, w.gsrc, 3 * nf, nf) || !walloc(c, w.grad, 3 * nf, nf) ||
-        !walloc(c, w.cls, w.z.cls()) || !walloc(c, w.adjR, w.z.nR, c->g.rn)) {
+        !walloc(c, w.gst, 6 * nf, nf) || !walloc(c, w.gsrc, 2 * nf, nf) || !walloc(c, w.grad, 3 * nf, nf) ||
+        !walloc(c, w.nbr, nf) || !walloc(c, w.adjR, w.z.nR, c->g.rn)) {
         swpc_adj_release(c);
         return ctx_fail(c, SWPC_ENOMEM, "adjoint: device memory for the adjoint fields");
     }
-    // the density kernels write every cell and never the halo, where the
-    // gathers then read zeros
-    if (zero(w.grad, 3 * nf, c->stream) != hipSuccess || zero(w.dens, 9 * nf, c->stream) != hipSuccess ||
-        zero(w.qq, 6 * nf, c->stream) != hipSuccess)
-        return SWPC_EHIP;
+    if (zero(w.grad, 3 * nf, c->stream) != hipSuccess) return SWPC_EHIP;
     return SWPC_OK;
 }
 
@@ -722,8 +747,8 @@ extern "C" int swpc_adj_release(swpc_ctx *c)
     AdjWorkspace &w = *c->adj_ws;
     const long long nf = w.z.nf;
     wfree(c, w.adjF, 9 * nf); wfree(c, w.adjA, w.z.na18); wfree(c, w.dens, 9 * nf);
-    wfree(c, w.qq, 6 * nf); wfree(c, w.gsrc, 3 * nf); wfree(c, w.grad, 3 * nf); wfree(c, w.adjR, w.z.nR);
-    wfree(c, w.cls, w.z.cls());
+    wfree(c, w.gst, 6 * nf); wfree(c, w.gsrc, 2 * nf); wfree(c, w.grad, 3 * nf); wfree(c, w.adjR, w.z.nR);
+    wfree(c, w.nbr, nf);
     wfree(c, w.ck, w.ck_n); wfree(c, w.seg, w.seg_n); wfree(c, w.obs, w.obs_n); wfree(c, w.rec, w.rec_n);
     delete c->adj_ws;
     c->adj_ws = nullptr;
@@ -978,27 +1003,27 @@ extern "C" int swpc_adj_accumulate(swpc_ctx *c, int nt, const float *obs, int ck
     a.npml = c->npml;
     a.has_pml = 1;
     a.gxc = c->gxc; a.gxe = c->gxe; a.gyc = c->gyc; a.gye = c->gye; a.gzc = c->gzc; a.gze = c->gze;
+    // the context's fields hold nothing that is read again until a checkpoint
+    // is loaded: the stress phase's densities go there.  Density kernels write
+    // every cell and never the halo, where the gathers read zeros.
     for (int q = 0; q < 9; ++q) {
         a.aF[q] = w.adjF + q * nf;
-        a.D[q] = w.dens + q * nf;
+        a.W[q] = w.dens + q * nf;
+        a.D[q] = c->fields[q];
     }
-    for (int q = 0; q < 6; ++q) a.q[q] = w.qq + q * nf;
-    a.cls = (const unsigned char *)w.cls;
-    {
-        const float h[3] = {a.hx, a.hy, a.hz};
-        const float *p40[3] = {c->coef.re40x, c->coef.re40y, c->coef.re40z};
-        const float *p41[3] = {c->coef.re41x, c->coef.re41y, c->coef.re41z};
-        for (int ax = 0; ax < 3; ++ax) {
-            const float ta[4] = {0.0f, p40[ax][0], p40[ax][1], h[ax]}, tb[4] = {0.0f, p41[ax][0], p41[ax][1], 0.0f};
-            for (int q = 0; q < 4; ++q) { a.tA[ax][q] = ta[q]; a.tB[ax][q] = tb[q]; }
-        }
+    for (int q = 0; q < 3; ++q) {
+        a.gb[q] = w.gst + q * nf;
+        a.gh[q] = w.gst + (3 + q) * nf;
     }
+    a.nbr = (const unsigned *)w.nbr;
+    a.ratio = 1.0f / 27.0f;
     a.aA = w.adjA;
-    a.g_lam = w.gsrc; a.g_mu = w.gsrc + nf; a.g_rho = w.gsrc + 2 * nf;
+    a.g_lam = w.gsrc; a.g_mu = w.gsrc + nf;
     if (zero(w.adjF, 9 * nf, s) != hipSuccess || zero(w.adjA, na18, s) != hipSuccess ||
-        zero(w.gsrc, 3 * nf, s) != hipSuccess || (nR && zero(w.adjR, nR, s) != hipSuccess))
+        zero(w.dens, 9 * nf, s) != hipSuccess || zero(w.gst, 6 * nf, s) != hipSuccess ||
+        zero(w.gsrc, 2 * nf, s) != hipSuccess || (nR && zero(w.adjR, nR, s) != hipSuccess))
         return SWPC_EHIP;
-    hipLaunchKernelGGL(k_adj_class, dim3(1024), dim3(256), 0, s, a, (unsigned char *)w.cls);
+    hipLaunchKernelGGL(k_adj_nbr, dim3(4096), dim3(256), 0, s, a, (unsigned *)w.nbr);
     if (hipGetLastError() != hipSuccess) return SWPC_EHIP;
     const dim3 blk(64, 4, 1), grd(((((g.nx + 63) / 64) * ((g.ny + 3) / 4) + 7) & ~7) * g.nz);
     // record table: the distinct (field, point) targets of the stations'
@@ -1054,25 +1079,38 @@ extern "C" int swpc_adj_accumulate(swpc_ctx *c, int nt, const float *obs, int ck
     // the adjoint of steps n1-1 down to n0 from their records
     auto backward = [&](int n0, int n1) -> hipError_t {
         hipError_t e = hipSuccess;
+        auto stress_record = [&](int n) {   // S_{n+1} and the stress auxiliaries aS_n
+            const float *st = w.seg + (size_t)(n - n0) * sstep;
+            for (int q = 3; q < 9; ++q) a.fF[q] = st + q * nf;
+            a.fA = st + 9 * nf + na9;
+        };
+        // velocity densities of the last step (before the first injection the adjoint fields and densities are zero)
+        if (n1 < nt) {
+            stress_record(n1 - 1);
+            hipLaunchKernelGGL((k_adj_v<false, true>), grd, blk, 0, s, a);
+        }
         for (int n = n1 - 1; n >= n0 && e == hipSuccess; --n) {
             const float *st = w.seg + (size_t)(n - n0) * sstep;
-            for (int q = 0; q < 9; ++q) a.fF[q] = st + q * nf;
-            a.fA = st + 9 * nf + na9;      // stress auxiliaries aS_n
-            hipLaunchKernelGGL(k_adj_vel_dens, grd, blk, 0, s, a);
-            hipLaunchKernelGGL(k_adj_vel_gather, grd, blk, 0, s, a);
+            for (int q = 0; q < 3; ++q) a.fF[q] = st + q * nf;
             a.fA = st + 9 * nf;            // velocity auxiliaries aV_n
             switch (a.nm) {
 #define SWPC_ADJ_CASE(NMV) \
-    case NMV: hipLaunchKernelGGL((k_adj_stress_dens<NMV>), grd, blk, 0, s, a); break;
+    case NMV: hipLaunchKernelGGL((k_adj_s<NMV>), grd, blk, 0, s, a); break;
                 SWPC_ADJ_CASE(0) SWPC_ADJ_CASE(1) SWPC_ADJ_CASE(2) SWPC_ADJ_CASE(3) SWPC_ADJ_CASE(4)
                 SWPC_ADJ_CASE(5) SWPC_ADJ_CASE(6) SWPC_ADJ_CASE(7) SWPC_ADJ_CASE(8)
 #undef SWPC_ADJ_CASE
             default: break;
             }
-            hipLaunchKernelGGL(k_adj_stress_gather, grd, blk, 0, s, a);
+            // the traces sampled V_n, which the stress update of step n has read as well
             if (n % c->ntdec_w == 0 && n / c->ntdec_w < c->ntw)
                 hipLaunchKernelGGL(k_adj_record, dim3((ntgt + 63) / 64), dim3(64), 0, s, a, ntgt, rec_tgt, rec_ptr,
                                    rec_src, c->d_wav[0], w.obs, c->ntw, n / c->ntdec_w, sc);
+            if (n > n0) {
+                stress_record(n - 1);
+                hipLaunchKernelGGL((k_adj_v<true, true>), grd, blk, 0, s, a);
+            } else {
+                hipLaunchKernelGGL((k_adj_v<true, false>), grd, blk, 0, s, a);
+            }
             e = hipGetLastError();
         }
         return e;
@@ -1098,7 +1136,7 @@ extern "C" int swpc_adj_accumulate(swpc_ctx *c, int nt, const float *obs, int ck
         }
     }
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_add, dim3(1024), dim3(256), 0, s, w.grad, w.gsrc, 3 * nf);
+        hipLaunchKernelGGL(k_adj_finish, grd, blk, 0, s, a, w.grad, w.grad + nf, w.grad + 2 * nf);
         e = hipGetLastError();
     }
     if (e != hipSuccess) return ctx_fail(c, SWPC_EHIP, hipGetErrorString(e));
