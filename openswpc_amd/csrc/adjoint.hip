@@ -257,6 +257,11 @@ __device__ static inline void hmean4_w(float a, float b, float c, float d, float
     gr[3] = (4.0f * a * b * c * Dn - N * (a * b + a * c + b * c)) * r;
 }
 
+// Where an axis does not damp (the auxiliary's gain, entry 4, is zero) the
+// recorded auxiliaries are zero and their adjoints reach nothing: both stay
+// unread, and the adjoints unwritten, as the forward's auxiliaries do.
+__device__ __forceinline__ bool aux_on(const float4 &gc, const float4 &ge) { return gc.w != 0.0f || ge.w != 0.0f; }
+
 // k_adj_v: G gathers the stress phase into the velocity adjoints; D takes them
 // on to the velocity update of the step before: densities, stress-auxiliary
 // adjoints and the buoyancy gradients (D without G starts a segment of
@@ -322,12 +327,19 @@ __global__ void __launch_bounds__(256) k_adj_v(AdjArgs a)
             const float der[9] = {FWD2(Sxx, 1, 0, 0, a.hx), BWD2(Sxy, 0, 1, 0, a.hy), BWD2(Sxz, 0, 0, 1, a.hz),
                                   BWD2(Sxy, 1, 0, 0, a.hx), FWD2(Syy, 0, 1, 0, a.hy), BWD2(Syz, 0, 0, 1, a.hz),
                                   BWD2(Sxz, 1, 0, 0, a.hx), BWD2(Syz, 0, 1, 0, a.hy), FWD2(Szz, 0, 0, 1, a.hz)};
+            const bool on[3] = {aux_on(gp[3], gp[0]), aux_on(gp[1], gp[4]), aux_on(gp[2], gp[8])};
             float ahat[9], fa[9];
 #pragma unroll
-            for (int c = 0; c < 9; ++c) {
-                ahat[c] = a.aA[(long long)(A_axSxx + c) * n + q];
-                fa[c] = a.fA[(long long)c * n + q];
-            }
+            for (int c = 0; c < 9; ++c) ahat[c] = fa[c] = 0.0f;
+#pragma unroll
+            for (int ax = 0; ax < 3; ++ax)
+                if (on[ax]) {
+#pragma unroll
+                    for (int c = ax; c < 9; c += 3) {
+                        ahat[c] = a.aA[(long long)(A_axSxx + c) * n + q];
+                        fa[c] = a.fA[(long long)c * n + q];
+                    }
+                }
             float f[3] = {0.0f, 0.0f, 0.0f}, d[9];
 #pragma unroll
             for (int c = 0; c < 9; ++c) {
@@ -335,7 +347,12 @@ __global__ void __launch_bounds__(256) k_adj_v(AdjArgs a)
                 f[c / 3] += gp[c].x * der[c] + gp[c].y * fa[c];
             }
 #pragma unroll
-            for (int c = 0; c < 9; ++c) a.aA[(long long)(A_axSxx + c) * n + q] = gp[c].y * w[c] + gp[c].z * ahat[c];
+            for (int ax = 0; ax < 3; ++ax)
+                if (on[ax]) {
+#pragma unroll
+                    for (int c = ax; c < 9; c += 3)
+                        a.aA[(long long)(A_axSxx + c) * n + q] = gp[c].y * w[c] + gp[c].z * ahat[c];
+                }
 #pragma unroll
             for (int c = 0; c < 9; ++c) st<false>(a.W[c], p, d[c]);
             fx = f[0]; fy = f[1]; fz = f[2];
@@ -474,19 +491,33 @@ __global__ void __launch_bounds__(256) k_adj_s(AdjArgs a)
             const float der[9] = {BWD2(Vx, 1, 0, 0, a.hx), BWD2(Vy, 0, 1, 0, a.hy), BWD2(Vz, 0, 0, 1, a.hz),
                                   FWD2(Vz, 0, 1, 0, a.hy), FWD2(Vy, 0, 0, 1, a.hz), FWD2(Vz, 1, 0, 0, a.hx),
                                   FWD2(Vx, 0, 0, 1, a.hz), FWD2(Vy, 1, 0, 0, a.hx), FWD2(Vx, 0, 1, 0, a.hy)};
+            const int axis[9] = {0, 1, 2, 1, 2, 0, 2, 0, 1};
+            const bool on[3] = {aux_on(gp[0], gp[5]), aux_on(gp[1], gp[3]), aux_on(gp[2], gp[4])};
             float ahat[9], fa[9], t[9];
 #pragma unroll
-            for (int c = 0; c < 9; ++c) {
-                ahat[c] = a.aA[(long long)ai[c] * n + q];
-                fa[c] = a.fA[(long long)ai[c] * n + q];
-            }
+            for (int c = 0; c < 9; ++c) ahat[c] = fa[c] = 0.0f;
+#pragma unroll
+            for (int ax = 0; ax < 3; ++ax)
+                if (on[ax]) {
+#pragma unroll
+                    for (int c = 0; c < 9; ++c) {
+                        if (axis[c] != ax) continue;
+                        ahat[c] = a.aA[(long long)ai[c] * n + q];
+                        fa[c] = a.fA[(long long)ai[c] * n + q];
+                    }
+                }
 #pragma unroll
             for (int c = 0; c < 9; ++c) {
                 d[c] = gp[c].x * w[c] + gp[c].w * a.dt * ahat[c];
                 t[c] = gp[c].x * der[c] + gp[c].y * fa[c];
             }
 #pragma unroll
-            for (int c = 0; c < 9; ++c) a.aA[(long long)ai[c] * n + q] = gp[c].y * w[c] + gp[c].z * ahat[c];
+            for (int ax = 0; ax < 3; ++ax)
+                if (on[ax]) {
+#pragma unroll
+                    for (int c = 0; c < 9; ++c)
+                        if (axis[c] == ax) a.aA[(long long)ai[c] * n + q] = gp[c].y * w[c] + gp[c].z * ahat[c];
+                }
             ex = t[0]; ey = t[1]; ez = t[2];
             tyz = t[3] + t[4]; txz = t[5] + t[6]; txy = t[7] + t[8];
             dgl = a.dt * (ex + ey + ez) * (sxx + syy + szz);
@@ -945,6 +976,7 @@ extern "C" int swpc_adj_accumulate(swpc_ctx *c, int nt, const float *obs, int ck
     hipError_t e = hipSuccess;
     for (int q = 0; q < SWPC_NFIELD && e == hipSuccess; ++q) e = zero(c->fields[q], nf, s);
     if (e == hipSuccess) e = zero(c->ade, na18, s);
+    c->aux_still = true;   // from zero under the profiles as they are
     if (e == hipSuccess && nR) e = zero(c->R, nR, s);
     if (e == hipSuccess && c->d_uacc) e = zero(c->d_uacc, 3LL * c->nst, s);
     if (e == hipSuccess && c->d_eacc) e = zero(c->d_eacc, 6LL * c->nst, s);

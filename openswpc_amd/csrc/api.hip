@@ -361,6 +361,7 @@ extern "C" int swpc_create(const swpc_desc *d, swpc_ctx **out)
             c->box[q] = b[q];
         }
         c->npml = off;
+        c->aux_still = true;
         ALLOC_STRIPED(c->ade, (size_t)A_N * c->npml * sizeof(float), kAuxRegion, A_N, (size_t)c->npml * sizeof(float));
         ALLOC(c->gxc, (size_t)nx * sizeof(float4));
         ALLOC(c->gxe, (size_t)nx * sizeof(float4));
@@ -530,6 +531,7 @@ extern "C" int swpc_set_pml(swpc_ctx *c, const float *gxc, const float *gxe, con
     HIPCHK(c, hipMemcpyAsync(c->gzc, gzc, (size_t)g.nz * 16, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipMemcpyAsync(c->gze, gze, (size_t)g.nz * 16, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    if (c->aux_moved) c->aux_still = false;
     c->has_pml = true;
     reset_graph(c);
     return SWPC_OK;

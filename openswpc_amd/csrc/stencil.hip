@@ -110,6 +110,7 @@ struct StepArgs {
     int ntiles;
     int sideb;           // blocks of a launch that walk the side tiles (a multiple of 8, >= ntiles; 0: none)
     int has_pml, mask;
+    int still;           // see aux_on
     // Cerjan profiles at cell centres (c) and boundaries (b), halo of 3: entry of cell n is n + 2
     const float *cgx_c, *cgx_b, *cgy_c, *cgy_b, *cgz_c, *cgz_b;
     // interior launch shape
@@ -164,11 +165,25 @@ __device__ static inline PmlBox pick_box(const StepArgs &a, int q)
     return q == 0 ? a.box[0] : q == 1 ? a.box[1] : q == 2 ? a.box[2] : q == 3 ? a.box[3] : a.box[4];
 }
 
+// Whether a cell's auxiliaries of one axis take part.  Where the axis does not
+// damp (profile entry 4, the gain of the auxiliary, is zero at the centre and
+// at the edge) they start at zero and stay there, and a zero adds nothing to
+// the derivative: neither they nor their update is needed.  Only the cells in
+// the edges and corners of the zones keep all nine of a phase; a cell of a
+// face keeps three, 24 of 72 bytes (us per step with all nine and with the
+// ones that take part: 128^3 557 -> 528, elastic 256 x 256 x 192 522 -> 469,
+// 768 x 768 x 448 13260 -> 12770).  still: no auxiliary has moved under other
+// profiles (swpc_set_pml).
+__device__ __forceinline__ bool aux_on(const StepArgs &a, const float4 &gc, const float4 &ge)
+{
+    return !(a.still && gc.w == 0.0f && ge.w == 0.0f);
+}
+
 // absorb_p__update_stress for one cell, m_absorb_p.f90:455-517.  The caller
 // passes its z-queue values: V at k (and k+1 for Vx, Vy; k-1 for Vz) and mu
 // on planes k, k+1.
 template <bool NT, bool OOP>
-__device__ __forceinline__ void pml_stress_cell(const StepArgs &a, const Loc &p, const Loc &q, int k, float vx_0,
+__device__ __forceinline__ void pml_stress_cell(const StepArgs &a, Loc p, Loc q, int k, float vx_0,
                                                 float vx_p1, float vy_0, float vy_p1, float vz_m1, float vz_0,
                                                 float mu00, float mu00n, float mu10, float mu10n, float mu01,
                                                 float mu01n, float mu11, float4 gxc, float4 gxe, float4 gyc,
@@ -189,10 +204,23 @@ __device__ __forceinline__ void pml_stress_cell(const StepArgs &a, const Loc &p,
     const float vx_jp1 = ld(Vx, p, 0, 0, 1), vz_jp1 = ld(Vz, p, 0, 0, 1);
     const float4 gzc = ldp(a.gzc + (k - 1)), gze = ldp(a.gze + (k - 1));
     const float lam0 = ld<NT>(a.m.lam, p);
-    const float axVx = ld<NT>(AI, q, A_axVx * n), ayVy = ld<NT>(AI, q, A_ayVy * n), azVz = ld<NT>(AI, q, A_azVz * n);
-    const float ayVx = ld<NT>(AI, q, A_ayVx * n), azVx = ld<NT>(AI, q, A_azVx * n);
-    const float axVy = ld<NT>(AI, q, A_axVy * n), azVy = ld<NT>(AI, q, A_azVy * n);
-    const float axVz = ld<NT>(AI, q, A_axVz * n), ayVz = ld<NT>(AI, q, A_ayVz * n);
+    const bool onx = aux_on(a, gxc, gxe), ony = aux_on(a, gyc, gye), onz = aux_on(a, gzc, gze);
+    float axVx = 0.0f, axVy = 0.0f, axVz = 0.0f;
+    float ayVx = 0.0f, ayVy = 0.0f, ayVz = 0.0f;
+    float azVx = 0.0f, azVy = 0.0f, azVz = 0.0f;
+    if (onx) {
+        fresh(q);
+        axVx = ld<NT>(AI, q, A_axVx * n); axVy = ld<NT>(AI, q, A_axVy * n); axVz = ld<NT>(AI, q, A_axVz * n);
+    }
+    if (ony) {
+        fresh(q);
+        ayVx = ld<NT>(AI, q, A_ayVx * n); ayVy = ld<NT>(AI, q, A_ayVy * n); ayVz = ld<NT>(AI, q, A_ayVz * n);
+    }
+    if (onz) {
+        fresh(q);
+        azVx = ld<NT>(AI, q, A_azVx * n); azVy = ld<NT>(AI, q, A_azVy * n); azVz = ld<NT>(AI, q, A_azVz * n);
+    }
+    fresh(p);
     float *__restrict__ Sxx = a.f.Sxx;
     float *__restrict__ Syy = a.f.Syy;
     float *__restrict__ Szz = a.f.Szz;
@@ -221,9 +249,6 @@ __device__ __forceinline__ void pml_stress_cell(const StepArgs &a, const Loc &p,
     st<NT>(Sxx, p, sxx + (lam2mu_R * dxVx_ade + lam_R * (dyVy_ade + dzVz_ade)) * dt);
     st<NT>(Syy, p, syy + (lam2mu_R * dyVy_ade + lam_R * (dxVx_ade + dzVz_ade)) * dt);
     st<NT>(Szz, p, szz + (lam2mu_R * dzVz_ade + lam_R * (dxVx_ade + dyVy_ade)) * dt);
-    st<NT>(A, q, gxc.z * axVx + gxc.w * dxVx * dt, A_axVx * n);
-    st<NT>(A, q, gyc.z * ayVy + gyc.w * dyVy * dt, A_ayVy * n);
-    st<NT>(A, q, gzc.z * azVz + gzc.w * dzVz * dt, A_azVz * n);
 
     // shear components
     const float dxVy = (vy_ip1 - vy_0) * a.r20x;
@@ -238,18 +263,30 @@ __device__ __forceinline__ void pml_stress_cell(const StepArgs &a, const Loc &p,
     st<NT>(Syz, p, syz + muyz * (gye.x * dyVz + gze.x * dzVy + gye.y * ayVz + gze.y * azVy) * dt);
     st<NT>(Sxz, p, sxz + muxz * (gxe.x * dxVz + gze.x * dzVx + gxe.y * axVz + gze.y * azVx) * dt);
     st<NT>(Sxy, p, sxy + muxy * (gxe.x * dxVy + gye.x * dyVx + gxe.y * axVy + gye.y * ayVx) * dt);
-    st<NT>(A, q, gye.z * ayVx + gye.w * dyVx * dt, A_ayVx * n);
-    st<NT>(A, q, gze.z * azVx + gze.w * dzVx * dt, A_azVx * n);
-    st<NT>(A, q, gxe.z * axVy + gxe.w * dxVy * dt, A_axVy * n);
-    st<NT>(A, q, gze.z * azVy + gze.w * dzVy * dt, A_azVy * n);
-    st<NT>(A, q, gxe.z * axVz + gxe.w * dxVz * dt, A_axVz * n);
-    st<NT>(A, q, gye.z * ayVz + gye.w * dyVz * dt, A_ayVz * n);
+    if (onx) {
+        fresh(q);
+        st<NT>(A, q, gxc.z * axVx + gxc.w * dxVx * dt, A_axVx * n);
+        st<NT>(A, q, gxe.z * axVy + gxe.w * dxVy * dt, A_axVy * n);
+        st<NT>(A, q, gxe.z * axVz + gxe.w * dxVz * dt, A_axVz * n);
+    }
+    if (ony) {
+        fresh(q);
+        st<NT>(A, q, gyc.z * ayVy + gyc.w * dyVy * dt, A_ayVy * n);
+        st<NT>(A, q, gye.z * ayVx + gye.w * dyVx * dt, A_ayVx * n);
+        st<NT>(A, q, gye.z * ayVz + gye.w * dyVz * dt, A_ayVz * n);
+    }
+    if (onz) {
+        fresh(q);
+        st<NT>(A, q, gzc.z * azVz + gzc.w * dzVz * dt, A_azVz * n);
+        st<NT>(A, q, gze.z * azVx + gze.w * dzVx * dt, A_azVx * n);
+        st<NT>(A, q, gze.z * azVy + gze.w * dzVy * dt, A_azVy * n);
+    }
 }
 
 // absorb_p__update_vel for one cell, m_absorb_p.f90:267-304.  Queue values:
 // Szz on k, k+1; Syz, Sxz on k-1, k; rho on k, k+1.
 template <bool OOP>
-__device__ __forceinline__ void pml_vel_cell(const StepArgs &a, const Loc &p, const Loc &q, int k, float szz_0,
+__device__ __forceinline__ void pml_vel_cell(const StepArgs &a, Loc p, Loc q, int k, float szz_0,
                                              float szz_p1, float syz_m1, float syz_0, float sxz_m1, float sxz_0,
                                              float rho0, float rho_kp, float4 gxc, float4 gxe, float4 gyc,
                                              float4 gye)
@@ -271,9 +308,23 @@ __device__ __forceinline__ void pml_vel_cell(const StepArgs &a, const Loc &p, co
     const float sxy_0 = ld(Sxy, p), sxy_im1 = ld(Sxy, p, 0, -1), sxy_jm1 = ld(Sxy, p, 0, 0, -1);
     const float rho_ip = ld(rho, p, 0, 1), rho_jp = ld(rho, p, 0, 0, 1);
     const float4 gzc = ldp(a.gzc + (k - 1)), gze = ldp(a.gze + (k - 1));
-    const float axSxx = ld<true>(AI, q, A_axSxx * n), aySxy = ld<true>(AI, q, A_aySxy * n), azSxz = ld<true>(AI, q, A_azSxz * n);
-    const float axSxy = ld<true>(AI, q, A_axSxy * n), aySyy = ld<true>(AI, q, A_aySyy * n), azSyz = ld<true>(AI, q, A_azSyz * n);
-    const float axSxz = ld<true>(AI, q, A_axSxz * n), aySyz = ld<true>(AI, q, A_aySyz * n), azSzz = ld<true>(AI, q, A_azSzz * n);
+    const bool onx = aux_on(a, gxc, gxe), ony = aux_on(a, gyc, gye), onz = aux_on(a, gzc, gze);
+    float axSxx = 0.0f, axSxy = 0.0f, axSxz = 0.0f;
+    float aySxy = 0.0f, aySyy = 0.0f, aySyz = 0.0f;
+    float azSxz = 0.0f, azSyz = 0.0f, azSzz = 0.0f;
+    if (onx) {
+        fresh(q);
+        axSxx = ld<true>(AI, q, A_axSxx * n); axSxy = ld<true>(AI, q, A_axSxy * n); axSxz = ld<true>(AI, q, A_axSxz * n);
+    }
+    if (ony) {
+        fresh(q);
+        aySxy = ld<true>(AI, q, A_aySxy * n); aySyy = ld<true>(AI, q, A_aySyy * n); aySyz = ld<true>(AI, q, A_aySyz * n);
+    }
+    if (onz) {
+        fresh(q);
+        azSxz = ld<true>(AI, q, A_azSxz * n); azSyz = ld<true>(AI, q, A_azSyz * n); azSzz = ld<true>(AI, q, A_azSzz * n);
+    }
+    fresh(p);
     float *__restrict__ Vx = a.f.Vx;
     float *__restrict__ Vy = a.f.Vy;
     float *__restrict__ Vz = a.f.Vz;
@@ -299,15 +350,24 @@ __device__ __forceinline__ void pml_vel_cell(const StepArgs &a, const Loc &p, co
                                                 + gxc.y * axSxy + gye.y * aySyy + gzc.y * azSyz) * dt);
     st<true>(Vz, p, vz + bz * (gxc.x * dxSxz + gyc.x * dySyz + gze.x * dzSzz
                                                 + gxc.y * axSxz + gyc.y * aySyz + gze.y * azSzz) * dt);
-    st<true>(A, q, gxe.z * axSxx + gxe.w * dxSxx * dt, A_axSxx * n);
-    st<true>(A, q, gyc.z * aySxy + gyc.w * dySxy * dt, A_aySxy * n);
-    st<true>(A, q, gzc.z * azSxz + gzc.w * dzSxz * dt, A_azSxz * n);
-    st<true>(A, q, gxc.z * axSxy + gxc.w * dxSxy * dt, A_axSxy * n);
-    st<true>(A, q, gye.z * aySyy + gye.w * dySyy * dt, A_aySyy * n);
-    st<true>(A, q, gzc.z * azSyz + gzc.w * dzSyz * dt, A_azSyz * n);
-    st<true>(A, q, gxc.z * axSxz + gxc.w * dxSxz * dt, A_axSxz * n);
-    st<true>(A, q, gyc.z * aySyz + gyc.w * dySyz * dt, A_aySyz * n);
-    st<true>(A, q, gze.z * azSzz + gze.w * dzSzz * dt, A_azSzz * n);
+    if (onx) {
+        fresh(q);
+        st<true>(A, q, gxe.z * axSxx + gxe.w * dxSxx * dt, A_axSxx * n);
+        st<true>(A, q, gxc.z * axSxy + gxc.w * dxSxy * dt, A_axSxy * n);
+        st<true>(A, q, gxc.z * axSxz + gxc.w * dxSxz * dt, A_axSxz * n);
+    }
+    if (ony) {
+        fresh(q);
+        st<true>(A, q, gyc.z * aySxy + gyc.w * dySxy * dt, A_aySxy * n);
+        st<true>(A, q, gye.z * aySyy + gye.w * dySyy * dt, A_aySyy * n);
+        st<true>(A, q, gyc.z * aySyz + gyc.w * dySyz * dt, A_aySyz * n);
+    }
+    if (onz) {
+        fresh(q);
+        st<true>(A, q, gzc.z * azSxz + gzc.w * dzSxz * dt, A_azSxz * n);
+        st<true>(A, q, gzc.z * azSyz + gzc.w * dzSyz * dt, A_azSyz * n);
+        st<true>(A, q, gze.z * azSzz + gze.w * dzSzz * dt, A_azSzz * n);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1075,6 +1135,8 @@ void fill_step_args(swpc_ctx *c, StepArgs &a, int mask)
     a.sideb = 0;
     a.cgx_c = c->cgx_c; a.cgx_b = c->cgx_b; a.cgy_c = c->cgy_c; a.cgy_b = c->cgy_b; a.cgz_c = c->cgz_c; a.cgz_b = c->cgz_b;
     a.has_pml = (c->desc.abc == SWPC_ABC_PML && c->npml > 0) ? 1 : 0;
+    a.still = c->aux_still ? 1 : 0;
+    c->aux_moved = true;
     a.mask = mask;
     a.by = c->by;
     a.zc = c->d_zchunks;

@@ -130,6 +130,9 @@ struct swpc_ctx {
     PmlBox box[5];
     long long npml;
     float *ade;
+    // every auxiliary on an axis that does not damp its cell is zero: true
+    // until the profiles are replaced after a step (aux_moved)
+    bool aux_still, aux_moved;
     float4 *gxc, *gxe, *gyc, *gye, *gzc, *gze;
     int *d_pml_tiles;  // int4 (i0 | width << 20 | xslab << 28, j0, k0, k1) per side-column tile
     int npml_tiles;

@@ -62,3 +62,27 @@ def test_taper_applied_by_the_update(orc, nx, ny, nz, kchunk, force):
         h.source_bodyforce(it)
     for n in O.FIELDS_V + O.FIELDS_S:
         assert np.array_equal(h.get_field(n), g.get_field(n)), n
+
+
+@pytest.mark.parametrize("nx,ny,nz,na", [(40, 36, 32, 8), (67, 13, 14, 6), (9, 70, 12, 4)])
+def test_profiles_replaced_between_steps(orc, nx, ny, nz, na):
+    """The auxiliaries of an axis that does not damp a cell are left alone,
+    unless they have moved under earlier profiles: a context whose profiles
+    are set again after an update of a field at rest takes every auxiliary
+    from then on, and both forms agree before and after the damping moves to
+    other cells."""
+    m = _model(nx=nx, ny=ny, nz=nz, na=na, nm=1, sources=[MT])
+    run = O.OracleRun(m, 32)
+    run.run(12)
+    prof = [m.gxc, m.gxe, m.gyc, m.gye, m.gzc, m.gze]
+    moved = [np.roll(p, 3 * 4) for p in prof]   # four numbers a cell
+    g, h = gpu_from_model(m), gpu_from_model(m)
+    h.update_stress()
+    h.set_pml(*prof)
+    for c in (g, h):
+        c.step(1, 12)
+        _same(c, run, f"{nx}x{ny}x{nz} na={na}")
+        c.set_pml(*moved)
+        c.step(1, 6)
+    for n in O.FIELDS_V + O.FIELDS_S:
+        assert np.array_equal(h.get_field(n), g.get_field(n)), n
