@@ -171,7 +171,7 @@ __device__ static inline PmlBox pick_box(const StepArgs &a, int q)
 // the derivative: neither they nor their update is needed.  Only the cells in
 // the edges and corners of the zones keep all nine of a phase; a cell of a
 // face keeps three, 24 of 72 bytes (us per step with all nine and with the
-// ones that take part: 128^3 557 -> 528, elastic 256 x 256 x 192 522 -> 469,
+// ones that take part: 128^3 139 -> 132, elastic 256 x 256 x 192 522 -> 469,
 // 768 x 768 x 448 13260 -> 12770).  still: no auxiliary has moved under other
 // profiles (swpc_set_pml).
 __device__ __forceinline__ bool aux_on(const StepArgs &a, const float4 &gc, const float4 &ge)
