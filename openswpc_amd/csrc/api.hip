@@ -9,7 +9,7 @@
 #include <utility>
 #include <vector>
 
-#include "swpc_internal.h"
+#include "outputs.h"
 
 static int fail(swpc_ctx *c, int code, const char *fmt, ...)
 {
@@ -1017,8 +1017,9 @@ extern "C" int swpc_wav_store(swpc_ctx *c, int it)
 }
 
 // one step in the order of src/swpc_3d/main.f90:122-138.  d_it != nullptr:
-// kernels read the step number from device memory and the step ends by
-// advancing it (graph-capturable).  marks != nullptr: an event is recorded
+// the step number is the one in device memory plus it (graph-capturable: it
+// is the step's place in the block, and the block ends by advancing the
+// counter; advancing it by a launch per step took 4.6 us of each).  marks != nullptr: an event is recorded
 // before the step and after each of the SWPC_NTIMER launch slots.
 static hipError_t enqueue_step(swpc_ctx *c, int it, const int *d_it, hipEvent_t *marks = nullptr)
 {
@@ -1031,12 +1032,17 @@ static hipError_t enqueue_step(swpc_ctx *c, int it, const int *d_it, hipEvent_t 
     int slot = 0;
     auto mark = [&]() -> hipError_t { return marks ? hipEventRecord(marks[slot++], c->stream) : hipSuccess; };
     if ((e = mark()) != hipSuccess) return e;
-    if ((e = launch_green_store(c, it, d_it)) != hipSuccess) return e;
-    if ((e = launch_wav_store(c, it, d_it)) != hipSuccess || (e = mark()) != hipSuccess) return e;
-    if ((e = launch_snap(c, it, d_it)) != hipSuccess || (e = mark()) != hipSuccess) return e;
-    if (marks && (e = launch_stress(c, pml, 0)) != hipSuccess) return e;
-    if ((e = mark()) != hipSuccess) return e;
-    if ((e = launch_stress(c, pml && !marks, pml ? 3 : marks ? 1 : 5)) != hipSuccess) return e;
+    OutArgs out;
+    out.nblk = 0;
+    if (marks) {
+        if ((e = launch_green_store(c, it, d_it)) != hipSuccess) return e;
+        if ((e = launch_wav_store(c, it, d_it)) != hipSuccess || (e = mark()) != hipSuccess) return e;
+        if ((e = launch_snap(c, it, d_it)) != hipSuccess || (e = mark()) != hipSuccess) return e;
+        if ((e = launch_stress(c, pml, 0)) != hipSuccess || (e = mark()) != hipSuccess) return e;
+    } else if ((e = launch_outputs(c, it, d_it, out)) != hipSuccess) {
+        return e;
+    }
+    if ((e = launch_stress(c, pml && !marks, pml ? 3 : marks ? 1 : 5, &out)) != hipSuccess) return e;
     if ((e = mark()) != hipSuccess) return e;
     if (!pml && marks && (e = launch_cerjan_stress(c)) != hipSuccess) return e;
     if ((e = mark()) != hipSuccess) return e;
@@ -1048,9 +1054,8 @@ static hipError_t enqueue_step(swpc_ctx *c, int it, const int *d_it, hipEvent_t 
     if (!pml && marks && (e = launch_cerjan_vel(c)) != hipSuccess) return e;
     if ((e = mark()) != hipSuccess) return e;
     if ((e = launch_bodyforce(c, it, d_it)) != hipSuccess) return e;
-    if ((e = launch_green_source(c, it, d_it)) != hipSuccess || (e = mark()) != hipSuccess) return e;
-    if (d_it) e = launch_step_advance(c);
-    return e;
+    if ((e = launch_green_source(c, it, d_it)) != hipSuccess) return e;
+    return mark();
 }
 
 // variant bit 7: the velocity update of a step and the stress update of the
@@ -1082,13 +1087,12 @@ static hipError_t enqueue_fused_steps(swpc_ctx *c, int it, int n, const int *d_i
         for (int q = 3; q < SWPC_NFIELD; ++q) c->fields[q] = s[q];
         for (int q = 0; q < SWPC_NFIELD; ++q) c->fields_in[q] = in ? in[q] : nullptr;
     };
-    auto step_no = [&](int s) { return d_it ? 0 : it + s; };
     hipError_t e;
     // step it up to its stress glut, as in enqueue_step
-    if ((e = launch_green_store(c, step_no(0), d_it)) != hipSuccess ||
-        (e = launch_wav_store(c, step_no(0), d_it)) != hipSuccess || (e = launch_snap(c, step_no(0), d_it)) != hipSuccess ||
+    if ((e = launch_green_store(c, it, d_it)) != hipSuccess ||
+        (e = launch_wav_store(c, it, d_it)) != hipSuccess || (e = launch_snap(c, it, d_it)) != hipSuccess ||
         (e = launch_stress(c, true, 3)) != hipSuccess ||
-        (e = launch_stressglut(c, step_no(0), d_it)) != hipSuccess)
+        (e = launch_stressglut(c, it, d_it)) != hipSuccess)
         return e;
     const int nf = (n - 1) & ~1;
     for (int s = 0; s < nf && e == hipSuccess; ++s) {
@@ -1102,22 +1106,21 @@ static hipError_t enqueue_fused_steps(swpc_ctx *c, int it, int n, const int *d_i
         if ((e = launch_fused(c)) != hipSuccess) break;
         // step it+s+1: stresses of the side columns and the bottom band
         if ((e = launch_stress(c, true, 2)) != hipSuccess) break;
-        if (d_it && (e = launch_step_advance(c)) != hipSuccess) break;
         view(nxt, cur, nullptr);
-        if ((e = launch_wav_store(c, step_no(s + 1), d_it)) != hipSuccess ||
-            (e = launch_snap(c, step_no(s + 1), d_it)) != hipSuccess)
+        if ((e = launch_wav_store(c, it + s + 1, d_it)) != hipSuccess ||
+            (e = launch_snap(c, it + s + 1, d_it)) != hipSuccess)
             break;
         view(nxt, nxt, nullptr);
-        e = launch_stressglut(c, step_no(s + 1), d_it);
+        e = launch_stressglut(c, it + s + 1, d_it);
     }
     view(A, A, nullptr);
     if (e != hipSuccess) return e;
     // step it+nf from its velocity update on, in place
     if ((e = launch_vel(c, true, 3)) != hipSuccess ||
-        (e = launch_bodyforce(c, step_no(nf), d_it)) != hipSuccess ||
-        (e = launch_green_source(c, step_no(nf), d_it)) != hipSuccess || (d_it && (e = launch_step_advance(c)) != hipSuccess))
+        (e = launch_bodyforce(c, it + nf, d_it)) != hipSuccess ||
+        (e = launch_green_source(c, it + nf, d_it)) != hipSuccess)
         return e;
-    for (int s = nf + 1; s < n && e == hipSuccess; ++s) e = enqueue_step(c, step_no(s), d_it);
+    for (int s = nf + 1; s < n && e == hipSuccess; ++s) e = enqueue_step(c, it + s, d_it);
     return e;
 }
 
@@ -1125,7 +1128,7 @@ static hipError_t enqueue_steps(swpc_ctx *c, int it, int n, const int *d_it)
 {
     if (n >= 3 && fused_ready(c)) return enqueue_fused_steps(c, it, n, d_it);
     hipError_t e = hipSuccess;
-    for (int s = 0; s < n && e == hipSuccess; ++s) e = enqueue_step(c, d_it ? 0 : it + s, d_it);
+    for (int s = 0; s < n && e == hipSuccess; ++s) e = enqueue_step(c, it + s, d_it);
     return e;
 }
 
@@ -1149,6 +1152,7 @@ extern "C" int swpc_step(swpc_ctx *c, int it0, int nsteps, int use_graph, int bl
             hipGraph_t graph;
             HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
             hipError_t e = enqueue_steps(c, 0, block, c->d_it);
+            if (e == hipSuccess) e = launch_counter_advance(c->d_it, block, c->stream);
             hipError_t e2 = hipStreamEndCapture(c->stream, &graph);
             if (e != hipSuccess) return fail(c, SWPC_EHIP, "graph capture: %s", hipGetErrorString(e));
             if (e2 != hipSuccess) return fail(c, SWPC_EHIP, "graph capture end: %s", hipGetErrorString(e2));

@@ -10,7 +10,7 @@
 #include <cstring>
 #include <mutex>
 
-#include "swpc_internal.h"
+#include "outputs.h"
 
 // --------------------------------------------------------------------------
 // source__stressglut, m_source.f90:776-848
@@ -28,8 +28,6 @@ struct SrcArgs {
     int it;
     const int *d_it;
 };
-
-__device__ static inline int step_of(const SrcArgs &a) { return a.d_it ? *a.d_it : a.it; }
 
 // target t of one context's stress glut at step it
 __device__ static inline void stressglut_body(const SrcArgs &a, int t, int it)
@@ -51,7 +49,7 @@ __device__ static inline void stressglut_body(const SrcArgs &a, int t, int it)
     f[tg.idx] = v;
 }
 
-__global__ void k_stressglut(SrcArgs a) { stressglut_body(a, blockIdx.x * blockDim.x + threadIdx.x, step_of(a)); }
+__global__ void k_stressglut(SrcArgs a) { stressglut_body(a, blockIdx.x * blockDim.x + threadIdx.x, step_number(a.it, a.d_it)); }
 
 // source__bodyforce, m_source.f90:850-898
 __device__ static inline void bodyforce_body(const SrcArgs &a, int t, int it)
@@ -72,16 +70,16 @@ __device__ static inline void bodyforce_body(const SrcArgs &a, int t, int it)
     f[tg.idx] = v;
 }
 
-__global__ void k_bodyforce(SrcArgs a) { bodyforce_body(a, blockIdx.x * blockDim.x + threadIdx.x, step_of(a)); }
+__global__ void k_bodyforce(SrcArgs a) { bodyforce_body(a, blockIdx.x * blockDim.x + threadIdx.x, step_number(a.it, a.d_it)); }
 
 // batched launches: context m = blockIdx.y, its arguments in HBM
 __global__ void k_stressglut_b(const SrcArgs *__restrict__ args, int it, const int *d_it)
 {
-    stressglut_body(args[blockIdx.y], blockIdx.x * blockDim.x + threadIdx.x, d_it ? *d_it : it);
+    stressglut_body(args[blockIdx.y], blockIdx.x * blockDim.x + threadIdx.x, step_number(it, d_it));
 }
 __global__ void k_bodyforce_b(const SrcArgs *__restrict__ args, int it, const int *d_it)
 {
-    bodyforce_body(args[blockIdx.y], blockIdx.x * blockDim.x + threadIdx.x, d_it ? *d_it : it);
+    bodyforce_body(args[blockIdx.y], blockIdx.x * blockDim.x + threadIdx.x, step_number(it, d_it));
 }
 
 static void srcargs_fill(swpc_ctx *c, SrcArgs &a, int it, const int *d_it)
@@ -120,113 +118,19 @@ hipError_t launch_bodyforce(swpc_ctx *c, int it, const int *d_it, hipStream_t s)
 }
 
 // --------------------------------------------------------------------------
-// wav__store, m_wav.f90:397-625 (one thread per station)
+// receivers (outputs.h)
 // --------------------------------------------------------------------------
-struct WavArgs {
-    Grid g;
-    const float *Vx, *Vy, *Vz, *Sxx, *Syy, *Szz, *Syz, *Sxz, *Sxy;
-    const int *ist, *jst, *kst;
-    float *uacc, *eacc;
-    float *wv, *wu, *ws, *we;
-    int nst, what, ntdec, ntw;
-    float M0, UC, dt;
-    float r40x, r40y, r40z, r41x, r41y, r41z;
-    int it;
-    const int *d_it;
-};
-
-// station n of one context at step it
-__device__ static inline void wav_store_body(const WavArgs &a, int n, int it)
-{
-    if (n >= a.nst) return;
-    const Grid &g = a.g;
-    const int i = a.ist[n], j = a.jst[n], k = a.kst[n];
-    const long long P = g.plane;
-    const int Y = g.pitch;
-    const long long p = gidx(g, i, j, k);
-    const float dt = a.dt;
-    if (a.what & SWPC_WAV_U) {
-        a.uacc[3 * n + 0] = a.uacc[3 * n + 0] + (a.Vx[p] + a.Vx[p - 1]) * 0.5f * dt;
-        a.uacc[3 * n + 1] = a.uacc[3 * n + 1] + (a.Vy[p] + a.Vy[p - Y]) * 0.5f * dt;
-        a.uacc[3 * n + 2] = a.uacc[3 * n + 2] - (a.Vz[p] + a.Vz[p - P]) * 0.5f * dt;
-    }
-    if (a.what & SWPC_WAV_STRAIN) {
-        const float *Vx = a.Vx, *Vy = a.Vy, *Vz = a.Vz;
-        const float r40x = a.r40x, r40y = a.r40y, r40z = a.r40z, r41x = a.r41x, r41y = a.r41y, r41z = a.r41z;
-#define AT(F, di, dj, dk) F[p + (di) + (long long)(dj) * Y + (long long)(dk) * P]
-        const float dxVx = (AT(Vx, 0, 0, 0) - AT(Vx, -1, 0, 0)) * r40x - (AT(Vx, 1, 0, 0) - AT(Vx, -2, 0, 0)) * r41x;
-        const float dyVy = (AT(Vy, 0, 0, 0) - AT(Vy, 0, -1, 0)) * r40y - (AT(Vy, 0, 1, 0) - AT(Vy, 0, -2, 0)) * r41y;
-        const float dzVz = (AT(Vz, 0, 0, 0) - AT(Vz, 0, 0, -1)) * r40z - (AT(Vz, 0, 0, 1) - AT(Vz, 0, 0, -2)) * r41z;
-        const float dxVy = ((AT(Vy, 1, 0, 0) - AT(Vy, 0, 0, 0)) * r40x - (AT(Vy, 2, 0, 0) - AT(Vy, -1, 0, 0)) * r41x
-                          + (AT(Vy, 1, -1, 0) - AT(Vy, 0, -1, 0)) * r40x - (AT(Vy, 2, -1, 0) - AT(Vy, -1, -1, 0)) * r41x
-                          + (AT(Vy, 0, 0, 0) - AT(Vy, -1, 0, 0)) * r40x - (AT(Vy, 1, 0, 0) - AT(Vy, -2, 0, 0)) * r41x
-                          + (AT(Vy, 0, -1, 0) - AT(Vy, -1, -1, 0)) * r40x - (AT(Vy, 1, -1, 0) - AT(Vy, -2, -1, 0)) * r41x) / 4.0f;
-        const float dxVz = ((AT(Vz, 1, 0, 0) - AT(Vz, 0, 0, 0)) * r40x - (AT(Vz, 2, 0, 0) - AT(Vz, -1, 0, 0)) * r41x
-                          + (AT(Vz, 1, 0, -1) - AT(Vz, 0, 0, -1)) * r40x - (AT(Vz, 2, 0, -1) - AT(Vz, -1, 0, -1)) * r41x
-                          + (AT(Vz, 0, 0, 0) - AT(Vz, -1, 0, 0)) * r40x - (AT(Vz, 1, 0, 0) - AT(Vz, -2, 0, 0)) * r41x
-                          + (AT(Vz, 0, 0, -1) - AT(Vz, -1, 0, -1)) * r40x - (AT(Vz, 1, 0, -1) - AT(Vz, -2, 0, -1)) * r41x) / 4.0f;
-        const float dyVx = ((AT(Vx, 0, 1, 0) - AT(Vx, 0, 0, 0)) * r40y - (AT(Vx, 0, 2, 0) - AT(Vx, 0, -1, 0)) * r41y
-                          + (AT(Vx, -1, 1, 0) - AT(Vx, -1, 0, 0)) * r40y - (AT(Vx, -1, 2, 0) - AT(Vx, -1, -1, 0)) * r41y
-                          + (AT(Vx, 0, 0, 0) - AT(Vx, 0, -1, 0)) * r40y - (AT(Vx, 0, 1, 0) - AT(Vx, 0, -2, 0)) * r41y
-                          + (AT(Vx, -1, 0, 0) - AT(Vx, -1, -1, 0)) * r40y - (AT(Vx, -1, 1, 0) - AT(Vx, -1, -2, 0)) * r41y) / 4.0f;
-        const float dyVz = ((AT(Vz, 0, 1, 0) - AT(Vz, 0, 0, 0)) * r40y - (AT(Vz, 0, 2, 0) - AT(Vz, 0, -1, 0)) * r41y
-                          + (AT(Vz, 0, 1, -1) - AT(Vz, 0, 0, -1)) * r40y - (AT(Vz, 0, 2, -1) - AT(Vz, 0, -1, -1)) * r41y
-                          + (AT(Vz, 0, 0, 0) - AT(Vz, 0, -1, 0)) * r40y - (AT(Vz, 0, 1, 0) - AT(Vz, 0, -2, 0)) * r41y
-                          + (AT(Vz, 0, 0, -1) - AT(Vz, 0, -1, -1)) * r40y - (AT(Vz, 0, 1, -1) - AT(Vz, 0, -2, -1)) * r41y) / 4.0f;
-        const float dzVx = ((AT(Vx, 0, 0, 1) - AT(Vx, 0, 0, 0)) * r40z - (AT(Vx, 0, 0, 2) - AT(Vx, 0, 0, -1)) * r41z
-                          + (AT(Vx, -1, 0, 1) - AT(Vx, -1, 0, 0)) * r40z - (AT(Vx, -1, 0, 2) - AT(Vx, -1, 0, -1)) * r41z
-                          + (AT(Vx, 0, 0, 0) - AT(Vx, 0, 0, -1)) * r40z - (AT(Vx, 0, 0, 1) - AT(Vx, 0, 0, -2)) * r41z
-                          + (AT(Vx, -1, 0, 0) - AT(Vx, -1, 0, -1)) * r40z - (AT(Vx, -1, 0, 1) - AT(Vx, -1, 0, -2)) * r41z) / 4.0f;
-        const float dzVy = ((AT(Vy, 0, 0, 1) - AT(Vy, 0, 0, 0)) * r40z - (AT(Vy, 0, 0, 2) - AT(Vy, 0, 0, -1)) * r41z
-                          + (AT(Vy, 0, -1, 1) - AT(Vy, 0, -1, 0)) * r40z - (AT(Vy, 0, -1, 2) - AT(Vy, 0, -1, -1)) * r41z
-                          + (AT(Vy, 0, 0, 0) - AT(Vy, 0, 0, -1)) * r40z - (AT(Vy, 0, 0, 1) - AT(Vy, 0, 0, -2)) * r41z
-                          + (AT(Vy, 0, -1, 0) - AT(Vy, 0, -1, -1)) * r40z - (AT(Vy, 0, -1, 1) - AT(Vy, 0, -1, -2)) * r41z) / 4.0f;
-#undef AT
-        float *e = a.eacc + 6 * n;
-        e[0] = e[0] + dxVx * dt;
-        e[1] = e[1] + dyVy * dt;
-        e[2] = e[2] + dzVz * dt;
-        e[3] = e[3] + (dyVz + dzVy) / 2.0f * dt;
-        e[4] = e[4] + (dxVz + dzVx) / 2.0f * dt;
-        e[5] = e[5] + (dxVy + dyVx) / 2.0f * dt;
-    }
-    if ((it - 1) % a.ntdec != 0) return;
-    const int itw = (it - 1) / a.ntdec;
-    if (itw < 0 || itw >= a.ntw) return;
-    const float M0 = a.M0, UC = a.UC;
-    const long long ntw = a.ntw;
-    if (a.what & SWPC_WAV_V) {
-        a.wv[(n * 3LL + 0) * ntw + itw] = (a.Vx[p] + a.Vx[p - 1]) / 2.0f * M0 * UC * 1e9f;
-        a.wv[(n * 3LL + 1) * ntw + itw] = (a.Vy[p] + a.Vy[p - Y]) / 2.0f * M0 * UC * 1e9f;
-        a.wv[(n * 3LL + 2) * ntw + itw] = -((a.Vz[p] + a.Vz[p - P]) / 2.0f * M0 * UC * 1e9f);
-    }
-    if (a.what & SWPC_WAV_U) {
-        for (int q = 0; q < 3; ++q) a.wu[(n * 3LL + q) * ntw + itw] = a.uacc[3 * n + q] * M0 * UC * 1e9f;
-    }
-    if (a.what & SWPC_WAV_STRESS) {
-        a.ws[(n * 6LL + 0) * ntw + itw] = a.Sxx[p] * M0 * UC * 1e6f;
-        a.ws[(n * 6LL + 1) * ntw + itw] = a.Syy[p] * M0 * UC * 1e6f;
-        a.ws[(n * 6LL + 2) * ntw + itw] = a.Szz[p] * M0 * UC * 1e6f;
-        a.ws[(n * 6LL + 3) * ntw + itw] = (a.Syz[p] + a.Syz[p - Y] + a.Syz[p - P] + a.Syz[p - Y - P]) / 4.0f * M0 * UC * 1e6f;
-        a.ws[(n * 6LL + 4) * ntw + itw] = (a.Sxz[p] + a.Sxz[p - 1] + a.Sxz[p - P] + a.Sxz[p - 1 - P]) / 4.0f * M0 * UC * 1e6f;
-        a.ws[(n * 6LL + 5) * ntw + itw] = (a.Sxy[p] + a.Sxy[p - Y] + a.Sxy[p - 1] + a.Sxy[p - 1 - Y]) / 4.0f * M0 * UC * 1e6f;
-    }
-    if (a.what & SWPC_WAV_STRAIN) {
-        for (int q = 0; q < 6; ++q) a.we[(n * 6LL + q) * ntw + itw] = a.eacc[6 * n + q] * M0 * UC * 1e-3f;
-    }
-}
-
 __global__ void k_wav_store(WavArgs a)
 {
-    wav_store_body(a, blockIdx.x * blockDim.x + threadIdx.x, a.d_it ? *a.d_it : a.it);
+    wav_store_body(a, blockIdx.x * blockDim.x + threadIdx.x, step_number(a.it, a.d_it));
 }
 
 __global__ void k_wav_store_b(const WavArgs *__restrict__ args, int it, const int *d_it)
 {
-    wav_store_body(args[blockIdx.y], blockIdx.x * blockDim.x + threadIdx.x, d_it ? *d_it : it);
+    wav_store_body(args[blockIdx.y], blockIdx.x * blockDim.x + threadIdx.x, step_number(it, d_it));
 }
 
-static void wavargs_fill(swpc_ctx *c, WavArgs &a, int it, const int *d_it)
+void wavargs_fill(swpc_ctx *c, WavArgs &a, int it, const int *d_it)
 {
     a.g = c->g;
     a.Vx = c->fields[SWPC_VX]; a.Vy = c->fields[SWPC_VY]; a.Vz = c->fields[SWPC_VZ];
@@ -296,20 +200,14 @@ hipError_t launch_batch_aux(int kind, const void *d_args, int nmem, int nmax, in
 // --------------------------------------------------------------------------
 // device step counter used by graph-captured step blocks
 // --------------------------------------------------------------------------
-__global__ void k_step_advance(int *d_it)
+__global__ void k_step_advance(int *d_it, int n)
 {
-    if (threadIdx.x == 0 && blockIdx.x == 0) *d_it = *d_it + 1;
+    if (threadIdx.x == 0 && blockIdx.x == 0) *d_it = *d_it + n;
 }
 
-hipError_t launch_step_advance(swpc_ctx *c)
+hipError_t launch_counter_advance(int *d, int n, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_step_advance, dim3(1), dim3(64), 0, c->stream, c->d_it);
-    return hipGetLastError();
-}
-
-hipError_t launch_counter_advance(int *d, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_step_advance, dim3(1), dim3(64), 0, s, d);
+    hipLaunchKernelGGL(k_step_advance, dim3(1), dim3(64), 0, s, d, n);
     return hipGetLastError();
 }
 

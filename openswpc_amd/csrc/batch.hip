@@ -291,8 +291,7 @@ static hipError_t enqueue_batch_step(swpc_batch *b, int it, const int *d_it)
     if ((e = launch_batch_aux(BATCH_AUX_GREEN_SOURCE, b->d_aux[BATCH_AUX_GREEN_SOURCE],
                               b->naux[BATCH_AUX_GREEN_SOURCE], b->maxaux[BATCH_AUX_GREEN_SOURCE], it, d_it, s)) != hipSuccess)
         return e;
-    if (d_it) e = launch_counter_advance(b->d_it, s);
-    return e;
+    return hipSuccess;
 }
 
 extern "C" const char *swpc_batch_last_error(const swpc_batch *b) { return b ? b->err : "null batch"; }
@@ -382,7 +381,8 @@ extern "C" int swpc_batch_step(swpc_batch *b, int it0, int nsteps, int use_graph
             hipGraph_t graph;
             BCHK(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
             hipError_t e = hipSuccess;
-            for (int s = 0; s < block && e == hipSuccess; ++s) e = enqueue_batch_step(b, 0, b->d_it);
+            for (int s = 0; s < block && e == hipSuccess; ++s) e = enqueue_batch_step(b, s, b->d_it);
+            if (e == hipSuccess) e = launch_counter_advance(b->d_it, block, b->stream);
             hipError_t e2 = hipStreamEndCapture(b->stream, &graph);
             if (e != hipSuccess) return bfail(b, SWPC_EHIP, "batch graph capture: %s", hipGetErrorString(e));
             if (e2 != hipSuccess) return bfail(b, SWPC_EHIP, "batch graph capture end: %s", hipGetErrorString(e2));

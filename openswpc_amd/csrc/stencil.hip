@@ -18,6 +18,7 @@
 // before it stores; called routine by routine it is a sweep of its own, as in
 // the reference.
 #include "device_access.h"
+#include "outputs.h"
 #include "swpc_internal.h"
 
 #define BX 64
@@ -108,6 +109,7 @@ struct StepArgs {
     float r20x, r20y, r20z;
     const int4 *tiles;   // side-column PML tiles: (i0 | width << 20, j0, k0, k1)
     int ntiles;
+    int first;           // blocks of the launch before the tiles' (the step's outputs, k_stress)
     int sideb;           // blocks of a launch that walk the side tiles (a multiple of 8, >= ntiles; 0: none)
     int has_pml, mask;
     int still;           // see aux_on
@@ -190,7 +192,6 @@ __device__ __forceinline__ void pml_stress_cell(const StepArgs &a, Loc p, Loc q,
                                                 float4 gye)
 {
     const long long P = a.g.plane;
-    const int Y = a.g.pitch;
     const float *__restrict__ Vx = a.f.Vx;
     const float *__restrict__ Vy = a.f.Vy;
     const float *__restrict__ Vz = a.f.Vz;
@@ -291,7 +292,6 @@ __device__ __forceinline__ void pml_vel_cell(const StepArgs &a, Loc p, Loc q, in
                                              float rho0, float rho_kp, float4 gxc, float4 gxe, float4 gyc,
                                              float4 gye)
 {
-    const int Y = a.g.pitch;
     const float *__restrict__ Sxx = a.f.Sxx;
     const float *__restrict__ Syy = a.f.Syy;
     const float *__restrict__ Syz = a.f.Syz;
@@ -515,7 +515,8 @@ __device__ __forceinline__ void stress_cell(const StepArgs &a, const Loc &p, con
 // its side blocks): blocks of one XCD take a contiguous run of tiles, x fastest
 __device__ static inline void plain_tile(const StepArgs &a, int &bx, int &byy, int &bz)
 {
-    const int bid = xcd_remap(blockIdx.x - a.sideb, gridDim.x - a.sideb);
+    const int b0 = a.first + a.sideb;
+    const int bid = xcd_remap(blockIdx.x - b0, gridDim.x - b0);
     bx = bid % a.nbx;
     const int t = bid / a.nbx;
     byy = t % a.nby;
@@ -538,7 +539,6 @@ __device__ __forceinline__ void stress_int_body(const StepArgs &a, int bx, int b
     const int ks = ka1 >= k0 ? k0 : kb0;
 
     const long long P = g.plane;
-    const int Y = g.pitch;
     const float *__restrict__ Vx = a.f.Vx;
     const float *__restrict__ Vy = a.f.Vy;
     const float *__restrict__ Vz = a.f.Vz;
@@ -636,7 +636,6 @@ __device__ __forceinline__ void vel_int_body(const StepArgs &a, int bx, int byy,
     const int ks = ka1 >= k0 ? k0 : kb0;
 
     const long long P = g.plane;
-    const int Y = g.pitch;
     const float *__restrict__ Sxx = a.f.Sxx;
     const float *__restrict__ Syy = a.f.Syy;
     const float *__restrict__ Szz = a.f.Szz;
@@ -982,7 +981,6 @@ __device__ __forceinline__ void stress_pml_body(const StepArgs &a, const int4 tl
     const Grid &g = a.g;
     const int i = L.i, j = L.j;
     const long long P = g.plane;
-    const int Y = g.pitch;
     const float *__restrict__ Vx = a.f.Vx;
     const float *__restrict__ Vy = a.f.Vy;
     const float *__restrict__ Vz = a.f.Vz;
@@ -1040,11 +1038,22 @@ __device__ __forceinline__ void vel_pml_body(const StepArgs &a, const int4 tl)
 // eighth of both.  Launched one after the other, each kind's last blocks leave
 // CUs idle: 128^3 took 140 us/step in two launches per phase and 127 in one,
 // elastic 256 x 256 x 192 525 and 505, 768 x 768 x 448 13.26 and 13.21 ms.
+//
+// In place, the stress update's first blocks take the outputs that the step
+// samples from V (outputs.h), which would otherwise be launches of 4.6 to 13
+// us that leave the device idle.
 template <int NM, bool NT, bool OOP, bool TP>
-__global__ void __launch_bounds__(256) WAVES_NM k_stress(StepArgs a)
+__global__ void __launch_bounds__(256) WAVES_NM k_stress(StepArgs a, OutArgs o)
 {
-    if ((int)blockIdx.x < a.sideb) {
-        const int t = xcd_remap(blockIdx.x, a.sideb);
+    const int blk = (int)blockIdx.x - a.first;
+    if constexpr (NT && !OOP) {
+        if (blk < 0) {
+            outputs_body(o, blockIdx.x, threadIdx.y * blockDim.x + threadIdx.x);
+            return;
+        }
+    }
+    if (blk < a.sideb) {
+        const int t = xcd_remap(blk, a.sideb);
         if (t < a.ntiles) stress_pml_body<OOP>(a, uni(a.tiles[t]));
         return;
     }
@@ -1132,6 +1141,7 @@ void fill_step_args(swpc_ctx *c, StepArgs &a, int mask)
     a.r20z = 1.0f / (float)c->desc.dz;
     a.tiles = (const int4 *)c->d_pml_tiles;
     a.ntiles = c->npml_tiles;
+    a.first = 0;
     a.sideb = 0;
     a.cgx_c = c->cgx_c; a.cgx_b = c->cgx_b; a.cgy_c = c->cgy_c; a.cgy_b = c->cgy_b; a.cgz_c = c->cgz_c; a.cgz_b = c->cgz_b;
     a.has_pml = (c->desc.abc == SWPC_ABC_PML && c->npml > 0) ? 1 : 0;
@@ -1170,20 +1180,66 @@ static bool phase_grid(swpc_ctx *c, StepArgs &a, int phase, bool side, int mask,
     return grid.x > 0;
 }
 
-hipError_t launch_stress(swpc_ctx *c, bool side, int mask)
+void green_store_fill(swpc_ctx *c, GreenArgs &a, int it, const int *d_it);
+void wavargs_fill(swpc_ctx *c, WavArgs &a, int it, const int *d_it);
+void snap_fill(swpc_ctx *c, SnapArgs &a, int it, const int *d_it);
+
+// The step's outputs before its stress update: returns those that read V only
+// in o, for the update's launch, and launches the others (receivers that
+// record stresses, sections of div and rot, which mask with S) or, where the
+// launch does not take any (variant without bit 0, blocks of another size),
+// all of them.
+hipError_t launch_outputs(swpc_ctx *c, int it, const int *d_it, OutArgs &o)
+{
+    o.ng = o.nw = o.ns = o.nblk = 0;
+    const bool in = (c->variant & 1) && !c->fields_in[0] && c->by * BX == 256;
+    hipError_t e = hipSuccess;
+    if (in && c->green_on && c->green_ng > 0) {
+        green_store_fill(c, o.green, it, d_it);
+        o.ng = (c->green_ng + 255) / 256;
+    } else if ((e = launch_green_store(c, it, d_it)) != hipSuccess) {
+        return e;
+    }
+    if (in && c->nst > 0 && !(c->wav_what & SWPC_WAV_STRESS)) {
+        wavargs_fill(c, o.wav, it, d_it);
+        o.nw = (c->nst + 255) / 256;
+    } else if ((e = launch_wav_store(c, it, d_it)) != hipSuccess) {
+        return e;
+    }
+    bool v_only = true;
+    for (int t = 0; t < c->snap_ntask; ++t) v_only = v_only && c->snap_task[t].q != SWPC_SNP_PS;
+    if (in && c->snap_ntask > 0 && v_only) {
+        snap_fill(c, o.snap, it, d_it);
+        o.ns = c->snap_nblk;
+    } else if ((e = launch_snap(c, it, d_it)) != hipSuccess) {
+        return e;
+    }
+    o.nblk = (o.ng + o.nw + o.ns + 7) & ~7;
+    return hipSuccess;
+}
+
+hipError_t launch_stress(swpc_ctx *c, bool side, int mask, const OutArgs *out)
 {
     StepArgs a;
+    OutArgs o;
     dim3 grid, block;
-    if (!phase_grid(c, a, 0, side, mask, grid, block)) return hipSuccess;
+    const bool tiles = phase_grid(c, a, 0, side, mask, grid, block);
+    if (out && out->nblk > 0) {
+        o = *out;
+        a.first = o.nblk;
+        grid.x += a.first;
+    } else if (!tiles) {
+        return hipSuccess;
+    }
     const bool nt = (c->variant & 1) != 0;
     const bool oop = c->fields_in[0] != nullptr;   // out of place: non-temporal streams as well
     const bool tp = (mask & MASK_TAPER) != 0;
 #define SWPC_STRESS_CASE(NMV)                                                                              \
     case NMV:                                                                                              \
-        if (oop) hipLaunchKernelGGL((k_stress<NMV, true, true, false>), grid, block, 0, c->stream, a);       \
-        else if (tp) hipLaunchKernelGGL((k_stress<NMV, true, false, true>), grid, block, 0, c->stream, a);   \
-        else if (nt) hipLaunchKernelGGL((k_stress<NMV, true, false, false>), grid, block, 0, c->stream, a);  \
-        else hipLaunchKernelGGL((k_stress<NMV, false, false, false>), grid, block, 0, c->stream, a);         \
+        if (oop) hipLaunchKernelGGL((k_stress<NMV, true, true, false>), grid, block, 0, c->stream, a, o);       \
+        else if (tp) hipLaunchKernelGGL((k_stress<NMV, true, false, true>), grid, block, 0, c->stream, a, o);   \
+        else if (nt) hipLaunchKernelGGL((k_stress<NMV, true, false, false>), grid, block, 0, c->stream, a, o);  \
+        else hipLaunchKernelGGL((k_stress<NMV, false, false, false>), grid, block, 0, c->stream, a, o);         \
         break;
     switch (c->g.nm) {
         SWPC_STRESS_CASE(0) SWPC_STRESS_CASE(1) SWPC_STRESS_CASE(2) SWPC_STRESS_CASE(3) SWPC_STRESS_CASE(4)

@@ -230,7 +230,9 @@ bool arena_free(void *p);
 // one launch of the stress or velocity update: the side columns when `side`,
 // and of the interior columns mask 1 the interior planes, 2 the bottom PML
 // band, 3 both, 0 none
-hipError_t launch_stress(swpc_ctx *c, bool side, int mask);
+struct OutArgs;
+hipError_t launch_stress(swpc_ctx *c, bool side, int mask, const OutArgs *out = nullptr);
+hipError_t launch_outputs(swpc_ctx *c, int it, const int *d_it, OutArgs &o);
 hipError_t launch_vel(swpc_ctx *c, bool side, int mask);
 hipError_t launch_fused(swpc_ctx *c);
 hipError_t launch_cerjan_stress(swpc_ctx *c);
@@ -240,11 +242,10 @@ hipError_t launch_bodyforce(swpc_ctx *c, int it, const int *d_it, hipStream_t s 
 hipError_t launch_wav_store(swpc_ctx *c, int it, const int *d_it, hipStream_t s = nullptr);
 hipError_t launch_green_store(swpc_ctx *c, int it, const int *d_it, hipStream_t s = nullptr);
 hipError_t launch_green_source(swpc_ctx *c, int it, const int *d_it, hipStream_t s = nullptr);
-hipError_t launch_step_advance(swpc_ctx *c);
 hipError_t launch_snap(swpc_ctx *c, int it, const int *d_it, hipStream_t s = nullptr);
 
 hipError_t launch_set_counter(int *d, int v, hipStream_t s);
-hipError_t launch_counter_advance(int *d, hipStream_t s);
+hipError_t launch_counter_advance(int *d, int n, hipStream_t s);
 
 // ---- batched launches (stencil.hip) ----
 size_t step_args_size();

@@ -86,3 +86,52 @@ def test_profiles_replaced_between_steps(orc, nx, ny, nz, na):
         c.step(1, 6)
     for n in O.FIELDS_V + O.FIELDS_S:
         assert np.array_equal(h.get_field(n), g.get_field(n)), n
+
+
+@pytest.mark.parametrize("by,variant", [(0, -1), (2, -1), (0, 0)])
+@pytest.mark.parametrize("flags,sections", [(1 | 2 | 8, ["xy_v", "fs_u", "ob_v", "yz_u"]), (15, ["fs_v"]), (3, ["xz_ps", "fs_v"]),
+                                            (8, [])])
+def test_outputs_in_the_stress_launch(orc, flags, sections, by, variant):
+    """Receivers, sections and Green's-function cells, more than one block of
+    each, taken by the stress update's launch or beside it, against the same
+    step made of the single routines: step blocks in a graph, more than one
+    block of them, and the steps left over."""
+    nt = 11
+    rng = np.random.default_rng(3)
+    st = [(float(x), float(y), 0.0, "fsb") for x, y in rng.uniform(-3.0, 3.0, (300, 2))]
+    m = O.build_model(small_config(nt=nt, nx=37, ny=34, nz=24, na=5, nm=1, zbeg=-1.0, stations=st, wav_flags=flags, ntdec_w=2,
+                                   sources=[MT]))
+    cells = [rng.integers(3, n - 2, 290) for n in (37, 34, 24)]
+    stf = rng.standard_normal(nt).astype(np.float32)
+
+    def make(**kw):
+        g = gpu_from_model(m, **kw)
+        if sections:
+            g.set_snapshots(sections, m.kfs, k0_xy=5, i0_yz=17, j0_xz=15, ntdec_s=3, nframe=4, M0=m.M0, UC=m.UC)
+        g.set_green(*cells, 18, 16, 9, "z", True, 2, 6, stf)
+        return g
+
+    g, h = make(by=by, variant=variant), make()
+    g.step(1, nt, use_graph=True, block=4)
+    for it in range(1, nt + 1):
+        h.green_store(it)
+        h.wav_store(it)
+        if sections:
+            h.snap_write(it)
+        h.update_stress()
+        h.source_stressglut(it)
+        h.update_vel()
+        h.source_bodyforce(it)
+        h.green_source(it)
+    kinds = [k for k, bit in (("vel", 1), ("disp", 2), ("stress", 4), ("strain", 8)) if flags & bit]
+    for k in kinds:
+        assert np.any(h.seismograms(k) != 0)
+        assert np.array_equal(g.seismograms(k), h.seismograms(k)), k
+    for s in sections:
+        for f in range(4):
+            assert np.array_equal(g.snapshot(s, f), h.snapshot(s, f)), (s, f)
+        if s[:2] in ("fs", "ob") and s[3:] != "ps":
+            assert np.array_equal(g.snap_max(s), h.snap_max(s)), s
+    assert np.any(h.green() != 0) and np.array_equal(g.green(), h.green())
+    for n in O.FIELDS_V + O.FIELDS_S:
+        assert np.array_equal(g.get_field(n), h.get_field(n)), n
