@@ -286,7 +286,7 @@ __device__ __forceinline__ void pml_stress_cell(const StepArgs &a, Loc p, Loc q,
 
 // absorb_p__update_vel for one cell, m_absorb_p.f90:267-304.  Queue values:
 // Szz on k, k+1; Syz, Sxz on k-1, k; rho on k, k+1.
-template <bool OOP>
+template <bool NT, bool OOP>
 __device__ __forceinline__ void pml_vel_cell(const StepArgs &a, Loc p, Loc q, int k, float szz_0,
                                              float szz_p1, float syz_m1, float syz_0, float sxz_m1, float sxz_0,
                                              float rho0, float rho_kp, float4 gxc, float4 gxe, float4 gyc,
@@ -314,22 +314,22 @@ __device__ __forceinline__ void pml_vel_cell(const StepArgs &a, Loc p, Loc q, in
     float azSxz = 0.0f, azSyz = 0.0f, azSzz = 0.0f;
     if (onx) {
         fresh(q);
-        axSxx = ld<true>(AI, q, A_axSxx * n); axSxy = ld<true>(AI, q, A_axSxy * n); axSxz = ld<true>(AI, q, A_axSxz * n);
+        axSxx = ld<NT>(AI, q, A_axSxx * n); axSxy = ld<NT>(AI, q, A_axSxy * n); axSxz = ld<NT>(AI, q, A_axSxz * n);
     }
     if (ony) {
         fresh(q);
-        aySxy = ld<true>(AI, q, A_aySxy * n); aySyy = ld<true>(AI, q, A_aySyy * n); aySyz = ld<true>(AI, q, A_aySyz * n);
+        aySxy = ld<NT>(AI, q, A_aySxy * n); aySyy = ld<NT>(AI, q, A_aySyy * n); aySyz = ld<NT>(AI, q, A_aySyz * n);
     }
     if (onz) {
         fresh(q);
-        azSxz = ld<true>(AI, q, A_azSxz * n); azSyz = ld<true>(AI, q, A_azSyz * n); azSzz = ld<true>(AI, q, A_azSzz * n);
+        azSxz = ld<NT>(AI, q, A_azSxz * n); azSyz = ld<NT>(AI, q, A_azSyz * n); azSzz = ld<NT>(AI, q, A_azSzz * n);
     }
     fresh(p);
     float *__restrict__ Vx = a.f.Vx;
     float *__restrict__ Vy = a.f.Vy;
     float *__restrict__ Vz = a.f.Vz;
-    const float vx = ld<true>(OOP ? a.fin.Vx : Vx, p), vy = ld<true>(OOP ? a.fin.Vy : Vy, p);
-    const float vz = ld<true>(OOP ? a.fin.Vz : Vz, p);
+    const float vx = ld<NT>(OOP ? a.fin.Vx : Vx, p), vy = ld<NT>(OOP ? a.fin.Vy : Vy, p);
+    const float vz = ld<NT>(OOP ? a.fin.Vz : Vz, p);
 
     const float dxSxx = (sxx_ip1 - sxx_0) * a.r20x;
     const float dySyy = (syy_jp1 - syy_0) * a.r20y;
@@ -344,29 +344,29 @@ __device__ __forceinline__ void pml_vel_cell(const StepArgs &a, Loc p, Loc q, in
     const float by = 2.0f / (rho0 + rho_jp);
     const float bz = 2.0f / (rho0 + rho_kp);
 
-    st<true>(Vx, p, vx + bx * (gxe.x * dxSxx + gyc.x * dySxy + gzc.x * dzSxz
+    st<NT>(Vx, p, vx + bx * (gxe.x * dxSxx + gyc.x * dySxy + gzc.x * dzSxz
                                                 + gxe.y * axSxx + gyc.y * aySxy + gzc.y * azSxz) * dt);
-    st<true>(Vy, p, vy + by * (gxc.x * dxSxy + gye.x * dySyy + gzc.x * dzSyz
+    st<NT>(Vy, p, vy + by * (gxc.x * dxSxy + gye.x * dySyy + gzc.x * dzSyz
                                                 + gxc.y * axSxy + gye.y * aySyy + gzc.y * azSyz) * dt);
-    st<true>(Vz, p, vz + bz * (gxc.x * dxSxz + gyc.x * dySyz + gze.x * dzSzz
+    st<NT>(Vz, p, vz + bz * (gxc.x * dxSxz + gyc.x * dySyz + gze.x * dzSzz
                                                 + gxc.y * axSxz + gyc.y * aySyz + gze.y * azSzz) * dt);
     if (onx) {
         fresh(q);
-        st<true>(A, q, gxe.z * axSxx + gxe.w * dxSxx * dt, A_axSxx * n);
-        st<true>(A, q, gxc.z * axSxy + gxc.w * dxSxy * dt, A_axSxy * n);
-        st<true>(A, q, gxc.z * axSxz + gxc.w * dxSxz * dt, A_axSxz * n);
+        st<NT>(A, q, gxe.z * axSxx + gxe.w * dxSxx * dt, A_axSxx * n);
+        st<NT>(A, q, gxc.z * axSxy + gxc.w * dxSxy * dt, A_axSxy * n);
+        st<NT>(A, q, gxc.z * axSxz + gxc.w * dxSxz * dt, A_axSxz * n);
     }
     if (ony) {
         fresh(q);
-        st<true>(A, q, gyc.z * aySxy + gyc.w * dySxy * dt, A_aySxy * n);
-        st<true>(A, q, gye.z * aySyy + gye.w * dySyy * dt, A_aySyy * n);
-        st<true>(A, q, gyc.z * aySyz + gyc.w * dySyz * dt, A_aySyz * n);
+        st<NT>(A, q, gyc.z * aySxy + gyc.w * dySxy * dt, A_aySxy * n);
+        st<NT>(A, q, gye.z * aySyy + gye.w * dySyy * dt, A_aySyy * n);
+        st<NT>(A, q, gyc.z * aySyz + gyc.w * dySyz * dt, A_aySyz * n);
     }
     if (onz) {
         fresh(q);
-        st<true>(A, q, gzc.z * azSxz + gzc.w * dzSxz * dt, A_azSxz * n);
-        st<true>(A, q, gzc.z * azSyz + gzc.w * dzSyz * dt, A_azSyz * n);
-        st<true>(A, q, gze.z * azSzz + gze.w * dzSzz * dt, A_azSzz * n);
+        st<NT>(A, q, gzc.z * azSxz + gzc.w * dzSxz * dt, A_azSxz * n);
+        st<NT>(A, q, gzc.z * azSyz + gzc.w * dzSyz * dt, A_azSyz * n);
+        st<NT>(A, q, gze.z * azSzz + gze.w * dzSzz * dt, A_azSzz * n);
     }
 }
 
@@ -511,12 +511,10 @@ __device__ __forceinline__ void stress_cell(const StepArgs &a, const Loc &p, con
     st<NT>(Sxy, p, sxy);
 }
 
-// logical tile (bx, by, bz) of the interior blocks of a launch (those after
-// its side blocks): blocks of one XCD take a contiguous run of tiles, x fastest
-__device__ static inline void plain_tile(const StepArgs &a, int &bx, int &byy, int &bz)
+// logical tile (bx, by, bz) of interior tile bid, x fastest; xcd_remap gives
+// the blocks of one XCD a contiguous run of them
+__device__ static inline void plain_tile(const StepArgs &a, int bid, int &bx, int &byy, int &bz)
 {
-    const int b0 = a.first + a.sideb;
-    const int bid = xcd_remap(blockIdx.x - b0, gridDim.x - b0);
     bx = bid % a.nbx;
     const int t = bid / a.nbx;
     byy = t % a.nby;
@@ -725,7 +723,7 @@ __device__ __forceinline__ void vel_int_body(const StepArgs &a, int bx, int byy,
             fresh(q);
             const float sxz_p1 = ld(Sxz, p, P), syz_p1 = ld(Syz, p, P), szz_p2 = ld(Szz, p, 2 * P);
             const float rho_kp = ld(rho, p, P);
-            pml_vel_cell<OOP>(a, p, q, k, szz_0, szz_p1, syz_m1, syz_0, sxz_m1, sxz_0, rho0, rho_kp, gxc, gxe, gyc, gye);
+            pml_vel_cell<true, OOP>(a, p, q, k, szz_0, szz_p1, syz_m1, syz_0, sxz_m1, sxz_0, rho0, rho_kp, gxc, gxe, gyc, gye);
             sxz_m2 = sxz_m1; sxz_m1 = sxz_0; sxz_0 = sxz_p1;
             syz_m2 = syz_m1; syz_m1 = syz_0; syz_0 = syz_p1;
             szz_m1 = szz_0; szz_0 = szz_p1; szz_p1 = szz_p2;
@@ -737,7 +735,7 @@ __device__ __forceinline__ void vel_int_body(const StepArgs &a, int bx, int byy,
 template <bool TP>
 __global__ void __launch_bounds__(256) WAVES4 k_vel_int_b(const StepArgs *__restrict__ mem, const int4 *__restrict__ tiles)
 {
-    const int4 t = uni(tiles[xcd_remap(blockIdx.x, gridDim.x)]);
+    const int4 t = uni(tiles[xcd_remap_rev(blockIdx.x, gridDim.x)]);
     vel_int_body<false, TP>(mem[t.x], t.y, t.z, t.w);
 }
 
@@ -763,7 +761,7 @@ __global__ void __launch_bounds__(256) k_fused(StepArgs a)
     constexpr int TY = 4 * SR, VR = TY + 4, NS = 6;
     __shared__ float vs[NS][3][VR][BX];
     int bx, byy, bz;
-    plain_tile(a, bx, byy, bz);
+    plain_tile(a, xcd_remap(blockIdx.x, gridDim.x), bx, byy, bz);
     const Grid &g = a.g;
     const int tx = threadIdx.x, ty = threadIdx.y;
     const int i0 = g.ib + bx * FW, j0 = g.jb + byy * TY;
@@ -972,7 +970,7 @@ __device__ static inline bool pml_lane(const StepArgs &a, const int4 tl, PmlLane
     return L.kb <= L.ke;
 }
 
-// absorb_p__update_stress, m_absorb_p.f90:448-519
+// absorb_p__update_stress, m_absorb_p.f90:448-519.
 template <bool OOP>
 __device__ __forceinline__ void stress_pml_body(const StepArgs &a, const int4 tl)
 {
@@ -1026,13 +1024,13 @@ __device__ __forceinline__ void vel_pml_body(const StepArgs &a, const int4 tl)
         fresh(p);
         fresh(q);
         const float szz_p1 = ld(Szz, p, P), syz_0 = ld(Syz, p), sxz_0 = ld(Sxz, p), rho_kp = ld(rho, p, P);
-        pml_vel_cell<OOP>(a, p, q, k, szz_0, szz_p1, syz_m1, syz_0, sxz_m1, sxz_0, rho0, rho_kp, gxc, gxe, gyc, gye);
+        pml_vel_cell<true, OOP>(a, p, q, k, szz_0, szz_p1, syz_m1, syz_0, sxz_m1, sxz_0, rho0, rho_kp, gxc, gxe, gyc, gye);
         szz_0 = szz_p1; syz_m1 = syz_0; sxz_m1 = sxz_0; rho0 = rho_kp;
     }
 }
 
-// One launch of a phase: its first sideb blocks walk the side tiles, the rest
-// the interior columns.  The two kinds update disjoint cells from the other
+// One launch of a phase: sideb blocks walk the side tiles, the rest the
+// interior columns.  The two kinds update disjoint cells from the other
 // phase's fields, so their order does not change any result.  Each kind is
 // dealt to the XCDs by itself (sideb is a multiple of 8), so every XCD gets an
 // eighth of both.  Launched one after the other, each kind's last blocks leave
@@ -1058,20 +1056,27 @@ __global__ void __launch_bounds__(256) WAVES_NM k_stress(StepArgs a, OutArgs o)
         return;
     }
     int bx, byy, bz;
-    plain_tile(a, bx, byy, bz);
+    plain_tile(a, xcd_remap(blk - a.sideb, gridDim.x - a.first - a.sideb), bx, byy, bz);
     stress_int_body<NM, NT, OOP, TP>(a, bx, byy, bz);
 }
 
+// The stress update's blocks backwards: it starts on the stresses written
+// last and ends on the velocities that the next stress update reads first,
+// which the 256 MB cache in front of HBM still holds (us per step forwards and
+// backwards: elastic 256 x 256 x 192 439 and 428, 384 x 384 x 256 1870 and
+// 1838, 128^3 110.7 and 108.8, twelve small members 3105 and
+// 3060, 768 x 768 x 448 within the noise).
 template <bool OOP, bool TP>
 __global__ void __launch_bounds__(256) WAVES4 k_vel(StepArgs a)
 {
-    if ((int)blockIdx.x < a.sideb) {
-        const int t = xcd_remap(blockIdx.x, a.sideb);
+    const int n = gridDim.x - a.sideb;
+    if ((int)blockIdx.x >= n) {
+        const int t = xcd_remap_rev(blockIdx.x - n, a.sideb);
         if (t < a.ntiles) vel_pml_body<OOP>(a, uni(a.tiles[t]));
         return;
     }
     int bx, byy, bz;
-    plain_tile(a, bx, byy, bz);
+    plain_tile(a, xcd_remap_rev(blockIdx.x, n), bx, byy, bz);
     vel_int_body<OOP, TP>(a, bx, byy, bz);
 }
 
@@ -1086,7 +1091,7 @@ __global__ void __launch_bounds__(256) k_stress_pml_b(const StepArgs *__restrict
 
 __global__ void __launch_bounds__(256) k_vel_pml_b(const StepArgs *__restrict__ mem, const int4 *__restrict__ tiles)
 {
-    const int4 t = uni(tiles[xcd_remap(blockIdx.x, gridDim.x)]);
+    const int4 t = uni(tiles[xcd_remap_rev(blockIdx.x, gridDim.x)]);
     vel_pml_body<false>(mem[t.w], unpack_bside(t));
 }
 
@@ -1104,7 +1109,7 @@ __global__ void __launch_bounds__(256) WAVES_NM k_stress_all_b(const StepArgs *_
 template <bool TP>
 __global__ void __launch_bounds__(256) WAVES4 k_vel_all_b(const StepArgs *__restrict__ mem, const int4 *__restrict__ tiles)
 {
-    const int4 t = uni(tiles[xcd_remap(blockIdx.x, gridDim.x)]);
+    const int4 t = uni(tiles[xcd_remap_rev(blockIdx.x, gridDim.x)]);
     if (t.x >= 0) vel_int_body<false, TP>(mem[t.x], t.y, t.z, t.w);
     else vel_pml_body<false>(mem[-t.x - 1], make_int4(t.y, t.z, t.w & 0xFFFF, t.w >> 16));
 }

@@ -48,6 +48,13 @@ __device__ static inline int xcd_remap(int b, int n)
     const int q = n >> 3, r = n & 7;
     return x < r ? x * (q + 1) + t : r * (q + 1) + (x - r) * q + t;
 }
+// the same runs, each from its end
+__device__ static inline int xcd_remap_rev(int b, int n)
+{
+    const int x = b & 7, t = b >> 3;
+    const int q = n >> 3, r = n & 7;
+    return x < r ? x * (q + 1) + q - t : r * (q + 1) + (x - r) * q + q - 1 - t;
+}
 
 // one of the five PML boxes (m_global.f90:334-343 kbeg_a partition)
 struct PmlBox {
