@@ -970,7 +970,12 @@ __device__ static inline bool pml_lane(const StepArgs &a, const int4 tl, PmlLane
     return L.kb <= L.ke;
 }
 
-// absorb_p__update_stress, m_absorb_p.f90:448-519.
+// absorb_p__update_stress, m_absorb_p.f90:448-519.  Side tiles use ordinary
+// loads and stores: a row of an x slab ends inside a 128-byte line whose rest
+// belongs to an interior tile, and a non-temporal store gives the line up
+// before that arrives.  us with non-temporal and ordinary accesses: 768 x 768
+// x 448 688 and 588 (velocity 550 and 492), 384 x 384 x 256 206 and 178 (166
+// and 149), twelve small members 3250 and 3040 per step.
 template <bool OOP>
 __device__ __forceinline__ void stress_pml_body(const StepArgs &a, const int4 tl)
 {
@@ -995,7 +1000,7 @@ __device__ __forceinline__ void stress_pml_body(const StepArgs &a, const int4 tl
         const float vx_p1 = ld(Vx, p, P), vy_p1 = ld(Vy, p, P), vz_0 = ld(Vz, p);
         const float mu00n = ld(mu, p, P), mu10n = ld(mu, p, P, 1), mu01n = ld(mu, p, P, 0, 1);
         const float mu11n = ld(mu, p, P, 1, 1);
-        pml_stress_cell<true, OOP>(a, p, q, k, vx_0, vx_p1, vy_0, vy_p1, vz_m1, vz_0, mu00, mu00n, mu10, mu10n, mu01,
+        pml_stress_cell<false, OOP>(a, p, q, k, vx_0, vx_p1, vy_0, vy_p1, vz_m1, vz_0, mu00, mu00n, mu10, mu10n, mu01,
                               mu01n, mu11, gxc, gxe, gyc, gye);
         vx_0 = vx_p1; vy_0 = vy_p1; vz_m1 = vz_0;
         mu00 = mu00n; mu10 = mu10n; mu01 = mu01n; mu11 = mu11n;
@@ -1024,7 +1029,7 @@ __device__ __forceinline__ void vel_pml_body(const StepArgs &a, const int4 tl)
         fresh(p);
         fresh(q);
         const float szz_p1 = ld(Szz, p, P), syz_0 = ld(Syz, p), sxz_0 = ld(Sxz, p), rho_kp = ld(rho, p, P);
-        pml_vel_cell<true, OOP>(a, p, q, k, szz_0, szz_p1, syz_m1, syz_0, sxz_m1, sxz_0, rho0, rho_kp, gxc, gxe, gyc, gye);
+        pml_vel_cell<false, OOP>(a, p, q, k, szz_0, szz_p1, syz_m1, syz_0, sxz_m1, sxz_0, rho0, rho_kp, gxc, gxe, gyc, gye);
         szz_0 = szz_p1; syz_m1 = syz_0; sxz_m1 = sxz_0; rho0 = rho_kp;
     }
 }
