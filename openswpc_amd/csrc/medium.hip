@@ -321,5 +321,5 @@ extern "C" int swpc_medium_layered(swpc_ctx *c, const float *prof, const float *
     vrange[1] = ext[2] ? vmax : -1.0f;
     c->has_medium = true;
     ctx_reset_graph(c);
-    return SWPC_OK;
+    return ctx_find_tau(c);
 }

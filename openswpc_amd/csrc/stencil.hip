@@ -113,6 +113,7 @@ struct StepArgs {
     int sideb;           // blocks of a launch that walk the side tiles (a multiple of 8, >= ntiles; 0: none)
     int has_pml, mask;
     int still;           // see aux_on
+    int tau;             // NM = 0: whether taup or taus is anything but zero
     // Cerjan profiles at cell centres (c) and boundaries (b), halo of 3: entry of cell n is n + 2
     const float *cgx_c, *cgx_b, *cgy_c, *cgy_b, *cgz_c, *cgz_b;
     // interior launch shape
@@ -417,8 +418,11 @@ __device__ __forceinline__ void stress_cell(const StepArgs &a, const Loc &p, con
     // every load comes before the first store: the fields may alias for the
     // compiler, and a load left between two stores waits for both
     const float lam1 = ld<NT>(a.m.lam, p);
-    const float taup1 = ld<NT>(a.m.taup, p);
-    const float taus1 = ld<NT>(a.m.taus, p);
+    float taup1 = 0.0f, taus1 = 0.0f;
+    if (NM > 0 || a.tau) {
+        taup1 = ld<NT>(a.m.taup, p);
+        taus1 = ld<NT>(a.m.taus, p);
+    }
     float sxx = ld<NT>(SxxI, p), syy = ld<NT>(SyyI, p), szz = ld<NT>(SzzI, p);
     float syz = ld<NT>(SyzI, p), sxz = ld<NT>(SxzI, p), sxy = ld<NT>(SxyI, p);
     RCell<NM> R;
@@ -1156,6 +1160,7 @@ void fill_step_args(swpc_ctx *c, StepArgs &a, int mask)
     a.cgx_c = c->cgx_c; a.cgx_b = c->cgx_b; a.cgy_c = c->cgy_c; a.cgy_b = c->cgy_b; a.cgz_c = c->cgz_c; a.cgz_b = c->cgz_b;
     a.has_pml = (c->desc.abc == SWPC_ABC_PML && c->npml > 0) ? 1 : 0;
     a.still = c->aux_still ? 1 : 0;
+    a.tau = c->tau ? 1 : 0;
     c->aux_moved = true;
     a.mask = mask;
     a.by = c->by;

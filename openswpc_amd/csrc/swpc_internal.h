@@ -132,6 +132,7 @@ struct swpc_ctx {
     float *R;          // 6*nm*rn
     ViscoCoef visco;
     bool has_medium, has_visco, has_pml, has_cerjan;
+    bool tau;          // taup, taus have to be read (without memory variables they are zero as a rule)
 
     // PML
     PmlBox box[5];
@@ -217,6 +218,7 @@ struct swpc_ctx {
 int ctx_fail(swpc_ctx *c, int code, const char *msg);
 // launch arguments changed: drops the captured graphs (api.hip)
 void ctx_reset_graph(swpc_ctx *c);
+int ctx_find_tau(swpc_ctx *c);
 
 // ---- striped device arena (arena.hip) ----
 // memory from the arena reserved on the device, or nullptr when there is

@@ -135,3 +135,27 @@ def test_outputs_in_the_stress_launch(orc, flags, sections, by, variant):
     assert np.any(h.green() != 0) and np.array_equal(g.green(), h.green())
     for n in O.FIELDS_V + O.FIELDS_S:
         assert np.array_equal(g.get_field(n), h.get_field(n)), n
+
+
+@pytest.mark.parametrize("at", [None, (0, 0, 0), (12, 20, 18), (-1, -1, -1)])
+def test_relaxation_times_without_memory_variables(orc, at):
+    """taup and taus are read where one of them is not zero anywhere, halo
+    included, and no longer once they are zero again"""
+    m = _model(nx=33, ny=30, nz=22, na=5, nm=0, sources=[MT])
+    run = O.OracleRun(m, 32)
+    run.run(12)
+    g = gpu_from_model(m)
+    if at is not None:
+        for q in (m.taup, m.taus):
+            h = gpu_from_model(m)
+            tau = [np.zeros_like(m.taup), np.zeros_like(m.taus)]
+            tau[0 if q is m.taup else 1][at] = 0.25
+            h.set_medium(m.rho, m.lam, m.mu, *tau, m.kfs_top, m.kfs_bot, m.kob_top, m.kob_bot, m.kob)
+            h.step(1, 12)
+            inside = at == (12, 20, 18)
+            assert inside == any(not np.array_equal(h.get_field(n), run.field(n)) for n in O.FIELDS_S)
+            h.close()
+        g.set_medium(m.rho, m.lam, m.mu, *tau, m.kfs_top, m.kfs_bot, m.kob_top, m.kob_bot, m.kob)
+        g.set_medium(m.rho, m.lam, m.mu, m.taup, m.taus, m.kfs_top, m.kfs_bot, m.kob_top, m.kob_bot, m.kob)
+    g.step(1, 12)
+    _same(g, run, f"tau at {at}")
