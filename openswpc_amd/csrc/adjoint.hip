@@ -262,6 +262,11 @@ __device__ static inline void hmean4_w(float a, float b, float c, float d, float
 // unread, and the adjoints unwritten, as the forward's auxiliaries do.
 __device__ __forceinline__ bool aux_on(const float4 &gc, const float4 &ge) { return gc.w != 0.0f || ge.w != 0.0f; }
 
+// What only its own cell reads (adjoint fields, gradients, neighbour words)
+// goes past the caches: ordinary accesses 189.6 and 106.6 ms per gradient at
+// 256 x 256 x 192 elastic and 176 x 160 x 128 with three memory variables,
+// non-temporal ones 186.9 and 102.7 (medians of three).
+
 // k_adj_v: G gathers the stress phase into the velocity adjoints; D takes them
 // on to the velocity update of the step before: densities, stress-auxiliary
 // adjoints and the buoyancy gradients (D without G starts a segment of
@@ -283,24 +288,24 @@ template <bool G, bool D>
 __global__ void __launch_bounds__(256) k_adj_v(AdjArgs a)
 {
     ADJ_CELL(a) {
-        float vx = ld(a.aF[FVX], p), vy = ld(a.aF[FVY], p), vz = ld(a.aF[FVZ], p);
+        float vx = ld<true>(a.aF[FVX], p), vy = ld<true>(a.aF[FVY], p), vz = ld<true>(a.aF[FVZ], p);
         if (G) {
-            const unsigned m = __float_as_uint(ld((const float *)a.nbr, p));
+            const unsigned m = __float_as_uint(ld<true>((const float *)a.nbr, p));
             if (__any(m & NBR_ANY_PML)) gather_vel<true>(a, p, m, vx, vy, vz);
             else gather_vel<false>(a, p, m, vx, vy, vz);
         }
         if (!D) {
             fresh(p);
-            st<false>(a.aF[FVX], p, vx);
-            st<false>(a.aF[FVY], p, vy);
-            st<false>(a.aF[FVZ], p, vz);
+            st<true>(a.aF[FVX], p, vx);
+            st<true>(a.aF[FVY], p, vy);
+            st<true>(a.aF[FVZ], p, vz);
             return;
         }
         fresh(p);
         const int kind = cell_kind(a, i, j, k);
         const float r0 = ld(a.rho, p);
         const float sx = r0 + AT(a.rho, 1, 0, 0), sy = r0 + AT(a.rho, 0, 1, 0), sz = r0 + AT(a.rho, 0, 0, 1);
-        const float bx = ld(a.gb[0], p), by = ld(a.gb[1], p), bz = ld(a.gb[2], p);
+        const float bx = ld<true>(a.gb[0], p), by = ld<true>(a.gb[1], p), bz = ld<true>(a.gb[2], p);
         const float wx = 2.0f / sx * a.dt * vx, wy = 2.0f / sy * a.dt * vy, wz = 2.0f / sz * a.dt * vz;
         const float *Sxx = a.fF[FSXX], *Syy = a.fF[FSYY], *Szz = a.fF[FSZZ];
         const float *Syz = a.fF[FSYZ], *Sxz = a.fF[FSXZ], *Sxy = a.fF[FSXY];
@@ -359,13 +364,13 @@ __global__ void __launch_bounds__(256) k_adj_v(AdjArgs a)
         }
         fresh(p);
         if (G) {
-            st<false>(a.aF[FVX], p, vx);
-            st<false>(a.aF[FVY], p, vy);
-            st<false>(a.aF[FVZ], p, vz);
+            st<true>(a.aF[FVX], p, vx);
+            st<true>(a.aF[FVY], p, vy);
+            st<true>(a.aF[FVZ], p, vz);
         }
-        st<false>(a.gb[0], p, bx + -2.0f / (sx * sx) * a.dt * fx * vx);
-        st<false>(a.gb[1], p, by + -2.0f / (sy * sy) * a.dt * fy * vy);
-        st<false>(a.gb[2], p, bz + -2.0f / (sz * sz) * a.dt * fz * vz);
+        st<true>(a.gb[0], p, bx + -2.0f / (sx * sx) * a.dt * fx * vx);
+        st<true>(a.gb[1], p, by + -2.0f / (sy * sy) * a.dt * fy * vy);
+        st<true>(a.gb[2], p, bz + -2.0f / (sz * sz) * a.dt * fz * vz);
     }
 }
 
@@ -393,10 +398,10 @@ template <int NM>
 __global__ void __launch_bounds__(256) k_adj_s(AdjArgs a)
 {
     ADJ_CELL(a) {
-        const unsigned m = __float_as_uint(ld((const float *)a.nbr, p));
+        const unsigned m = __float_as_uint(ld<true>((const float *)a.nbr, p));
         float s[6];   // xx yy zz yz xz xy
 #pragma unroll
-        for (int c = 0; c < 6; ++c) s[c] = ld(a.aF[FSXX + c], p);
+        for (int c = 0; c < 6; ++c) s[c] = ld<true>(a.aF[FSXX + c], p);
         if (__any(m & NBR_ANY_PML)) gather_str<true>(a, p, m, s);
         else gather_str<false>(a, p, m, s);
         fresh(p);
@@ -414,8 +419,8 @@ __global__ void __launch_bounds__(256) k_adj_s(AdjArgs a)
         const float hxy = hmean4(mu, m100, m010, m110);
         const float Wyz = a.dt * hyz * syz, Wxz = a.dt * hxz * sxz, Wxy = a.dt * hxy * sxy;
         const float *Vx = a.fF[FVX], *Vy = a.fF[FVY], *Vz = a.fF[FVZ];
-        const float glo = ld(a.g_lam, p), gmo = ld(a.g_mu, p);
-        const float hyo = ld(a.gh[0], p), hxo = ld(a.gh[1], p), hzo = ld(a.gh[2], p);
+        const float glo = ld<true>(a.g_lam, p), gmo = ld<true>(a.g_mu, p);
+        const float hyo = ld<true>(a.gh[0], p), hxo = ld<true>(a.gh[1], p), hzo = ld<true>(a.gh[2], p);
         float ex, ey, ez, tyz, txz, txy;
         float qyz, qxz, qxy;   // gradients of the three shear moduli
         float d[9], dgl, dgm;
@@ -538,12 +543,12 @@ __global__ void __launch_bounds__(256) k_adj_s(AdjArgs a)
         }
         fresh(p);
 #pragma unroll
-        for (int c = 0; c < 6; ++c) st<false>(a.aF[FSXX + c], p, s[c]);
-        st<false>(a.g_lam, p, glo + dgl);
-        st<false>(a.g_mu, p, gmo + dgm);
-        st<false>(a.gh[0], p, hyo + qyz);
-        st<false>(a.gh[1], p, hxo + qxz);
-        st<false>(a.gh[2], p, hzo + qxy);
+        for (int c = 0; c < 6; ++c) st<true>(a.aF[FSXX + c], p, s[c]);
+        st<true>(a.g_lam, p, glo + dgl);
+        st<true>(a.g_mu, p, gmo + dgm);
+        st<true>(a.gh[0], p, hyo + qyz);
+        st<true>(a.gh[1], p, hxo + qxz);
+        st<true>(a.gh[2], p, hzo + qxy);
     }
 }
 
