@@ -861,7 +861,7 @@ extern "C" int swpc_adj_accumulate(swpc_ctx *c, int nt, const float *obs, int ck
     const long long per_state = w.z.state(), sstep = w.z.sstep();
     const long long nck = scheme_ck_slots(nt, c1, c2), nout = (nt + c1 - 1) / c1;
     const long long nobs = (long long)c->ntw * 3 * c->nst;
-    const float *seg_before = w.seg;
+    const bool seg_new = !w.seg || w.seg_n < scheme_seg_slots(nt, c1, c2) * sstep;
     if (!wgrow(c, w.ck, w.ck_n, nck * per_state, nf) ||
         !wgrow(c, w.seg, w.seg_n, scheme_seg_slots(nt, c1, c2) * sstep, nf) ||
         !wgrow(c, w.obs, w.obs_n, nobs))
@@ -870,7 +870,7 @@ extern "C" int swpc_adj_accumulate(swpc_ctx *c, int nt, const float *obs, int ck
     // the steps recorded in place of the records never write the halo of a
     // field, which the next step's stencils read as zero: a new store starts
     // at zero and its halos stay so
-    if (w.seg != seg_before && zero(w.seg, w.seg_n, s) != hipSuccess) return SWPC_EHIP;
+    if (seg_new && zero(w.seg, w.seg_n, s) != hipSuccess) return SWPC_EHIP;
     float *outer_ck = w.ck, *inner_ck = w.ck + nout * per_state;
     if (hipMemcpyAsync(w.obs, obs, nobs * sizeof(float), hipMemcpyHostToDevice, s) != hipSuccess) return SWPC_EHIP;
 

@@ -19,7 +19,10 @@
 // (a multi-stream array such as the packed memory variables names one
 // region per stream segment); smaller arrays are sub-allocated from
 // per-region slabs.  When the arena is missing or full, allocation falls
-// back to hipMalloc.  The arena is process-wide, one per device; contexts
+// back to hipMalloc.  A freed range of granules stays mapped, and counts as
+// free, until its granules are needed for another one: unmapping 16 GiB takes
+// 16 ms and mapping them again 5, which a gradient paid for its checkpoint
+// and record stores on every call (see take_parked).  The arena is process-wide, one per device; contexts
 // hold no reference to it, so swpc_stripe_release refuses while any of its
 // memory is in use.  A large context created on a device without an arena
 // reserves a private one sized for itself (swpc_create), which only that
@@ -52,9 +55,17 @@ struct Region {
 struct Live {
     bool big = false;
     size_t bytes = 0;  // big: mapped bytes; small: block bytes
-    std::vector<std::pair<int, hipMemGenericAllocationHandle_t>> granules;  // big: (region, handle) per granule
+    std::vector<std::pair<int, hipMemGenericAllocationHandle_t>> granules;  // big: of the range
     Slab *slab = nullptr;
     size_t off = 0;
+};
+
+using Granules = std::vector<std::pair<int, hipMemGenericAllocationHandle_t>>;  // (region, handle) per granule
+
+// a freed range that is still mapped
+struct Parked {
+    char *va;
+    Granules granules;
 };
 
 struct Arena {
@@ -65,7 +76,54 @@ struct Arena {
     hipMemAccessDesc access{};
     Region reg[kMaxRegions];
     std::map<char *, Live> live;
+    std::vector<Parked> parked;  // oldest first
 };
+
+size_t parked_granules(const Arena &a, int region)
+{
+    size_t n = 0;
+    for (const Parked &p : a.parked)
+        for (const auto &g : p.granules) n += g.first == region;
+    return n;
+}
+
+// unmap a parked range; its granules can go anywhere
+void unpark(Arena &a, size_t i)
+{
+    const Parked p = std::move(a.parked[i]);
+    a.parked.erase(a.parked.begin() + (long)i);
+    (void)hipMemUnmap(p.va, p.granules.size() * a.gran);
+    (void)hipMemAddressFree(p.va, p.granules.size() * a.gran);
+    for (const auto &g : p.granules) a.reg[g.first].granules.push_back(g.second);
+}
+
+// the parked range whose granules lie in exactly these regions, if there is one
+bool take_parked(Arena &a, const std::vector<int> &rk, Parked &out)
+{
+    for (size_t i = a.parked.size(); i-- > 0;) {
+        const Granules &g = a.parked[i].granules;
+        if (g.size() != rk.size()) continue;
+        bool same = true;
+        for (size_t k = 0; k < rk.size() && same; ++k) same = g[k].first == rk[k];
+        if (!same) continue;
+        out = std::move(a.parked[i]);
+        a.parked.erase(a.parked.begin() + (long)i);
+        return true;
+    }
+    return false;
+}
+
+// granules of a region to map: parked ranges that hold some give theirs up, oldest first
+bool want_granules(Arena &a, int region, size_t n)
+{
+    for (size_t i = 0; a.reg[region].granules.size() < n && i < a.parked.size();) {
+        bool has = false;
+        for (const auto &g : a.parked[i].granules) has = has || g.first == region;
+        if (has) unpark(a, i);
+        else ++i;
+    }
+    return a.reg[region].granules.size() >= n;
+}
 
 std::mutex g_mu;
 std::map<int, Arena *> g_arena;
@@ -115,7 +173,7 @@ void *alloc_big(Arena &a, size_t bytes, const int *seg_region, int nseg, size_t 
     size_t need[kMaxRegions] = {};
     std::vector<int> rk(ng);
     size_t avail[kMaxRegions] = {};
-    for (int r = 0; r < a.nreg; ++r) avail[r] = a.reg[r].granules.size();
+    for (int r = 0; r < a.nreg; ++r) avail[r] = a.reg[r].granules.size() + parked_granules(a, r);
     for (size_t k = 0; k < ng; ++k) {
         // the granule's segment names its region (no table: segments rotate
         // over the regions); a region that has run out yields to the region
@@ -131,6 +189,17 @@ void *alloc_big(Arena &a, size_t bytes, const int *seg_region, int nseg, size_t 
         rk[k] = r;
         ++need[r];
     }
+    Parked old;
+    if (take_parked(a, rk, old)) {
+        Live L;
+        L.big = true;
+        L.bytes = ng * a.gran;
+        L.granules = std::move(old.granules);
+        a.live[old.va] = std::move(L);
+        return old.va;
+    }
+    for (int r = 0; r < a.nreg; ++r)
+        if (!want_granules(a, r, need[r])) return nullptr;
     void *va = nullptr;
     if (hipMemAddressReserve(&va, ng * a.gran, 0, nullptr, 0) != hipSuccess) {
         (void)hipGetLastError();
@@ -169,7 +238,7 @@ void *alloc_small(Arena &a, size_t bytes, int region)
         if (f != s->free_.end()) { slab = s; break; }
     }
     if (!slab) {
-        if (R.granules.empty()) return nullptr;
+        if (!want_granules(a, r, 1)) return nullptr;
         void *va = nullptr;
         if (hipMemAddressReserve(&va, a.gran, 0, nullptr, 0) != hipSuccess) {
             (void)hipGetLastError();
@@ -204,6 +273,7 @@ void *alloc_small(Arena &a, size_t bytes, int region)
 
 void release_all(Arena &a)
 {
+    while (!a.parked.empty()) unpark(a, a.parked.size() - 1);
     for (int r = 0; r < a.nreg; ++r) {
         for (Slab *s : a.reg[r].slabs) {
             (void)hipMemUnmap(s->va, a.gran);
@@ -243,7 +313,8 @@ int64_t arena_granule_bytes(int device, const void *who)
     auto it = g_arena.find(device);
     if (it == g_arena.end() || (it->second->owner && it->second->owner != who)) return 0;
     int64_t b = 0;
-    for (int r = 0; r < it->second->nreg; ++r) b += (int64_t)(it->second->reg[r].granules.size() * it->second->gran);
+    const Arena &a = *it->second;
+    for (int r = 0; r < a.nreg; ++r) b += (int64_t)((a.reg[r].granules.size() + parked_granules(a, r)) * a.gran);
     return b;
 }
 
@@ -260,9 +331,7 @@ bool arena_free(void *p)
         DeviceScope ds(a.device);
         (void)hipDeviceSynchronize();
         if (L.big) {
-            (void)hipMemUnmap(p, L.bytes);
-            (void)hipMemAddressFree(p, L.bytes);
-            for (auto &g : L.granules) a.reg[g.first].granules.push_back(g.second);
+            a.parked.push_back({(char *)p, std::move(L.granules)});
         } else {
             Slab *s = L.slab;
             size_t off = L.off, sz = L.bytes;
@@ -375,7 +444,7 @@ extern "C" int64_t swpc_stripe_free_bytes(int device, int region)
     if (it == g_arena.end()) return 0;
     const Arena &a = *it->second;
     if (region < 0 || region >= a.nreg) return SWPC_EINVAL;
-    int64_t b = (int64_t)(a.reg[region].granules.size() * a.gran);
+    int64_t b = (int64_t)((a.reg[region].granules.size() + parked_granules(a, region)) * a.gran);
     for (const Slab *s : a.reg[region].slabs)
         for (const auto &f : s->free_) b += (int64_t)f.second;
     return b;
