@@ -146,7 +146,8 @@ def measure_batch(steps, warmup, block_req):
     n_int = sum(cell_counts(sp.nx, sp.ny, sp.nz, sp.na)[0] for sp in specs)
     n_pml = cells - n_int
     b_si, b_vi, b_sp, b_vp = bytes_model(nm)
-    bytes_step = n_int * (b_si + b_vi) + n_pml * (b_sp + b_vp)
+    bytes_step = n_int * (b_si + b_vi) + n_pml * (b_sp + b_vp) \
+        + 2 * ADE_BYTES * sum(ade_axes(sp.nx, sp.ny, sp.nz, sp.na) for sp in specs)
     for s in sims:
         s.close()
     stripe_off(placement)
@@ -436,7 +437,7 @@ def run_rmedia(args):
     shape = (518, 1030, 1030)
     cells = shape[0] * shape[1] * shape[2]
     kw = dict(d=(0.25, 0.25, 0.25), a=(5.0, 5.0, 5.0), epsil=0.05, kappa=0.5)
-    rmedia_3d("vonkarman", (64, 64, 64), seed=1, **kw)   # first use: library and FFT plan set-up
+    rmedia_3d("vonkarman", (64, 64, 64), seed=1, **kw)   # first use: library set-up
     times = []
     for rep in range(3):
         t = time.perf_counter()
@@ -474,9 +475,17 @@ def bytes_model(nm):
     once per phase, stencil neighbours free)."""
     stress_int = 4 * (3 + 4 + 2 * 6 + 2 * 6 * nm)   # V3 read; lam,mu,taup,taus; S6 RMW; R(6 nm) RMW
     vel_int = 4 * (6 + 1 + 2 * 3)                   # S6 read; rho; V3 RMW
-    stress_pml = 4 * (3 + 2 + 2 * 6 + 2 * 9)        # V3; lam, mu; S6 RMW; 9 ADE RMW
-    vel_pml = 4 * (6 + 1 + 2 * 3 + 2 * 9)           # S6; rho; V3 RMW; 9 ADE RMW
+    stress_pml = 4 * (3 + 2 + 2 * 6)                # V3; lam, mu; S6 RMW; and the ADE auxiliaries (ade_axes)
+    vel_pml = 4 * (6 + 1 + 2 * 3)                   # S6; rho; V3 RMW; and the ADE auxiliaries
     return stress_int, vel_int, stress_pml, vel_pml
+
+
+ADE_BYTES = 4 * 2 * 3   # per PML cell, phase and axis that damps it: 3 ADE RMW
+
+
+def ade_axes(nx, ny, nz, na):
+    """damping axes summed over the PML cells (x and y zones on both sides, z at the bottom)"""
+    return 2 * na * ny * nz + 2 * na * nx * nz + na * nx * ny
 
 
 # ---------------------------------------------------------------------------
@@ -540,7 +549,7 @@ def cpu_baseline(target_s=12.0):
 def read_traffic(workload):
     """HBM bytes per launch of the dominant kernel from committed rocprofv3
     --pmc summaries (FETCH_SIZE + WRITE_SIZE), if present."""
-    p = os.path.join(ROOT, "profiles", f"k_stress_int_{workload}_pmc.txt")
+    p = os.path.join(ROOT, "profiles", f"k_stress_{workload}_pmc.txt")
     if not os.path.exists(p):
         return None
     for line in open(p):
@@ -665,10 +674,11 @@ def main():
     n_int, n_pml = cell_counts(nx, ny, nz, na)
     n_bot = (nx - 2 * na) * (ny - 2 * na) * na      # bottom PML band of the interior columns
     b_si, b_vi, b_sp, b_vp = bytes_model(nm)
-    bytes_step = n_int * (b_si + b_vi) + n_pml * (b_sp + b_vp)
-    # dominant launch: interior columns of the stress phase = kernel__update_stress
-    # over the interior plus absorb__update_stress over their bottom band
-    bytes_launch = n_int * b_si + n_bot * b_sp
+    bytes_step = n_int * (b_si + b_vi) + n_pml * (b_sp + b_vp) + 2 * ADE_BYTES * ade_axes(nx, ny, nz, na)
+    # dominant launch (timed steps launch it by itself): interior columns of
+    # the stress phase = kernel__update_stress over the interior plus
+    # absorb__update_stress over their bottom band, which z alone damps
+    bytes_launch = n_int * b_si + n_bot * (b_sp + ADE_BYTES)
     achieved = bytes_launch / (kms["stress"] * 1e-3)
     value = nx * ny * nz / (ms_per_step * 1e-3) / 1e9
     step_bw = bytes_step / (ms_per_step * 1e-3)
@@ -706,7 +716,7 @@ def main():
         },
         "roofline": {
             "bound": "hbm",
-            "kernel": "k_stress_int<3,true> (kernel__update_stress + bottom band of absorb__update_stress)",
+            "kernel": "k_stress<3,true>, interior columns (kernel__update_stress + bottom band of absorb__update_stress)",
             "achieved": round(achieved / 1e9, 2),
             "peak": HBM_PEAK / 1e9,
             "unit": "GB/s",
