@@ -15,7 +15,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIBDIR, "libswpc_gpu.so")
 SOURCES = ["api.hip", "stencil.hip", "aux.hip", "snap.hip", "green.hip", "batch.hip", "adjoint.hip", "rmedia.hip", "medium.hip", "arena.hip"]
-# hipFFT for the random-media generator
+# hipFFT for random media with lines that do not fit in LDS
 LIBS = ["-L/opt/rocm/lib", "-lhipfft", "-Wl,-rpath,/opt/rocm/lib"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("SWPC_OFFLOAD_ARCH", "gfx950")

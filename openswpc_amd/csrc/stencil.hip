@@ -1,7 +1,8 @@
 // stencil.hip -- velocity/stress updates of OpenSWPC's 3D loop on gfx950.
 //
-// Each phase is two z-marching kernels: the interior (4th order + Zener
-// memory variables, m_kernel) and the ADE-CFS PML (2nd order, m_absorb_p).
+// Each phase is one launch of z-marching tiles: the interior (4th order +
+// Zener memory variables, m_kernel) and the ADE-CFS PML (2nd order,
+// m_absorb_p).
 // A thread owns one (i,j) column of a 64 x BY tile of full-width rows whose
 // first cell sits on a 128-byte line, and marches a chunk of planes along z,
 // keeping the z-neighbours of its column in a rotating register queue while
@@ -10,9 +11,9 @@
 // store, so every load of an iteration is in flight at once: with each stress
 // component loaded between the stores of its neighbours a wave made six
 // memory round trips per cell (elastic 256 x 256 x 192, 20-cell PML: stress
-// launch 262 us, 195 us with the loads first).  Every arithmetic expression keeps the reference's FP32
-// evaluation order; the library is compiled with -ffp-contract=off so no FMA
-// changes the rounding.
+// launch 262 us, 195 us with the loads first).  Every arithmetic expression
+// keeps the reference's FP32 evaluation order; the library is compiled with
+// -ffp-contract=off so no FMA changes the rounding.
 //
 // A whole step's Cerjan taper (m_absorb_c) is applied by the update itself
 // before it stores; called routine by routine it is a sweep of its own, as in
@@ -25,7 +26,6 @@
 #define MASK_INT 1
 #define MASK_PML 2
 #define MASK_TAPER 4  // the update applies the Cerjan taper to the values it stores
-
 
 // Four waves per SIMD: 128 registers, which every NM <= 4 form fits without a
 // spill; asking for no more lets the scheduler keep a cell's loads together.
@@ -1073,8 +1073,8 @@ __global__ void __launch_bounds__(256) WAVES_NM k_stress(StepArgs a, OutArgs o)
 // last and ends on the velocities that the next stress update reads first,
 // which the 256 MB cache in front of HBM still holds (us per step forwards and
 // backwards: elastic 256 x 256 x 192 439 and 428, 384 x 384 x 256 1870 and
-// 1838, 128^3 110.7 and 108.8, twelve small members 3105 and
-// 3060, 768 x 768 x 448 within the noise).
+// 1838, 128^3 110.7 and 108.8, twelve small members 3105 and 3060, 768 x 768 x
+// 448 within the noise).
 template <bool OOP, bool TP>
 __global__ void __launch_bounds__(256) WAVES4 k_vel(StepArgs a)
 {
