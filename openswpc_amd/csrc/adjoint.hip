@@ -693,6 +693,7 @@ struct AdjWorkspace {
     float *grad = nullptr;  // the sums over sources
     float *nbr = nullptr;   // neighbour words
     float *ck = nullptr, *seg = nullptr, *obs = nullptr;
+    bool seg_zero = false;  // the record store was cleared after it was allocated
     // record table for 6 nst targets: tgt (long long) | ptr (6 nst + 1 int) | src (6 nst int)
     float *rec = nullptr;
     long long ck_n = 0, seg_n = 0, obs_n = 0, rec_n = 0;
@@ -861,16 +862,19 @@ extern "C" int swpc_adj_accumulate(swpc_ctx *c, int nt, const float *obs, int ck
     const long long per_state = w.z.state(), sstep = w.z.sstep();
     const long long nck = scheme_ck_slots(nt, c1, c2), nout = (nt + c1 - 1) / c1;
     const long long nobs = (long long)c->ntw * 3 * c->nst;
-    const bool seg_new = !w.seg || w.seg_n < scheme_seg_slots(nt, c1, c2) * sstep;
+    const long long nseg = scheme_seg_slots(nt, c1, c2) * sstep;
+    if (!w.seg || w.seg_n < nseg) w.seg_zero = false;
     if (!wgrow(c, w.ck, w.ck_n, nck * per_state, nf) ||
-        !wgrow(c, w.seg, w.seg_n, scheme_seg_slots(nt, c1, c2) * sstep, nf) ||
+        !wgrow(c, w.seg, w.seg_n, nseg, nf) ||
         !wgrow(c, w.obs, w.obs_n, nobs))
         return ctx_fail(c, SWPC_ENOMEM, "swpc_adj_accumulate: device memory for the checkpoints "
                                         "(swpc_adj_plan finds a scheme that fits)");
     // the steps recorded in place of the records never write the halo of a
     // field, which the next step's stencils read as zero: a new store starts
-    // at zero and its halos stay so
-    if (seg_new && zero(w.seg, w.seg_n, s) != hipSuccess) return SWPC_EHIP;
+    // at zero and its halos stay so.  (A call that fails before this leaves a
+    // store that the next call still has to clear.)
+    if (!w.seg_zero && zero(w.seg, w.seg_n, s) != hipSuccess) return SWPC_EHIP;
+    w.seg_zero = true;
     float *outer_ck = w.ck, *inner_ck = w.ck + nout * per_state;
     if (hipMemcpyAsync(w.obs, obs, nobs * sizeof(float), hipMemcpyHostToDevice, s) != hipSuccess) return SWPC_EHIP;
 
