@@ -87,6 +87,15 @@ int swpc_set_visco(swpc_ctx *ctx, const float *c1, const float *c2, const float 
 int swpc_set_pml(swpc_ctx *ctx, const float *gxc, const float *gxe, const float *gyc, const float *gye,
                  const float *gzc, const float *gze);
 
+/* 1 when the updates leave the PML auxiliaries of axes that do not damp their
+   cell alone (they are zero and stay so: a face cell moves 12 of 36 words a
+   step), 0 when they take all of them.  All are taken, from then on, once
+   swpc_set_pml undamps an axis of a cell where steps have run with it damped;
+   setting the same profiles again changes nothing, and a gradient, which
+   starts from rest, brings 1 back.  The results do not depend on it.  0
+   without a PML. */
+int swpc_pml_axes_skipped(const swpc_ctx *ctx);
+
 /* Cerjan sponge profiles with the 3-cell halo (n+6 each)
    (src/swpc_3d/m_absorb_c.f90:27-101). */
 int swpc_set_cerjan(swpc_ctx *ctx, const float *gx_c, const float *gx_b, const float *gy_c, const float *gy_b,

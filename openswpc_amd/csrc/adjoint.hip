@@ -985,7 +985,10 @@ extern "C" int swpc_adj_accumulate(swpc_ctx *c, int nt, const float *obs, int ck
     hipError_t e = hipSuccess;
     for (int q = 0; q < SWPC_NFIELD && e == hipSuccess; ++q) e = zero(c->fields[q], nf, s);
     if (e == hipSuccess) e = zero(c->ade, na18, s);
-    c->aux_still = true;   // from zero under the profiles as they are
+    if (e == hipSuccess) {   // from zero under the profiles as they are
+        c->aux_still = true;
+        for (int n = 0; n < g.nx + g.ny + g.nz; ++n) c->aux_axis[n] &= 1;
+    }
     if (e == hipSuccess && nR) e = zero(c->R, nR, s);
     if (e == hipSuccess && c->d_uacc) e = zero(c->d_uacc, 3LL * c->nst, s);
     if (e == hipSuccess && c->d_eacc) e = zero(c->d_eacc, 6LL * c->nst, s);

@@ -362,6 +362,7 @@ extern "C" int swpc_create(const swpc_desc *d, swpc_ctx **out)
         }
         c->npml = off;
         c->aux_still = true;
+        if (!(c->aux_axis = (unsigned char *)calloc((size_t)nx + ny + nz, 1))) { rc = SWPC_ENOMEM; goto bad; }
         ALLOC_STRIPED(c->ade, (size_t)A_N * c->npml * sizeof(float), kAuxRegion, A_N, (size_t)c->npml * sizeof(float));
         ALLOC(c->gxc, (size_t)nx * sizeof(float4));
         ALLOC(c->gxe, (size_t)nx * sizeof(float4));
@@ -436,6 +437,7 @@ extern "C" int swpc_destroy(swpc_ctx *c)
     for (int q = 0; q < SWPC_NFIELD; ++q) dfree(c->fields[q]);
     for (int q = 0; q < SWPC_NFIELD; ++q) dfree(c->fields2[q]);
     dfree(c->d_fzc);
+    free(c->aux_axis);
     dfree(c->rho); dfree(c->lam); dfree(c->mu); dfree(c->taup); dfree(c->taus);
     dfree(c->kfs_top); dfree(c->kfs_bot); dfree(c->kob_top); dfree(c->kob_bot); dfree(c->kob);
     dfree(c->R); dfree(c->ade); dfree(c->d_pml_tiles); dfree(c->d_zchunks);
@@ -556,10 +558,26 @@ extern "C" int swpc_set_pml(swpc_ctx *c, const float *gxc, const float *gxe, con
     HIPCHK(c, hipMemcpyAsync(c->gzc, gzc, (size_t)g.nz * 16, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipMemcpyAsync(c->gze, gze, (size_t)g.nz * 16, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    if (c->aux_moved) c->aux_still = false;
+    const float *const prof[3][2] = {{gxc, gxe}, {gyc, gye}, {gzc, gze}};
+    const int len[3] = {g.nx, g.ny, g.nz};
+    unsigned char *ax = c->aux_axis;
+    for (int q = 0; q < 3; ++q)
+        for (int n = 0; n < len[q]; ++n, ++ax) {
+            const bool on = prof[q][0][4 * n + 3] != 0.0f || prof[q][1][4 * n + 3] != 0.0f;   // aux_on (stencil.hip)
+            const bool was = (*ax & 2) || (c->aux_moved && (*ax & 1));
+            if (was && !on) c->aux_still = false;
+            *ax = (unsigned char)((was ? 2 : 0) | (on ? 1 : 0));
+        }
+    c->aux_moved = false;   // the graphs dropped below are captured anew, which sets it
     c->has_pml = true;
     reset_graph(c);
     return SWPC_OK;
+}
+
+extern "C" int swpc_pml_axes_skipped(const swpc_ctx *c)
+{
+    if (!c) return SWPC_EINVAL;
+    return c->desc.abc == SWPC_ABC_PML && c->npml > 0 && c->aux_still ? 1 : 0;
 }
 
 extern "C" int swpc_set_cerjan(swpc_ctx *c, const float *gx_c, const float *gx_b, const float *gy_c,

@@ -374,6 +374,8 @@ extern "C" int swpc_batch_step(swpc_batch *b, int it0, int nsteps, int use_graph
         if (c->snap_ntask > 0 && nsteps > 0 && it0 + nsteps - 1 >= 1 &&
             (it0 + nsteps - 2) / c->snap.ntdec_s >= c->snap.nframe)
             return bfail(b, SWPC_EINVAL, "a member's snapshot frame store is too small for these steps");
+    if (nsteps > 0)
+        for (swpc_ctx *c : b->mem) c->aux_moved = true;
     int done = 0;
     if (use_graph && block > 0 && nsteps >= block) {
         if (!b->graph || b->graph_block != block) {
@@ -431,6 +433,8 @@ extern "C" int swpc_batch_tune(swpc_batch *b, int trial_steps, int *kchunk_out, 
     BCHK(b, hipSetDevice(b->device));
     int rc;
     if ((rc = batch_sync_members(b))) return rc;
+    // a caller may tune on a field that is not at rest, which the trials move
+    for (swpc_ctx *c : b->mem) c->aux_moved = true;
     const int kc_cand[] = {4, 6, 8, 12, 16, 24, 32};
     const int by_cand[] = {2, 4};
     const int w_cand[] = {64, 32};

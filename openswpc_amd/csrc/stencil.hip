@@ -1123,10 +1123,7 @@ __global__ void __launch_bounds__(256) WAVES4 k_vel_all_b(const StepArgs *__rest
     else vel_pml_body<false>(mem[-t.x - 1], make_int4(t.y, t.z, t.w & 0xFFFF, t.w >> 16));
 }
 
-void fill_step_args(swpc_ctx *c, StepArgs &a, int mask);
-static void step_args(swpc_ctx *c, StepArgs &a, int mask) { fill_step_args(c, a, mask); }
-
-void fill_step_args(swpc_ctx *c, StepArgs &a, int mask)
+static void step_args(const swpc_ctx *c, StepArgs &a, int mask)
 {
     a.g = c->g;
     a.f.Vx = c->fields[SWPC_VX]; a.f.Vy = c->fields[SWPC_VY]; a.f.Vz = c->fields[SWPC_VZ];
@@ -1161,7 +1158,6 @@ void fill_step_args(swpc_ctx *c, StepArgs &a, int mask)
     a.has_pml = (c->desc.abc == SWPC_ABC_PML && c->npml > 0) ? 1 : 0;
     a.still = c->aux_still ? 1 : 0;
     a.tau = c->tau ? 1 : 0;
-    c->aux_moved = true;
     a.mask = mask;
     a.by = c->by;
     a.zc = c->d_zchunks;
@@ -1180,7 +1176,7 @@ void fill_step_args(swpc_ctx *c, StepArgs &a, int mask)
 // interior planes (mask & MASK_INT) and their bottom PML band (mask &
 // MASK_PML), or over all of them.  The batch's and the fused launch's tiles
 // use the same bodies.
-static bool phase_grid(swpc_ctx *c, StepArgs &a, int phase, bool side, int mask, dim3 &grid, dim3 &block)
+static bool phase_grid(const swpc_ctx *c, StepArgs &a, int phase, bool side, int mask, dim3 &grid, dim3 &block)
 {
     step_args(c, a, mask);
     if (phase == 1) a.zc = c->d_zchunks + c->nbz + 1;
@@ -1249,6 +1245,7 @@ hipError_t launch_stress(swpc_ctx *c, bool side, int mask, const OutArgs *out)
     const bool nt = (c->variant & 1) != 0;
     const bool oop = c->fields_in[0] != nullptr;   // out of place: non-temporal streams as well
     const bool tp = (mask & MASK_TAPER) != 0;
+    c->aux_moved = true;
 #define SWPC_STRESS_CASE(NMV)                                                                              \
     case NMV:                                                                                              \
         if (oop) hipLaunchKernelGGL((k_stress<NMV, true, true, false>), grid, block, 0, c->stream, a, o);       \
@@ -1270,6 +1267,7 @@ hipError_t launch_vel(swpc_ctx *c, bool side, int mask)
     StepArgs a;
     dim3 grid, block;
     if (!phase_grid(c, a, 1, side, mask, grid, block)) return hipSuccess;
+    c->aux_moved = true;
     if (c->fields_in[0]) hipLaunchKernelGGL((k_vel<true, false>), grid, block, 0, c->stream, a);
     else if (mask & MASK_TAPER) hipLaunchKernelGGL((k_vel<false, true>), grid, block, 0, c->stream, a);
     else hipLaunchKernelGGL((k_vel<false, false>), grid, block, 0, c->stream, a);
@@ -1290,6 +1288,7 @@ hipError_t launch_fused(swpc_ctx *c)
     a.nby = (g.nyk + 4 * sr - 1) / (4 * sr);
     a.nbz = c->nfz;
     const dim3 grid(a.nbx * a.nby * a.nbz), block(BX, 4);
+    c->aux_moved = true;
 #define SWPC_FUSED_CASE(NMV)                                                                          \
     case NMV:                                                                                         \
         if (sr == 2) hipLaunchKernelGGL((k_fused<NMV, 2>), grid, block, 0, c->stream, a);              \
@@ -1389,7 +1388,7 @@ size_t step_args_size() { return sizeof(StepArgs); }
 
 // arguments of one member for the stress (phase 0) or velocity (phase 1)
 // launches of a whole step
-void fill_batch_args(swpc_ctx *c, void *out, int phase)
+void fill_batch_args(const swpc_ctx *c, void *out, int phase)
 {
     StepArgs a;
     step_args(c, a, MASK_INT | (c->desc.abc == SWPC_ABC_PML ? MASK_PML : MASK_TAPER));
@@ -1398,7 +1397,7 @@ void fill_batch_args(swpc_ctx *c, void *out, int phase)
 }
 
 // interior-column grid of one member: tiles (bx, by, bz)
-void member_tiles(swpc_ctx *c, int &nbx, int &nby, int &nbz)
+void member_tiles(const swpc_ctx *c, int &nbx, int &nby, int &nbz)
 {
     StepArgs a;
     step_args(c, a, MASK_INT | MASK_PML);

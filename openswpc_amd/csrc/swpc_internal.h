@@ -138,9 +138,13 @@ struct swpc_ctx {
     PmlBox box[5];
     long long npml;
     float *ade;
-    // every auxiliary on an axis that does not damp its cell is zero: true
-    // until the profiles are replaced after a step (aux_moved)
+    // aux_still: every auxiliary on an axis that does not damp its cell is
+    // zero.  True until a step has moved an auxiliary (aux_moved: an update has
+    // been enqueued since the profiles were set) and its axis then stops
+    // damping that cell.  aux_axis, per cell of the x, y and z axis: 1 damps
+    // now, 2 damped under earlier profiles that steps ran with.
     bool aux_still, aux_moved;
+    unsigned char *aux_axis;
     float4 *gxc, *gxe, *gyc, *gye, *gzc, *gze;
     int *d_pml_tiles;  // int4 (i0 | width << 20 | xslab << 28, j0, k0, k1) per side-column tile
     int npml_tiles;
@@ -258,8 +262,8 @@ hipError_t launch_counter_advance(int *d, int n, hipStream_t s);
 
 // ---- batched launches (stencil.hip) ----
 size_t step_args_size();
-void fill_batch_args(swpc_ctx *c, void *out, int phase);
-void member_tiles(swpc_ctx *c, int &nbx, int &nby, int &nbz);
+void fill_batch_args(const swpc_ctx *c, void *out, int phase);
+void member_tiles(const swpc_ctx *c, int &nbx, int &nby, int &nbz);
 // batched receivers, sources, Green's-function stores and sources (aux.hip,
 // green.hip): kinds of per-member argument arrays
 enum { BATCH_AUX_WAV = 0, BATCH_AUX_GLUT = 1, BATCH_AUX_BODYFORCE = 2, BATCH_AUX_GREEN_STORE = 3,

@@ -79,6 +79,7 @@ def load_library(path: str = LIB_PATH) -> C.CDLL:
     L.swpc_set_medium.argtypes = [vp, fp, fp, fp, fp, fp, ip, ip, ip, ip, ip]
     L.swpc_set_visco.argtypes = [vp, fp, fp, fp, f]
     L.swpc_set_pml.argtypes = [vp, fp, fp, fp, fp, fp, fp]
+    L.swpc_pml_axes_skipped.argtypes = [vp]
     L.swpc_set_cerjan.argtypes = [vp, fp, fp, fp, fp, fp, fp]
     L.swpc_set_sources.argtypes = [vp, i, i, ip, ip, ip, fp, fp, f, i, fp]
     L.swpc_set_receivers.argtypes = [vp, i, ip, ip, ip, i, i, i, f, f]
@@ -191,6 +192,10 @@ class SwpcGPU:
 
     def set_pml(self, gxc, gxe, gyc, gye, gzc, gze):
         self._chk(self.L.swpc_set_pml(self.h, _f32(gxc), _f32(gxe), _f32(gyc), _f32(gye), _f32(gzc), _f32(gze)))
+
+    def pml_axes_skipped(self):
+        """whether the updates leave the auxiliaries of undamped axes alone"""
+        return self.L.swpc_pml_axes_skipped(self.h) == 1
 
     def set_cerjan(self, gx_c, gx_b, gy_c, gy_b, gz_c, gz_b):
         self._chk(self.L.swpc_set_cerjan(self.h, _f32(gx_c), _f32(gx_b), _f32(gy_c), _f32(gy_b), _f32(gz_c),

@@ -86,6 +86,10 @@ module m_swpc_gpu
             real(c_float), intent(in) :: c1(*), c2(*), d1(*)
             real(c_float), value :: d2
         end function
+        integer(c_int) function swpc_pml_axes_skipped(ctx) bind(C, name='swpc_pml_axes_skipped')
+            import :: c_int, c_ptr
+            type(c_ptr), value :: ctx
+        end function
         integer(c_int) function swpc_set_pml(ctx, gxc, gxe, gyc, gye, gzc, gze) bind(C, name='swpc_set_pml')
             import :: c_int, c_ptr, c_float
             type(c_ptr), value :: ctx
