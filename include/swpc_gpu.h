@@ -421,11 +421,16 @@ int64_t swpc_stripe_free_bytes(int device, int region);
    a step and the stress update of the next in one interior launch (PML runs
    without body forces or the reciprocity mode; the context then holds a
    second set of the 9 fields, taken from the striped arena when it has room;
-   kchunk sets the launch's chunk depth), bit 8 = that launch with 8-row
-   tiles instead of 4; other bits have no effect.  All variants give
-   bit-identical results.  Fails with SWPC_ENOMEM when the second field set
-   does not fit. */
+   kchunk sets the launch's chunk depth, by default 16 halved until it has 7/4
+   blocks per CU), bit 8 = that launch with 8-row tiles instead of 4; other
+   bits have no effect.  All variants give bit-identical results.  Fails with
+   SWPC_ENOMEM when the second field set does not fit. */
 int swpc_set_tuning(swpc_ctx *ctx, int kchunk, int by, int variant);
+
+/* The launch shape in use: k-planes per thread block, rows per tile, variant
+   flags and the k-planes per block of the launch of variant bit 7; any of the
+   pointers may be NULL. */
+int swpc_get_tuning(const swpc_ctx *ctx, int *kchunk, int *by, int *variant, int *kchunk_fused);
 
 /* The HIP stream the context launches on (hipStream_t as void*), so a
    caller can time or order work against it. */

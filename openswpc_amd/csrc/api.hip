@@ -150,6 +150,38 @@ static int build_pml_tiles(swpc_ctx *c)
     return SWPC_OK;
 }
 
+static int compute_units(const swpc_ctx *c)
+{
+    int ncu = 0;
+    if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess || ncu <= 0) {
+        (void)hipGetLastError();
+        ncu = 256;
+    }
+    return ncu;
+}
+
+// The default chunk of the fused launch: 16 planes, halved until it has 7/4
+// blocks per CU (5/4 with 8-row tiles).  Each chunk computes the velocities of
+// four planes more than it updates, so it wants deeper chunks than the phase
+// launches, whose depth this was: us/step at the phase launches' depth and at
+// this one
+//   96^3 (NM = 2, 10-cell PML)    133, 107     128^3 (NM = 0)             152, 136
+//   128^3 (NM = 3)                175, 158     200 x 170 x 90 (NM = 2)    211, 206
+//   220 x 240 x 120 (NM = 0)      362, 333     256 x 256 x 192 (NM = 0)   631, 616
+//   256 x 256 x 192 (NM = 3)      802, 810     448 x 400 x 300 (NM = 1) 2431, 2441
+static int default_kfused(const swpc_ctx *c)
+{
+    const Grid &g = c->g;
+    const bool tall = (c->variant & 256) != 0;
+    const int rows = tall ? 8 : 4, nk = g.ke - g.kb + 1;
+    if (g.nxk <= 0 || g.nyk <= 0 || nk <= 0) return c->kchunk;
+    const long long tiles = (long long)((g.nxk + 59) / 60) * ((g.nyk + rows - 1) / rows);   // 60: FW (stencil.hip)
+    const long long want = (tall ? 5LL : 7LL) * compute_units(c);
+    int kc = 16;
+    while (kc > 1 && 4 * tiles * ((nk + kc - 1) / kc) < want) kc /= 2;
+    return kc;
+}
+
 // k chunks of the interior-column kernels.  Blocks of one chunk form a
 // contiguous run of logical tiles, so each XCD takes whole chunks; a plane
 // of the bottom PML band costs a different time than an interior plane (more
@@ -186,10 +218,11 @@ static int build_zchunks(swpc_ctx *c)
                 break;
             }
     }
-    // fused launch: chunks of kchunk planes over the interior planes kb..ke
+    // fused launch: chunks of kfused planes over the interior planes kb..ke
     // (each chunk recomputes the velocities of two planes on either side)
     const int nki = g.ke - g.kb + 1;
-    const int nfz = nki > 0 ? (nki + c->kchunk - 1) / c->kchunk : 0;
+    c->kfused = c->kchunk_auto ? default_kfused(c) : c->kchunk;
+    const int nfz = nki > 0 ? (nki + c->kfused - 1) / c->kfused : 0;
     std::vector<int> fz(nfz + 1);
     for (int b = 0; b <= nfz; ++b) fz[b] = g.kb + (int)((long long)nki * b / std::max(nfz, 1));
     if (c->d_zchunks) c->bytes -= 2LL * (c->nbz + 1) * (long long)sizeof(int);
@@ -240,11 +273,7 @@ extern "C" void *swpc_staging_buffer(swpc_ctx *ctx, int64_t *nfloats)
 static int default_kchunk(const swpc_ctx *c)
 {
     const Grid &g = c->g;
-    int ncu = 0;
-    if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess || ncu <= 0) {
-        (void)hipGetLastError();
-        ncu = 256;
-    }
+    const int ncu = compute_units(c);
     // tiles of one chunk: interior columns, and the side columns' y and x slabs
     long long tiles =
         g.nxk > 0 && g.nyk > 0 ? (long long)((g.ie - 1) / 64 - (g.ib - 1) / 64 + 1) * ((g.nyk + 3) / 4) : 0;
@@ -295,6 +324,7 @@ extern "C" int swpc_create(const swpc_desc *d, swpc_ctx **out)
     g.nxk = g.ie - g.ib + 1;
     g.nyk = g.je - g.jb + 1;
     c->kchunk = default_kchunk(c);
+    c->kchunk_auto = true;
     g.nzk = g.ke - g.kb + 1;
     // memory variables keep full-width rows (i = 1 at offset 0) so that they
     // align with the field rows; only interior cells are ever touched
@@ -1315,6 +1345,16 @@ extern "C" int swpc_synchronize(swpc_ctx *c)
     return SWPC_OK;
 }
 
+extern "C" int swpc_get_tuning(const swpc_ctx *c, int *kchunk, int *by, int *variant, int *kchunk_fused)
+{
+    if (!c) return SWPC_EINVAL;
+    if (kchunk) *kchunk = c->kchunk;
+    if (by) *by = c->by;
+    if (variant) *variant = c->variant;
+    if (kchunk_fused) *kchunk_fused = c->kfused;
+    return SWPC_OK;
+}
+
 extern "C" int swpc_set_tuning(swpc_ctx *c, int kchunk, int by, int variant)
 {
     if (!c) return SWPC_EINVAL;
@@ -1324,8 +1364,10 @@ extern "C" int swpc_set_tuning(swpc_ctx *c, int kchunk, int by, int variant)
     // the tables rebuilt below may be read by work on any stream of the
     // device (the context's own, a batch's that steps this member)
     HIPCHK(c, hipDeviceSynchronize());
-    if (kchunk > 0) c->kchunk = kchunk;
-    else if (kchunk == -1) c->kchunk = default_kchunk(c);
+    if (kchunk != 0) {
+        c->kchunk = kchunk > 0 ? kchunk : default_kchunk(c);
+        c->kchunk_auto = kchunk < 0;
+    }
     if (by > 0) c->by = by;
     if (variant >= 0) c->variant = variant;
     reset_graph(c);

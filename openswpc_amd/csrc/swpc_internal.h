@@ -203,6 +203,8 @@ struct swpc_ctx {
     float *d_vmax;
 
     int kchunk, by;
+    bool kchunk_auto;  // the default chunk, not one the caller set
+    int kfused;        // planes per chunk of the fused launch
     int nbz;           // k chunks of the interior-column kernels
     int *d_zchunks;    // first plane of each chunk, stress phase then velocity phase (2 x (nbz+1))
     int zband[2];      // per phase, the first chunk that holds planes of the bottom PML band

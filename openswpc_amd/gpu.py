@@ -110,6 +110,7 @@ def load_library(path: str = LIB_PATH) -> C.CDLL:
     L.swpc_device_bytes.argtypes = [vp]
     L.swpc_device_bytes.restype = C.c_int64
     L.swpc_set_tuning.argtypes = [vp, i, i, i]
+    L.swpc_get_tuning.argtypes = [vp] + [C.POINTER(C.c_int)] * 4
     L.swpc_stream.argtypes = [vp]
     L.swpc_stream.restype = vp
     L.swpc_adj_gradient.argtypes = [vp, i, fp, i, C.POINTER(C.c_double), vp, vp, vp]
@@ -447,6 +448,12 @@ class SwpcGPU:
 
     def set_tuning(self, kchunk=0, by=0, variant=-1):
         self._chk(self.L.swpc_set_tuning(self.h, int(kchunk), int(by), int(variant)))
+
+    def tuning(self):
+        """(k chunk, tile rows, variant, k chunk of the fused launch) in use"""
+        v = [C.c_int() for _ in range(4)]
+        self._chk(self.L.swpc_get_tuning(self.h, *(C.byref(q) for q in v)))
+        return tuple(q.value for q in v)
 
     def stream(self):
         return self.L.swpc_stream(self.h)

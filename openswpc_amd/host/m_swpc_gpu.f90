@@ -367,6 +367,11 @@ module m_swpc_gpu
             type(c_ptr), value :: ctx
             integer(c_int), value :: kchunk, by, variant
         end function
+        integer(c_int) function swpc_get_tuning(ctx, kchunk, by, variant, kchunk_fused) bind(C, name='swpc_get_tuning')
+            import :: c_int, c_ptr
+            type(c_ptr), value :: ctx
+            integer(c_int), intent(out) :: kchunk, by, variant, kchunk_fused
+        end function
         type(c_ptr) function swpc_stream(ctx) bind(C, name='swpc_stream')
             import :: c_ptr
             type(c_ptr), value :: ctx
