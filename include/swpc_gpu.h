@@ -333,6 +333,12 @@ int swpc_batch_tune(swpc_batch *batch, int trial_steps, int *kchunk, int *by, in
    rows they border (one launch per phase).  Results do not depend on it. */
 int swpc_batch_set_packing(swpc_batch *batch, int packing);
 int swpc_batch_get_packing(const swpc_batch *batch);
+
+/* The k-planes per thread block of a member's tiles in the batch: what
+   swpc_set_tuning set for the member, or, where the member has the default,
+   one depth for all such members by the tiles of the whole batch (4 planes, 8
+   when nm = 0, halved until its launches have 50 or 40 blocks per CU). */
+int swpc_batch_get_kchunk(const swpc_batch *batch, int member);
 void *swpc_batch_stream(swpc_batch *batch);
 
 /* ---- discrete adjoint (ADE-CFS PML; elastic or with Zener memory variables) ----

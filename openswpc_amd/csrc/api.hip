@@ -107,8 +107,33 @@ static void reset_graph(swpc_ctx *c)
     c->graph_block = 0;
 }
 
-// Tiles (64 x by columns, one k chunk) that hold PML cells: side columns
-// over the full depth, interior columns over the bottom na planes.
+// Tiles (64 x by columns, one k chunk of kc planes) of the side columns, over
+// the full depth: (i0 | width << 20 | xslab << 28, j0, k0, k1) each.  The
+// bottom band of interior columns is marched by the interior kernels.
+std::vector<int> side_tiles(const Grid &g, int by, int kc)
+{
+    const int nx = g.nx, ny = g.ny, nz = g.nz, na = g.na;
+    std::vector<int> t;
+    auto add = [&](int i0, int w, int xslab, int j0, int k0, int k1) {
+        t.push_back(i0 | (w << 20) | (xslab << 28)); t.push_back(j0); t.push_back(k0); t.push_back(k1);
+    };
+    // x slabs (side columns of interior rows), width na, several rows per block
+    const int slab_rows = (64 * by) / na;
+    for (int k0 = 1; k0 <= nz; k0 += kc) {
+        const int k1 = std::min(nz, k0 + kc - 1);
+        // y-slab rows as full-row tiles, each within its slab
+        for (int j0 = 1; j0 <= na; j0 += by)
+            for (int i0 = 1; i0 <= nx; i0 += 64) add(i0, 64, 0, j0, k0, k1);
+        for (int j0 = ny - na + 1; j0 <= ny; j0 += by)
+            for (int i0 = 1; i0 <= nx; i0 += 64) add(i0, 64, 0, j0, k0, k1);
+        for (int j0 = na + 1; j0 <= ny - na; j0 += slab_rows) {
+            add(1, na, 1, j0, k0, k1);
+            add(nx - na + 1, na, 1, j0, k0, k1);
+        }
+    }
+    return t;
+}
+
 static int build_pml_tiles(swpc_ctx *c)
 {
     if (c->d_pml_tiles) c->bytes -= (long long)c->npml_tiles * 4 * (long long)sizeof(int);
@@ -116,32 +141,8 @@ static int build_pml_tiles(swpc_ctx *c)
     c->d_pml_tiles = nullptr;
     c->npml_tiles = 0;
     if (c->desc.abc != SWPC_ABC_PML || c->npml == 0) return SWPC_OK;
-    const int nx = c->g.nx, ny = c->g.ny, nz = c->g.nz, na = c->g.na, by = c->by, kc = c->kchunk;
-    std::vector<int> t;
-    // tile = (i0 | width << 20 | xslab << 28, j0, k0, k1)
-    auto add = [&](int i0, int w, int xslab, int j0, int k0, int k1) {
-        t.push_back(i0 | (w << 20) | (xslab << 28)); t.push_back(j0); t.push_back(k0); t.push_back(k1);
-    };
-    // x slabs (side columns of interior rows), width na, several rows per block
-    const int slab_rows = (64 * by) / std::max(na, 1);
-    const bool slab_tiles = na > 0 && na <= 64 && slab_rows > 0;
-    for (int k0 = 1; k0 <= nz; k0 += kc) {
-        const int k1 = std::min(nz, k0 + kc - 1);
-        // y-slab rows as full-row tiles over the full depth, each within its
-        // slab; the bottom band of interior columns is marched by the interior
-        // kernels
-        for (int j0 = 1; j0 <= na; j0 += by)
-            for (int i0 = 1; i0 <= nx; i0 += 64) add(i0, 64, 0, j0, k0, k1);
-        for (int j0 = ny - na + 1; j0 <= ny; j0 += by)
-            for (int i0 = 1; i0 <= nx; i0 += 64) add(i0, 64, 0, j0, k0, k1);
-        if (slab_tiles)
-            for (int j0 = na + 1; j0 <= ny - na; j0 += slab_rows) {
-                add(1, na, 1, j0, k0, k1);
-                add(nx - na + 1, na, 1, j0, k0, k1);
-            }
-    }
-    if (!slab_tiles && na > 0) return fail(c, SWPC_EINVAL, "PML thickness na must be 1..64");
-    if (t.empty()) return SWPC_OK;
+    if (c->g.na > 64) return fail(c, SWPC_EINVAL, "PML thickness na must be 1..64");
+    const std::vector<int> t = side_tiles(c->g, c->by, c->kchunk);
     if (dalloc(c, (void **)&c->d_pml_tiles, t.size() * sizeof(int)) != hipSuccess)
         return fail(c, SWPC_ENOMEM, "PML tile list allocation failed");
     HIPCHK(c, hipMemcpyAsync(c->d_pml_tiles, t.data(), t.size() * sizeof(int), hipMemcpyHostToDevice, c->stream));
@@ -150,7 +151,7 @@ static int build_pml_tiles(swpc_ctx *c)
     return SWPC_OK;
 }
 
-static int compute_units(const swpc_ctx *c)
+int compute_units(const swpc_ctx *c)
 {
     int ncu = 0;
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess || ncu <= 0) {
@@ -186,18 +187,21 @@ static int default_kfused(const swpc_ctx *c)
 // contiguous run of logical tiles, so each XCD takes whole chunks; a plane
 // of the bottom PML band costs a different time than an interior plane (more
 // in the velocity phase, about the same in the stress phase), so chunk
-// boundaries equalise estimated time per chunk rather than planes.
-static int build_zchunks(swpc_ctx *c)
+// boundaries equalise estimated time per chunk rather than planes.  Returns
+// the number of chunks and, in zc, the first plane of each and nz + 1, for the
+// stress phase and then for the velocity phase; zband: per phase, the first
+// chunk with planes of the band.
+int zchunk_table(const swpc_ctx *c, int kchunk, std::vector<int> &zc, int zband[2])
 {
     const Grid &g = c->g;
     const int nz = g.nz, nm = g.nm;
-    const int nbz = std::max(1, std::min(nz, (nz + c->kchunk - 1) / c->kchunk));
+    const int nbz = std::max(1, std::min(nz, (nz + kchunk - 1) / kchunk));
     const bool pml = c->desc.abc == SWPC_ABC_PML && c->npml > 0;
     // relative time per cell: algorithmic bytes over the streaming rate the
     // two loops reach (interior ~4.7 TB/s, PML band ~3.0 TB/s on MI355X)
     const double w_int[2] = {4.0 * (3 + 4 + 12 + 12 * nm), 4.0 * (6 + 1 + 6)};   // stress, velocity
     const double w_pml[2] = {4.0 * (3 + 2 + 12 + 18) * 1.55, 4.0 * (6 + 1 + 6 + 18) * 1.55};
-    std::vector<int> zc(2 * (nbz + 1));
+    zc.assign(2 * (nbz + 1), 0);
     for (int ph = 0; ph < 2; ++ph) {
         std::vector<double> W(nz + 1, 0.0);
         for (int k = 1; k <= nz; ++k) W[k] = W[k - 1] + ((pml && k > g.ke) ? w_pml[ph] : w_int[ph]);
@@ -211,13 +215,21 @@ static int build_zchunks(swpc_ctx *c)
             z[b] = std::min(std::max(k + 1, z[b - 1] + 1), nz - (nbz - b) + 1);
         }
         z[nbz] = nz + 1;
-        c->zband[ph] = 0;
+        zband[ph] = 0;
         for (int b = 0; b < nbz; ++b)
             if (pml && z[b + 1] - 1 > g.ke) {
-                c->zband[ph] = b;
+                zband[ph] = b;
                 break;
             }
     }
+    return nbz;
+}
+
+static int build_zchunks(swpc_ctx *c)
+{
+    const Grid &g = c->g;
+    std::vector<int> zc;
+    const int nbz = zchunk_table(c, c->kchunk, zc, c->zband);
     // fused launch: chunks of kfused planes over the interior planes kb..ke
     // (each chunk recomputes the velocities of two planes on either side)
     const int nki = g.ke - g.kb + 1;
@@ -259,6 +271,18 @@ extern "C" void *swpc_staging_buffer(swpc_ctx *ctx, int64_t *nfloats)
     return ctx ? (void *)ctx->staging : nullptr;
 }
 
+// tiles of one chunk of a phase (64 wide, 4 rows): interior columns, and the
+// side columns' y and x slabs
+long long phase_tiles(const swpc_ctx *c)
+{
+    const Grid &g = c->g;
+    long long tiles =
+        g.nxk > 0 && g.nyk > 0 ? (long long)((g.ie - 1) / 64 - (g.ib - 1) / 64 + 1) * ((g.nyk + 3) / 4) : 0;
+    if (c->desc.abc == SWPC_ABC_PML && g.na > 0 && g.na <= 64)
+        tiles += 2LL * ((g.na + 3) / 4) * ((g.nx + 63) / 64) + 2LL * ((g.nyk + 256 / g.na - 1) / (256 / g.na));
+    return tiles;
+}
+
 // The default k chunk of a context: 16 planes, halved until a phase's launch
 // has 14 blocks per CU (four are resident at a time), down to one plane.  A
 // march spares reading its z neighbours again, but its planes follow one
@@ -273,14 +297,9 @@ extern "C" void *swpc_staging_buffer(swpc_ctx *ctx, int64_t *nfloats)
 static int default_kchunk(const swpc_ctx *c)
 {
     const Grid &g = c->g;
-    const int ncu = compute_units(c);
-    // tiles of one chunk: interior columns, and the side columns' y and x slabs
-    long long tiles =
-        g.nxk > 0 && g.nyk > 0 ? (long long)((g.ie - 1) / 64 - (g.ib - 1) / 64 + 1) * ((g.nyk + 3) / 4) : 0;
-    if (c->desc.abc == SWPC_ABC_PML && g.na > 0 && g.na <= 64)
-        tiles += 2LL * ((g.na + 3) / 4) * ((g.nx + 63) / 64) + 2LL * ((g.nyk + 256 / g.na - 1) / (256 / g.na));
+    const long long tiles = phase_tiles(c), want = 14LL * compute_units(c);
     int kc = 16;
-    while (tiles > 0 && kc > 1 && tiles * ((g.nz + kc - 1) / kc) < 14LL * ncu) kc /= 2;
+    while (tiles > 0 && kc > 1 && tiles * ((g.nz + kc - 1) / kc) < want) kc /= 2;
     return kc;
 }
 

@@ -35,6 +35,8 @@ struct swpc_batch {
     hipStream_t stream;
     int nm, by;
     bool tp;                       // Cerjan members: the update applies their taper
+    std::vector<int> kchunk;       // planes per chunk of each member's tiles
+    int *d_zc;                     // the chunks' first planes
     int packing;                   // tile order of the tables (see above)
     void *d_args[2];               // StepArgs of every member: stress, velocity
     int4 *d_cols, *d_side;
@@ -89,6 +91,9 @@ static void free_tables(swpc_batch *b)
     bfree(p);
     b->d_cols = b->d_side = nullptr;
     b->ncols = b->nside = 0;
+    p = b->d_zc;
+    bfree(p);
+    b->d_zc = nullptr;
     p = b->d_all;
     bfree(p);
     b->d_all = nullptr;
@@ -105,6 +110,28 @@ static void free_tables(swpc_batch *b)
 // interior tile width of the members (variant bit 2: 32 cells, else 64)
 static int batch_bxw(const swpc_batch *b) { return (b->mem[0]->variant & 4) ? 32 : 64; }
 
+// The chunk of members that have the default one: the batch's launches hold
+// all members' tiles, so it goes by the tiles of all of them, and it is the
+// same for all, as each XCD takes an equal run of tiles whatever their depth:
+// 4 planes (8 without memory variables, where a chunk's first loads weigh
+// more), halved until there are 50 (40) blocks per CU.  us/step, packing 0,
+// with each member's own default and with this one:
+//   12 members of 96 to 256 cells an axis (NM = 2)  4460 (4 and 8 planes), 3785 (4)
+//   8 of 150 to 250 (NM = 3)     3733, 3488 (4)     64 of 64 to 128 (NM = 3)  3260, 3106 (4)
+//   14 of 64 to 120 (NM = 1)     610 (1), 602 (4)   32 of 48 to 80 (NM = 3)   566 (1), 559 (2)
+//   4 of 64 to 100 (NM = 2)      156 (1), 156 (1)   2 of 180 to 240 (NM = 0)  748, 755 (8)
+//   3 of 100 to 140 (NM = 0)     237, 238 (2)       24 of 40 to 60 (NM = 1)   212 (1), 208 (1)
+static int batch_kchunk(const swpc_batch *b)
+{
+    const long long want = (b->nm > 0 ? 50LL : 40LL) * compute_units(b->mem[0]);
+    for (int kc = b->nm > 0 ? 4 : 8; kc > 1; kc /= 2) {
+        long long blocks = 0;
+        for (const swpc_ctx *c : b->mem) blocks += phase_tiles(c) * ((c->g.nz + kc - 1) / kc);
+        if (blocks >= want) return kc;
+    }
+    return 1;
+}
+
 // (re)build the argument arrays and tile tables from the members' current state
 static int build_tables(swpc_batch *b)
 {
@@ -119,6 +146,20 @@ static int build_tables(swpc_batch *b)
         const Grid &gx = b->mem[x]->g, &gy = b->mem[y]->g;
         return (long long)gx.nx * gx.ny * gx.nz > (long long)gy.nx * gy.ny * gy.nz;
     });
+    // the members' chunks
+    b->kchunk.assign(n, batch_kchunk(b));
+    std::vector<std::vector<int>> zc(n);
+    std::vector<size_t> zoff(n);
+    std::vector<int> zall;
+    for (int m = 0; m < n; ++m) {
+        if (!b->mem[m]->kchunk_auto) b->kchunk[m] = b->mem[m]->kchunk;
+        int zband[2];
+        zchunk_table(b->mem[m], b->kchunk[m], zc[m], zband);
+        zoff[m] = zall.size();
+        zall.insert(zall.end(), zc[m].begin(), zc[m].end());
+    }
+    BCHK(b, hipMalloc((void **)&b->d_zc, zall.size() * sizeof(int)));
+    BCHK(b, hipMemcpy(b->d_zc, zall.data(), zall.size() * sizeof(int), hipMemcpyHostToDevice));
     const size_t asz = step_args_size();
     std::vector<char> args[2] = {std::vector<char>(asz * n), std::vector<char>(asz * n)};
     // per member, its interior tiles and side tiles grouped by k chunk
@@ -127,11 +168,12 @@ static int build_tables(swpc_batch *b)
     for (int m : order) {
         swpc_ctx *c = b->mem[m];
         if (c->by != b->by) return bfail(b, SWPC_ESTATE, "member %d has tile rows %d, batch %d", m, c->by, b->by);
-        fill_batch_args(c, args[0].data() + asz * m, 0);
-        fill_batch_args(c, args[1].data() + asz * m, 1);
-        int nbx, nby, nbz;
-        member_tiles(c, nbx, nby, nbz);
-        const int nch = (c->g.nz + c->kchunk - 1) / c->kchunk;
+        const int kc = b->kchunk[m], nbz = (int)zc[m].size() / 2 - 1;
+        fill_batch_args(c, args[0].data() + asz * m, b->d_zc + zoff[m]);
+        fill_batch_args(c, args[1].data() + asz * m, b->d_zc + zoff[m] + nbz + 1);
+        int nbx, nby;
+        member_tiles(c, nbx, nby);
+        const int nch = (c->g.nz + kc - 1) / kc;
         mcols[m].assign(std::max(nbz, nch), {});
         mside[m].assign(std::max(nbz, nch), {});
         maxchunks = std::max(maxchunks, (int)mcols[m].size());
@@ -140,11 +182,11 @@ static int build_tables(swpc_batch *b)
                 for (int by = 0; by < nby; ++by)
                     for (int bx = 0; bx < nbx; ++bx) mcols[m][bz].push_back(make_int4(m, bx, by, bz));
         if (c->desc.abc == SWPC_ABC_PML && c->npml_tiles > 0) {
-            std::vector<int4> t(c->npml_tiles);
-            BCHK(b, hipMemcpy(t.data(), c->d_pml_tiles, t.size() * sizeof(int4), hipMemcpyDeviceToHost));
-            for (const int4 &x : t) {
+            const std::vector<int> t = side_tiles(c->g, b->by, kc);
+            for (size_t q = 0; q < t.size(); q += 4) {
+                const int4 x = make_int4(t[q], t[q + 1], t[q + 2], t[q + 3]);
                 if (x.z > 0xFFFF || x.w > 0x7FFF) return bfail(b, SWPC_EINVAL, "member %d: nz too large", m);
-                const int ch = std::min((x.z - 1) / c->kchunk, (int)mside[m].size() - 1);
+                const int ch = std::min((x.z - 1) / kc, (int)mside[m].size() - 1);
                 mside[m][ch].push_back(make_int4(x.x, x.y, x.z | (x.w << 16), m));
             }
         }
@@ -411,6 +453,11 @@ extern "C" int swpc_batch_set_packing(swpc_batch *b, int packing)
     if (packing == b->packing) return SWPC_OK;
     b->packing = packing;
     return build_tables(b);
+}
+
+extern "C" int swpc_batch_get_kchunk(const swpc_batch *b, int member)
+{
+    return b && member >= 0 && member < (int)b->kchunk.size() ? b->kchunk[member] : SWPC_EINVAL;
 }
 
 extern "C" int swpc_batch_get_packing(const swpc_batch *b) { return b ? b->packing : SWPC_EINVAL; }

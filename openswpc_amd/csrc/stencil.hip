@@ -1386,24 +1386,23 @@ hipError_t launch_cerjan_vel(swpc_ctx *c)
 // ---------------------------------------------------------------------------
 size_t step_args_size() { return sizeof(StepArgs); }
 
-// arguments of one member for the stress (phase 0) or velocity (phase 1)
-// launches of a whole step
-void fill_batch_args(const swpc_ctx *c, void *out, int phase)
+// arguments of one member for the launches of a whole step's phase, whose
+// chunks start at the planes in zc
+void fill_batch_args(const swpc_ctx *c, void *out, const int *zc)
 {
     StepArgs a;
     step_args(c, a, MASK_INT | (c->desc.abc == SWPC_ABC_PML ? MASK_PML : MASK_TAPER));
-    if (phase == 1) a.zc = c->d_zchunks + c->nbz + 1;
+    a.zc = zc;
     *(StepArgs *)out = a;
 }
 
-// interior-column grid of one member: tiles (bx, by, bz)
-void member_tiles(const swpc_ctx *c, int &nbx, int &nby, int &nbz)
+// interior-column tiles of one member's chunk: (bx, by)
+void member_tiles(const swpc_ctx *c, int &nbx, int &nby)
 {
     StepArgs a;
     step_args(c, a, MASK_INT | MASK_PML);
     nbx = a.nbx;
     nby = a.nby;
-    nbz = a.nbz;
 }
 
 // one launch per phase for both kinds of tiles (the batch's packing 2)

@@ -14,6 +14,8 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+
+#include <vector>
 #include <stdint.h>
 
 #include "../../include/swpc_gpu.h"
@@ -224,6 +226,11 @@ struct swpc_ctx {
 int ctx_fail(swpc_ctx *c, int code, const char *msg);
 // launch arguments changed: drops the captured graphs (api.hip)
 void ctx_reset_graph(swpc_ctx *c);
+// launch shapes of a context (api.hip)
+int compute_units(const swpc_ctx *c);
+long long phase_tiles(const swpc_ctx *c);
+std::vector<int> side_tiles(const Grid &g, int by, int kc);
+int zchunk_table(const swpc_ctx *c, int kchunk, std::vector<int> &zc, int zband[2]);
 int ctx_find_tau(swpc_ctx *c);
 
 // ---- striped device arena (arena.hip) ----
@@ -264,8 +271,8 @@ hipError_t launch_counter_advance(int *d, int n, hipStream_t s);
 
 // ---- batched launches (stencil.hip) ----
 size_t step_args_size();
-void fill_batch_args(const swpc_ctx *c, void *out, int phase);
-void member_tiles(const swpc_ctx *c, int &nbx, int &nby, int &nbz);
+void fill_batch_args(const swpc_ctx *c, void *out, const int *zc);
+void member_tiles(const swpc_ctx *c, int &nbx, int &nby);
 // batched receivers, sources, Green's-function stores and sources (aux.hip,
 // green.hip): kinds of per-member argument arrays
 enum { BATCH_AUX_WAV = 0, BATCH_AUX_GLUT = 1, BATCH_AUX_BODYFORCE = 2, BATCH_AUX_GREEN_STORE = 3,

@@ -134,6 +134,7 @@ def load_library(path: str = LIB_PATH) -> C.CDLL:
     L.swpc_batch_stream.argtypes = [vp]
     L.swpc_batch_set_packing.argtypes = [vp, i]
     L.swpc_batch_get_packing.argtypes = [vp]
+    L.swpc_batch_get_kchunk.argtypes = [vp, i]
     L.swpc_batch_stream.restype = vp
     L.swpc_stripe_reserve.argtypes = [i, C.c_int64, i]
     L.swpc_stripe_release.argtypes = [i]
@@ -493,6 +494,10 @@ class SwpcBatch:
 
     def set_packing(self, packing):
         self._chk(self.L.swpc_batch_set_packing(self.h, int(packing)))
+
+    def kchunks(self):
+        """planes per block of each member's tiles"""
+        return [int(self.L.swpc_batch_get_kchunk(self.h, m)) for m in range(len(self.members))]
 
     def packing(self):
         return int(self.L.swpc_batch_get_packing(self.h))

@@ -335,6 +335,11 @@ module m_swpc_gpu
             import :: c_int, c_ptr
             type(c_ptr), value :: batch
         end function
+        integer(c_int) function swpc_batch_get_kchunk(batch, member) bind(C, name='swpc_batch_get_kchunk')
+            import :: c_int, c_ptr
+            type(c_ptr), value :: batch
+            integer(c_int), value :: member
+        end function
         type(c_ptr) function swpc_batch_stream(batch) bind(C, name='swpc_batch_stream')
             import :: c_ptr
             type(c_ptr), value :: batch
