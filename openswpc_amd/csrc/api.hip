@@ -184,9 +184,8 @@ static int default_kfused(const swpc_ctx *c)
 }
 
 // k chunks of the interior-column kernels.  Blocks of one chunk form a
-// contiguous run of logical tiles, so each XCD takes whole chunks; a plane
-// of the bottom PML band costs a different time than an interior plane (more
-// in the velocity phase, about the same in the stress phase), so chunk
+// contiguous run of logical tiles, so each XCD takes whole chunks; a plane of
+// the bottom PML band costs a different time than an interior plane, so chunk
 // boundaries equalise estimated time per chunk rather than planes.  Returns
 // the number of chunks and, in zc, the first plane of each and nz + 1, for the
 // stress phase and then for the velocity phase; zband: per phase, the first
@@ -197,10 +196,18 @@ int zchunk_table(const swpc_ctx *c, int kchunk, std::vector<int> &zc, int zband[
     const int nz = g.nz, nm = g.nm;
     const int nbz = std::max(1, std::min(nz, (nz + kchunk - 1) / kchunk));
     const bool pml = c->desc.abc == SWPC_ABC_PML && c->npml > 0;
-    // relative time per cell: algorithmic bytes over the streaming rate the
-    // two loops reach (interior ~4.7 TB/s, PML band ~3.0 TB/s on MI355X)
-    const double w_int[2] = {4.0 * (3 + 4 + 12 + 12 * nm), 4.0 * (6 + 1 + 6)};   // stress, velocity
-    const double w_pml[2] = {4.0 * (3 + 2 + 12 + 18) * 1.55, 4.0 * (6 + 1 + 6 + 18) * 1.55};
+    // relative time per cell: the words it moves (in the band the auxiliaries
+    // of z, the one axis that damps most of its cells; taup and taus only with
+    // memory variables), a band cell's stress update at 1 / 1.2 of the
+    // interior's rate.  Best ratios of a band plane to an interior one when
+    // swept: velocity 1.5 everywhere; stress 1.3, 1.0, 0.8, 0.5 at NM = 0, 1,
+    // 2, 3.  us per launch, stress and velocity, with all 18 words at 1 / 1.55
+    // and with these: 256 x 256 x 192 (NM = 0) 167, 139 and 152, 122; 448 x
+    // 400 x 300 (NM = 1) 1054, 570 and 1034, 529; 512 x 512 x 256 (NM = 2)
+    // 1740, 735 and 1724, 666; 640 x 640 x 400 (NM = 3) 5340, 1712 and 5320,
+    // 1620.
+    const double w_int[2] = {3.0 + 2 + (nm > 0 ? 2 : 0) + 12 + 12 * nm, 6.0 + 1 + 6};   // stress, velocity
+    const double w_pml[2] = {(3.0 + 2 + 12 + 6) * 1.2, 6.0 + 1 + 6 + 6};
     zc.assign(2 * (nbz + 1), 0);
     for (int ph = 0; ph < 2; ++ph) {
         std::vector<double> W(nz + 1, 0.0);
