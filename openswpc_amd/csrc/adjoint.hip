@@ -217,10 +217,11 @@ __device__ static inline float4 prof(const float4 *p, int n) { return p[n - 1]; 
 // The blocks form a 1D grid, plane after plane, each plane's tiles padded to
 // a multiple of 8 blocks: block b goes to XCD b % 8, so a tile and the same
 // tile one plane up or down share an XCD and its L2, and each plane still
-// spreads over all eight XCDs.  (A thread marching over several planes keeps
-// the 64-bit addresses of every array and offset live across its loop and
-// halves the occupancy; keeping whole planes on one XCD overflows its L2
-// with the z neighbours of nine density arrays.  Both measured slower.
+// spreads over all eight XCDs.  (Keeping whole planes on one XCD overflows its
+// L2 with the z neighbours of nine density arrays: measured slower.  So was a
+// thread marching over several planes while every array took a 64-bit address
+// of its own, which halved the occupancy; with the present addresses a march
+// has not been tried.
 // Giving each XCD a contiguous eighth of a plane's tiles keeps halo rows in
 // one L2: 2.79 against 2.84 ms per gradient step at 256 x 256 x 192, but
 // 10.04 against 9.93 ms per source-step at 384 x 384 x 256, NM = 3.  With

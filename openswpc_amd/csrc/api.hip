@@ -202,10 +202,10 @@ int zchunk_table(const swpc_ctx *c, int kchunk, std::vector<int> &zc, int zband[
     // interior's rate.  Best ratios of a band plane to an interior one when
     // swept: velocity 1.5 everywhere; stress 1.3, 1.0, 0.8, 0.5 at NM = 0, 1,
     // 2, 3.  us per launch, stress and velocity, with all 18 words at 1 / 1.55
-    // and with these: 256 x 256 x 192 (NM = 0) 167, 139 and 152, 122; 448 x
-    // 400 x 300 (NM = 1) 1054, 570 and 1034, 529; 512 x 512 x 256 (NM = 2)
-    // 1740, 735 and 1724, 666; 640 x 640 x 400 (NM = 3) 5340, 1712 and 5320,
-    // 1620.
+    // and with these: 256 x 256 x 192 (NM = 0) 167, 139 and 155, 123; 448 x
+    // 400 x 300 (NM = 1) 1054, 570 and 1042, 532; 512 x 512 x 256 (NM = 2)
+    // 1740, 735 and 1733, 670; 640 x 640 x 400 (NM = 3) 5340, 1712 and 5316,
+    // 1630.
     const double w_int[2] = {3.0 + 2 + (nm > 0 ? 2 : 0) + 12 + 12 * nm, 6.0 + 1 + 6};   // stress, velocity
     const double w_pml[2] = {(3.0 + 2 + 12 + 6) * 1.2, 6.0 + 1 + 6 + 6};
     zc.assign(2 * (nbz + 1), 0);
@@ -294,13 +294,14 @@ long long phase_tiles(const swpc_ctx *c)
 // has 14 blocks per CU (four are resident at a time), down to one plane.  A
 // march spares reading its z neighbours again, but its planes follow one
 // another, so a grid that gives the chip few blocks waits for them: us/step
-// at 16, 8, 4, 2, 1 planes per chunk
-//   48 x 44 x 40   (NM = 3):  -, 88, 41, 19, 17
-//   128^3          (NM = 3):  162 (8), 129 (4), 127 (2)
-//   168 x 152 x 120 (NM = 2): 183 (8), 173 (4), 175 (2)
-//   256 x 256 x 192 (NM = 0): 510 (16), 505 (8), 510 (4)
-//   384 x 384 x 256 (NM = 3): 2020 (16), 2010 (8), 2320 (4)
-// and 13.21, 13.29, 13.32 ms at 16, 12 and 24 on 768 x 768 x 448.
+// at 16, 8, 4, 2, 1 planes per chunk, the default in brackets
+//   48 x 44 x 40 (NM = 3)        -, 35, 22, 16, [12]
+//   128^3 (NM = 3)             118, 117, 109, [107], 118
+//   168 x 152 x 120 (NM = 2)   170, 159, [154], 154, 165
+//   256 x 256 x 192 (NM = 0)   406, [405], 408, 426
+//   384 x 384 x 256 (NM = 3)  [1810], 1806, 1793
+// and 12.52, 12.46, [12.44], 12.43, 12.48 ms at 8, 12, 16, 24, 32 planes on 768
+// x 768 x 448 (NM = 3).  Tiles count as 64 x 4 cells whatever their shape.
 static int default_kchunk(const swpc_ctx *c)
 {
     const Grid &g = c->g;

@@ -21,7 +21,7 @@
 // per-region slabs.  When the arena is missing or full, allocation falls
 // back to hipMalloc.  A freed range of granules stays mapped, and counts as
 // free, until its granules are needed for another one: unmapping 16 GiB takes
-// 16 ms and mapping them again 5, which a gradient paid for its checkpoint
+// 16 ms and mapping them again 3 (17 the first time), which a gradient paid for its checkpoint
 // and record stores on every call (see take_parked).  The arena is process-wide, one per device; contexts
 // hold no reference to it, so swpc_stripe_release refuses while any of its
 // memory is in use.  A large context created on a device without an arena

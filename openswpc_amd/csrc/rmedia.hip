@@ -6,8 +6,8 @@
 // Noise comes from a counter-based generator (one 64-bit mix per cell), so a
 // realisation depends on the seed and the grid only, not on launch shapes.
 // Transforms are double-precision and of any size (the reference's radix-2
-// FFT, m_rfft.f90:46, needs powers of two); sums are deterministic two-pass
-// reductions.  The field is written as float.  Grids whose lines fit in LDS
+// FFT, m_rfft.f90:46, needs powers of two); sums are deterministic, per block
+// and then over the blocks.  The field is written as float.  Grids whose lines fit in LDS
 // are transformed by the kernels here; the others by hipFFT.
 #include <hipfft/hipfft.h>
 

@@ -192,7 +192,6 @@ __device__ __forceinline__ void pml_stress_cell(const StepArgs &a, Loc p, Loc q,
                                                 float mu01n, float mu11, float4 gxc, float4 gxe, float4 gyc,
                                                 float4 gye)
 {
-    const long long P = a.g.plane;
     const float *__restrict__ Vx = a.f.Vx;
     const float *__restrict__ Vy = a.f.Vy;
     const float *__restrict__ Vz = a.f.Vz;
@@ -200,7 +199,6 @@ __device__ __forceinline__ void pml_stress_cell(const StepArgs &a, Loc p, Loc q,
     float *__restrict__ A = a.ade;
     const float *__restrict__ AI = OOP ? a.ade_in : A;
     const float dt = a.dt;
-    (void)P;
     const float vx_im1 = ld(Vx, p, 0, -1), vy_jm1 = ld(Vy, p, 0, 0, -1);
     const float vy_ip1 = ld(Vy, p, 0, 1), vz_ip1 = ld(Vz, p, 0, 1);
     const float vx_jp1 = ld(Vx, p, 0, 0, 1), vz_jp1 = ld(Vz, p, 0, 0, 1);
