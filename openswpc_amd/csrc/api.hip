@@ -188,9 +188,8 @@ static int default_kfused(const swpc_ctx *c)
 // the bottom PML band costs a different time than an interior plane, so chunk
 // boundaries equalise estimated time per chunk rather than planes.  Returns
 // the number of chunks and, in zc, the first plane of each and nz + 1, for the
-// stress phase and then for the velocity phase; zband: per phase, the first
-// chunk with planes of the band.
-int zchunk_table(const swpc_ctx *c, int kchunk, std::vector<int> &zc, int zband[2])
+// stress phase and then for the velocity phase.
+int zchunk_table(const swpc_ctx *c, int kchunk, std::vector<int> &zc)
 {
     const Grid &g = c->g;
     const int nz = g.nz, nm = g.nm;
@@ -222,12 +221,6 @@ int zchunk_table(const swpc_ctx *c, int kchunk, std::vector<int> &zc, int zband[
             z[b] = std::min(std::max(k + 1, z[b - 1] + 1), nz - (nbz - b) + 1);
         }
         z[nbz] = nz + 1;
-        zband[ph] = 0;
-        for (int b = 0; b < nbz; ++b)
-            if (pml && z[b + 1] - 1 > g.ke) {
-                zband[ph] = b;
-                break;
-            }
     }
     return nbz;
 }
@@ -236,7 +229,13 @@ static int build_zchunks(swpc_ctx *c)
 {
     const Grid &g = c->g;
     std::vector<int> zc;
-    const int nbz = zchunk_table(c, c->kchunk, zc, c->zband);
+    const int nbz = zchunk_table(c, c->kchunk, zc);
+    // the band without the interior (the absorbing routines by themselves, the
+    // fused steps): a few planes a chunk, half the depth of a whole phase's up
+    // to three.  us per stress routine at 1, 3 and 7 planes: 96^3 (NM = 2) 18.7,
+    // 21.0, 23.3; 256 x 256 x 192 99, 99, 103; 512 x 512 x 256 342, 324, 325.
+    const int nband = g.nz - g.ke, kb = std::max(1, std::min(c->kchunk / 2, 3)), nbb = (nband + kb - 1) / kb;
+    for (int b = 0; b <= nbb; ++b) zc.push_back(g.ke + 1 + nband * b / std::max(nbb, 1));
     // fused launch: chunks of kfused planes over the interior planes kb..ke
     // (each chunk recomputes the velocities of two planes on either side)
     const int nki = g.ke - g.kb + 1;
@@ -244,10 +243,11 @@ static int build_zchunks(swpc_ctx *c)
     const int nfz = nki > 0 ? (nki + c->kfused - 1) / c->kfused : 0;
     std::vector<int> fz(nfz + 1);
     for (int b = 0; b <= nfz; ++b) fz[b] = g.kb + (int)((long long)nki * b / std::max(nfz, 1));
-    if (c->d_zchunks) c->bytes -= 2LL * (c->nbz + 1) * (long long)sizeof(int);
+    if (c->d_zchunks) c->bytes -= (2LL * (c->nbz + 1) + c->nbb + 1) * (long long)sizeof(int);
     dfree(c->d_zchunks);
     c->d_zchunks = nullptr;
     c->nbz = nbz;
+    c->nbb = nbb;
     if (dalloc(c, (void **)&c->d_zchunks, zc.size() * sizeof(int)) != hipSuccess)
         return fail(c, SWPC_ENOMEM, "k-chunk table allocation failed");
     HIPCHK(c, hipMemcpyAsync(c->d_zchunks, zc.data(), zc.size() * sizeof(int), hipMemcpyHostToDevice, c->stream));

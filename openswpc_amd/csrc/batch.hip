@@ -153,8 +153,7 @@ static int build_tables(swpc_batch *b)
     std::vector<int> zall;
     for (int m = 0; m < n; ++m) {
         if (!b->mem[m]->kchunk_auto) b->kchunk[m] = b->mem[m]->kchunk;
-        int zband[2];
-        zchunk_table(b->mem[m], b->kchunk[m], zc[m], zband);
+        zchunk_table(b->mem[m], b->kchunk[m], zc[m]);
         zoff[m] = zall.size();
         zall.insert(zall.end(), zc[m].begin(), zc[m].end());
     }

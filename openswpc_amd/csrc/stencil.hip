@@ -1178,9 +1178,9 @@ static bool phase_grid(const swpc_ctx *c, StepArgs &a, int phase, bool side, int
 {
     step_args(c, a, mask);
     if (phase == 1) a.zc = c->d_zchunks + c->nbz + 1;
-    if (mask == MASK_PML) {   // the bottom band alone: only the chunks that reach below the interior box
-        a.zc += c->zband[phase];
-        a.nbz -= c->zband[phase];
+    if (mask == MASK_PML) {   // the bottom band without the interior
+        a.zc = c->d_zchunks + 2 * (c->nbz + 1);
+        a.nbz = c->nbb;
     }
     const bool cols = c->g.nxk > 0 && c->g.nyk > 0 && ((mask & MASK_INT) || ((mask & MASK_PML) && a.has_pml));
     a.sideb = side && a.has_pml ? (c->npml_tiles + 7) & ~7 : 0;

@@ -208,8 +208,8 @@ struct swpc_ctx {
     bool kchunk_auto;  // the default chunk, not one the caller set
     int kfused;        // planes per chunk of the fused launch
     int nbz;           // k chunks of the interior-column kernels
-    int *d_zchunks;    // first plane of each chunk, stress phase then velocity phase (2 x (nbz+1))
-    int zband[2];      // per phase, the first chunk that holds planes of the bottom PML band
+    int nbb;           // chunks of the bottom PML band in launches of the band without the interior
+    int *d_zchunks;    // first plane of each chunk: stress phase, velocity phase (nbz+1 each), band (nbb+1)
     int *d_fzc;        // chunks of the fused launch over the interior planes (nfz + 1 entries)
     int nfz;
     float *fields2[SWPC_NFIELD];  // second field set of the fused steps (variant bit 7)
@@ -230,7 +230,7 @@ void ctx_reset_graph(swpc_ctx *c);
 int compute_units(const swpc_ctx *c);
 long long phase_tiles(const swpc_ctx *c);
 std::vector<int> side_tiles(const Grid &g, int by, int kc);
-int zchunk_table(const swpc_ctx *c, int kchunk, std::vector<int> &zc, int zband[2]);
+int zchunk_table(const swpc_ctx *c, int kchunk, std::vector<int> &zc);
 int ctx_find_tau(swpc_ctx *c);
 
 // ---- striped device arena (arena.hip) ----

@@ -1,8 +1,8 @@
 """Chunk boundaries of the interior columns, which weigh a plane of the bottom
 absorber against an interior one by what each moves: absorbers thinner and
 thicker than the planes above them, every depth that divides them and not, in
-step blocks, in the fused launch and timed (where the bottom band and the side
-columns are launches of their own).  Bit for bit against the FP32 oracle."""
+step blocks, in the fused launch, by the separate routines and timed (where the
+bottom band and the side columns are launches of their own).  Bit for bit against the FP32 oracle."""
 import numpy as np
 import pytest
 
@@ -25,7 +25,14 @@ def test_boundaries(orc, nm, nz, na):
         for variant in (1, 129):
             g = gpu_from_model(m, kchunk=kchunk, variant=variant)
             g.step(1, 5, use_graph=True, block=5)
-            g.step_timed(6, nt - 5)
+            g.wav_store(6)                   # step 6 by the separate routines: the band and the side columns alone
+            g.kernel_update_stress()
+            g.absorb_update_stress()
+            g.source_stressglut(6)
+            g.kernel_update_vel()
+            g.absorb_update_vel()
+            g.source_bodyforce(6)
+            g.step_timed(7, nt - 6)
             for n, (ulp, rel) in compare_fields(g, run).items():
                 assert ulp == 0, (kchunk, variant, n, ulp, rel)
             assert np.array_equal(g.seismograms("vel"), run.wav["vel"])
