@@ -632,8 +632,8 @@ def main():
     setup_again = None
     if not args.host_medium:
         # the same set-up once more in this process: the first one includes
-        # the FFT library's compilation of its kernels (once per machine and
-        # user, then read from its cache)
+        # the arena's reservation and the device's first allocations, which
+        # take longer where its memory was in use before
         sim.close()
         t1 = time.perf_counter()
         sim, inp = make_simulation_device(spec)
